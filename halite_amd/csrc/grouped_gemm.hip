@@ -26,6 +26,7 @@ struct GroupedArgs {
   void* Y;
   int ldy, y_group_cols, y_col0, y_dtype, y_add;
   int M, N, K, G;
+  int x_rows;
   const int* group_offsets;  // [G + 1] or null
   const int* tile_offsets;   // [G + 1] with group_offsets
   const int* row_src;        // or null
@@ -283,6 +284,242 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
     }
 }
 
+// The experts' products of prompts (rows sorted by group): tiles of up to 256 rows x 256 W rows (GATED:
+// 128 of the gate's weight and the same 128 of the up projection's) by eight waves, a wave half the
+// tile's rows x 64 W rows, one workgroup a compute unit.
+//
+// What bounds it: what a compute unit gets from the second-level cache, 16 to 20 bytes a clock whatever
+// the kernel around it looked like (some seventy 128-byte requests in flight, 570 clocks each), and a
+// tile of 128 x 128 asks for twice as much a product.  So the tile is as large as the registers hold, K
+// goes 64 at a time (whole 128-byte lines: half lines are as many requests for half the bytes) through
+// two LDS buffers that the loads fill by themselves, and no load is waited for before a whole step's
+// products have run: a step's one barrier stands in the middle of its second half's products, and
+// behind it the buffer just read is filled anew and the next operands are read while the rest of
+// them runs.  W rows are the instruction's first operand, so lane l of a result holds row l % 16 and the
+// four neighbouring columns 4 * (l / 16) .. + 3: one vector store.
+//
+// A group's rows are cut into the fewest tiles of at most 256 and these are made equally high, in
+// steps of 32 rows, so that workgroups take equally long.  Workgroup b runs on compute die b % 8, and
+// each die has an L2 of its own, so die x takes the x-th eighth of the list of all tiles, which goes
+// through a group's row tiles (eight at a time) column by column: one die reads an expert's weights,
+// once (tiles of two experts side by side cost a third more reads from memory and 8% of the time).
+//
+// LDS holds 8 rows x 64 k as one KiB, eight lanes of a load a row: the piece of eight k that lies
+// at place p of row r is piece p ^ gw_turn(r % 16).  A 16-byte read of a wave goes through LDS in turns of
+// sixteen lanes, lanes 0-3, 12-15 and 20-27 in one and 4-11, 16-19 and 28-31 in the next (and so on from
+// lane 32); each turn then meets all 64 banks once.
+//
+// Measured beside tiles of 128 x 128 in registers and LDS (grouped_mfma_kernel): 9,000 rows of 16 experts,
+// 4096 x 4096: 469 -> 300 us (644 -> 1,007 TFLOP/s); 18,000 rows of 64 experts, gate and up 1024 x 4096
+// each: 537 -> 400 us, down 4096 x 1024 into float32 rows 352 -> 280 us; 49,152 rows of 64: 1,127 -> 745 us;
+// 2,400 rows of 64 (the weights' 1.07 GB once): 252 -> 200 us.
+#define GW_ROWS 256
+#define GW_COLS 256
+#define GW_TK 64
+#define GW_PANEL 8
+#define GW_A_BYTES (GW_ROWS * GW_TK * 2)
+#define GW_BUFFER ((GW_ROWS + GW_COLS) * GW_TK * 2)
+
+// column n and the three behind it of the row that goes to row dst
+template <bool GATED>
+__device__ __forceinline__ void gw_store(const GroupedArgs& a, int dst, int n, gg_f32x4 v, gg_f32x4 v2) {
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    if (GATED) {
+      const float gg = fminf(v[j], a.limit);
+      const float uu = fminf(fmaxf(v2[j], -a.limit), a.limit);
+      v[j] = gg * gg_sigmoid(a.alpha * gg) * (uu + a.up_shift);
+    } else if (a.act == 1) {
+      const float p = fmaxf(v[j], 0.f);
+      v[j] = p * p;
+    }
+  }
+  const size_t at = (size_t)dst * a.ldy + a.y_col0 + n;
+  if (a.y_dtype == HAL_F32) *(gg_f32x4*)((float*)a.Y + at) = v;
+  else *(uint2*)((bf16_t*)a.Y + at) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
+}
+
+// 16 bytes a lane from memory straight into LDS: from byte `each` (a lane's own) + `all` of `from`, lane l's to
+// `to` (the same in all lanes) + 16 l.  (Buffer loads: the compiler waits for every load where it meets
+// one in the flat form that goes into LDS.)
+typedef __amdgpu_buffer_rsrc_t gw_rows;
+__device__ __forceinline__ gw_rows gw_rows_at(const void* p, uint32_t bytes) {
+  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
+}
+__device__ __forceinline__ void gw_load_lds(gw_rows from, uint32_t each, uint32_t all, char* to) {
+  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, each, all, 0, 0);
+}
+__device__ __forceinline__ int gw_turn(int r) { return ((r >> 1) & 1) | ((r >> 2) & 2) | (((r >> 1) ^ r) & 4); }
+// Until all but the last `left` loads of this wave are there, and then until every wave is here.
+template <int LEFT>
+__device__ __forceinline__ void gw_meet() {
+  __builtin_amdgcn_sched_barrier(0);
+  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
+  __builtin_amdgcn_sched_barrier(0);
+}
+
+// What one wave does for a tile of at most 32 * NI rows.  The two buffers are two arrays, so that the
+// compiler can tell a load into one from a read of the other.
+template <bool GATED, int NI>
+__device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1) {
+  constexpr int AI = (NI + 1) / 2, LOADS = AI + 4;  // a wave's loads a step: 8 rows of every 64 of X, and of W
+  const int steps = a.K / GW_TK;                    // even
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), wm = wave / 4, wn = wave % 4;
+  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ gw_turn(lr % 16)) * 16;
+  // (GATED: of every 64 W rows, a wave's, the first 32 are the gate's and the others the up projection's)
+  const void* w0 = GATED && wave >= 4 ? a.W2 : a.W;
+  const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
+  const gw_rows X = gw_rows_at((const bf16_t*)a.X + a.x_col0, (uint32_t)a.x_rows * a.ldx * 2 - a.x_col0 * 2);
+  uint32_t xo[AI], wo[4];
+  // rows and columns past the end are read from the last one: nothing of them is stored
+#pragma unroll
+  for (int i = 0; i < AI; ++i) {
+    int r = row0 + lr + 64 * i;
+    r = r < row_end ? r : row_end - 1;
+    xo[i] = (uint32_t)(a.row_src ? a.row_src[r] / a.src_div : r) * (uint32_t)(a.ldx * 2) + c;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int n = GATED ? n0 + i * 32 + lr % 32 : n0 + i * 64 + lr;
+    n = n < a.N ? n : a.N - 1;
+    wo[i] = (uint32_t)n * (uint32_t)(a.ldw * 2) + c;
+  }
+  // (no branch: past the end the last step's pieces come again and are not multiplied)
+  auto bring = [&](char* lds, int step) {
+    const uint32_t at = (uint32_t)(step < steps ? step : steps - 1) * (GW_TK * 2);
+#pragma unroll
+    for (int i = 0; i < AI; ++i) gw_load_lds(X, xo[i], at, lds + (i * 8 + wave) * 1024);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) gw_load_lds(W, wo[i], at, lds + GW_A_BYTES + (i * 8 + wave) * 1024);
+  };
+  const int q = lane / 16, r16 = lane % 16;
+  const int get[2] = {r16 * 128 + (q ^ gw_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ gw_turn(r16)) * 16};
+  struct Operands {
+    gg_bf16x8 w[4], x[NI];
+  };
+  auto read = [&](const char* lds, int half, Operands& o) {  // the operands of 32 of a step's 64 k
+#pragma unroll
+    for (int j = 0; j < 4; ++j) o.w[j] = *(const gg_bf16x8*)(lds + GW_A_BYTES + (wn * 4 + j) * 2048 + get[half]);
+#pragma unroll
+    for (int i = 0; i < NI; ++i) o.x[i] = *(const gg_bf16x8*)(lds + (wm * NI + i) * 2048 + get[half]);
+  };
+  gg_f32x4 acc[NI][4];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 4; ++j) acc[i][j] = gg_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const Operands& o, int from, int to) {
+#pragma unroll
+    for (int i = from; i < to; ++i)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[j], o.x[i], acc[i][j], 0, 0, 0);
+  };
+  constexpr int HALF = NI / 2, REST = NI - HALF;
+  Operands low, high;
+  // One step: the operands of its first half are in `low`, the rest is in `mine`, the next step in `next`.
+  auto advance = [&](int s, char* mine, char* next) {
+    read(mine, 1, high);
+    multiply(low, 0, NI);
+#pragma unroll
+    for (int k = 0; k < NI; ++k) {  // (the order that the compiler is to emit)
+      __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + NI - 1) / NI, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    }
+    multiply(high, 0, HALF);
+    gw_meet<0>();
+    bring(mine, s + 2);
+    read(next, 0, low);
+    multiply(high, HALF, NI);
+    __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
+#pragma unroll
+    for (int k = 0; k < REST; ++k) {
+      __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + REST - 1) / REST, 0);
+      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+    }
+  };
+  bring(b0, 0);
+  bring(b1, 1);
+  gw_meet<LOADS>();
+  read(b0, 0, low);
+  for (int s = 0; s < steps; s += 2) {
+    advance(s, b0, b1);
+    advance(s + 1, b1, b0);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // LDS is not given back while loads are on their way into it
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = row0 + (wm * NI + i) * 16 + r16;
+    if (r >= row_end) continue;
+    const int dst = a.row_dst ? a.row_dst[r] : r;
+#pragma unroll
+    for (int j = 0; j < (GATED ? 2 : 4); ++j) {
+      const int n = n0 + wn * (GATED ? 32 : 64) + j * 16 + q * 4;
+      if (n < a.N) gw_store<GATED>(a, dst, n, acc[i][j], GATED ? acc[i][j + 2] : acc[i][j]);
+    }
+  }
+}
+
+template <bool GATED>
+__global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int col_tiles) {
+  __shared__ __attribute__((aligned(16))) char b0[GW_BUFFER], b1[GW_BUFFER];
+  __shared__ __attribute__((aligned(64))) int found[4];  // group, first row, end row, column tile
+  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
+  if (wave == 0) {
+    auto tiles_of = [&](int g) { return g < a.G ? (a.group_offsets[g + 1] - a.group_offsets[g] + GW_ROWS - 1) / GW_ROWS : 0; };
+    int tiles = 0;
+    for (int c = 0; c < a.G; c += 64) {
+      int n = tiles_of(c + lane);
+#pragma unroll
+      for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+      tiles += n;
+    }
+    const long long units = (long long)tiles * col_tiles;
+    const int die = blockIdx.x % 8;
+    const long long unit = units * die / 8 + blockIdx.x / 8;
+    if (lane == 0) found[0] = -1;
+    if (unit < units * (die + 1) / 8) {
+      int before = 0;  // row tiles of the groups before
+      for (int c = 0; c < a.G; c += 64) {
+        const int n = tiles_of(c + lane);
+        int upto = n;
+#pragma unroll
+        for (int off = 1; off < 64; off <<= 1) {
+          const int v = __shfl_up(upto, off, 64);
+          if (lane >= off) upto += v;
+        }
+        upto += before;
+        if (unit >= (long long)(upto - n) * col_tiles && unit < (long long)upto * col_tiles) {
+          const int in_group = (int)(unit - (long long)(upto - n) * col_tiles);
+          const int panel = in_group / (GW_PANEL * col_tiles), in_panel = in_group % (GW_PANEL * col_tiles);
+          const int high = min(GW_PANEL, n - panel * GW_PANEL);  // row tiles of this panel
+          const int g = c + lane, begin = a.group_offsets[g], end = a.group_offsets[g + 1];
+          const int rows = ((end - begin + n - 1) / n + 31) / 32 * 32;  // of each of the group's tiles
+          found[0] = g;
+          found[1] = begin + (panel * GW_PANEL + in_panel % high) * rows;
+          found[2] = min(end, found[1] + rows);
+          found[3] = in_panel / high;
+        }
+        before = __shfl(upto, 63, 64);
+      }
+    }
+  }
+  __syncthreads();
+  const int g = __builtin_amdgcn_readfirstlane(found[0]);
+  if (g < 0) return;
+  const int row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
+  const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GW_COLS / 2 : GW_COLS);
+  const int rows = row_end - row0;
+  if (rows <= 0) return;  // (equal heights in steps of 32 can leave a group's last tile empty)
+#define GW_WAVE(NI_) gw_wave<GATED, NI_>(a, g, row0, row_end, n0, b0, b1)
+  if (rows <= 64) GW_WAVE(2);
+  else if (rows <= 128) GW_WAVE(4);
+  else if (rows <= 160) GW_WAVE(5);
+  else if (rows <= 192) GW_WAVE(6);
+  else if (rows <= 224) GW_WAVE(7);
+  else GW_WAVE(8);
+#undef GW_WAVE
+}
+
 // bf16, few rows a group (decode steps): a workgroup takes 64 rows of W (GATED: 32 of the
 // gate's weight and the same 32 of the up projection's) and the tile's rows 16 at a time.  Its
 // four waves split K between them and read both operands straight from memory in the
@@ -358,7 +595,7 @@ __global__ void __launch_bounds__(256) grouped_skinny_kernel(GroupedArgs a) {
 extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_col0, const void* W,
                                 const void* W2, long long w_group_stride, int ldw, int dtype,
                                 void* Y, int ldy, int y_group_cols, int y_col0, int y_dtype,
-                                int y_add, int M, int N, int K, int G, const int* group_offsets,
+                                int y_add, int M, int N, int K, int G, int x_rows, const int* group_offsets,
                                 const int* tile_offsets, const int* row_src, int src_div,
                                 const int* row_dst, const float* gate, int ldg, int gate_per_group,
                                 float limit, float up_shift,
@@ -380,6 +617,7 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   a.Y = Y; a.ldy = ldy; a.y_group_cols = y_group_cols; a.y_col0 = y_col0; a.y_dtype = y_dtype;
   a.y_add = y_add;
   a.M = M; a.N = N; a.K = K; a.G = G;
+  a.x_rows = x_rows;
   a.group_offsets = group_offsets; a.tile_offsets = tile_offsets;
   a.row_src = row_src; a.src_div = src_div; a.row_dst = row_dst;
   a.gate = gate; a.ldg = ldg; a.limit = limit; a.alpha = alpha; a.act = act; a.up_shift = up_shift;
@@ -393,12 +631,23 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   const bool aligned = K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && x_group_cols % 8 == 0 &&
                        x_col0 % 8 == 0 && w_group_stride % 8 == 0 && ((uintptr_t)X % 16 == 0) &&
                        ((uintptr_t)W % 16 == 0) && (W2 == nullptr || (uintptr_t)W2 % 16 == 0);
-  // few rows a group: the kernel that keeps many loads in flight instead of staging tiles
+  // few rows a group: the kernel that keeps many loads in flight instead of staging tiles; experts with
+  // more: the wide tiles wherever sizes and addresses are such that their loads and vector stores need
+  // no bounds (faster at every size measured, from 47 rows a group on); heads, narrow weights and the
+  // rest: tiles of 128
   const long long rows_per_group = group_offsets ? M / G : M;
   if (dtype == HAL_BF16 && allow_mfma && aligned && rows_per_group <= 16) {
     grid.x = W2 ? (N + 31) / 32 : (N + 63) / 64;
     if (W2) hipLaunchKernelGGL(grouped_skinny_kernel<true>, grid, dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(grouped_skinny_kernel<false>, grid, dim3(256), 0, stream, a);
+  } else if (dtype == HAL_BF16 && allow_mfma && aligned && group_offsets && K % (2 * GW_TK) == 0 && N >= GW_COLS &&
+             gate == nullptr && !y_add && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 && (uintptr_t)Y % 16 == 0 &&
+             x_group_cols == 0 && y_group_cols == 0 && (long long)N * ldw * 2 < (1ll << 31) && (long long)x_rows * ldx * 2 < (1ll << 31)) {
+    const int cols = W2 ? GW_COLS / 2 : GW_COLS, col_tiles = (N + cols - 1) / cols;
+    const long long units = ((long long)(M + GW_ROWS - 1) / GW_ROWS + G) * col_tiles, blocks = 8 * ((units + 7) / 8);
+    HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
+    if (W2) hipLaunchKernelGGL(grouped_wide_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, a, col_tiles);
+    else hipLaunchKernelGGL(grouped_wide_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, a, col_tiles);
   } else if (dtype == HAL_BF16 && allow_mfma && aligned) {
     grid.x = W2 ? (N + GG_ROWS / 2 - 1) / (GG_ROWS / 2) : (N + GG_ROWS - 1) / GG_ROWS;
     if (W2) hipLaunchKernelGGL(grouped_mfma_kernel<true>, grid, dim3(256), 0, stream, a);

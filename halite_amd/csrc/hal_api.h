@@ -142,7 +142,7 @@ int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const floa
 // ---- products in groups (grouped_gemm.hip) ---------------------------------------------
 // Y_g = X_g * W_g^T for G groups in one launch, float32 accumulation; operands of `dtype`.
 // Group g reads the columns from g * x_group_cols + x_col0 of X's rows (row length ldx) and
-// W + g * w_group_stride ([N, K], row length ldw), and writes the columns from
+// W + g * w_group_stride ([N, K], row length ldw; X has x_rows rows), and writes the columns from
 // g * y_group_cols + y_col0 of Y's rows (row length ldy, element type y_dtype; y_add: added
 // into a float32 Y).  group_offsets == null: every group has the rows 0 .. M-1.  Otherwise
 // group g has the rows group_offsets[g] .. group_offsets[g + 1] - 1 of a list of M rows in
@@ -156,7 +156,7 @@ int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const floa
 int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_col0, const void* W,
                      const void* W2, long long w_group_stride, int ldw, int dtype, void* Y, int ldy,
                      int y_group_cols, int y_col0, int y_dtype, int y_add, int M, int N, int K,
-                     int G, const int* group_offsets, const int* tile_offsets, const int* row_src,
+                     int G, int x_rows, const int* group_offsets, const int* tile_offsets, const int* row_src,
                      int src_div, const int* row_dst, const float* gate, int ldg, int gate_per_group,
                      float limit, float up_shift, float alpha, int act, int allow_mfma,
                      hipStream_t stream);

@@ -895,7 +895,7 @@ def grouped_gemm(
     _check(lib, lib.hal_grouped_gemm(
         _ptr(x), x.stride(0), x_group_cols, x_col0, _ptr(w), _ptr(w_up), ctypes.c_longlong(n * k), k,
         dtype_code(x.dtype), _ptr(y), y.stride(0), y_group_cols, y_col0, dtype_code(y.dtype), 1 if add else 0,
-        n_rows, n, k, g, _ptr(group_offsets), _ptr(tile_offsets), _ptr(row_src), src_div, _ptr(row_dst),
+        n_rows, n, k, g, x.shape[0], _ptr(group_offsets), _ptr(tile_offsets), _ptr(row_src), src_div, _ptr(row_dst),
         _ptr(gate), 0 if gate is None else gate.stride(0), 1 if gate_per_group else 0, ctypes.c_float(limit),
         ctypes.c_float(up_shift), ctypes.c_float(alpha),
         1 if relu_squared else 0, 1 if mfma else 0, _stream()))
