@@ -83,12 +83,14 @@ class LayerPages:
     transposed, ``[pages, K, D, page_size]``.  With ``tiled`` the bytes of one
     (page, kv head) are the same in number but lie in blocks of 32 tokens, keys as
     ``[block][16-key tile][32-dim step][dim quad][key][8 dims]`` and values as
-    ``[block][16-dim tile][8-key group][dim][8 keys]``."""
+    ``[block][16-dim tile][8-key group][dim][8 keys]``.  ``value_from``: the values' dimensions
+    before it are zeros in every token."""
 
     group_id: int
     k: torch.Tensor | None
     v: torch.Tensor | None
     tiled: bool = False
+    value_from: int = 0
 
 
 @dataclass

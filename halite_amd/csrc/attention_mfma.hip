@@ -118,12 +118,16 @@ __device__ __forceinline__ void load_to_lds(const bf16_t* src, void* lds) {
 // Two waves per SIMD leave 256 registers each, which keeps the accumulators in VGPRs (no
 // copies to and from AGPRs around every MFMA); the largest head sizes need more.
 #define MIN_WAVES_PER_SIMD (D > 160 ? 1 : 2)
+// The same for the kernel with LDS: its two halves are two waves per SIMD.
+#define MIN_WAVES_OF(SHARED_, HALVES_) (SHARED_ ? HALVES_ : MIN_WAVES_PER_SIMD)
 // RULED: the scores follow a rule beyond scale, causal mask and window (`hal_score_rule`): a
 // bias by distance (the table comes multiplied by log2 e), a sink in the denominator; a
 // chunked mask needs no build of its own.  KEPT: the first `rule.keep` keys stay visible under the
-// window, and the items say which of them a wave walks in front of its range.
-template <int RT, bool POW2, bool PAGE32, bool SHARED, bool TILED, int KB, int HALVES, bool RULED, bool KEPT>
-__global__ void __launch_bounds__(256 * HALVES, MIN_WAVES_PER_SIMD)
+// window, and the items say which of them a wave walks in front of its range.  VT0: the first VT0 x 16
+// dimensions of every value are zeros: they are neither loaded nor multiplied, and the result's are
+// zeros (a latent attention's values, whose rotated part is none).
+template <int RT, bool POW2, bool PAGE32, bool SHARED, bool TILED, int KB, int HALVES, bool RULED, bool KEPT, int VT0>
+__global__ void __launch_bounds__(256 * HALVES, MIN_WAVES_OF(SHARED, HALVES))
 attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __restrict__ out,
                       int out_row_stride, const int* __restrict__ items,
                       const int* __restrict__ n_items_ptr, const int* __restrict__ seg_q_start,
@@ -139,6 +143,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
   // empty); their sums are joined through LDS at the end and the first wave writes the
   // result, to the output or to the partial slot that its item names.
   constexpr bool JOIN = !SHARED;
+  constexpr int DV = DT - VT0;  // tiles of the head dimension that the values have something in
   static_assert(!JOIN || RT == 1, "pieces are joined in the kernel for one tile per wave");
   // wave: within its half (it names the item and the fragments the wave loads)
   const int lane = threadIdx.x % HAL_WAVE;
@@ -261,7 +266,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
   // (KEPT) the row sees the item's keys from see_from on, see_span more of them, and n_kept from kept_begin on
   int see_from[RT], see_span[RT], n_kept[RT];
   bf16x8 bq[RT][KT];  // Q^T as the B operand: lane holds Q[row][ks*32 + quad*8 .. +8]
-  f32x4 o[RT][DT];
+  f32x4 o[RT][DV];
   float m[RT], l[RT];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt) {
@@ -285,7 +290,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       bq[rt][ks] = (row_ok[rt] && (D % 32 == 0 || d0 < D)) ? ld16(qp + d0) : zero8();
     }
 #pragma unroll
-    for (int dt = 0; dt < DT; ++dt) o[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (int dt = 0; dt < DV; ++dt) o[rt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
     m[rt] = -INFINITY;
     l[rt] = 0.f;
   }
@@ -505,7 +510,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
     for (int rt = 0; rt < RT; ++rt) {
       if (__builtin_amdgcn_ballot_w64(alpha[rt] != 1.f) != 0) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) o[rt][dt][r] *= alpha[rt];
       }
@@ -521,8 +526,8 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
   };
 
   constexpr int FK = 2 * KT;                       // key fragments of a block of 32 keys
-  constexpr int NFK = SUBS * FK, NFV = SUBS * DT;  // key and value fragments of a step
-  constexpr int XCH_VALUES = RT * DT * 4 + 2 * RT;
+  constexpr int NFK = SUBS * FK, NFV = SUBS * DV;  // key and value fragments of a step
+  constexpr int XCH_VALUES = RT * DV * 4 + 2 * RT;
   constexpr int XCH_BYTES = HALVES == 2 ? WAVES * XCH_VALUES * HAL_WAVE * 4 : 0;
   // With LDS: [half of the workgroup][keys: two buffers of NFK fragments, values: two of
   // NFV][lane]: a fragment lies there in lane order, as the MFMA wants it back.  At the end,
@@ -574,7 +579,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       for (int i = 0; i < (NFV + WAVES - 1) / WAVES; ++i) {
         const int f = wave + WAVES * i;
         if (f < NFV)
-          load_to_lds(value_frag_ptr(j0 + 32 * (f / DT), pages[f / DT], f % DT), vbuf + b * NFV + f);
+          load_to_lds(value_frag_ptr(j0 + 32 * (f / DV), pages[f / DV], VT0 + f % DV), vbuf + b * NFV + f);
       }
     };
     // the values of keys past the request's end are cleared where they landed, by the wave
@@ -583,10 +588,10 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
 #pragma unroll
       for (int i = 0; i < (NFV + WAVES - 1) / WAVES; ++i) {
         const int f = wave + WAVES * i;
-        if (f < NFV && j0 + 32 * (f / DT) + 32 > kv_len) {
+        if (f < NFV && j0 + 32 * (f / DV) + 32 > kv_len) {
           u32x4* at = &vbuf[b * NFV + f][lane];
           *at = __builtin_bit_cast(
-              u32x4, clear_unwritten(j0 + 32 * (f / DT), __builtin_bit_cast(bf16x8, *at)));
+              u32x4, clear_unwritten(j0 + 32 * (f / DV), __builtin_bit_cast(bf16x8, *at)));
         }
       }
     };
@@ -603,7 +608,12 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       __syncthreads();
       __builtin_amdgcn_sched_barrier(0);
     };
-    constexpr int FR = FK > DT ? FK : DT;
+    // Heads of more than 128 dimensions leave no registers for all fragments of a block: they take
+    // them CHUNK at a time, a chunk of values or keys being read while the one before is multiplied.
+    constexpr bool CHUNKED = D > 128;
+    static_assert(!CHUNKED || SUBS == 1, "large heads take 32 keys a step");
+    constexpr int CHUNK = 4, VALUE_CHUNKS = (DV + CHUNK - 1) / CHUNK, KEY_CHUNKS = (FK + CHUNK - 1) / CHUNK;
+    constexpr int FR = CHUNKED ? CHUNK : (FK > DV ? FK : DV);
     bf16x8 fa[FR], fb[FR];  // two sets of fragment registers, filled in turn
     auto read_keys = [&](bf16x8 (&f)[FR], int b, int u) {
 #pragma unroll
@@ -611,7 +621,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
     };
     auto read_values = [&](bf16x8 (&f)[FR], int b, int u) {
 #pragma unroll
-      for (int x = 0; x < DT; ++x) f[x] = __builtin_bit_cast(bf16x8, vbuf[b * NFV + u * DT + x][lane]);
+      for (int x = 0; x < DV; ++x) f[x] = __builtin_bit_cast(bf16x8, vbuf[b * NFV + u * DV + x][lane]);
     };
     f32x4 s[RT][SUBS][2];
     // consecutive products go to different sums, so none waits for the one before it
@@ -628,10 +638,61 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
     bf16x8 pb[RT][SUBS];
     auto probabilities_times_values = [&](const bf16x8 (&f)[FR], int u) {
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
         for (int rt = 0; rt < RT; ++rt)
           o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[dt], pb[rt][u], o[rt][dt], 0, 0, 0);
+    };
+
+    // (CHUNKED) chunk c of a run of products: the values in buffer vb, then the keys in buffer kb, these
+    // in the order (32-wide step, tile)
+    auto read_chunk = [&](bf16x8 (&f)[FR], int c, int vb, int kb) {
+#pragma unroll
+      for (int x = 0; x < CHUNK; ++x) {
+        if (c < VALUE_CHUNKS) {
+          if (c * CHUNK + x < DV) f[x] = __builtin_bit_cast(bf16x8, vbuf[vb * NFV + c * CHUNK + x][lane]);
+        } else {
+          const int k = (c - VALUE_CHUNKS) * CHUNK + x;
+          if (k < FK) f[x] = __builtin_bit_cast(bf16x8, kbuf[kb * NFK + (k % 2) * KT + k / 2][lane]);
+        }
+      }
+    };
+    auto multiply_chunk = [&](const bf16x8 (&f)[FR], int c) {
+#pragma unroll
+      for (int x = 0; x < CHUNK; ++x)
+#pragma unroll
+        for (int rt = 0; rt < RT; ++rt) {
+          if (c < VALUE_CHUNKS) {
+            const int dt = c * CHUNK + x;
+            if (dt < DV) o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(f[x], pb[rt][0], o[rt][dt], 0, 0, 0);
+          } else {
+            const int k = (c - VALUE_CHUNKS) * CHUNK + x;
+            if (k < FK)
+              s[rt][0][k % 2] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(
+                  f[x], bq[rt][k / 2], k < 2 ? f32x4{0.f, 0.f, 0.f, 0.f} : s[rt][0][k % 2], 0, 0, 0);
+          }
+        }
+    };
+    // the chunks from `first` to the last, the first one's fragments in fa already
+    auto run_chunks = [&](auto first, int vb, int kb) {
+      constexpr int LAST = VALUE_CHUNKS + KEY_CHUNKS;
+#pragma unroll
+      for (int c = first; c < LAST; c += 2) {
+        if (c + 1 < LAST) read_chunk(fb, c + 1, vb, kb);
+        __builtin_amdgcn_sched_barrier(0);
+        multiply_chunk(fa, c);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + 2 < LAST) read_chunk(fa, c + 2, vb, kb);
+        __builtin_amdgcn_sched_barrier(0);
+        if (c + 1 < LAST) multiply_chunk(fb, c + 1);
+        __builtin_amdgcn_sched_barrier(0);
+      }
+    };
+    struct FirstValue {
+      constexpr operator int() const { return 0; }
+    };
+    struct FirstKey {
+      constexpr operator int() const { return VALUE_CHUNKS; }
     };
 
     {  // (pages_1, pages_2: of the next step and of the one after it)
@@ -644,10 +705,15 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
     if constexpr (HALVES == 2) {
       if (half_id == 1) turn_barrier();
     }
-    read_keys(fa, 0, 0);
-    if constexpr (SUBS == 2) read_keys(fb, 0, 1);
-    keys_times_queries(fa, 0);
-    if constexpr (SUBS == 2) keys_times_queries(fb, 1);
+    if constexpr (CHUNKED) {
+      read_chunk(fa, VALUE_CHUNKS, 0, 0);
+      run_chunks(FirstKey(), 0, 0);
+    } else {
+      read_keys(fa, 0, 0);
+      if constexpr (SUBS == 2) read_keys(fb, 0, 1);
+      keys_times_queries(fa, 0);
+      if constexpr (SUBS == 2) keys_times_queries(fb, 1);
+    }
 
     for (int i = 0; i < n_steps; ++i) {
       const int j0 = j_of(i), b = i & 1;
@@ -672,13 +738,16 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       // the scores of a step that does not exist are computed from what the buffer holds
       // and never looked at: the run of products has no branch)
       __builtin_amdgcn_s_setprio(2);  // the products go first where both halves could issue
-      read_values(fa, b, 0);
+      if constexpr (CHUNKED) read_chunk(fa, 0, b, b ^ 1);
+      else read_values(fa, b, 0);
       if constexpr (SUBS == 2) read_values(fb, b, 1);
       __builtin_amdgcn_sched_barrier(0);
       if (i + 2 < n_steps) ask_keys(j_of(i + 2), pages_2, b);
       if (i + 1 < n_steps) ask_values(j_of(i + 1), pages_1, b ^ 1);
       __builtin_amdgcn_sched_barrier(0);
-      if constexpr (SUBS == 2) {
+      if constexpr (CHUNKED) {
+        run_chunks(FirstValue(), b, b ^ 1);
+      } else if constexpr (SUBS == 2) {
         probabilities_times_values(fa, 0);
         __builtin_amdgcn_sched_barrier(0);
         read_keys(fa, b ^ 1, 0);
@@ -712,7 +781,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
     // Without LDS: this block's values and the next block's keys (a second buffer) are asked
     // for at the block's start; deeper or shallower schedules measured the same or worse.
     int page_0 = page_at(key_at(0)), page_1 = page_at(key_at(32)), page_2 = page_at(key_at(64));
-    bf16x8 kcur[2][KT], knext[2][KT], vf[DT];
+    bf16x8 kcur[2][KT], knext[2][KT], vf[DV];
 #pragma unroll
     for (int t = 0; t < 2; ++t)
 #pragma unroll
@@ -724,7 +793,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       const bool more = x + KB < walk_keys;
       const int page_3 = page_at(key_at(x + 96));
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) vf[dt] = load_value_frag(j0, page_0, dt);
+      for (int dt = 0; dt < DV; ++dt) vf[dt] = load_value_frag(j0, page_0, VT0 + dt);
       if (more) {
 #pragma unroll
         for (int t = 0; t < 2; ++t)
@@ -756,13 +825,13 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       // ---- O^T += V^T P^T ----------------------------------------------------------
       if (tail) {
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt) vf[dt] = clear_unwritten(j0, vf[dt]);
+        for (int dt = 0; dt < DV; ++dt) vf[dt] = clear_unwritten(j0, vf[dt]);
       }
 #pragma unroll
       for (int rt = 0; rt < RT; ++rt) {
         if (!active[rt]) continue;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DV; ++dt)
           o[rt][dt] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(vf[dt], pb[rt][0], o[rt][dt], 0, 0, 0);
       }
 #pragma unroll
@@ -787,9 +856,9 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
         xch[(2 * rt) * HAL_WAVE] = m[rt];
         xch[(2 * rt + 1) * HAL_WAVE] = l[rt];
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
-          for (int r = 0; r < 4; ++r) xch[(2 * RT + (rt * DT + dt) * 4 + r) * HAL_WAVE] = o[rt][dt][r];
+          for (int r = 0; r < 4; ++r) xch[(2 * RT + (rt * DV + dt) * 4 + r) * HAL_WAVE] = o[rt][dt][r];
       }
     }
     __syncthreads();
@@ -803,10 +872,10 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       l[rt] = l[rt] * a0 + l1 * a1;
       m[rt] = m_new;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt)
+      for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
         for (int r = 0; r < 4; ++r)
-          o[rt][dt][r] = o[rt][dt][r] * a0 + xch[(2 * RT + (rt * DT + dt) * 4 + r) * HAL_WAVE] * a1;
+          o[rt][dt][r] = o[rt][dt][r] * a0 + xch[(2 * RT + (rt * DV + dt) * 4 + r) * HAL_WAVE] * a1;
     }
   }
 
@@ -814,7 +883,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
   if constexpr (JOIN) {
     // lane to lane: the four waves have the same rows in the same lanes.  Joined by the
     // log-sum-exp rule, in wave order; the result is the first wave's.
-    constexpr int JV = DT * 4 + 2;
+    constexpr int JV = DV * 4 + 2;
     __shared__ float joined[WAVES - 1][JV][HAL_WAVE];
     __shared__ int arrived_before;
     float lt = l[0];
@@ -825,7 +894,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
         joined[wave - 1][0][lane] = m[0];
         joined[wave - 1][1][lane] = lt;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
           for (int r = 0; r < 4; ++r) joined[wave - 1][2 + dt * 4 + r][lane] = o[0][dt][r];
       }
@@ -840,7 +909,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
         lt = lt * a0 + l1 * a1;
         m[0] = m_new;
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
           for (int r = 0; r < 4; ++r)
             o[0][dt][r] = o[0][dt][r] * a0 + joined[w][2 + dt * 4 + r][lane] * a1;
@@ -872,9 +941,9 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
         const size_t slot = (size_t)partial * K + g;
         const auto to = slot_sums(slot);
 #pragma unroll
-        for (int dt = 0; dt < DT; ++dt)
+        for (int dt = 0; dt < DV; ++dt)
           __builtin_amdgcn_raw_buffer_store_b128(__builtin_bit_cast(u32x4, o[0][dt]), to,
-                                                 (dt * HAL_WAVE + lane) * 16, 0, SC1);
+                                                 ((VT0 + dt) * HAL_WAVE + lane) * 16, 0, SC1);
         if (quad == 0) {
           float* pm = part_ml + (slot * 16 + col) * 2;
           put(pm, m[0]);
@@ -891,11 +960,11 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       m[0] = -INFINITY;
       lt = 0.f;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) o[0][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+      for (int dt = 0; dt < DV; ++dt) o[0][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
       // a wave takes every fourth piece, the loads of several in flight at a time
-      constexpr int U = DT <= 8 ? 4 : 2;
+      constexpr int U = DV <= 8 ? 4 : 2;
       for (int i0 = wave; i0 < n_pieces; i0 += WAVES * U) {
-        f32x4 po[U][DT];
+        f32x4 po[U][DV];
         float pm[U], pl[U];
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -905,9 +974,9 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
           pl[u] = get(part_ml + (slot * 16 + col) * 2 + 1);
           const auto from = slot_sums(slot);
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
+          for (int dt = 0; dt < DV; ++dt)
             po[u][dt] = __builtin_bit_cast(
-                f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, (dt * HAL_WAVE + lane) * 16, 0, SC1));
+                f32x4, __builtin_amdgcn_raw_buffer_load_b128(from, ((VT0 + dt) * HAL_WAVE + lane) * 16, 0, SC1));
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -918,7 +987,7 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
           lt = lt * a0 + pl[u] * a1;
           m[0] = m_new;
 #pragma unroll
-          for (int dt = 0; dt < DT; ++dt)
+          for (int dt = 0; dt < DV; ++dt)
 #pragma unroll
             for (int r = 0; r < 4; ++r) o[0][dt][r] = o[0][dt][r] * a0 + po[u][dt][r] * a1;
         }
@@ -950,17 +1019,21 @@ attention_mfma_kernel(const bf16_t* __restrict__ q, int q_row_stride, bf16_t* __
       }
       bf16_t* op = out + (size_t)(q_start + qi[rt]) * out_row_stride + (size_t)head[rt] * D;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) {
+      for (int dt = 0; dt < DV; ++dt) {
         uint2 w;
         w.x = pack2(o[rt][dt][0] * inv, o[rt][dt][1] * inv);
         w.y = pack2(o[rt][dt][2] * inv, o[rt][dt][3] * inv);
-        *(uint2*)(op + dt * 16 + quad * 4) = w;
+        *(uint2*)(op + (VT0 + dt) * 16 + quad * 4) = w;
       }
+#pragma unroll
+      for (int dt = 0; dt < VT0; ++dt) *(uint2*)(op + dt * 16 + quad * 4) = make_uint2(0u, 0u);
     } else {
       const size_t slot = (size_t)(partial + rt) * K + g;
       float* po = part_o + (slot * 16 + col) * D;
 #pragma unroll
-      for (int dt = 0; dt < DT; ++dt) *(f32x4*)(po + dt * 16 + quad * 4) = o[rt][dt];
+      for (int dt = 0; dt < DV; ++dt) *(f32x4*)(po + (VT0 + dt) * 16 + quad * 4) = o[rt][dt];
+#pragma unroll
+      for (int dt = 0; dt < VT0; ++dt) *(f32x4*)(po + dt * 16 + quad * 4) = f32x4{0.f, 0.f, 0.f, 0.f};
       if (quad == 0) {
         float* pm = part_ml + (slot * 16 + col) * 2;
         pm[0] = m[rt];
@@ -1124,12 +1197,16 @@ attention_merge_few_kernel(bf16_t* __restrict__ out, int out_row_stride,
 
 extern "C" int hal_attention_mfma_head_dim() { return D; }
 
-// How many 16-row tiles a wave takes in the kernel for long segments.
+// How many 16-row tiles a wave takes in the kernel for long segments.  (Heads of more than 128
+// dimensions: two, their fragments read a few at a time.  As one-tile items, which read all keys and
+// values for every 16 rows, a latent's 32 heads of 256 over one key/value head were bound by the
+// second-level cache: 785 us for a prompt of 3,000 tokens, 188 TFLOP/s; 128 rows a workgroup take 190 us,
+// 680 TFLOP/s counting the zeros of the values, which are not multiplied.)
 #ifndef HAL_RT_BIG
-#define HAL_RT_BIG (D <= 64 ? 4 : (D <= 128 ? 2 : 1))
+#define HAL_RT_BIG (D <= 64 ? 4 : 2)
 #endif
 #define RT_BIG HAL_RT_BIG
-// Keys per step of the kernel for long segments: 64 where two halves of that fit 64 KB of LDS.
+// Keys per step of that kernel: 64 where two halves of that fit 64 KB of LDS.
 #ifndef HAL_KB_BIG
 #define HAL_KB_BIG (D <= 128 ? 64 : 32)
 #endif
@@ -1141,11 +1218,22 @@ extern "C" int hal_attention_mfma_head_dim() { return D; }
 #endif
 #define HALVES_BIG HAL_HALVES_BIG
 
-extern "C" int hal_attention_mfma_rows_per_big_item() { return 16 * RT_BIG; }
+// Tiles of leading zeros in the values that there is a build for beside none (see VT0).
+#define VT0_BUILT (D == 256 ? 4 : 0)
+
+// The sums and queries of two tiles and two waves a SIMD fit the registers up to 224 dimensions, and at
+// 256 if a quarter of the values' are zeros (one wave a SIMD instead was slower than the kernel
+// without LDS on eight heads of 2,048 tokens, where its workgroups are half as many as the chip has
+// units).  Other heads have no kernel for long segments: their tiles are one-tile items, 16 rows each.
+#define BIG_BUILT(VT0_) (D - 8 * (VT0_) <= 224)
+
+extern "C" int hal_attention_mfma_rows_per_big_item(int value_from) {
+  return (VT0_BUILT > 0 && value_from >= 16 * VT0_BUILT) || BIG_BUILT(0) ? 16 * RT_BIG : 16;
+}
 
 // All arrays are device pointers.  `items` [max_items, 12] lists the work on segments of
 // at most 16 query rows (one tile per wave), `big_items` [max_big, 16] the work on longer
-// segments (hal_attention_mfma_rows_per_big_item() rows per wave), `merges`
+// segments (hal_attention_mfma_rows_per_big_item(value_from) rows per wave; 16: none), `merges`
 // [max_merges, 8] the row tiles whose key range was cut and whose partial results the merge
 // kernel joins.  counts = {items, big items, merges} holds the live numbers, so a captured
 // launch can serve varying counts.  `counters` [n_counters] (or null, if no item asks the
@@ -1165,13 +1253,14 @@ extern "C" int hal_attention_mfma(const void* q, int q_row_stride, void* out, in
                                   max_big, merges, max_merges, counts, seg_q_start, seg_q_len,
                                   seg_kv_len, block_table, bt_stride, k_pages, v_pages, part_o, part_ml,
                                   counters, n_counters, H, K, head_dim, page_size, tiled, scale, window,
-                                  0, nullptr, 0, 0, 0.f, nullptr, 0, merge_parts, stream);
+                                  0, nullptr, 0, 0, 0.f, nullptr, 0, 0, merge_parts, stream);
 }
 
 // The same with a rule for the scores.  `keep` (with a window): the first keys that stay visible;
 // the work lists name them.  `chunk`: the work lists must have been cut for it (a
 // tile's first key is no earlier than the start of its first row's chunk).  `bias_log2`:
-// float32 [H][bias_len], the bias by distance times log2 e.
+// float32 [H][bias_len], the bias by distance times log2 e.  `value_from`: the values' dimensions
+// before it are zeros on every page (they need not be read; the result's are zeros).
 extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out_row_stride,
                                         const int* items, int max_items, const int* big_items,
                                         int max_big, const int* merges, int max_merges,
@@ -1183,7 +1272,7 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
                                         int page_size, int tiled, float scale, int window, int chunk,
                                         const float* bias_log2, int bias_len, int sink,
                                         float softcap, const float* sink_log2, int keep,
-                                        int merge_parts, hipStream_t stream) {
+                                        int value_from, int merge_parts, hipStream_t stream) {
   HAL_REQUIRE(keep >= 0 && (keep == 0 || (window > 0 && chunk == 0)),
               "hal_attention_mfma: %d kept keys belong to a window alone (window %d, chunk %d)", keep, window, chunk);
   HAL_REQUIRE(chunk >= 0 && (bias_log2 == nullptr || bias_len > 0),
@@ -1214,20 +1303,20 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
   if ((page_size & (page_size - 1)) == 0)
     for (page_shift = 0; (1 << page_shift) < page_size; ++page_shift) {}
   const int waves = WAVES;
-#define PICK_ATTENTION(RT_, SHARED_, KB_, HV_, RU_, KE_)                                           \
+#define PICK_ATTENTION(RT_, SHARED_, KB_, HV_, RU_, KE_, VT_)                                       \
   {                                                                                               \
-    kernel = attention_mfma_kernel<RT_, false, false, SHARED_, false, KB_, HV_, RU_, KE_>;         \
-    if (tiled) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, D % 32 == 0, KB_, HV_, RU_, KE_>; \
-    else if (page_shift >= 5) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, false, KB_, HV_, RU_, KE_>; \
-    else if (page_shift >= 0) kernel = attention_mfma_kernel<RT_, true, false, SHARED_, false, KB_, HV_, RU_, KE_>; \
+    kernel = attention_mfma_kernel<RT_, false, false, SHARED_, false, KB_, HV_, RU_, KE_, VT_>;    \
+    if (tiled) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, D % 32 == 0, KB_, HV_, RU_, KE_, VT_>; \
+    else if (page_shift >= 5) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, false, KB_, HV_, RU_, KE_, VT_>; \
+    else if (page_shift >= 0) kernel = attention_mfma_kernel<RT_, true, false, SHARED_, false, KB_, HV_, RU_, KE_, VT_>; \
   }
-#define LAUNCH_ATTENTION(RT_, SHARED_, KB_, HV_, LIST, MAX, COUNT)                                 \
+#define LAUNCH_ATTENTION(RT_, SHARED_, KB_, HV_, VT_, LIST, MAX, COUNT)                            \
   {                                                                                               \
     dim3 grid(((MAX) + waves - 1) / waves, K);                                                    \
-    auto kernel = attention_mfma_kernel<RT_, false, false, SHARED_, false, KB_, HV_, false, false>; \
-    if (ruled) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, true, false)                                \
-    else if (keep > 0) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, true)                        \
-    else PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, false)                                     \
+    auto kernel = attention_mfma_kernel<RT_, false, false, SHARED_, false, KB_, HV_, false, false, VT_>; \
+    if (ruled) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, true, false, VT_)                           \
+    else if (keep > 0) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, true, VT_)                   \
+    else PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, false, VT_)                                \
     hipLaunchKernelGGL(kernel, grid, dim3(waves * HAL_WAVE * HV_), 0, stream, (const bf16_t*)q,   \
                        q_row_stride, (bf16_t*)out, out_row_stride, LIST, COUNT, seg_q_start,      \
                        seg_q_len, seg_kv_len, block_table, bt_stride, (const bf16_t*)k_pages,     \
@@ -1240,8 +1329,18 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
   HAL_REQUIRE(!counters || (part_o && part_ml && (long long)(max_items / WAVES) * K <= n_counters),
               "hal_attention_mfma: %d counters and the partial buffers do not serve %d items of %d "
               "kv heads", n_counters, max_items, K);
-  if (max_items > 0) LAUNCH_ATTENTION(1, false, 32, 1, items, max_items, counts)
-  if (max_big > 0) LAUNCH_ATTENTION(RT_BIG, true, KB_BIG, HALVES_BIG, big_items, max_big, counts + 1)
+  HAL_REQUIRE(value_from >= 0 && value_from < D, "hal_attention_mfma: values from dimension %d on of %d", value_from, D);
+  if (VT0_BUILT > 0 && value_from >= 16 * VT0_BUILT) {
+    if (max_items > 0) LAUNCH_ATTENTION(1, false, 32, 1, VT0_BUILT, items, max_items, counts)
+    if (max_big > 0) LAUNCH_ATTENTION(RT_BIG, true, KB_BIG, HALVES_BIG, VT0_BUILT, big_items, max_big, counts + 1)
+  } else {
+    if (max_items > 0) LAUNCH_ATTENTION(1, false, 32, 1, 0, items, max_items, counts)
+    if constexpr (BIG_BUILT(0)) {
+      if (max_big > 0) LAUNCH_ATTENTION(RT_BIG, true, KB_BIG, HALVES_BIG, 0, big_items, max_big, counts + 1)
+    } else {
+      HAL_REQUIRE(max_big == 0, "hal_attention_mfma: no kernel for long segments at head size %d", D);
+    }
+  }
 #undef LAUNCH_ATTENTION
 #undef PICK_ATTENTION
   if (max_merges > 0) {

@@ -429,7 +429,7 @@ int hal_wkv_step(const float* r, const float* k, const float* v, const float* ga
 
 // ---- the head-size-specific library (attention_mfma.hip) ---------------------------------
 int hal_attention_mfma_head_dim();
-int hal_attention_mfma_rows_per_big_item();
+int hal_attention_mfma_rows_per_big_item(int value_from);
 // merge_parts: the most partial results that any merge item joins, or 0 if not known (the
 // kernel for many partials is taken then).  Items of both lists come in runs of four, a
 // workgroup's waves (max_items and max_big are multiples of four): the one-tile items of a
@@ -448,6 +448,7 @@ int hal_attention_mfma(const void* q, int q_row_stride, void* out, int out_row_s
 
 // hal_attention_mfma with a rule for the scores (see hal_attention_simple_ruled); the bias
 // table and the sinks' values come multiplied by log2 e, and the work lists are cut for the chunk.
+// The values' dimensions before value_from are zeros on every page.
 int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out_row_stride,
                              const int* items, int max_items, const int* big_items, int max_big,
                              const int* merges, int max_merges, const int* counts,
@@ -457,6 +458,6 @@ int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out
                              int n_counters, int H, int K, int head_dim, int page_size, int tiled,
                              float scale, int window, int chunk, const float* bias_log2,
                              int bias_len, int sink, float softcap, const float* sink_log2,
-                             int keep, int merge_parts, hipStream_t stream);
+                             int keep, int value_from, int merge_parts, hipStream_t stream);
 
 }  // extern "C"

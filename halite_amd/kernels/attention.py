@@ -149,10 +149,37 @@ def mfma_supported(dtype: torch.dtype, head_dim: int, page_size: int) -> bool:
     return dtype == torch.bfloat16 and head_dim % 16 == 0 and 16 <= head_dim <= 256 and page_size % 8 == 0
 
 
-def rows_per_big_item(head_dim: int) -> int:
+def rows_per_big_item(head_dim: int, value_from: int = 0) -> int:
     """Rows that one wave takes of a long segment: the kernel library for this head size
-    says how it was built."""
-    return int(library.attention_library(head_dim).hal_attention_mfma_rows_per_big_item())
+    says how it was built (``value_from``: the values' dimensions before it are zeros).  16: long
+    segments are cut into one-tile items like short ones."""
+    return int(library.attention_library(head_dim).hal_attention_mfma_rows_per_big_item(value_from))
+
+
+# Heads of more than 128 dimensions: the kernel for long segments keeps the keys and values of a
+# block for 128 rows where the one for one-tile items reads them for 16, but its workgroups start and
+# end with more.  Measured on a latent's one key/value head of 256 (16 and 32 query heads): 18 against
+# 9 us at 128 tokens, 24 / 19 at 256, 27 / 24 and 28 / 45 at 512, 42 / 64 at 1,024, 190 / 785 at 3,000, and
+# with 4,096 tokens before them 30 / 24 and 34 / 38 at 64: the two meet at about six million (row, key)
+# pairs.  Heads with values in all dimensions have too few workgroups besides until there is one a
+# compute unit (160 dimensions, 2,048 tokens: 60 against 35 us with 128 workgroups, 59 / 79 with 256).
+LONG_ITEM_PAIRS = 6_000_000
+LONG_ITEM_ROWS = 128  # rows of such a workgroup
+
+
+def long_items_pay(seg_q_len, seg_kv_len, group_size: int, n_kv_heads: int, window: int, head_dim: int,
+                   value_from: int = 0) -> bool:
+    """Whether a step's long segments go to the kernel for long segments."""
+    if head_dim <= 128:
+        return True
+    ql, kl = np.asarray(seg_q_len, dtype=np.int64), np.asarray(seg_kv_len, dtype=np.int64)
+    keys = kl - ql // 2
+    if window > 0:
+        keys = np.minimum(keys, window)
+    rows = np.where(ql > 1, ql * group_size, 0)
+    if int((rows * keys).sum()) * n_kv_heads < LONG_ITEM_PAIRS:
+        return False
+    return value_from > 0 or int((-(-rows // LONG_ITEM_ROWS)).sum()) * n_kv_heads >= compute_units()
 
 
 def kept_units(keep: int) -> int:
@@ -457,7 +484,8 @@ def attention_mfma(q, q_row_stride, plan_dev, ctx, group, kv, n_heads, scale, wi
         P(group.block_table), group.block_table.shape[1], P(kv.k), P(kv.v), P(part_o), P(part_ml),
         P(counters), N_COUNTERS, n_heads, n_kv, head_dim, page_size, 1 if getattr(kv, "tiled", False) else 0,
         ctypes.c_float(scale), window, rule.chunk, P(bias), 0 if bias is None else bias.shape[1],
-        rule.weights_code(), ctypes.c_float(rule.softcap), P(sinks), rule.keep, plan.max_parts, ops._stream(),
+        rule.weights_code(), ctypes.c_float(rule.softcap), P(sinks), rule.keep, getattr(kv, "value_from", 0),
+        plan.max_parts, ops._stream(),
     )
     ops._check(lib, rc)
     return out

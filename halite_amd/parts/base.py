@@ -80,6 +80,8 @@ class PagedKVNeed(PagedNeed):
     # under a window: every later query sees the request's first tokens too, and the pages of
     # so many of them are kept
     keep: int = 0
+    # the values' dimensions before this one are zeros in every token (the attention kernel need not read them)
+    value_from: int = 0
 
     def page_tensors(self, page_size: int) -> dict[str, tuple[int, ...]]:
         k, d = self.n_kv_heads, self.head_dim
@@ -89,7 +91,7 @@ class PagedKVNeed(PagedNeed):
         from ..cache.pages import LayerPages, tiled_layout
 
         tiled = not self.plain_layout and tiled_layout(dtype, self.head_dim, page_size)
-        return LayerPages(group_id, tensors["k"], tensors["v"], tiled)
+        return LayerPages(group_id, tensors["k"], tensors["v"], tiled, self.value_from)
 
 
 @dataclass(frozen=True)

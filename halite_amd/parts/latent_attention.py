@@ -140,7 +140,8 @@ class LatentAttention(Mixer):
         return None  # no (heads, key/value heads, head size) in the sense of the options that name them
 
     def cache_need(self):
-        return PagedKVNeed(1, self.head_dim, self.p.window)
+        # (a cached value is [0 | latent | 0], the zeros where the key has its rotated part)
+        return PagedKVNeed(1, self.head_dim, self.p.window, value_from=self.p.rope_dim)
 
     def prepare(self, ctx, run):
         group = ctx.cache.groups[run.kv.group_id]
