@@ -15,6 +15,7 @@
 // cores (v_mfma_f32_16x16x32_bf16), K staged through LDS in the instruction's operand order.
 #include "hal_common.h"
 #include "hal_api.h"
+#include <math.h>
 
 struct GroupedArgs {
   const void* X;
@@ -459,50 +460,54 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
   }
 }
 
+// Which tile a workgroup takes, written to `found` (group, first row, end row, column tile; group -1: none)
+// by its first wave: the groups' rows in tiles of at most ROWS, equally high in steps of 32.
+template <int ROWS>
+__device__ __forceinline__ void gw_find(const GroupedArgs& a, int col_tiles, int* found) {
+  const int lane = threadIdx.x % 64;
+  auto tiles_of = [&](int g) { return g < a.G ? (a.group_offsets[g + 1] - a.group_offsets[g] + ROWS - 1) / ROWS : 0; };
+  int tiles = 0;
+  for (int c = 0; c < a.G; c += 64) {
+    int n = tiles_of(c + lane);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
+    tiles += n;
+  }
+  const long long units = (long long)tiles * col_tiles;
+  const int die = blockIdx.x % 8;
+  const long long unit = units * die / 8 + blockIdx.x / 8;
+  if (lane == 0) found[0] = -1;
+  if (unit >= units * (die + 1) / 8) return;
+  int before = 0;  // row tiles of the groups before
+  for (int c = 0; c < a.G; c += 64) {
+    const int n = tiles_of(c + lane);
+    int upto = n;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const int v = __shfl_up(upto, off, 64);
+      if (lane >= off) upto += v;
+    }
+    upto += before;
+    if (unit >= (long long)(upto - n) * col_tiles && unit < (long long)upto * col_tiles) {
+      const int in_group = (int)(unit - (long long)(upto - n) * col_tiles);
+      const int panel = in_group / (GW_PANEL * col_tiles), in_panel = in_group % (GW_PANEL * col_tiles);
+      const int high = min(GW_PANEL, n - panel * GW_PANEL);  // row tiles of this panel
+      const int g = c + lane, begin = a.group_offsets[g], end = a.group_offsets[g + 1];
+      const int rows = ((end - begin + n - 1) / n + 31) / 32 * 32;  // of each of the group's tiles
+      found[0] = g;
+      found[1] = begin + (panel * GW_PANEL + in_panel % high) * rows;
+      found[2] = min(end, found[1] + rows);
+      found[3] = in_panel / high;
+    }
+    before = __shfl(upto, 63, 64);
+  }
+}
+
 template <bool GATED>
 __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GW_BUFFER], b1[GW_BUFFER];
-  __shared__ __attribute__((aligned(64))) int found[4];  // group, first row, end row, column tile
-  const int lane = threadIdx.x % 64, wave = threadIdx.x / 64;
-  if (wave == 0) {
-    auto tiles_of = [&](int g) { return g < a.G ? (a.group_offsets[g + 1] - a.group_offsets[g] + GW_ROWS - 1) / GW_ROWS : 0; };
-    int tiles = 0;
-    for (int c = 0; c < a.G; c += 64) {
-      int n = tiles_of(c + lane);
-#pragma unroll
-      for (int off = 32; off > 0; off >>= 1) n += __shfl_xor(n, off, 64);
-      tiles += n;
-    }
-    const long long units = (long long)tiles * col_tiles;
-    const int die = blockIdx.x % 8;
-    const long long unit = units * die / 8 + blockIdx.x / 8;
-    if (lane == 0) found[0] = -1;
-    if (unit < units * (die + 1) / 8) {
-      int before = 0;  // row tiles of the groups before
-      for (int c = 0; c < a.G; c += 64) {
-        const int n = tiles_of(c + lane);
-        int upto = n;
-#pragma unroll
-        for (int off = 1; off < 64; off <<= 1) {
-          const int v = __shfl_up(upto, off, 64);
-          if (lane >= off) upto += v;
-        }
-        upto += before;
-        if (unit >= (long long)(upto - n) * col_tiles && unit < (long long)upto * col_tiles) {
-          const int in_group = (int)(unit - (long long)(upto - n) * col_tiles);
-          const int panel = in_group / (GW_PANEL * col_tiles), in_panel = in_group % (GW_PANEL * col_tiles);
-          const int high = min(GW_PANEL, n - panel * GW_PANEL);  // row tiles of this panel
-          const int g = c + lane, begin = a.group_offsets[g], end = a.group_offsets[g + 1];
-          const int rows = ((end - begin + n - 1) / n + 31) / 32 * 32;  // of each of the group's tiles
-          found[0] = g;
-          found[1] = begin + (panel * GW_PANEL + in_panel % high) * rows;
-          found[2] = min(end, found[1] + rows);
-          found[3] = in_panel / high;
-        }
-        before = __shfl(upto, 63, 64);
-      }
-    }
-  }
+  __shared__ __attribute__((aligned(64))) int found[4];
+  if (threadIdx.x < 64) gw_find<GW_ROWS>(a, col_tiles, found);
   __syncthreads();
   const int g = __builtin_amdgcn_readfirstlane(found[0]);
   if (g < 0) return;
@@ -518,6 +523,125 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
   else if (rows <= 224) GW_WAVE(7);
   else GW_WAVE(8);
 #undef GW_WAVE
+}
+
+// Groups of few rows (decode steps, short prompts): what counts is that the weights come at the memory's
+// rate, and come once.  Tiles of at most 64 rows x 128 W rows (GATED: 64 and 64) by four waves, a wave all
+// rows x 32 W rows; whole lines straight into three LDS buffers, two steps of 64 k under way while one is
+// multiplied, and two workgroups a compute unit.
+// Measured beside grouped_skinny_kernel, whose loads take half lines and which goes through the weights
+// once for every 16 rows, events around the call: 48 tokens, 4 of 16 experts of 4096 x 4096 (537 MB): 143 ->
+// 106 us; 16 tokens: 113 -> 104; 64 tokens: 178 -> 107; 48 tokens, 6 of 64 experts of 1024 x 4096, gate and
+// up: 211 -> 184; one token 37 -> 34.  All workgroups at one place of K (see `begin`): 122 instead of 106.
+#define GT_ROWS 64
+#define GT_ROWS_A_GROUP 48  // the streaming tiles are for fewer rows a group, on average
+#define GT_COLS 128
+#define GT_A_BYTES (GT_ROWS * GW_TK * 2)
+#define GT_BUFFER ((GT_ROWS + GT_COLS) * GW_TK * 2)
+template <bool GATED, int NI>
+__device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1,
+                                        char* b2) {
+  constexpr int AI = NI / 2, LOADS = AI + 4;
+  const int steps = a.K / GW_TK;
+  // Workgroups begin at different places of K and go round: rows of W that lie a power of two apart, all
+  // read at one place of K at a time, meet in a few of the memory's channels.
+  const int begin = (n0 / (GATED ? GT_COLS / 2 : GT_COLS) * 7 + g * 13) % steps;
+  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ gw_turn(lr % 16)) * 16;
+  // (GATED: of every 32 W rows, a wave's, the first 16 are the gate's and the others the up projection's)
+  const void* w0 = GATED && wave % 4 >= 2 ? a.W2 : a.W;
+  const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
+  const gw_rows X = gw_rows_at((const bf16_t*)a.X + a.x_col0, (uint32_t)a.x_rows * a.ldx * 2 - a.x_col0 * 2);
+  uint32_t xo[AI], wo[4];
+#pragma unroll
+  for (int i = 0; i < AI; ++i) {
+    int r = row0 + lr + 32 * i;
+    r = r < row_end ? r : row_end - 1;
+    xo[i] = (uint32_t)(a.row_src ? a.row_src[r] / a.src_div : r) * (uint32_t)(a.ldx * 2) + c;
+  }
+#pragma unroll
+  for (int i = 0; i < 4; ++i) {
+    int n = GATED ? n0 + i * 16 + lr % 16 : n0 + i * 32 + lr;
+    n = n < a.N ? n : a.N - 1;
+    wo[i] = (uint32_t)n * (uint32_t)(a.ldw * 2) + c;
+  }
+  auto bring = [&](char* lds, int step) {
+    step = (step < steps ? step : steps - 1) + begin;
+    const uint32_t at = (uint32_t)(step < steps ? step : step - steps) * (GW_TK * 2);
+#pragma unroll
+    for (int i = 0; i < AI; ++i) gw_load_lds(X, xo[i], at, lds + (i * 4 + wave) * 1024);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) gw_load_lds(W, wo[i], at, lds + GT_A_BYTES + (i * 4 + wave) * 1024);
+  };
+  const int q = lane / 16, r16 = lane % 16;
+  const int get[2] = {r16 * 128 + (q ^ gw_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ gw_turn(r16)) * 16};
+  gg_f32x4 acc[NI][2];
+#pragma unroll
+  for (int i = 0; i < NI; ++i)
+#pragma unroll
+    for (int j = 0; j < 2; ++j) acc[i][j] = gg_f32x4{0.f, 0.f, 0.f, 0.f};
+  auto multiply = [&](const char* lds) {
+#pragma unroll
+    for (int half = 0; half < 2; ++half) {
+      gg_bf16x8 w[2], x[NI];
+#pragma unroll
+      for (int j = 0; j < 2; ++j) w[j] = *(const gg_bf16x8*)(lds + GT_A_BYTES + (wave * 2 + j) * 2048 + get[half]);
+#pragma unroll
+      for (int i = 0; i < NI; ++i) x[i] = *(const gg_bf16x8*)(lds + i * 2048 + get[half]);
+#pragma unroll
+      for (int i = 0; i < NI; ++i)
+#pragma unroll
+        for (int j = 0; j < 2; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[j], x[i], acc[i][j], 0, 0, 0);
+    }
+  };
+  // the steps that do not fill a turn through the buffers, one at a time
+  const int odd = steps % 3;
+  for (int s = 0; s < odd; ++s) {
+    bring(b0, s);
+    gw_meet<0>();
+    multiply(b0);
+    gw_meet<0>();
+  }
+  bring(b0, odd);
+  bring(b1, odd + 1);
+  auto advance = [&](int s, const char* mine, char* free) {
+    gw_meet<LOADS>();  // (this step's pieces are there, the next one's may be on their way)
+    bring(free, s + 2);
+    multiply(mine);
+  };
+  for (int s = odd; s < steps; s += 3) {
+    advance(s, b0, b2);
+    advance(s + 1, b1, b0);
+    advance(s + 2, b2, b1);
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // LDS is not given back while loads are on their way into it
+#pragma unroll
+  for (int i = 0; i < NI; ++i) {
+    const int r = row0 + i * 16 + r16;
+    if (r >= row_end) continue;
+    const int dst = a.row_dst ? a.row_dst[r] : r;
+#pragma unroll
+    for (int j = 0; j < (GATED ? 1 : 2); ++j) {
+      const int n = n0 + wave * (GATED ? 16 : 32) + j * 16 + q * 4;
+      if (n < a.N) gw_store<GATED>(a, dst, n, acc[i][j], GATED ? acc[i][1] : acc[i][j]);
+    }
+  }
+}
+
+template <bool GATED>
+__global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, int col_tiles) {
+  __shared__ __attribute__((aligned(16))) char b0[GT_BUFFER], b1[GT_BUFFER], b2[GT_BUFFER];
+  __shared__ __attribute__((aligned(64))) int found[4];
+  if (threadIdx.x < 64) gw_find<GT_ROWS>(a, col_tiles, found);
+  __syncthreads();
+  const int g = __builtin_amdgcn_readfirstlane(found[0]);
+  if (g < 0) return;
+  const int row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
+  const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GT_COLS / 2 : GT_COLS);
+  const int rows = row_end - row0;
+  if (rows <= 0) return;
+  if (rows <= 32) gt_wave<GATED, 2>(a, g, row0, row_end, n0, b0, b1, b2);
+  else gt_wave<GATED, 4>(a, g, row0, row_end, n0, b0, b1, b2);
 }
 
 // bf16, few rows a group (decode steps): a workgroup takes 64 rows of W (GATED: 32 of the
@@ -592,6 +716,17 @@ __global__ void __launch_bounds__(256) grouped_skinny_kernel(GroupedArgs a) {
   }
 }
 
+// Whether the streaming tiles of `rows` listed rows of G groups leave a round of two workgroups a compute
+// unit just begun (about as many groups have rows as such a number of random picks meets): the kernel for
+// few rows, whose workgroups are smaller, then ends earlier (48 rows of 64 groups of 1024 x 4096, gate
+// and up: 1.06 rounds, 117 us against 116; 4096 x 1024: 2.1 rounds, 61 / 58; with 72 rows, 1.36 and 2.7
+// rounds, 135 / 152 and 77 / 81).
+static bool gt_round_just_begun(long long rows, int G, int col_tiles) {
+  const double reached = G * (1.0 - pow(1.0 - 1.0 / G, (double)rows));
+  const double rounds = reached * col_tiles / (2 * 256);
+  return rounds > 1.0 && rounds - floor(rounds) < 0.2;
+}
+
 extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_col0, const void* W,
                                 const void* W2, long long w_group_stride, int ldw, int dtype,
                                 void* Y, int ldy, int y_group_cols, int y_col0, int y_dtype,
@@ -631,18 +766,28 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   const bool aligned = K % 8 == 0 && ldx % 8 == 0 && ldw % 8 == 0 && x_group_cols % 8 == 0 &&
                        x_col0 % 8 == 0 && w_group_stride % 8 == 0 && ((uintptr_t)X % 16 == 0) &&
                        ((uintptr_t)W % 16 == 0) && (W2 == nullptr || (uintptr_t)W2 % 16 == 0);
-  // few rows a group: the kernel that keeps many loads in flight instead of staging tiles; experts with
-  // more: the wide tiles wherever sizes and addresses are such that their loads and vector stores need
-  // no bounds (faster at every size measured, from 47 rows a group on); heads, narrow weights and the
-  // rest: tiles of 128
+  // Experts (rows listed by group) whose sizes and addresses are such that loads and vector stores need no
+  // bounds: of few rows the streaming tiles (ahead of the wide ones up to 40 to 75 rows a group: 196 / 196
+  // us at 37 rows of 64 experts of 1024 x 4096, 224 / 203 at 56; 139 / 142 at 75 rows of 16 of
+  // 4096 x 4096, 187 / 148 at 150), of more the wide ones.  The others, and the heads: of few rows the kernel
+  // that keeps many loads in flight instead of staging tiles, of more tiles of 128.
   const long long rows_per_group = group_offsets ? M / G : M;
-  if (dtype == HAL_BF16 && allow_mfma && aligned && rows_per_group <= 16) {
+  const bool plain = dtype == HAL_BF16 && allow_mfma && aligned && group_offsets && gate == nullptr && !y_add && N % 4 == 0 &&
+                     ldy % 4 == 0 && y_col0 % 4 == 0 && (uintptr_t)Y % 16 == 0 && x_group_cols == 0 && y_group_cols == 0 &&
+                     (long long)N * ldw * 2 < (1ll << 31) && (long long)x_rows * ldx * 2 < (1ll << 31);
+  const int stream_tiles = W2 ? (N + GT_COLS / 2 - 1) / (GT_COLS / 2) : (N + GT_COLS - 1) / GT_COLS;
+  if (plain && K % GW_TK == 0 && K >= 4 * GW_TK && N >= GT_COLS && rows_per_group < GT_ROWS_A_GROUP &&
+      !(rows_per_group <= 16 && gt_round_just_begun(M, G, stream_tiles))) {
+    const int col_tiles = stream_tiles;
+    const long long units = ((long long)(M + GT_ROWS - 1) / GT_ROWS + G) * col_tiles, blocks = 8 * ((units + 7) / 8);
+    HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
+    if (W2) hipLaunchKernelGGL(grouped_stream_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
+    else hipLaunchKernelGGL(grouped_stream_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
+  } else if (dtype == HAL_BF16 && allow_mfma && aligned && rows_per_group <= 16) {
     grid.x = W2 ? (N + 31) / 32 : (N + 63) / 64;
     if (W2) hipLaunchKernelGGL(grouped_skinny_kernel<true>, grid, dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(grouped_skinny_kernel<false>, grid, dim3(256), 0, stream, a);
-  } else if (dtype == HAL_BF16 && allow_mfma && aligned && group_offsets && K % (2 * GW_TK) == 0 && N >= GW_COLS &&
-             gate == nullptr && !y_add && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 && (uintptr_t)Y % 16 == 0 &&
-             x_group_cols == 0 && y_group_cols == 0 && (long long)N * ldw * 2 < (1ll << 31) && (long long)x_rows * ldx * 2 < (1ll << 31)) {
+  } else if (plain && K % (2 * GW_TK) == 0 && N >= GW_COLS) {
     const int cols = W2 ? GW_COLS / 2 : GW_COLS, col_tiles = (N + cols - 1) / cols;
     const long long units = ((long long)(M + GW_ROWS - 1) / GW_ROWS + G) * col_tiles, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);

@@ -1,5 +1,6 @@
-"""The experts' products of prompts (``grouped_wide_kernel``): tiles of up to 256 rows whose height
-follows the groups' sizes, against the products in 64 bits."""
+"""The experts' products: of prompts (``grouped_wide_kernel``, tiles of up to 256 rows whose height
+follows the groups' sizes) and of few rows a group (``grouped_stream_kernel``), against the products in
+64 bits."""
 
 import pytest
 import torch
@@ -18,6 +19,8 @@ def gpu():
 # 192, 224, 256 rows), of a second, third and ninth tile (a panel of eight and one more), and a group whose
 # equal heights in steps of 32 leave its last tile short
 EDGES = [0, 1, 33, 64, 65, 128, 129, 160, 0, 161, 192, 193, 224, 225, 255, 256, 257, 512, 513, 545, 2049, 0]
+# fewer than 48 a group on average: the streaming tiles; none, one, at both sides of 32 and 64 rows, several tiles
+FEW = [0, 1, 31, 32, 33, 0, 63, 64, 65, 0, 0, 97, 129, 2, 16, 17, 0, 0, 200, 0]
 
 
 def listed(counts, device):
@@ -38,12 +41,10 @@ def compare(got, want, size, result_rounding):
     assert bool(((got.double() - want).abs() <= limit).all()), float(((got.double() - want).abs() / limit).max())
 
 
-@pytest.mark.parametrize("n, k", [(256, 128), (260, 384), (768, 256)])
-@pytest.mark.parametrize("counts", [EDGES, [300] * 70, [40, 17, 20]])
-def test_down_products_scatter_float32_rows(gpu, n, k, counts):
+@pytest.mark.parametrize("counts, n, k", [(EDGES, 256, 128), (EDGES, 260, 384), (EDGES, 768, 256), ([300] * 70, 256, 128),
+                                          (FEW, 128, 256), (FEW, 132, 320), (FEW, 300, 384), ([1] * 3 + [0] * 80 + [5] * 3, 256, 448)])
+def test_down_products_scatter_float32_rows(gpu, counts, n, k):
     """Rows and results with strides of their own, results at scattered rows, more groups than lanes of a wave."""
-    if len(counts) > 30 and n != 256:
-        pytest.skip("one width is enough for many groups")
     rows = sum(counts)
     offsets, group_offsets, tile_offsets = listed(counts, gpu)
     x = rand(rows, k + 24, seed=1).bfloat16().to(gpu)
@@ -58,10 +59,10 @@ def test_down_products_scatter_float32_rows(gpu, n, k, counts):
 
 
 @pytest.mark.parametrize("act", ["gated", "relu_squared"])
-@pytest.mark.parametrize("n, k", [(256, 128), (388, 256)])
-def test_up_products_gather_rows(gpu, act, n, k):
+@pytest.mark.parametrize("counts, n, k", [(EDGES, 256, 128), (EDGES, 388, 256), (FEW, 128, 256), (FEW, 200, 320), (FEW, 388, 384)])
+def test_up_products_gather_rows(gpu, act, counts, n, k):
     """Rows gathered through the sorted list, the activations in the epilogue, bf16 results."""
-    counts, top = EDGES, 2
+    top = 2
     rows = sum(counts)
     offsets, group_offsets, tile_offsets = listed(counts, gpu)
     tokens = -(-rows // top)
