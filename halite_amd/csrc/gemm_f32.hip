@@ -7,7 +7,7 @@
 // its lanes take every 64th group of four k each (the rows of A come through LDS, shared by
 // the workgroup's four waves), and the partial sums of the lanes, and of the waves that share
 // columns, are added in a fixed order.  17 to about 100 rows: the matrix cores, k split over a
-// workgroup's waves, each staging whole rows through LDS of its own.  More rows: tiles of 128 rows and 128 or 32
+// workgroup's waves, each staging whole rows through LDS of its own.  More rows: tiles of 128 rows and 128, 64 or 32
 // columns on the matrix cores, through LDS.  For sizes and addresses that are no multiples of
 // four: tiles of 64 x 64 on the vector units, each output element one chain of K
 // multiply-adds in index order.
@@ -94,16 +94,19 @@ gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ 
 #define MF_XCDS 8  // dies of the gfx950 parts that this library is built for (a wrong count costs cache hits only)
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-// BN: columns of a workgroup's tile, 128 (a wave takes 64 x 64 as 2 x 2 products) or 32 (a wave
-// takes 32 x 32): the narrow tile is for products of so few rows and columns that tiles of 128
-// columns would leave most of the chip empty.  An output element's sum is the same in both.
+// BN: columns of a workgroup's tile, 128 (four waves, a wave 64 x 64 as 2 x 2 products), 64 (eight
+// waves) or 32 (four; a wave 32 x 32): the narrower tiles are for products whose rows and columns would
+// leave units without a tile of 128.  What bounds them is the second-level cache (tiles of 32 columns
+// ask it for 20 bytes a clock and unit, all it gives; of 64 for 12).  An output element's sum is the same in all.
 template <int BN>
-__global__ void __launch_bounds__(256, 2)
+__global__ void __launch_bounds__(BN == 64 ? 512 : 256, BN == 64 ? 4 : 2)
 gemm_f32_mfma_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
                      float* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n) {
-  constexpr int NB = BN == 128 ? 2 : 1;     // 32 x 32 products of a wave, each way
-  constexpr int WV = BN * MF_KQ / 256;      // 16-byte vectors of W's stage per thread
-  static_assert(BN == 128 || BN == 32, "tiles of 128 or 32 columns");
+  constexpr int THREADS = BN == 64 ? 512 : 256;
+  constexpr int NB = BN == 128 ? 2 : 1;           // 32 x 32 products of a wave, each way
+  constexpr int AV = MF_BM * MF_KQ / THREADS;     // 16-byte vectors of A's stage per thread
+  constexpr int WV = BN * MF_KQ / THREADS;        // and of W's
+  static_assert(BN == 128 || BN == 64 || BN == 32, "tiles of 128, 64 or 32 columns");
   // [buffer][k / 4][row], a row more than there are so that the stores of a wave (a row's
   // eight vectors side by side) spread over the banks
   __shared__ float4 a_s[2][MF_KQ][MF_BM + 1];
@@ -117,30 +120,30 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, int lda, const float* __restri
   if (n_tiles % MF_XCDS == 0) id = (id % MF_XCDS) * (n_tiles / MF_XCDS) + id / MF_XCDS;
   const int m0 = (id % tiles_m) * MF_BM, n0 = (id / tiles_m) * BN;
 
-  float4 a_next[4], w_next[WV];
+  float4 a_next[AV], w_next[WV];
   auto ask = [&](int k0) {  // vector e of a stage: row e / 8, k0 + 4 (e % 8)
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + u * 256, r = e / MF_KQ, k = k0 + (e % MF_KQ) * 4;
+    for (int u = 0; u < AV; ++u) {
+      const int e = tid + u * THREADS, r = e / MF_KQ, k = k0 + (e % MF_KQ) * 4;
       const bool in = k < K && m0 + r < M;  // (K is a multiple of 4)
       a_next[u] = in ? *(const float4*)(A + (size_t)(m0 + r) * lda + k) : float4{0.f, 0.f, 0.f, 0.f};
     }
 #pragma unroll
     for (int u = 0; u < WV; ++u) {
-      const int e = tid + u * 256, r = e / MF_KQ, k = k0 + (e % MF_KQ) * 4;
+      const int e = tid + u * THREADS, r = e / MF_KQ, k = k0 + (e % MF_KQ) * 4;
       const bool in = k < K && n0 + r < N;
       w_next[u] = in ? *(const float4*)(W + (size_t)(n0 + r) * ldw + k) : float4{0.f, 0.f, 0.f, 0.f};
     }
   };
   auto put = [&](int buf) {
 #pragma unroll
-    for (int u = 0; u < 4; ++u) {
-      const int e = tid + u * 256;
+    for (int u = 0; u < AV; ++u) {
+      const int e = tid + u * THREADS;
       a_s[buf][e % MF_KQ][e / MF_KQ] = a_next[u];
     }
 #pragma unroll
     for (int u = 0; u < WV; ++u) {
-      const int e = tid + u * 256;
+      const int e = tid + u * THREADS;
       w_s[buf][e % MF_KQ][e / MF_KQ] = w_next[u];
     }
   };
@@ -156,7 +159,8 @@ gemm_f32_mfma_kernel(const float* __restrict__ A, int lda, const float* __restri
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[i][j][v] = total[i][j][v] = 0.f;
   // this wave's corner of the tile
-  const int wm = BN == 128 ? (wave / 2) * 64 : wave * 32, wn = BN == 128 ? (wave % 2) * 64 : 0;
+  const int wm = BN == 128 ? (wave / 2) * 64 : BN == 64 ? (wave / 2) * 32 : wave * 32;
+  const int wn = BN == 128 ? (wave % 2) * 64 : BN == 64 ? (wave % 2) * 32 : 0;
   const int rows = wm + lane % 32, cols = wn + lane % 32, half = lane / 32;
   const bool wave_has_rows = m0 + wm < M;  // (a wave whose rows are all beyond M only helps to load)
 
@@ -472,6 +476,19 @@ static void launch_skinny(const float* A, int lda, const float* W, int ldw, floa
                        A, lda, W, ldw, C, ldc, M, N, K);
 }
 
+// What tiles of BN columns cost, in microseconds at K = 4,096: rounds over the 256 compute units, a round
+// of tiles of 128 / 64 / 32 columns 270 / 147 / 83 (a compute unit whose only tile it is has too few waves
+// to hide what they wait for: 30 and 10 more; one or two tiles of 32 columns 125 and 183).  Measured at K =
+// 4,096 in tiles of 128 / 64 / 32: 500 rows x 4,096 columns 305 / 174 / 187 us, x 6,144 308 / 301 / 255,
+// x 28,672 1,085 / 1,017 / 1,129, x 32,000 1,093 / 1,161 / 1,285; 200 x 4,096 305 / 167 / 126; 1,500 x 4,096
+// 548 / 451 / 490; 2,048 x 4,096 554 / 594 / 661.
+static double mf_rounds_cost(long long tiles_m, int N, int BN) {
+  const double n = (double)((tiles_m * ((N + BN - 1) / BN) + 255) / 256);
+  if (BN == 128) return 30 + 270 * n;
+  if (BN == 64) return 10 + 147 * n;
+  return n <= 1 ? 125 : n <= 2 ? 183 : 83 * n;
+}
+
 extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
                             int M, int N, int K, hipStream_t stream) {
   HAL_REQUIRE(M >= 0 && N > 0 && K > 0, "hal_gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -500,17 +517,23 @@ extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, fl
       HAL_LAUNCH_CHECK();
       return 0;
     }
-    // more rows: the matrix cores, in tiles of 128 columns where those fill the chip
-    const long long tiles_m = (M + MF_BM - 1) / MF_BM, wide = (N + 127) / 128, narrow = (N + 31) / 32;
-    const bool use_wide = tiles_m * wide >= 256;
-    const long long tiles_n = use_wide ? wide : narrow;
+    // more rows: the matrix cores, in the tiles whose rounds over the compute units are expected to end first
+    const long long tiles_m = (M + MF_BM - 1) / MF_BM;
+    int bn = 128;
+    for (int other = 64; other >= 32; other /= 2)
+      if (mf_rounds_cost(tiles_m, N, other) < mf_rounds_cost(tiles_m, N, bn)) bn = other;
+    const long long tiles_n = (N + bn - 1) / bn;
     HAL_REQUIRE(tiles_m * tiles_n < (1ll << 31), "hal_gemm_f32: M=%d N=%d exceed the grid limit", M, N);
-    if (use_wide)
-      hipLaunchKernelGGL(gemm_f32_mfma_kernel<128>, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, A,
-                         lda, W, ldw, C, ldc, M, N, K, (int)tiles_m, (int)tiles_n);
+    const dim3 tiles((unsigned)(tiles_m * tiles_n));
+    if (bn == 128)
+      hipLaunchKernelGGL(gemm_f32_mfma_kernel<128>, tiles, dim3(256), 0, stream, A, lda, W, ldw, C, ldc, M, N, K,
+                         (int)tiles_m, (int)tiles_n);
+    else if (bn == 64)
+      hipLaunchKernelGGL(gemm_f32_mfma_kernel<64>, tiles, dim3(512), 0, stream, A, lda, W, ldw, C, ldc, M, N, K,
+                         (int)tiles_m, (int)tiles_n);
     else
-      hipLaunchKernelGGL(gemm_f32_mfma_kernel<32>, dim3((unsigned)(tiles_m * tiles_n)), dim3(256), 0, stream, A,
-                         lda, W, ldw, C, ldc, M, N, K, (int)tiles_m, (int)tiles_n);
+      hipLaunchKernelGGL(gemm_f32_mfma_kernel<32>, tiles, dim3(256), 0, stream, A, lda, W, ldw, C, ldc, M, N, K,
+                         (int)tiles_m, (int)tiles_n);
     HAL_LAUNCH_CHECK();
     return 0;
   }
