@@ -538,7 +538,13 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
 #define GT_COLS 128
 #define GT_A_BYTES (GT_ROWS * GW_TK * 2)
 #define GT_BUFFER ((GT_ROWS + GT_COLS) * GW_TK * 2)
-template <bool GATED, int NI>
+// HEADS: every group has all rows, columns of its own in X and Y, and perhaps a gate on its result.  The
+// tiles' shape is as good for many rows there, as K is a head's few hundred and the rows are what is read:
+// 32 heads of K = 192, N = 128 with a gate: 17 rows 13.6 -> 8.0 us, 64 26.0 -> 9.6, 1,000 38.7 -> 15.2, 3,000
+// 51.6 -> 34.6 beside the tiles of 128 (K = 128, N = 192: 10.1 -> 6.6, 17.2 -> 7.7, 21.3 -> 15.5, 41.5 -> 36.4),
+// whose loads go through registers and wait for each other.
+typedef __attribute__((ext_vector_type(4), aligned(4))) float gt_f32x4_any;  // (a gate's rows begin at any float)
+template <bool GATED, bool HEADS, int NI>
 __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1,
                                         char* b2) {
   constexpr int AI = NI / 2, LOADS = AI + 4;
@@ -551,7 +557,8 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
   // (GATED: of every 32 W rows, a wave's, the first 16 are the gate's and the others the up projection's)
   const void* w0 = GATED && wave % 4 >= 2 ? a.W2 : a.W;
   const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
-  const gw_rows X = gw_rows_at((const bf16_t*)a.X + a.x_col0, (uint32_t)a.x_rows * a.ldx * 2 - a.x_col0 * 2);
+  const int x_col0 = a.x_col0 + (HEADS ? g * a.x_group_cols : 0);
+  const gw_rows X = gw_rows_at((const bf16_t*)a.X + x_col0, (uint32_t)a.x_rows * a.ldx * 2 - x_col0 * 2);
   uint32_t xo[AI], wo[4];
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
@@ -623,25 +630,45 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
 #pragma unroll
     for (int j = 0; j < (GATED ? 1 : 2); ++j) {
       const int n = n0 + wave * (GATED ? 16 : 32) + j * 16 + q * 4;
-      if (n < a.N) gw_store<GATED>(a, dst, n, acc[i][j], GATED ? acc[i][1] : acc[i][j]);
+      if (n >= a.N) continue;
+      if (HEADS && a.gate) {
+        const float* at = a.gate + (size_t)dst * a.ldg + (size_t)g * a.gate_group_cols + (a.gate_cols ? n : 0);
+        gt_f32x4_any by;
+        if (a.gate_cols) by = *(const gt_f32x4_any*)at;
+        else by = gt_f32x4_any{at[0], at[0], at[0], at[0]};
+#pragma unroll
+        for (int v = 0; v < 4; ++v) acc[i][j][v] *= gg_sigmoid(by[v]);
+      }
+      gw_store<GATED>(a, dst, (HEADS ? g * a.y_group_cols : 0) + n, acc[i][j], GATED ? acc[i][1] : acc[i][j]);
     }
   }
 }
 
-template <bool GATED>
+template <bool GATED, bool HEADS>
 __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GT_BUFFER], b1[GT_BUFFER], b2[GT_BUFFER];
   __shared__ __attribute__((aligned(64))) int found[4];
-  if (threadIdx.x < 64) gw_find<GT_ROWS>(a, col_tiles, found);
-  __syncthreads();
-  const int g = __builtin_amdgcn_readfirstlane(found[0]);
-  if (g < 0) return;
-  const int row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
-  const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GT_COLS / 2 : GT_COLS);
+  int g, row0, row_end, col;
+  if (HEADS) {
+    // a die takes neighbouring heads, a head's columns beside each other: they read the same rows
+    const int in_group = (a.M + GT_ROWS - 1) / GT_ROWS * col_tiles, die = blockIdx.x % 8;
+    const long long units = (long long)a.G * in_group, unit = units * die / 8 + blockIdx.x / 8;
+    if (unit >= units * (die + 1) / 8) return;
+    g = (int)(unit / in_group), row0 = (int)(unit % in_group) / col_tiles * GT_ROWS;
+    row_end = min(a.M, row0 + GT_ROWS), col = (int)(unit % in_group) % col_tiles;
+  } else {
+    if (threadIdx.x < 64) gw_find<GT_ROWS>(a, col_tiles, found);
+    __syncthreads();
+    g = __builtin_amdgcn_readfirstlane(found[0]);
+    if (g < 0) return;
+    row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
+    col = __builtin_amdgcn_readfirstlane(found[3]);
+  }
+  const int n0 = col * (GATED ? GT_COLS / 2 : GT_COLS);
   const int rows = row_end - row0;
   if (rows <= 0) return;
-  if (rows <= 32) gt_wave<GATED, 2>(a, g, row0, row_end, n0, b0, b1, b2);
-  else gt_wave<GATED, 4>(a, g, row0, row_end, n0, b0, b1, b2);
+  if (rows <= 32) gt_wave<GATED, HEADS, 2>(a, g, row0, row_end, n0, b0, b1, b2);
+  else gt_wave<GATED, HEADS, 4>(a, g, row0, row_end, n0, b0, b1, b2);
 }
 
 // bf16, few rows a group (decode steps): a workgroup takes 64 rows of W (GATED: 32 of the
@@ -769,20 +796,27 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   // Experts (rows listed by group) whose sizes and addresses are such that loads and vector stores need no
   // bounds: of few rows the streaming tiles (ahead of the wide ones up to 40 to 75 rows a group: 196 / 196
   // us at 37 rows of 64 experts of 1024 x 4096, 224 / 203 at 56; 139 / 142 at 75 rows of 16 of
-  // 4096 x 4096, 187 / 148 at 150), of more the wide ones.  The others, and the heads: of few rows the kernel
-  // that keeps many loads in flight instead of staging tiles, of more tiles of 128.
+  // 4096 x 4096, 187 / 148 at 150), of more the wide ones; heads of more
+  // than 16 rows the streaming tiles (figures there; faster from 17 to 8,000 rows at K of 128 to 512).  The others:
+  // of few rows the kernel that keeps many loads in flight instead of staging tiles, of more tiles of 128.
   const long long rows_per_group = group_offsets ? M / G : M;
-  const bool plain = dtype == HAL_BF16 && allow_mfma && aligned && group_offsets && gate == nullptr && !y_add && N % 4 == 0 &&
-                     ldy % 4 == 0 && y_col0 % 4 == 0 && (uintptr_t)Y % 16 == 0 && x_group_cols == 0 && y_group_cols == 0 &&
-                     (long long)N * ldw * 2 < (1ll << 31) && (long long)x_rows * ldx * 2 < (1ll << 31);
+  const bool whole = dtype == HAL_BF16 && allow_mfma && aligned && !y_add && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 &&
+                     y_group_cols % 4 == 0 && (uintptr_t)Y % 16 == 0 && (long long)N * ldw * 2 < (1ll << 31) &&
+                     (long long)x_rows * ldx * 2 < (1ll << 31);
+  const bool plain = whole && group_offsets && gate == nullptr && x_group_cols == 0 && y_group_cols == 0;
+  const bool heads = whole && !group_offsets && !W2 && row_src == nullptr && row_dst == nullptr && (act == 0 || gate == nullptr);
   const int stream_tiles = W2 ? (N + GT_COLS / 2 - 1) / (GT_COLS / 2) : (N + GT_COLS - 1) / GT_COLS;
   if (plain && K % GW_TK == 0 && K >= 4 * GW_TK && N >= GT_COLS && rows_per_group < GT_ROWS_A_GROUP &&
       !(rows_per_group <= 16 && gt_round_just_begun(M, G, stream_tiles))) {
     const int col_tiles = stream_tiles;
     const long long units = ((long long)(M + GT_ROWS - 1) / GT_ROWS + G) * col_tiles, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    if (W2) hipLaunchKernelGGL(grouped_stream_kernel<true>, dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
-    else hipLaunchKernelGGL(grouped_stream_kernel<false>, dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
+    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
+    else hipLaunchKernelGGL((grouped_stream_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
+  } else if (heads && K % GW_TK == 0 && rows_per_group > 16) {
+    const long long units = (long long)((M + GT_ROWS - 1) / GT_ROWS) * G * stream_tiles, blocks = 8 * ((units + 7) / 8);
+    HAL_REQUIRE(blocks < (1ll << 31) && (long long)M * stream_tiles < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
+    hipLaunchKernelGGL((grouped_stream_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_tiles);
   } else if (dtype == HAL_BF16 && allow_mfma && aligned && rows_per_group <= 16) {
     grid.x = W2 ? (N + 31) / 32 : (N + 63) / 64;
     if (W2) hipLaunchKernelGGL(grouped_skinny_kernel<true>, grid, dim3(256), 0, stream, a);
