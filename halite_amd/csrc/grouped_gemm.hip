@@ -532,7 +532,7 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
 // Measured beside grouped_skinny_kernel, whose loads take half lines and which goes through the weights
 // once for every 16 rows, events around the call: 48 tokens, 4 of 16 experts of 4096 x 4096 (537 MB): 143 ->
 // 106 us; 16 tokens: 113 -> 104; 64 tokens: 178 -> 107; 48 tokens, 6 of 64 experts of 1024 x 4096, gate and
-// up: 211 -> 184; one token 37 -> 34.  All workgroups at one place of K (see `begin`): 122 instead of 106.
+// up: 211 -> 184.  All workgroups at one place of K (see `begin`): 122 instead of 106.
 #define GT_ROWS 64
 #define GT_ROWS_A_GROUP 48  // the streaming tiles are for fewer rows a group, on average
 #define GT_COLS 128
@@ -743,15 +743,18 @@ __global__ void __launch_bounds__(256) grouped_skinny_kernel(GroupedArgs a) {
   }
 }
 
-// Whether the streaming tiles of `rows` listed rows of G groups leave a round of two workgroups a compute
-// unit just begun (about as many groups have rows as such a number of random picks meets): the kernel for
-// few rows, whose workgroups are smaller, then ends earlier (48 rows of 64 groups of 1024 x 4096, gate
-// and up: 1.06 rounds, 117 us against 116; 4096 x 1024: 2.1 rounds, 61 / 58; with 72 rows, 1.36 and 2.7
-// rounds, 135 / 152 and 77 / 81).
-static bool gt_round_just_begun(long long rows, int G, int col_tiles) {
+// Whether the streaming tiles of `rows` listed rows of G groups fill the chip badly (about as many groups
+// have rows as such a number of random picks meets): fewer than 144 tiles, which leave compute units without
+// one, or a round of two workgroups a unit just begun.  The kernel for few rows, whose workgroups are smaller,
+// then ends earlier.  One row of 4 of 16 groups of 4096 x 4096 (116 tiles): 30.0 us against 35.8, two (206
+// tiles) 50.5 / 44.0; of 6 of 64 of 1024 x 4096, gate and up (92 tiles) 27.9 / 34.3, two (176) 49.3 / 39.1;
+// 4096 x 1024, one (185): 14.1 / 11.5.  48 rows of 64 groups of 1024 x 4096, gate and up: 1.06 rounds, 116
+// us against 117; 4096 x 1024: 2.1 rounds, 58 / 61; with 72 rows, 1.36 and 2.7 rounds, 152 / 135 and 81 / 77.
+#define GT_FEWEST_TILES 144
+static bool gt_fills_badly(long long rows, int G, int col_tiles) {
   const double reached = G * (1.0 - pow(1.0 - 1.0 / G, (double)rows));
-  const double rounds = reached * col_tiles / (2 * 256);
-  return rounds > 1.0 && rounds - floor(rounds) < 0.2;
+  const double tiles = reached * col_tiles, rounds = tiles / (2 * 256);
+  return tiles < GT_FEWEST_TILES || (rounds > 1.0 && rounds - floor(rounds) < 0.2);
 }
 
 extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_col0, const void* W,
@@ -807,7 +810,7 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   const bool heads = whole && !group_offsets && !W2 && row_src == nullptr && row_dst == nullptr && (act == 0 || gate == nullptr);
   const int stream_tiles = W2 ? (N + GT_COLS / 2 - 1) / (GT_COLS / 2) : (N + GT_COLS - 1) / GT_COLS;
   if (plain && K % GW_TK == 0 && K >= 4 * GW_TK && N >= GT_COLS && rows_per_group < GT_ROWS_A_GROUP &&
-      !(rows_per_group <= 16 && gt_round_just_begun(M, G, stream_tiles))) {
+      !(rows_per_group <= 16 && gt_fills_badly(M, G, stream_tiles))) {
     const int col_tiles = stream_tiles;
     const long long units = ((long long)(M + GT_ROWS - 1) / GT_ROWS + G) * col_tiles, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
