@@ -347,6 +347,11 @@ typedef __amdgpu_buffer_rsrc_t gw_rows;
 __device__ __forceinline__ gw_rows gw_rows_at(const void* p, uint32_t bytes) {
   return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
+// The rows of X, K columns from `col0` on: up to the end of the last row's, so that rows that overlap (a row
+// length below K, or 0 where one row stands for all) lie in the range like any others.
+__device__ __forceinline__ gw_rows gw_rows_of_x(const GroupedArgs& a, int col0) {
+  return gw_rows_at((const bf16_t*)a.X + col0, ((uint32_t)(a.x_rows - 1) * a.ldx + a.K) * 2);
+}
 __device__ __forceinline__ void gw_load_lds(gw_rows from, uint32_t each, uint32_t all, char* to) {
   __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, each, all, 0, 0);
 }
@@ -370,7 +375,7 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
   // (GATED: of every 64 W rows, a wave's, the first 32 are the gate's and the others the up projection's)
   const void* w0 = GATED && wave >= 4 ? a.W2 : a.W;
   const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
-  const gw_rows X = gw_rows_at((const bf16_t*)a.X + a.x_col0, (uint32_t)a.x_rows * a.ldx * 2 - a.x_col0 * 2);
+  const gw_rows X = gw_rows_of_x(a, a.x_col0);
   uint32_t xo[AI], wo[4];
   // rows and columns past the end are read from the last one: nothing of them is stored
 #pragma unroll
@@ -557,8 +562,7 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
   // (GATED: of every 32 W rows, a wave's, the first 16 are the gate's and the others the up projection's)
   const void* w0 = GATED && wave % 4 >= 2 ? a.W2 : a.W;
   const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
-  const int x_col0 = a.x_col0 + (HEADS ? g * a.x_group_cols : 0);
-  const gw_rows X = gw_rows_at((const bf16_t*)a.X + x_col0, (uint32_t)a.x_rows * a.ldx * 2 - x_col0 * 2);
+  const gw_rows X = gw_rows_of_x(a, a.x_col0 + (HEADS ? g * a.x_group_cols : 0));
   uint32_t xo[AI], wo[4];
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
@@ -803,9 +807,9 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   // than 16 rows the streaming tiles (figures there; faster from 17 to 8,000 rows at K of 128 to 512).  The others:
   // of few rows the kernel that keeps many loads in flight instead of staging tiles, of more tiles of 128.
   const long long rows_per_group = group_offsets ? M / G : M;
-  const bool whole = dtype == HAL_BF16 && allow_mfma && aligned && !y_add && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 &&
+  const bool whole = dtype == HAL_BF16 && allow_mfma && aligned && !y_add && x_rows > 0 && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 &&
                      y_group_cols % 4 == 0 && (uintptr_t)Y % 16 == 0 && (long long)N * ldw * 2 < (1ll << 31) &&
-                     (long long)x_rows * ldx * 2 < (1ll << 31);
+                     ((long long)x_rows * ldx + K) * 2 < (1ll << 31);
   const bool plain = whole && group_offsets && gate == nullptr && x_group_cols == 0 && y_group_cols == 0;
   const bool heads = whole && !group_offsets && !W2 && row_src == nullptr && row_dst == nullptr && (act == 0 || gate == nullptr);
   const int stream_tiles = W2 ? (N + GT_COLS / 2 - 1) / (GT_COLS / 2) : (N + GT_COLS - 1) / GT_COLS;
