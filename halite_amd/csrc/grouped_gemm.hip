@@ -8,11 +8,16 @@
 // of a float32 gate (heads), or compute the clamped gated activation of two products
 // (experts: W the gate's weight, W2 the up projection's), write float32 or bf16, or add
 // into a float32 destination.  Accumulation is float32 throughout; a row's result depends
-// on that row alone.
+// on that row alone, up to the order in which the kernels add its terms.
 //
-// Two kernels: tiles of 64 x 64 on the vector units for any element type and any sizes,
-// and for bf16 operands whose addresses allow 16-byte loads tiles of 128 x 128 on the matrix
-// cores (v_mfma_f32_16x16x32_bf16), K staged through LDS in the instruction's operand order.
+// Five kernels.  For any element type and any sizes tiles of 64 x 64 on the vector units
+// (grouped_fma_kernel).  For bf16 operands whose addresses allow 16-byte loads the matrix cores
+// (v_mfma_f32_16x16x32_bf16): a kernel for at most 16 rows a group that reads both operands straight
+// from memory (grouped_skinny_kernel), and tiles of 128 x 128 staged through registers and LDS
+// (grouped_mfma_kernel).  Where moreover whole lines can go straight into LDS (K of whole 64s) and
+// results leave as vector stores: streaming tiles of 64 x 128 for experts of few rows and for heads
+// (grouped_stream_kernel), and tiles of up to 256 x 256 for prompts' experts (grouped_wide_kernel).
+// gg_experts_kernel says which of the four takes an expert's product, and why.
 #include "hal_common.h"
 #include "hal_api.h"
 #include <math.h>
@@ -38,6 +43,7 @@ struct GroupedArgs {
   int gate_group_cols, gate_cols;  // the gate of group g, column n: gate[row][g * gate_group_cols + (gate_cols ? n : 0)]
   float limit, alpha, up_shift;
   int act;  // without W2: 0 the product as it is, 1 the square of its positive part
+  int turn;  // the streaming tiles begin at different places of K
 };
 
 #define GG_ROWS 128  // rows of a workgroup's tile (what the tile offsets count in)
@@ -552,9 +558,10 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
                                         char* b2) {
   constexpr int AI = NI / 2, LOADS = AI + 4;
   const int steps = a.K / GW_TK;
-  // Workgroups begin at different places of K and go round: rows of W that lie a power of two apart, all
-  // read at one place of K at a time, meet in a few of the memory's channels.
-  const int begin = (n0 / (GATED ? GT_COLS / 2 : GT_COLS) * 7 + g * 13) % steps;
+  // Few rows: workgroups begin at different places of K and go round, since rows of W that lie a power of two
+  // apart, all read at one place of K at a time, meet in a few of the memory's channels.  (Prompts' products add in
+  // the order of K, as in the other tiles: their bits do not depend on which of the three the rows' number takes.)
+  const int begin = a.turn ? (n0 / (GATED ? GT_COLS / 2 : GT_COLS) * 7 + g * 13) % steps : 0;
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ gw_turn(lr % 16)) * 16;
   // (GATED: of every 32 W rows, a wave's, the first 16 are the gate's and the others the up projection's)
@@ -753,18 +760,60 @@ static long long gw_most_tiles(int M, int G, int rows) {
   return n < M ? n : M;
 }
 
-// Whether the streaming tiles of `rows` listed rows of G groups fill the chip badly (about as many groups
-// have rows as such a number of random picks meets): fewer than 144 tiles, which leave compute units without
-// one, or a round of two workgroups a unit just begun.  The kernel for few rows, whose workgroups are smaller,
-// then ends earlier.  One row of 4 of 16 groups of 4096 x 4096 (116 tiles): 30.0 us against 35.8, two (206
-// tiles) 50.5 / 44.0; of 6 of 64 of 1024 x 4096, gate and up (92 tiles) 27.9 / 34.3, two (176) 49.3 / 39.1;
-// 4096 x 1024, one (185): 14.1 / 11.5.  48 rows of 64 groups of 1024 x 4096, gate and up: 1.06 rounds, 116
-// us against 117; 4096 x 1024: 2.1 rounds, 58 / 61; with 72 rows, 1.36 and 2.7 rounds, 152 / 135 and 81 / 77.
-#define GT_FEWEST_TILES 144
-static bool gt_fills_badly(long long rows, int G, int col_tiles) {
-  const double reached = G * (1.0 - pow(1.0 - 1.0 / G, (double)rows));
-  const double tiles = reached * col_tiles, rounds = tiles / (2 * 256);
-  return tiles < GT_FEWEST_TILES || (rounds > 1.0 && rounds - floor(rounds) < 0.2);
+// Which kernel takes experts' products whose sizes and addresses allow any of them (bf16, loads and vector
+// stores without bounds): M listed rows of G groups, N x K weights.  All sides were timed on 2 to 512 groups
+// of 256 to 14,336 x 256 to 14,336, rows dealt to the groups at random.
+//
+// Up to 16 rows a group: the streaming tiles, but not where they fill the chip badly (about as many
+// groups have rows as M random picks meet).  Fewer of them than half of the compute units: 4 rows of 16
+// groups of 4096 x 4096 (116 tiles) 26.9 us against 26.3 of the kernel for few rows, whose workgroups are
+// smaller; 8192 x 4096, 2 of 8 groups (60) 42.5 / 36.4; 2048 x 512, 4 of 32 (61) 7.3 / 6.5, but 4608 x 4096,
+// 4 of 16 (131) 36.4 / 45.8.  Or the second or third round of two tiles a unit just begun, with less than a
+// row a group (the others are bound by the reads of all weights): 80 rows of 512 groups of 512 x 2048, gate
+// and up (1.16 rounds) 62.7 / 57.7, 64 of 128 of 768 x 2048 (1.18) 64.1 / 61.7, 48 of 64 of 4096 x 1024 (2.1)
+// 64.3 / 61.8; with a row or more in a group 0.99 to 0.57 of the other's time at any fraction of a round
+// (4608 x 4096, 16 groups, 1.12 rounds: 48 rows 122 / 124, 256 rows 124 / 192).
+//
+// From 48 rows a group on the wide tiles, one a unit, where they fill the chip: below five eighths of a
+// round, and where a second round has just begun, the streaming tiles end earlier (200 rows of each of
+// 8 groups of 1024 x 4096, gate and up, 64 wide tiles: 102 us against 61; 16 of 256 x 2048, 32: 47.6 / 18.0;
+// with 256 tiles, 16 of 4096 x 4096 at 200 rows: 0.69 of the streaming tiles' time), and
+// where those would be more than one and a half rounds over a long K, tiles of 128 in registers (4096 x
+// 14336, 8 groups at 200 rows: wide 356, streaming 395, 128: 328; 512 x 2048, 32 groups, gate and up: 62.8,
+// 61.8, 56.3; over a short K, 2048 x 256, 16 groups, they take twice the streaming tiles' time).
+// The kernel for few rows and the tiles of 128 take what the others' conditions leave.
+// (the tiles that a group of `rows` rows on average has: the rows vary by their root, so that a group of about
+// a tile's has one tile or two)
+static double gg_tiles_a_group(double rows, int tile) {
+  double n = 0;
+  for (double k = 0; tile * k < rows + 4 * sqrt(rows); k += 1) n += 0.5 * erfc((tile * k - rows) / sqrt(2 * rows));
+  return n;
+}
+#define GG_UNITS 256  // compute units of the gfx950 parts that this library is built for
+enum { GG_FEW_ROWS = 0, GG_STREAM = 1, GG_WIDE = 2, GG_TILES_128 = 3 };
+static int gg_experts_kernel(int M, int N, int K, int G, bool gated) {
+  const double rows = (double)M / G;
+  const bool stream = K % GW_TK == 0 && K >= 4 * GW_TK && N >= GT_COLS, wide = K % (2 * GW_TK) == 0 && N >= GW_COLS;
+  const int n_of = gated ? 2 * N : N;  // W rows that tiles are cut from
+  const int stream_cols = (n_of + GT_COLS - 1) / GT_COLS, wide_cols = (n_of + GW_COLS - 1) / GW_COLS;
+  if (M / G <= 16) {
+    const double tiles = G * (1.0 - pow(1.0 - 1.0 / G, (double)M)) * stream_cols, rounds = tiles / (2 * GG_UNITS);
+    const bool begun = M < G && rounds > 1.0 && rounds < 3.0 && rounds - floor(rounds) < 0.2;
+    return stream && tiles >= GG_UNITS / 2 && !begun ? GG_STREAM : GG_FEW_ROWS;
+  }
+  if (stream && M / G < GT_ROWS_A_GROUP) return GG_STREAM;
+  const double wide_tiles = G * gg_tiles_a_group(rows, GW_ROWS) * wide_cols;
+  const double stream_tiles = G * gg_tiles_a_group(rows, GT_ROWS) * stream_cols;
+  // (groups of many tiles make these lower where one more is needed, and the round begun is a short one)
+  const bool begun = rows < 2 * GW_ROWS && wide_tiles > 1.02 * GG_UNITS && wide_tiles < 1.1 * GG_UNITS;
+  const bool wide_fills = wide_tiles >= 0.625 * GG_UNITS && !begun;
+  if (wide && (wide_fills || !stream)) return GG_WIDE;
+  return stream && (stream_tiles <= 3 * GG_UNITS || K < 2048 || rows >= 512) ? GG_STREAM : GG_TILES_128;
+}
+
+// The choice above, for tests.
+extern "C" int hal_grouped_gemm_experts_kernel(int M, int N, int K, int G, int gated) {
+  return gg_experts_kernel(M, N, K, G, gated != 0);
 }
 
 extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_col0, const void* W,
@@ -807,39 +856,36 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
                        x_col0 % 8 == 0 && w_group_stride % 8 == 0 && ((uintptr_t)X % 16 == 0) &&
                        ((uintptr_t)W % 16 == 0) && (W2 == nullptr || (uintptr_t)W2 % 16 == 0);
   // Experts (rows listed by group) whose sizes and addresses are such that loads and vector stores need no
-  // bounds: of few rows the streaming tiles (ahead of the wide ones up to 40 to 75 rows a group: 196 / 196
-  // us at 37 rows of 64 experts of 1024 x 4096, 224 / 203 at 56; 139 / 142 at 75 rows of 16 of
-  // 4096 x 4096, 187 / 148 at 150), of more the wide ones; heads of more
-  // than 16 rows the streaming tiles (figures there; faster from 17 to 8,000 rows at K of 128 to 512).  The others:
-  // of few rows the kernel that keeps many loads in flight instead of staging tiles, of more tiles of 128.
+  // bounds take one of four kernels (gg_experts_kernel), heads of more than 16 rows the streaming tiles (figures
+  // there; faster from 17 to 8,000 rows at K of 64 to 512).  The others: of few rows the kernel that keeps many
+  // loads in flight instead of staging tiles, of more tiles of 128.
   const long long rows_per_group = group_offsets ? M / G : M;
   const bool whole = dtype == HAL_BF16 && allow_mfma && aligned && !y_add && x_rows > 0 && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 &&
                      y_group_cols % 4 == 0 && (uintptr_t)Y % 16 == 0 && (long long)N * ldw * 2 < (1ll << 31) &&
                      ((long long)x_rows * ldx + K) * 2 < (1ll << 31);
   const bool plain = whole && group_offsets && gate == nullptr && x_group_cols == 0 && y_group_cols == 0;
   const bool heads = whole && !group_offsets && !W2 && row_src == nullptr && row_dst == nullptr && (act == 0 || gate == nullptr);
-  const int stream_tiles = W2 ? (N + GT_COLS / 2 - 1) / (GT_COLS / 2) : (N + GT_COLS - 1) / GT_COLS;
-  if (plain && K % GW_TK == 0 && K >= 4 * GW_TK && N >= GT_COLS && rows_per_group < GT_ROWS_A_GROUP &&
-      !(rows_per_group <= 16 && gt_fills_badly(M, G, stream_tiles))) {
-    const int col_tiles = stream_tiles;
-    const long long units = gw_most_tiles(M, G, GT_ROWS) * col_tiles, blocks = 8 * ((units + 7) / 8);
+  const int stream_cols = ((W2 ? 2 * N : N) + GT_COLS - 1) / GT_COLS, wide_cols = ((W2 ? 2 * N : N) + GW_COLS - 1) / GW_COLS;
+  const int kernel = plain ? gg_experts_kernel(M, N, K, G, W2 != nullptr) : rows_per_group <= 16 ? GG_FEW_ROWS : GG_TILES_128;
+  a.turn = heads || rows_per_group < GT_ROWS_A_GROUP;
+  if (kernel == GG_STREAM) {
+    const long long units = gw_most_tiles(M, G, GT_ROWS) * stream_cols, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
-    else hipLaunchKernelGGL((grouped_stream_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, col_tiles);
+    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+    else hipLaunchKernelGGL((grouped_stream_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+  } else if (kernel == GG_WIDE) {
+    const long long units = gw_most_tiles(M, G, GW_ROWS) * wide_cols, blocks = 8 * ((units + 7) / 8);
+    HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
+    if (W2) hipLaunchKernelGGL(grouped_wide_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, a, wide_cols);
+    else hipLaunchKernelGGL(grouped_wide_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, a, wide_cols);
   } else if (heads && K % GW_TK == 0 && rows_per_group > 16) {
-    const long long units = (long long)((M + GT_ROWS - 1) / GT_ROWS) * G * stream_tiles, blocks = 8 * ((units + 7) / 8);
-    HAL_REQUIRE(blocks < (1ll << 31) && (long long)M * stream_tiles < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    hipLaunchKernelGGL((grouped_stream_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_tiles);
-  } else if (dtype == HAL_BF16 && allow_mfma && aligned && rows_per_group <= 16) {
+    const long long units = (long long)((M + GT_ROWS - 1) / GT_ROWS) * G * stream_cols, blocks = 8 * ((units + 7) / 8);
+    HAL_REQUIRE(blocks < (1ll << 31) && (long long)M * stream_cols < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
+    hipLaunchKernelGGL((grouped_stream_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+  } else if (dtype == HAL_BF16 && allow_mfma && aligned && kernel == GG_FEW_ROWS) {
     grid.x = W2 ? (N + 31) / 32 : (N + 63) / 64;
     if (W2) hipLaunchKernelGGL(grouped_skinny_kernel<true>, grid, dim3(256), 0, stream, a);
     else hipLaunchKernelGGL(grouped_skinny_kernel<false>, grid, dim3(256), 0, stream, a);
-  } else if (plain && K % (2 * GW_TK) == 0 && N >= GW_COLS) {
-    const int cols = W2 ? GW_COLS / 2 : GW_COLS, col_tiles = (N + cols - 1) / cols;
-    const long long units = gw_most_tiles(M, G, GW_ROWS) * col_tiles, blocks = 8 * ((units + 7) / 8);
-    HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    if (W2) hipLaunchKernelGGL(grouped_wide_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, a, col_tiles);
-    else hipLaunchKernelGGL(grouped_wide_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, a, col_tiles);
   } else if (dtype == HAL_BF16 && allow_mfma && aligned) {
     grid.x = W2 ? (N + GG_ROWS / 2 - 1) / (GG_ROWS / 2) : (N + GG_ROWS - 1) / GG_ROWS;
     if (W2) hipLaunchKernelGGL(grouped_mfma_kernel<true>, grid, dim3(256), 0, stream, a);

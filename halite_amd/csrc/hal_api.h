@@ -160,6 +160,9 @@ int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_col0, const
                      int src_div, const int* row_dst, const float* gate, int ldg, int gate_per_group,
                      float limit, float up_shift, float alpha, int act, int allow_mfma,
                      hipStream_t stream);
+// Which kernel takes M listed rows of G groups, N x K bf16 weights (gated: two of them), whose addresses and
+// strides allow any: 0 that for few rows a group, 1 the streaming tiles, 2 the wide tiles, 3 tiles of 128.
+int hal_grouped_gemm_experts_kernel(int M, int N, int K, int G, int gated);
 
 // ---- around a latent attention and a mixture of experts (latent_moe.hip) -----------------
 // RMSNorm of rows of the float32 stream (rows[r] or r) with one or two weights, x * rstd * w
