@@ -552,6 +552,9 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
 // 32 heads of K = 192, N = 128 with a gate: 17 rows 13.6 -> 8.0 us, 64 26.0 -> 9.6, 1,000 38.7 -> 15.2, 3,000
 // 51.6 -> 34.6 beside the tiles of 128 (K = 128, N = 192: 10.1 -> 6.6, 17.2 -> 7.7, 21.3 -> 15.5, 41.5 -> 36.4),
 // whose loads go through registers and wait for each other.
+// A K of one step has no loads on their way while another step is multiplied: 128 heads of 64 x 64, 4,000 rows 67.3 us
+// against 67.6, but 8,000 rows 131 / 121.
+#define GT_ONE_STEP_ROWS 4096
 typedef __attribute__((ext_vector_type(4), aligned(4))) float gt_f32x4_any;  // (a gate's rows begin at any float)
 template <bool GATED, bool HEADS, int NI>
 __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1,
@@ -857,7 +860,7 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
                        ((uintptr_t)W % 16 == 0) && (W2 == nullptr || (uintptr_t)W2 % 16 == 0);
   // Experts (rows listed by group) whose sizes and addresses are such that loads and vector stores need no
   // bounds take one of four kernels (gg_experts_kernel), heads of more than 16 rows the streaming tiles (figures
-  // there; faster from 17 to 8,000 rows at K of 64 to 512).  The others: of few rows the kernel that keeps many
+  // there; faster from 17 to 8,000 rows at K of 128 to 512).  The others: of few rows the kernel that keeps many
   // loads in flight instead of staging tiles, of more tiles of 128.
   const long long rows_per_group = group_offsets ? M / G : M;
   const bool whole = dtype == HAL_BF16 && allow_mfma && aligned && !y_add && x_rows > 0 && N % 4 == 0 && ldy % 4 == 0 && y_col0 % 4 == 0 &&
@@ -878,7 +881,7 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
     if (W2) hipLaunchKernelGGL(grouped_wide_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, a, wide_cols);
     else hipLaunchKernelGGL(grouped_wide_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, a, wide_cols);
-  } else if (heads && K % GW_TK == 0 && rows_per_group > 16) {
+  } else if (heads && K % GW_TK == 0 && rows_per_group > 16 && (K > GW_TK || M <= GT_ONE_STEP_ROWS)) {
     const long long units = (long long)((M + GT_ROWS - 1) / GT_ROWS) * G * stream_cols, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31) && (long long)M * stream_cols < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
     hipLaunchKernelGGL((grouped_stream_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);

@@ -97,3 +97,18 @@ def test_wide_tiles_that_fill_the_chip(n, k):
         xs, ws = x[a:b, 8 : 8 + k].double(), w[g].double()
         limit = (k + 8) * 2.0**-23 * (xs.abs() @ ws.abs().T)  # (the matrix cores need not round to nearest)
         assert bool(((y[to[a:b].long(), 4 : 4 + n].double() - xs @ ws.T).abs() <= limit).all()), g
+
+
+@pytest.mark.parametrize("rows", [4096, 4097])
+def test_heads_of_one_step(rows):
+    """Heads whose K is one step of the streaming tiles, at both sides of the rows from which tiles of 128 take them."""
+    heads, n, k = 3, 68, 64
+    gen = torch.Generator().manual_seed(rows)
+    x = torch.randn(rows, heads * k, generator=gen).bfloat16().cuda()
+    w = torch.randn(heads, n, k, generator=gen).bfloat16().cuda()
+    y = torch.empty(rows, heads * n, device="cuda")
+    ops.grouped_gemm(x, w, y, n_rows=rows, x_group_cols=k, y_group_cols=n)
+    for h in range(heads):
+        a, b = x[:, h * k : (h + 1) * k].double(), w[h].double()
+        limit = (k + 8) * 2.0**-23 * (a.abs() @ b.abs().T)  # (the matrix cores need not round to nearest)
+        assert bool(((y[:, h * n : (h + 1) * n].double() - a @ b.T).abs() <= limit).all())
