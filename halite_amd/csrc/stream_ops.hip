@@ -472,12 +472,17 @@ __global__ void streams_step_kernel(float* __restrict__ x, size_t copy_stride, i
 // The same in rows of a multiple of four elements: a thread keeps V groups of four of every copy, asks for
 // all of them before it writes any (above, a group's loads wait for the stores of the one before), and reads
 // nothing back from LDS.  The squares are summed in groups of 256 elements, which are added in their order:
-// the sum is the same for every V.  A row is a chain of two waits on memory, so a few rows take all the
-// threads there can be (V of 1 or 2); many rows take more in flight from fewer threads, and more rows a
-// compute unit (V of 4).  Measured on two copies of rows of 4,096 with an update, the norm and bfloat16 out:
-// 48 rows 19.2 -> 5.3 us, 2,250 rows 54.7 -> 37.1 us (204 MB).
+// the sum is the same for every V.  A row is a chain of two waits on memory, so it gets all the threads there
+// can be, one group each up to 1,024 of them.  Two groups each from half the threads where all rows then run at
+// once and would not otherwise (of up to two copies: more of them leave too few registers for as many rows).
+// Measured, captured launches one behind the other, with an update, the norm and bfloat16 out, beside the kernel
+// above: two copies of 4,096: 48 rows 11.6 -> 4.5 us, 768 rows 22.1 -> 14.0 (one group each 15.4), 2,048 40.8 ->
+// 35.5, 4,096 85.4 -> 63.1; of 1,024: 768 rows 8.1 -> 6.1; of 8,192: 48 rows 19.9 -> 6.1, 2,048 109.5 -> 65.7.
+// Four copies of 4,096: 48 rows 14.4 -> 6.1, 1,024 39.7 -> 35.4.  Eight copies of one group a thread leave registers for a
+// single row a compute unit: 48 rows of 4,096 took 25.0 -> 12.0 us so, but 900 rows 60.7 -> 65.1, and of 1,028 24.2 ->
+// 32.4, and a row's bits are not to depend on the number of rows.  More than four copies stay above.
 template <typename TO, int MAXS, int V>
-__global__ void __launch_bounds__(V == 4 ? 512 : 1024)
+__global__ void __launch_bounds__(1024)
 streams_step_vec_kernel(float* __restrict__ x, size_t copy_stride, int S, const float* __restrict__ y,
                         const void* __restrict__ mix, const void* __restrict__ outw, float m,
                         const void* __restrict__ inw, int c_dtype, int read, const void* __restrict__ norm_w,
@@ -571,8 +576,9 @@ streams_step_vec_kernel(float* __restrict__ x, size_t copy_stride, int S, const 
   }
 }
 
-#define STREAMS_VEC_MOST 8192   // the widest row of the vector kernel: 32 groups of 256
-#define STREAMS_FEW_ROWS 512    // up to here one or two groups of four a thread: two such rows a compute unit fit
+#define STREAMS_VEC_MOST 8192     // the widest row of the vector kernel: 32 groups of 256
+#define STREAMS_VEC_COPIES 4      // and the most copies
+#define STREAMS_AT_ONCE (1 << 19)  // threads that the chip runs at once: 256 compute units of 2,048
 extern "C" int hal_streams_step(float* x, long long copy_stride, int S, const float* y, const void* mix,
                                 const void* outw, float m, const void* inw, int c_dtype, int read,
                                 const void* norm_w, int norm_dtype, float offset, float eps, void* result,
@@ -587,29 +593,24 @@ extern "C" int hal_streams_step(float* x, long long copy_stride, int S, const fl
   HAL_REQUIRE(result_dtype == HAL_F32 || result_dtype == HAL_BF16, "hal_streams_step: dtype %d", result_dtype);
   if (n_rows == 0) return 0;
   const uintptr_t result_size = result_dtype == HAL_F32 ? 16 : 8, norm_size = norm_dtype == HAL_F32 ? 16 : 8;
-  if (W % 4 == 0 && W <= STREAMS_VEC_MOST && copy_stride % 4 == 0 && ((uintptr_t)x | (uintptr_t)y) % 16 == 0 &&
+  const long long nv = W / 4, groups = (long long)n_rows * nv;
+  if (W % 4 == 0 && W <= STREAMS_VEC_MOST && S <= STREAMS_VEC_COPIES && copy_stride % 4 == 0 && ((uintptr_t)x | (uintptr_t)y) % 16 == 0 &&
       (!read || (ld_result % 4 == 0 && (uintptr_t)result % result_size == 0 && (uintptr_t)norm_w % norm_size == 0))) {
-    const int nv = W / 4, per = n_rows > STREAMS_FEW_ROWS ? 4 : nv <= 1024 ? 1 : 2;
-    const int threads = ((nv + per - 1) / per + HAL_WAVE - 1) / HAL_WAVE * HAL_WAVE;
+    const int per = nv > 1024 || (S <= 2 && groups > STREAMS_AT_ONCE && groups <= 2 * STREAMS_AT_ONCE) ? 2 : 1;
+    const int threads = (int)((nv + per - 1) / per + HAL_WAVE - 1) / HAL_WAVE * HAL_WAVE;
 #define STREAMS_LAUNCH(T_, M_, V_)                                                                                   \
   hipLaunchKernelGGL((streams_step_vec_kernel<T_, M_, V_>), dim3(n_rows), dim3(threads), 0, stream, x,               \
                      (size_t)copy_stride, S, y, mix, outw, m, inw, c_dtype, read, read ? norm_w : nullptr, norm_dtype, \
                      offset, eps, (T_*)result, ld_result, rows, W)
-#define STREAMS_BY_COUNT(T_, V_)                \
-  do {                                          \
-    if (S <= 2) STREAMS_LAUNCH(T_, 2, V_);      \
-    else if (S <= 4) STREAMS_LAUNCH(T_, 4, V_); \
-    else STREAMS_LAUNCH(T_, 8, V_);             \
+#define STREAMS_BY_COUNT(T_)                                  \
+  do {                                                        \
+    if (S <= 2 && per == 1) STREAMS_LAUNCH(T_, 2, 1);         \
+    else if (S <= 2) STREAMS_LAUNCH(T_, 2, 2);                \
+    else if (per == 1) STREAMS_LAUNCH(T_, 4, 1);              \
+    else STREAMS_LAUNCH(T_, 4, 2);                            \
   } while (0)
-#define STREAMS_BY_ROWS(T_)                     \
-  do {                                          \
-    if (per == 1) STREAMS_BY_COUNT(T_, 1);      \
-    else if (per == 2) STREAMS_BY_COUNT(T_, 2); \
-    else STREAMS_BY_COUNT(T_, 4);               \
-  } while (0)
-    if (result_dtype == HAL_F32) STREAMS_BY_ROWS(float);
-    else STREAMS_BY_ROWS(bf16_t);
-#undef STREAMS_BY_ROWS
+    if (result_dtype == HAL_F32) STREAMS_BY_COUNT(float);
+    else STREAMS_BY_COUNT(bf16_t);
 #undef STREAMS_BY_COUNT
 #undef STREAMS_LAUNCH
     HAL_LAUNCH_CHECK();
