@@ -1227,8 +1227,11 @@ extern "C" int hal_attention_mfma_head_dim() { return D; }
 // units).  Other heads have no kernel for long segments: their tiles are one-tile items, 16 rows each.
 #define BIG_BUILT(VT0_) (D - 8 * (VT0_) <= 224)
 
+// whether the values' dimensions before value_from, zeros, are left out
+extern "C" int hal_attention_mfma_skips_zeros(int value_from) { return VT0_BUILT > 0 && value_from >= 16 * VT0_BUILT; }
+
 extern "C" int hal_attention_mfma_rows_per_big_item(int value_from) {
-  return (VT0_BUILT > 0 && value_from >= 16 * VT0_BUILT) || BIG_BUILT(0) ? 16 * RT_BIG : 16;
+  return hal_attention_mfma_skips_zeros(value_from) || BIG_BUILT(0) ? 16 * RT_BIG : 16;
 }
 
 // All arrays are device pointers.  `items` [max_items, 12] lists the work on segments of
@@ -1330,7 +1333,7 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
               "hal_attention_mfma: %d counters and the partial buffers do not serve %d items of %d "
               "kv heads", n_counters, max_items, K);
   HAL_REQUIRE(value_from >= 0 && value_from < D, "hal_attention_mfma: values from dimension %d on of %d", value_from, D);
-  if (VT0_BUILT > 0 && value_from >= 16 * VT0_BUILT) {
+  if (hal_attention_mfma_skips_zeros(value_from)) {
     if (max_items > 0) LAUNCH_ATTENTION(1, false, 32, 1, VT0_BUILT, items, max_items, counts)
     if (max_big > 0) LAUNCH_ATTENTION(RT_BIG, true, KB_BIG, HALVES_BIG, VT0_BUILT, big_items, max_big, counts + 1)
   } else {

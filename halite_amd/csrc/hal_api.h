@@ -433,6 +433,7 @@ int hal_wkv_step(const float* r, const float* k, const float* v, const float* ga
 // ---- the head-size-specific library (attention_mfma.hip) ---------------------------------
 int hal_attention_mfma_head_dim();
 int hal_attention_mfma_rows_per_big_item(int value_from);
+int hal_attention_mfma_skips_zeros(int value_from);
 // merge_parts: the most partial results that any merge item joins, or 0 if not known (the
 // kernel for many partials is taken then).  Items of both lists come in runs of four, a
 // workgroup's waves (max_items and max_big are multiples of four): the one-tile items of a

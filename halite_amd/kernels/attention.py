@@ -156,30 +156,41 @@ def rows_per_big_item(head_dim: int, value_from: int = 0) -> int:
     return int(library.attention_library(head_dim).hal_attention_mfma_rows_per_big_item(value_from))
 
 
+def skips_leading_zeros(head_dim: int, value_from: int) -> bool:
+    """Whether the kernels for this head size leave out the values' dimensions before ``value_from``."""
+    return bool(library.attention_library(head_dim).hal_attention_mfma_skips_zeros(value_from))
+
+
 # Heads of more than 128 dimensions: the kernel for long segments keeps the keys and values of a
 # block for 128 rows where the one for one-tile items reads them for 16, but its workgroups start and
-# end with more.  Measured on a latent's one key/value head of 256 (16 and 32 query heads): 18 against
-# 9 us at 128 tokens, 24 / 19 at 256, 27 / 24 and 28 / 45 at 512, 42 / 64 at 1,024, 190 / 785 at 3,000, and
-# with 4,096 tokens before them 30 / 24 and 34 / 38 at 64: the two meet at about six million (row, key)
-# pairs.  Heads with values in all dimensions have too few workgroups besides until there is one a
-# compute unit (160 dimensions, 2,048 tokens: 60 against 35 us with 128 workgroups, 59 / 79 with 256).
+# end with more.  Measured on a latent's one key/value head of 256 whose values begin behind 64 zeros, with 16 and
+# 32 query heads, us against one-tile items, launches captured one behind the other: 28 / 21 and 27 / 39 at 512
+# tokens, 40 / 55 and 43 / 109 at 1,024, 97 / 338 and 173 / 673 at 3,000; with 4,096 tokens before them 33 / 20 and
+# 36 / 32 at 64, 43 / 48 and 57 / 91 at 256: the two meet at about six million (row, key) pairs.
+# Where values are read in all dimensions a workgroup takes longer, and one a compute unit is needed besides: a
+# latent's one head of 160 and 64 query heads, 256 tokens behind 4,096 (128 workgroups) 106 / 100, of 224 206 / 172;
+# 16 key/value heads of 160, 1,024 tokens (128) 36 / 23, 2,048 (256) 59 / 62; 8 of 160, 4,096 tokens (256) 105 / 105,
+# of 224 192 / 187; 16 of 192, 2,048 tokens 63 / 105.
 LONG_ITEM_PAIRS = 6_000_000
 LONG_ITEM_ROWS = 128  # rows of such a workgroup
 
 
 def long_items_pay(seg_q_len, seg_kv_len, group_size: int, n_kv_heads: int, window: int, head_dim: int,
-                   value_from: int = 0) -> bool:
+                   value_from: int = 0, chunk: int = 0) -> bool:
     """Whether a step's long segments go to the kernel for long segments."""
     if head_dim <= 128:
         return True
     ql, kl = np.asarray(seg_q_len, dtype=np.int64), np.asarray(seg_kv_len, dtype=np.int64)
     keys = kl - ql // 2
-    if window > 0:
-        keys = np.minimum(keys, window)
+    for most in (window, chunk):
+        if most > 0:
+            keys = np.minimum(keys, most)
     rows = np.where(ql > 1, ql * group_size, 0)
     if int((rows * keys).sum()) * n_kv_heads < LONG_ITEM_PAIRS:
         return False
-    return value_from > 0 or int((-(-rows // LONG_ITEM_ROWS)).sum()) * n_kv_heads >= compute_units()
+    if skips_leading_zeros(head_dim, value_from):
+        return True
+    return int((-(-rows // LONG_ITEM_ROWS)).sum()) * n_kv_heads >= compute_units()
 
 
 def kept_units(keep: int) -> int:
