@@ -1263,7 +1263,8 @@ extern "C" int hal_attention_mfma(const void* q, int q_row_stride, void* out, in
 // the work lists name them.  `chunk`: the work lists must have been cut for it (a
 // tile's first key is no earlier than the start of its first row's chunk).  `bias_log2`:
 // float32 [H][bias_len], the bias by distance times log2 e.  `value_from`: the values' dimensions
-// before it are zeros on every page (they need not be read; the result's are zeros).
+// before it are zeros on every page (they need not be read; the result's are zeros; with kept keys
+// they are read, and the work lists are made for a value_from of 0: no layer has both).
 extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out_row_stride,
                                         const int* items, int max_items, const int* big_items,
                                         int max_big, const int* merges, int max_merges,
@@ -1318,7 +1319,7 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
     dim3 grid(((MAX) + waves - 1) / waves, K);                                                    \
     auto kernel = attention_mfma_kernel<RT_, false, false, SHARED_, false, KB_, HV_, false, false, VT_>; \
     if (ruled) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, true, false, VT_)                           \
-    else if (keep > 0) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, true, VT_)                   \
+    else if (keep > 0) PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, VT_ == 0, VT_)               \
     else PICK_ATTENTION(RT_, SHARED_, KB_, HV_, false, false, VT_)                                \
     hipLaunchKernelGGL(kernel, grid, dim3(waves * HAL_WAVE * HV_), 0, stream, (const bf16_t*)q,   \
                        q_row_stride, (bf16_t*)out, out_row_stride, LIST, COUNT, seg_q_start,      \
@@ -1333,7 +1334,7 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
               "hal_attention_mfma: %d counters and the partial buffers do not serve %d items of %d "
               "kv heads", n_counters, max_items, K);
   HAL_REQUIRE(value_from >= 0 && value_from < D, "hal_attention_mfma: values from dimension %d on of %d", value_from, D);
-  if (hal_attention_mfma_skips_zeros(value_from)) {
+  if (keep == 0 && hal_attention_mfma_skips_zeros(value_from)) {
     if (max_items > 0) LAUNCH_ATTENTION(1, false, 32, 1, VT0_BUILT, items, max_items, counts)
     if (max_big > 0) LAUNCH_ATTENTION(RT_BIG, true, KB_BIG, HALVES_BIG, VT0_BUILT, big_items, max_big, counts + 1)
   } else {

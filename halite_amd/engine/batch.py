@@ -191,7 +191,7 @@ class StepContext:
             return
         if self._dev is not None and not late:
             return
-        value_from = getattr(self.cache.groups[group_id].need, "value_from", 0)
+        value_from = 0 if keep else getattr(self.cache.groups[group_id].need, "value_from", 0)
         rows_big = attention_kernels.rows_per_big_item(head_dim, value_from)
         lens = (self.seg_q_len_host, self.seg_kv_len_host, n_heads // n_kv_heads, n_kv_heads, window)
         if not attention_kernels.long_items_pay(*lens, head_dim, value_from, chunk):

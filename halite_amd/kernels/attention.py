@@ -495,7 +495,7 @@ def attention_mfma(q, q_row_stride, plan_dev, ctx, group, kv, n_heads, scale, wi
         P(group.block_table), group.block_table.shape[1], P(kv.k), P(kv.v), P(part_o), P(part_ml),
         P(counters), N_COUNTERS, n_heads, n_kv, head_dim, page_size, 1 if getattr(kv, "tiled", False) else 0,
         ctypes.c_float(scale), window, rule.chunk, P(bias), 0 if bias is None else bias.shape[1],
-        rule.weights_code(), ctypes.c_float(rule.softcap), P(sinks), rule.keep, getattr(kv, "value_from", 0),
+        rule.weights_code(), ctypes.c_float(rule.softcap), P(sinks), rule.keep, 0 if rule.keep else getattr(kv, "value_from", 0),
         plan.max_parts, ops._stream(),
     )
     ops._check(lib, rc)

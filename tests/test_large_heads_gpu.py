@@ -70,7 +70,8 @@ SEGS = [[(0, 1)], [(0, 70)], [(63, 1), (0, 33), (64, 64), (129, 2), (200, 1)], [
 def test_values_that_begin_behind_zeros(H, K, segs):
     gpu = torch.device("cuda:0")
     for page, window, tiled in ((16, 0, False), (64, 0, True), (24, 0, False), (64, 300, True), (64, 37, False)):
-        case(gpu, H, K, 256, page, segs, window, tiled, FROM, 50, poison=True)
+        n_big = case(gpu, H, K, 256, page, segs, window, tiled, FROM, 50, poison=True)
+        assert len(n_big) == 2 and (max(n_big) > 0) == any(new > 1 and new * (H // K) > 16 for _, new in segs)
 
 
 @pytest.mark.gpu
