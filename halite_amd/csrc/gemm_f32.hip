@@ -489,6 +489,15 @@ static double mf_rounds_cost(long long tiles_m, int N, int BN) {
   return n <= 1 ? 125 : n <= 2 ? 183 : 83 * n;
 }
 
+// The columns of the tiles that M rows by N columns take on the matrix cores (100 rows and fewer: see below).
+extern "C" int hal_gemm_f32_tile_columns(int M, int N) {
+  const long long tiles_m = (M + MF_BM - 1) / MF_BM;
+  int bn = 128;
+  for (int other = 64; other >= 32; other /= 2)
+    if (mf_rounds_cost(tiles_m, N, other) < mf_rounds_cost(tiles_m, N, bn)) bn = other;
+  return bn;
+}
+
 extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
                             int M, int N, int K, hipStream_t stream) {
   HAL_REQUIRE(M >= 0 && N > 0 && K > 0, "hal_gemm_f32: bad sizes M=%d N=%d K=%d", M, N, K);
@@ -518,11 +527,8 @@ extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, fl
       return 0;
     }
     // more rows: the matrix cores, in the tiles whose rounds over the compute units are expected to end first
-    const long long tiles_m = (M + MF_BM - 1) / MF_BM;
-    int bn = 128;
-    for (int other = 64; other >= 32; other /= 2)
-      if (mf_rounds_cost(tiles_m, N, other) < mf_rounds_cost(tiles_m, N, bn)) bn = other;
-    const long long tiles_n = (N + bn - 1) / bn;
+    const int bn = hal_gemm_f32_tile_columns(M, N);
+    const long long tiles_m = (M + MF_BM - 1) / MF_BM, tiles_n = (N + bn - 1) / bn;
     HAL_REQUIRE(tiles_m * tiles_n < (1ll << 31), "hal_gemm_f32: M=%d N=%d exceed the grid limit", M, N);
     const dim3 tiles((unsigned)(tiles_m * tiles_n));
     if (bn == 128)

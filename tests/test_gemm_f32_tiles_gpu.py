@@ -4,15 +4,16 @@ columns that end inside a tile, against the product in 64 bits."""
 import pytest
 import torch
 
-from halite_amd.kernels import ops
+from halite_amd.kernels import library, ops
 
 pytestmark = pytest.mark.gpu
 
 
-# 130 x 4,000: tiles of 32 (one round); 300 x 4,100 and 500 x 4,090: of 64 (one round); 260 x 28,004: of
-# 128; 700 x 4,033: of 32 (three rounds); 1,030 x 4,161: of 64 (three rounds)
-@pytest.mark.parametrize("m, n, k", [(130, 4000, 36), (300, 4100, 1028), (500, 4090, 544), (260, 28004, 64), (700, 4033, 96), (1030, 4161, 512)])
-def test_tiles(m, n, k):
+# tiles of 32 in one, three and five rounds, of 64 in one and three, and of 128
+@pytest.mark.parametrize("m, n, k, columns", [(130, 4000, 36, 32), (300, 4100, 1028, 64), (500, 4090, 544, 64), (260, 28004, 64, 128),
+                                              (700, 4033, 96, 32), (1030, 4161, 512, 32), (1500, 4090, 1028, 64)])
+def test_tiles(m, n, k, columns):
+    assert library.core_library().hal_gemm_f32_tile_columns(m, n) == columns
     gen = torch.Generator().manual_seed(m)
     a, w = torch.randn(m, k, generator=gen).cuda(), torch.randn(n, k, generator=gen).cuda()
     got = ops.gemm_f32(a, w).double()

@@ -79,20 +79,23 @@ def test_which_kernel():
 EDGES = 3 * [0, 1, 33, 64, 65, 128, 129, 160, 0, 161, 192, 193, 224, 225, 255, 256, 257, 512, 513, 545, 2049, 0]
 
 
-@pytest.mark.parametrize("n, k", [(260, 384), (512, 256)])
-def test_wide_tiles_that_fill_the_chip(n, k):
+@pytest.mark.parametrize("n, k, kernel", [(260, 384, WIDE), (512, 256, WIDE), (132, 320, STREAM)])
+def test_tiles_of_prompts(n, k, kernel):
+    """Against 64 bits; and the bits of the tiles of 128, which a result that begins at an odd column gets."""
     ends = [0, *torch.tensor(EDGES).cumsum(0).tolist()]
     rows = ends[-1]
-    assert kernel_of(rows, n, k, len(EDGES)) == WIDE
+    assert kernel_of(rows, n, k, len(EDGES)) == kernel
     gen = torch.Generator().manual_seed(n)
     x = torch.randn(rows, k + 24, generator=gen).bfloat16().cuda()
     w = (0.1 * torch.randn(len(EDGES), n, k, generator=gen)).bfloat16().cuda()
     to = torch.randperm(rows, generator=gen).int().cuda()
     tiles = [0, *(-(-torch.tensor(EDGES) // ops.GROUP_TILE_ROWS)).cumsum(0).tolist()]
-    y = torch.full((rows, n + 12), 7.0, device="cuda")
-    ops.grouped_gemm(x, w, y, n_rows=rows, x_col0=8, y_col0=4, group_offsets=torch.tensor(ends).int().cuda(),
-                     tile_offsets=torch.tensor(tiles).int().cuda(), row_dst=to)
+    y, general = (torch.full((rows, n + 12), 7.0, device="cuda") for _ in range(2))
+    how = dict(n_rows=rows, x_col0=8, group_offsets=torch.tensor(ends).int().cuda(), tile_offsets=torch.tensor(tiles).int().cuda(), row_dst=to)
+    ops.grouped_gemm(x, w, y, y_col0=4, **how)
+    ops.grouped_gemm(x, w, general, y_col0=5, **how)
     assert bool((y[:, :4] == 7).all()) and bool((y[:, 4 + n :] == 7).all())
+    assert torch.equal(y[:, 4 : 4 + n], general[:, 5 : 5 + n])
     for g, (a, b) in enumerate(zip(ends, ends[1:])):
         xs, ws = x[a:b, 8 : 8 + k].double(), w[g].double()
         limit = (k + 8) * 2.0**-23 * (xs.abs() @ ws.abs().T)  # (the matrix cores need not round to nearest)

@@ -1,6 +1,6 @@
-"""The experts' products: of prompts (``grouped_wide_kernel``, tiles of up to 256 rows whose height
-follows the groups' sizes) and of few rows a group (``grouped_stream_kernel``), against the products in
-64 bits."""
+"""The experts' products: of prompts (tiles of up to 256 rows whose height follows the groups' sizes, and
+streaming tiles where those would not fill the chip) and of few rows a group (streaming tiles, and the
+kernel for few rows), against the products in 64 bits."""
 
 import pytest
 import torch
@@ -19,7 +19,7 @@ def gpu():
 # 192, 224, 256 rows), of a second, third and ninth tile (a panel of eight and one more), and a group whose
 # equal heights in steps of 32 leave its last tile short
 EDGES = [0, 1, 33, 64, 65, 128, 129, 160, 0, 161, 192, 193, 224, 225, 255, 256, 257, 512, 513, 545, 2049, 0]
-# fewer than 48 a group on average: the streaming tiles; none, one, at both sides of 32 and 64 rows, several tiles
+# fewer than 48 a group on average: the streaming tiles (the long list of single rows: the kernel for few rows); none, one, at both sides of 32 and 64 rows, several tiles
 FEW = [0, 1, 31, 32, 33, 0, 63, 64, 65, 0, 0, 97, 129, 2, 16, 17, 0, 0, 200, 0]
 
 
@@ -89,8 +89,8 @@ def test_up_products_gather_rows(gpu, act, counts, n, k):
 
 
 def test_a_row_does_not_depend_on_its_neighbours(gpu):
-    """The same rows in groups of other sizes, and through the kernel for tiles of 128 (K that is no multiple
-    of 128 takes it: the added columns are zeros), give the same bits."""
+    """The same rows in groups of other sizes, and with a K of another number of steps (the added columns are
+    zeros), give the same bits."""
     n, k, rows = 256, 256, 700
     x, w = rand(rows, k, seed=7).bfloat16().to(gpu), rand(1, n, k, seed=8, scale=0.1).bfloat16().to(gpu)
     whole = torch.empty((rows, n), device=gpu)
