@@ -1221,10 +1221,12 @@ extern "C" int hal_attention_mfma_head_dim() { return D; }
 // Tiles of leading zeros in the values that there is a build for beside none (see VT0).
 #define VT0_BUILT (D == 256 ? 4 : 0)
 
-// The sums and queries of two tiles and two waves a SIMD fit the registers up to 224 dimensions, and at
-// 256 if a quarter of the values' are zeros (one wave a SIMD instead was slower than the kernel
+// The sums and queries of two tiles and two waves a SIMD fit the registers up to 192 dimensions; at 208, 224 and
+// 256 with a quarter of the values' dimensions zeros the builds spill 2 to 33 of them, which costs less than one-tile
+// items do (16 key/value heads, 2,048 tokens, us against one-tile items: 208 dimensions 72 / 163, 224 103 / 120; 32 heads over 8,
+// 4,096 tokens: 208 274 / 1,084, 224 397 / 704).  At 256 without zeros (one wave a SIMD instead was slower than the kernel
 // without LDS on eight heads of 2,048 tokens, where its workgroups are half as many as the chip has
-// units).  Other heads have no kernel for long segments: their tiles are one-tile items, 16 rows each.
+// units) and at 240 there is no kernel for long segments: their tiles are one-tile items, 16 rows each.
 #define BIG_BUILT(VT0_) (D - 8 * (VT0_) <= 224)
 
 // whether the values' dimensions before value_from, zeros, are left out

@@ -770,11 +770,11 @@ static long long gw_most_tiles(int M, int G, int rows) {
 // Up to 16 rows a group: the streaming tiles, but not where they fill the chip badly (about as many
 // groups have rows as M random picks meet).  Fewer of them than half of the compute units: 4 rows of 16
 // groups of 4096 x 4096 (116 tiles) 26.9 us against 26.3 of the kernel for few rows, whose workgroups are
-// smaller; 8192 x 4096, 2 of 8 groups (60) 42.5 / 36.4; 2048 x 512, 4 of 32 (61) 7.3 / 6.5, but 4608 x 4096,
+// smaller; 4096 x 8192, 2 of 8 groups (60) 42.5 / 36.4; 2048 x 512, 4 of 32 (61) 7.3 / 6.5, but 4608 x 4096,
 // 4 of 16 (131) 36.4 / 45.8.  Or the second or third round of two tiles a unit just begun, with less than a
 // row a group (the others are bound by the reads of all weights): 80 rows of 512 groups of 512 x 2048, gate
 // and up (1.16 rounds) 62.7 / 57.7, 64 of 128 of 768 x 2048 (1.18) 64.1 / 61.7, 48 of 64 of 4096 x 1024 (2.1)
-// 64.3 / 61.8; with a row or more in a group 0.99 to 0.57 of the other's time at any fraction of a round
+// 64.3 / 61.8; with a row or more in a group 1.02 to 0.57 of the other's time at any fraction of a round
 // (4608 x 4096, 16 groups, 1.12 rounds: 48 rows 122 / 124, 256 rows 124 / 192).
 //
 // From 48 rows a group on the wide tiles, one a unit, where they fill the chip: below five eighths of a
@@ -783,7 +783,7 @@ static long long gw_most_tiles(int M, int G, int rows) {
 // with 256 tiles, 16 of 4096 x 4096 at 200 rows: 0.69 of the streaming tiles' time), and
 // where those would be more than one and a half rounds over a long K, tiles of 128 in registers (4096 x
 // 14336, 8 groups at 200 rows: wide 356, streaming 395, 128: 328; 512 x 2048, 32 groups, gate and up: 62.8,
-// 61.8, 56.3; over a short K, 2048 x 256, 16 groups, they take twice the streaming tiles' time).
+// 61.8, 56.3; over a short K, 2048 x 256, 16 groups: 20.4, 18.2, 25.6).
 // The kernel for few rows and the tiles of 128 take what the others' conditions leave.
 // (the tiles that a group of `rows` rows on average has: the rows vary by their root, so that a group of about
 // a tile's has one tile or two)

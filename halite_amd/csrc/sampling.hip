@@ -377,8 +377,8 @@ __device__ __forceinline__ int part_share(int V) { return ((V + ROW_PARTS - 1) /
 // The logits begin + tid, begin + tid + PART_THREADS, ... below `end`, PART_BATCH of them asked for
 // before the first is worked on (a share of a vocabulary of up to 131,072 is one batch): these passes are
 // bound by the trips to memory, which a load at a time takes one after the other.  64 rows of 128,256 with
-// top-p: a pass over the rows 10.6 -> 9.0 us, the first one, which keeps its batch, 20.9 -> 13.8 us, a
-// histogram 19.4 -> 12.2 us on average (where it also leaves out what the row does not search by).  Places of the
+// top-p: a pass over the rows 10.6 -> 10.1 us, the first one, which keeps its batch, 20.9 -> 15.1 us, a
+// histogram 19.4 -> 12.7 us on average (where it also leaves out what the row does not search by).  Places of the
 // batch that lie past the share are passed over by all threads at once: worked through by none of them, 200 rows
 // of 1,000 logits without filters took 23.0 us, of 32,000 29.9, and take 16.5 and 23.4 so.
 #define PART_BATCH 16
