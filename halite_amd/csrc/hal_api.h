@@ -285,6 +285,17 @@ int hal_delta_rule(const float* r, int ldr, const float* k, int ldk, const float
                    float unit_eps, float* pre, float* state, const int* seg_q_start,
                    const int* seg_q_len, const int* token_slot, float* o, int n_tokens, int n_segs,
                    int H, int D, hipStream_t stream);
+// The same in chunks of 16 tokens on the matrix cores, with the heads' norm, weight and gate:
+// out[t] = norm over each head of o[t], times weight [H * D], times sigmoid(z) (delta_chunks.hip).
+// records: scratch of hal_delta_chunks_room floats; hal_delta_chunks_fit says which sizes it takes.
+int hal_delta_chunks_fit(int D, float decay_rate, const float* v, int ldv, const float* z, int ldz);
+long long hal_delta_chunks_room(int n_tokens, int n_segs, int H);
+int hal_delta_chunks(const float* r, int ldr, const float* k, int ldk, const float* v, int ldv, const float* a_raw,
+                     int lda, const float* x1, int ldx1, const void* w2, const void* w0, const void* a_bias,
+                     int w_dtype, int lora, float decay_rate, float unit_eps, float* records, float* state,
+                     const int* seg_q_start, const int* seg_q_len, const int* token_slot, const float* z, int ldz,
+                     const void* weight, int weight_dtype, float eps, void* out, int dtype, int n_tokens, int n_segs,
+                     int H, int D, hipStream_t stream);
 // What takes the requests' states through their chunks: S <- decays[c][h] S + sums[c][h] chunk by chunk of
 // a segment, leaving in sums the state that each chunk starts from (NP numbers a head).
 int hal_ssd_carry(float* state, float* sums, const float* decays, const int* seg_chunks, const int* seg_q_start,

@@ -49,6 +49,7 @@ CORE_SOURCES = [
     "recurrent.hip",
     "decay_chunks.hip",
     "delta_rule.hip",
+    "delta_chunks.hip",
     "time_mix.hip",
 ]
 ATTENTION_SOURCES = ["runtime.hip", "attention_mfma.hip"]

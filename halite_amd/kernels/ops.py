@@ -1308,6 +1308,9 @@ def gated_part_norm(y: torch.Tensor, z: torch.Tensor, weight: torch.Tensor, eps:
 
 # -- the generalized delta rule; copies of the stream; per-head norms and gates -------------------
 
+DELTA_CHUNK_TOKENS = 8  # tokens a segment, on average, from which on chunks beat the walk token by token
+DELTA_CHUNK_GROUPS = 512  # (segment, head) pairs up to which they do whatever the segments' lengths
+
 
 def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch.Tensor, x1: torch.Tensor,
                w2: torch.Tensor, w0: torch.Tensor, a_bias: torch.Tensor, state: torch.Tensor,
@@ -1343,6 +1346,49 @@ def delta_rule(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch.T
         ctypes.c_float(decay_rate), ctypes.c_float(unit_eps), _ptr(pre), _ptr(state), _ptr(seg_q_start),
         _ptr(seg_q_len), _ptr(token_slot), _ptr(o), n, seg_q_start.numel(), heads, d, _stream()))
     return o
+
+
+def delta_chunks_fit(v: torch.Tensor, z: torch.Tensor, n_segs: int, heads: int, dim: int, decay_rate: float) -> bool:
+    """Whether ``delta_rule`` and ``head_norm_gate`` over values ``v`` and gates ``z`` are better made by ``delta_chunks``:
+    where it has a kernel, and a segment's chunk, which costs the same for one token as for sixteen, is filled or the
+    segments' workgroups are two a compute unit at most."""
+    # (64 heads, both sides in us: 4 segments of 4 tokens 34 / 24; 8 of which one has 9 tokens and the others one 33 / 31;
+    # 16 of 4 37 / 49, of 8 47 / 50, of 16 62 / 50; 64 of 6 139 / 128, of 12 204 / 129; 63 of one beside one of 200 681 / 293)
+    if not (n_segs * heads <= DELTA_CHUNK_GROUPS or v.shape[0] >= DELTA_CHUNK_TOKENS * n_segs):
+        return False
+    return bool(library.core_library().hal_delta_chunks_fit(dim, ctypes.c_float(decay_rate), _ptr(v), v.stride(0), _ptr(z), z.stride(0)))
+
+
+def delta_chunks(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch.Tensor, x1: torch.Tensor,
+                 w2: torch.Tensor, w0: torch.Tensor, a_bias: torch.Tensor, state: torch.Tensor,
+                 seg_q_start: torch.Tensor, seg_q_len: torch.Tensor, token_slot: torch.Tensor,
+                 decay_rate: float, unit_eps: float, z: torch.Tensor, weight: torch.Tensor, eps: float,
+                 out_dtype: torch.dtype) -> torch.Tensor:
+    """``head_norm_gate(delta_rule(...), z, weight, eps, heads, out_dtype)`` in chunks of tokens as float32 products
+    on the matrix cores, for the sizes that ``delta_chunks_fit`` names."""
+    lib = library.core_library()
+    _, heads, d, d2 = state.shape
+    n, inner, lora, n_segs = r.shape[0], heads * d, x1.shape[1], seg_q_start.numel()
+    for t, what in ((r, "r"), (k, "k"), (v, "v"), (a_raw, "a"), (z, "z")):
+        _rows_f32(t, inner, f"delta_chunks {what}")
+        _need(t.shape[0] == n, "delta_chunks: one row a token")
+    _rows_f32(x1, lora, "delta_chunks x1")
+    _dev(w2, w0, a_bias, state, seg_q_start, seg_q_len, token_slot, weight)
+    _i32(seg_q_start, "seg_q_start"), _i32(seg_q_len, "seg_q_len"), _i32(token_slot, "token_slot")
+    _need(state.dtype == torch.float32 and d == d2, "delta_chunks: a float32 state [slots, heads, dim, dim]")
+    _need(w2.shape == (inner, lora) and w0.numel() == inner and a_bias.numel() == inner
+          and w2.dtype == w0.dtype == a_bias.dtype, "delta_chunks: w2 [heads * dim, rank], w0 and a_bias [heads * dim] of one type")
+    _need(token_slot.numel() == n and n_segs == seg_q_len.numel() and weight.numel() == inner, "delta_chunks: the step's arrays")
+    lib.hal_delta_chunks_room.restype = ctypes.c_longlong
+    records = torch.empty(lib.hal_delta_chunks_room(n, n_segs, heads), dtype=torch.float32, device=r.device)
+    out = torch.empty((n, inner), dtype=out_dtype, device=r.device)
+    _check(lib, lib.hal_delta_chunks(
+        _ptr(r), r.stride(0), _ptr(k), k.stride(0), _ptr(v), v.stride(0), _ptr(a_raw), a_raw.stride(0),
+        _ptr(x1), x1.stride(0), _ptr(w2), _ptr(w0), _ptr(a_bias), dtype_code(w2.dtype), lora,
+        ctypes.c_float(decay_rate), ctypes.c_float(unit_eps), _ptr(records), _ptr(state), _ptr(seg_q_start),
+        _ptr(seg_q_len), _ptr(token_slot), _ptr(z), z.stride(0), _ptr(weight), dtype_code(weight.dtype),
+        ctypes.c_float(eps), _ptr(out), dtype_code(out_dtype), n, n_segs, heads, d, _stream()))
+    return out
 
 
 def head_norm_gate(y: torch.Tensor, z: torch.Tensor | None, weight: torch.Tensor | None, eps: float, heads: int,

@@ -92,7 +92,11 @@ class GeneralDelta(Mixer):
         a = ops.linear(x, self.w_in, out_dtype=torch.float32, tiled=self.t_in)
         r, k, v, a_raw, gate = (a[:, i * n : (i + 1) * n] for i in range(5))
         x1 = a[:, 5 * n :]
-        o = ops.delta_rule(r, k, v, a_raw, x1, self.w_decay_up_weight, self.w_decay_bias, self.w_a_bias,
-                           run.state["state"], ctx.seg_q_start, ctx.seg_q_len, ctx.token_slot, p.decay_rate, p.unit_eps)
-        y = ops.head_norm_gate(o, gate, self.w_norm_weight, p.eps, p.n_heads, x.dtype)
+        rule = (r, k, v, a_raw, x1, self.w_decay_up_weight, self.w_decay_bias, self.w_a_bias,
+                run.state["state"], ctx.seg_q_start, ctx.seg_q_len, ctx.token_slot, p.decay_rate, p.unit_eps)
+        n_segs = ctx.seg_q_start.numel()
+        if n_segs < x.shape[0] and ops.delta_chunks_fit(v, gate, n_segs, p.n_heads, p.head_dim, p.decay_rate):
+            y = ops.delta_chunks(*rule, gate, self.w_norm_weight, p.eps, x.dtype)
+        else:
+            y = ops.head_norm_gate(ops.delta_rule(*rule), gate, self.w_norm_weight, p.eps, p.n_heads, x.dtype)
         return ops.linear(y, self.w_out_weight, out_dtype=torch.float32, tiled=self.t_out)
