@@ -133,12 +133,12 @@ int hal_sample_unfiltered(const float* logits, int ld, int n_rows, int V, const 
 
 // Rows with filters spread over 32 blocks a pass.  any_late: some row has top-k, top-p and
 // min-p all at once (searched twice).  parts: n_rows * 32 * 4 floats; kept: n_rows * 32
-// floats; state: n_rows * 20 words; hist: n_rows * 2 * 2048 64-bit words.
+// floats; state: n_rows * 6 words; hist: n_rows * 2 * 256 64-bit words; lists: n_rows * V words.
 int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const float* temperature,
                       const int* top_k, const float* top_p, const float* min_p,
                       const uint64_t* seeds, const int* draw_index, float* parts, float* kept,
-                      void* state, void* hist, int any_late, int* out_token, float* out_logprob,
-                      hipStream_t stream);
+                      void* state, void* hist, uint32_t* lists, int any_late, int* out_token,
+                      float* out_logprob, hipStream_t stream);
 
 // ---- products in groups (grouped_gemm.hip) ---------------------------------------------
 // Y_g = X_g * W_g^T for G groups in one launch, float32 accumulation; operands of `dtype`.

@@ -587,49 +587,127 @@ row_join_kernel(const float* __restrict__ logits, int ld, int V, const float* __
 }
 
 // ---- rows with filters, spread over many blocks -----------------------------------------
-// The one-block kernel above spends most of its time in the first histogram: a row's keys
-// crowd into a few dozen of the 2,048 bins, and a block's atomics on one bin wait for each
-// other.  Here a row's keys are split over ROW_PARTS blocks for every pass; a block builds
-// its histogram in LDS and adds the bins it has filled to the row's histogram in memory
-// (integers: the order does not matter), and a one-block kernel per row walks that histogram
-// exactly as the kernel above walks its own.  Thresholds are therefore the same keys as
-// there; the drawn token may differ where the draw is within rounding of a token's edge,
-// since the kept masses are added in another order.  A row with top-k, top-p and min-p all
-// at once, where top-p refers to what top-k kept, is searched twice: top-k first, then (the
-// `late` passes) the mass that top-k kept and top-p within it.
+// A row's passes are shared by ROW_PARTS blocks each; what a pass over 64 rows of 128,256 costs is its
+// launch, the logits' way from memory (33 MB, 6.5 us) and about fifty instructions a logit where it takes
+// an exponential.  So a row is passed over four times, and once with its share alone:
+//   filt_max_kernel     its maximum;
+//   filt_coarse_kernel  the sum of exponentials, and how many logits and what mass lie in each of 256 bins of
+//                       the distance from the maximum (an eighth wide; the last takes the rest);
+//   filt_list_kernel    the keys in the bin that holds the threshold, as a list in memory;
+//   filt_find_kernel    (a block a row) the threshold among them, by radix selection over the bits in which
+//                       they differ;
+//   filt_mass_kernel    the kept mass of every share;
+//   filt_pick_kernel    the draw.
+// Distances are monotone in the keys, so the bins hold the keys in order, and counts and masses are integers: the
+// thresholds are the same keys as the one-block kernel's.  The drawn token may differ where the draw is within
+// rounding of a token's edge, since the kept masses are added in another order.  A row with top-k, top-p and min-p
+// all at once, where top-p refers to what top-k kept, is searched twice: top-k first, then (`late`) top-p
+// of the mass that top-k kept.
+// Before (three levels of 2,048 bins of the keys' bits, ten launches): 64 rows of 128,256 with top-p 112 us of kernels,
+// now 13.1 + 15.5 + 12.1 + 11.9 + 10.5 + 8.2 = 71.
 struct FiltRow {
-  float m, total;  // maximum of z and sum of exp(z - m) over the row
-  int best;        // first index of the maximum
-  int flags;       // FILT_*
-  uint32_t prefix[2];
+  float m;        // maximum of z
+  int best;       // its first index
+  int listed;     // keys in the row's list
   uint32_t key_min;
-  uint32_t unused;
-  unsigned long long above[2], target[2];
   unsigned long long kept_by_k;  // late rows: the mass of the keys that top-k kept
-  unsigned long long unused2;
 };
-static_assert(sizeof(FiltRow) == 80, "FiltRow is 20 words");
+static_assert(sizeof(FiltRow) == 24, "FiltRow is 6 words");
+#define FILT_BINS 256
 // greedy; top-k is searched; top-p is searched beside it; top-p is searched after it (late)
 enum { FILT_GREEDY = 1, FILT_K = 2, FILT_P = 4, FILT_P_LATE = 8 };
 
-__device__ __forceinline__ int level_shift(int level) { return level == 0 ? 21 : (level == 1 ? 10 : 0); }
-__device__ __forceinline__ int level_up(int level) { return level == 0 ? 32 : (level == 1 ? 21 : 10); }
+struct FiltParams {
+  const float *temperature, *top_p, *min_p;
+  const int* top_k;
+};
 
-__global__ void __launch_bounds__(HAL_WAVE)
-filt_join_kernel(const float* __restrict__ parts, const float* __restrict__ temperature,
-                 const int* __restrict__ top_k, const float* __restrict__ top_p,
-                 const float* __restrict__ min_p, int V, FiltRow* __restrict__ rows,
-                 unsigned long long* __restrict__ hist) {
-  const int row = blockIdx.x, lane = threadIdx.x;
-  // the row's histogram starts at zero (the searches leave it so, but the room may be new)
-  for (int b = lane; b < 2 * SAMPLE_BINS; b += HAL_WAVE) hist[(size_t)row * 2 * SAMPLE_BINS + b] = 0ull;
+__device__ __forceinline__ int filt_flags(const FiltParams& p, int V, int row) {
+  if (row_scale_of(p.temperature, p.top_k, row) == 0.f) return FILT_GREEDY;
+  const int k = p.top_k[row];
+  const bool want_k = k > 0 && k < V, want_p = p.top_p[row] < 1.f;
+  // with min_p the reference renormalises after top-k, so top-p refers to what top-k kept
+  const bool late = want_k && want_p && p.min_p[row] > 0.f;
+  return (want_k ? FILT_K : 0) | (want_p ? (late ? FILT_P_LATE : FILT_P) : 0);
+}
+
+// the bin of a z (the last one also where there is no distance: a maximum that is infinite)
+__device__ __forceinline__ int filt_bin(float z, float m) { return (int)fminf((m - z) * 8.0f, (float)(FILT_BINS - 1)); }
+// a key's mass, in units of 2^-40 of the largest
+__device__ __forceinline__ unsigned long long filt_fixed(float e) { return (unsigned long long)(e * 1099511627776.0f); }
+
+__global__ void __launch_bounds__(PART_THREADS, 8)  // (eight blocks a compute unit: 64 rows at once)
+filt_max_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, float* __restrict__ parts,
+                unsigned long long* __restrict__ hist) {  // [rows][2][FILT_BINS]
+  __shared__ ArgMax amax_s[PART_THREADS / HAL_WAVE];
+  const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
+  const int lane = tid % HAL_WAVE, wave = tid / HAL_WAVE;
+  constexpr int MINE = 2 * FILT_BINS / ROW_PARTS;  // of the row's bins, which start at zero
+  if (tid < MINE) hist[(size_t)row * 2 * FILT_BINS + part * MINE + tid] = 0ull;
+  const int share = part_share(V);
+  const int begin = part * share;
+  const int end = begin + share < V ? begin + share : V;
+  const float* x = logits + (size_t)row * ld;
+  const float T = row_scale_of(params.temperature, params.top_k, row);
+  const float scale = T == 0.f ? 1.f : T;
+  // The quotient rises with the logit, so the largest logit has the largest z, and only logits next to it can
+  // share that z: those alone are divided to find the first (all, where quotients run into the type's ends).
   ArgMax am = {-INFINITY, 0x7fffffff};
-  float sum = 0.f;
+  float held[PART_BATCH];
+  float top = -INFINITY;
+  const bool one_batch = share <= PART_BATCH * PART_THREADS;
+  for_part(x, begin, end, [&](float v, int, int u) {
+    held[u] = clean_logit(v);
+    top = fmaxf(top, held[u]);
+  });
+  am.v = top / scale;
+  const float near = fabsf(am.v) > 1e-30f && fabsf(am.v) < INFINITY ? top - fabsf(top) * 1e-6f : -INFINITY;
+  auto first = [&](float v, int i) {
+    if (v >= near && am.i == 0x7fffffff && am.v > -INFINITY && v / scale == am.v) am.i = i;
+  };
+  if (one_batch) {
+#pragma unroll
+    for (int u = 0; u < PART_BATCH; ++u) {
+      const int i = begin + tid + u * PART_THREADS;
+      if (i < end) first(held[u], i);
+    }
+  } else {
+    for_part(x, begin, end, [&](float v, int i, int) { first(clean_logit(v), i); });
+  }
+#pragma unroll
+  for (int off = HAL_WAVE / 2; off > 0; off >>= 1) {
+    ArgMax o;
+    o.v = __shfl_xor(am.v, off, HAL_WAVE);
+    o.i = __shfl_xor(am.i, off, HAL_WAVE);
+    am = argmax_merge(am, o);
+  }
+  if (lane == 0) amax_s[wave] = am;
+  __syncthreads();
+  if (tid != 0) return;
+  for (int w = 1; w < PART_THREADS / HAL_WAVE; ++w) am = argmax_merge(am, amax_s[w]);
+  float* p = parts + ((size_t)row * ROW_PARTS + part) * 4;
+  p[0] = am.v;
+  p[1] = __int_as_float(am.i);
+}
+
+__global__ void __launch_bounds__(PART_THREADS)
+filt_coarse_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, float* __restrict__ parts,
+                   FiltRow* __restrict__ rows, unsigned long long* __restrict__ hist) {
+  __shared__ uint32_t count_s[FILT_BINS];
+  __shared__ unsigned long long mass_s[FILT_BINS];
+  __shared__ float red[16];
+  static_assert(FILT_BINS == PART_THREADS, "a thread a bin");
+  const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x, lane = tid % HAL_WAVE;
+  const int flags = filt_flags(params, V, row);
+  const bool on_k = (flags & FILT_K) != 0, on_p = (flags & (FILT_P | FILT_P_LATE)) != 0;
+  count_s[tid] = 0u;
+  mass_s[tid] = 0ull;
+  // every wave joins the shares' maxima for itself
+  ArgMax best = {-INFINITY, 0x7fffffff};
   if (lane < ROW_PARTS) {
     const float* p = parts + ((size_t)row * ROW_PARTS + lane) * 4;
-    am.v = p[0], am.i = __float_as_int(p[1]), sum = p[2];
+    best.v = p[0], best.i = __float_as_int(p[1]);
   }
-  ArgMax best = am;
 #pragma unroll
   for (int off = HAL_WAVE / 2; off > 0; off >>= 1) {
     ArgMax o;
@@ -637,216 +715,292 @@ filt_join_kernel(const float* __restrict__ parts, const float* __restrict__ temp
     o.i = __shfl_xor(best.i, off, HAL_WAVE);
     best = argmax_merge(best, o);
   }
-  const float scaled = (am.v == -INFINITY) ? 0.f : sum * expf(am.v - best.v);
-  const float total = wave_sum(scaled);
-  if (lane != 0) return;
-  const bool greedy = row_scale_of(temperature, top_k, row) == 0.f;
-  const int k = top_k[row];
-  FiltRow r;
-  r.m = best.v, r.total = total, r.best = best.i;
-  const bool want_k = k > 0 && k < V, want_p = top_p[row] < 1.f;
-  // with min_p the reference renormalises after top-k, so top-p refers to what top-k kept
-  const bool late = want_k && want_p && min_p[row] > 0.f;
-  r.flags = greedy ? FILT_GREEDY : ((want_k ? FILT_K : 0) | (want_p ? (late ? FILT_P_LATE : FILT_P) : 0));
-  r.prefix[0] = r.prefix[1] = 0u, r.key_min = 0u, r.unused = 0u, r.kept_by_k = 0ull, r.unused2 = 0ull;
-  r.above[0] = r.above[1] = 0ull;
-  r.target[0] = (unsigned long long)(k > 0 ? k : 0), r.target[1] = ~0ull;  // top_p of the whole mass, set at level 0
-  rows[row] = r;
-}
-
-// One level of the search: the histogram of a share of the row, added to the row's.
-__global__ void __launch_bounds__(PART_THREADS)
-filt_hist_kernel(const float* __restrict__ logits, int ld, int V,
-                 const float* __restrict__ temperature, const FiltRow* __restrict__ rows, int level,
-                 int late, unsigned long long* __restrict__ hist) {  // [rows][2][SAMPLE_BINS]
-  __shared__ uint32_t count_s[SAMPLE_BINS];
-  __shared__ unsigned long long mass_s[SAMPLE_BINS];
-  const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
-  const FiltRow r = rows[row];
-  const bool on_k = !late && (r.flags & FILT_K) != 0;
-  const bool on_p = (r.flags & (late ? FILT_P_LATE : FILT_P)) != 0;
-  if (!on_k && !on_p) return;
-  if (on_k)
-    for (int b = tid; b < SAMPLE_BINS; b += PART_THREADS) count_s[b] = 0u;
-  if (on_p)
-    for (int b = tid; b < SAMPLE_BINS; b += PART_THREADS) mass_s[b] = 0ull;
-  __syncthreads();
-  const int share = part_share(V);
-  const int begin = part * share, end = begin + share < V ? begin + share : V;
-  const float* x = logits + (size_t)row * ld;
-  const float T = temperature[row];
-  const int shift = level_shift(level), up = level_up(level);
-  for_part(x, begin, end, [&](float v, int, int) {
-    const uint32_t key = sort_key(clean_logit(v) / T);
-    const uint32_t high = level == 0 ? 0u : key >> up;
-    const uint32_t bin = (key >> shift) & (SAMPLE_BINS - 1) & ((1u << (up - shift)) - 1u);
-    if (on_k && high == r.prefix[0]) atomicAdd(&count_s[bin], 1u);
-    if (on_p && high == r.prefix[1])
-      atomicAdd(&mass_s[bin], (unsigned long long)(expf(key_value(key) - r.m) * 1099511627776.0f));
-  });
-  __syncthreads();
-  unsigned long long* h = hist + (size_t)row * 2 * SAMPLE_BINS;
-  if (on_k)
-    for (int b = tid; b < SAMPLE_BINS; b += PART_THREADS)
-      if (count_s[b]) atomicAdd(&h[b], (unsigned long long)count_s[b]);
-  if (on_p)
-    for (int b = tid; b < SAMPLE_BINS; b += PART_THREADS)
-      if (mass_s[b]) atomicAdd(&h[SAMPLE_BINS + b], mass_s[b]);
-}
-
-// The walk over the row's histogram of one level (as in sample_kernel); leaves the
-// histogram cleared for the next level, and after the last level the smallest kept key.
-__global__ void __launch_bounds__(SAMPLE_THREADS)
-filt_find_kernel(FiltRow* __restrict__ rows, unsigned long long* __restrict__ hist,
-                 const float* __restrict__ top_p, int level, int late) {
-  __shared__ unsigned long long scan_tmp[SAMPLE_THREADS / HAL_WAVE];
-  __shared__ unsigned long long whole_mass;
-  __shared__ unsigned long long found_above[2];
-  __shared__ uint32_t found_bin[2];
-  __shared__ int found_any[2];
-  const int row = blockIdx.x, tid = threadIdx.x;
-  FiltRow r = rows[row];
-  const bool on[2] = {!late && (r.flags & FILT_K) != 0, (r.flags & (late ? FILT_P_LATE : FILT_P)) != 0};
-  if (!on[0] && !on[1]) return;
-  unsigned long long* h = hist + (size_t)row * 2 * SAMPLE_BINS;
-  const int shift = level_shift(level), up = level_up(level);
-  if (level == 0 && late) {
-    // top-p of what top-k kept
-    r.target[1] = (unsigned long long)((double)top_p[row] * (double)r.kept_by_k);
-  } else if (level == 0 && on[1]) {
-    // the whole mass, as the histogram has it: the reference of top-p
-    unsigned long long all = h[SAMPLE_BINS + 2 * tid] + h[SAMPLE_BINS + 2 * tid + 1];
-    all += block_suffix_u64(all, scan_tmp);
-    if (tid == 0) whole_mass = all;
-    __syncthreads();
-    r.target[1] = (unsigned long long)((double)top_p[row] * (double)whole_mass);
-  }
-#pragma unroll
-  for (int sidx = 0; sidx < 2; ++sidx) {
-    if (!on[sidx]) continue;
-    // bins in descending order: thread t has bins 2t+1 and 2t
-    const unsigned long long h1 = h[sidx * SAMPLE_BINS + 2 * tid + 1], h0 = h[sidx * SAMPLE_BINS + 2 * tid];
-    const unsigned long long higher = r.above[sidx] + block_suffix_u64(h1 + h0, scan_tmp);
-    if (tid == 0) found_bin[sidx] = 0u, found_above[sidx] = r.above[sidx], found_any[sidx] = 0;
-    __syncthreads();
-    if (higher < r.target[sidx] && higher + h1 >= r.target[sidx]) {
-      found_bin[sidx] = 2 * tid + 1, found_above[sidx] = higher, found_any[sidx] = 1;
-    } else if (higher + h1 < r.target[sidx] && higher + h1 + h0 >= r.target[sidx]) {
-      found_bin[sidx] = 2 * tid, found_above[sidx] = higher + h1, found_any[sidx] = 1;
-    }
-    __syncthreads();
-    // a target of zero, or one beyond the whole sum, is met by no bin: the first keeps the
-    // largest key only, the second every key
-    if (!found_any[sidx]) {
-      if (r.target[sidx] == 0ull) {
-        int top = -1;
-        if (h1 != 0ull) top = 2 * tid + 1; else if (h0 != 0ull) top = 2 * tid;
-        if (top >= 0) atomicMax(&found_bin[sidx], (uint32_t)top);
-      }
-      __syncthreads();
-    }
-    r.prefix[sidx] = (r.prefix[sidx] << (up - shift)) | found_bin[sidx];
-    r.above[sidx] = found_above[sidx];
-    __syncthreads();
-  }
-  // cleared for the next level (every thread has read its bins)
-  h[2 * tid] = h[2 * tid + 1] = 0ull;
-  h[SAMPLE_BINS + 2 * tid] = h[SAMPLE_BINS + 2 * tid + 1] = 0ull;
-  if (tid == 0) {
-    if (level == 2) {
-      if (!late) r.key_min = on[0] ? r.prefix[0] : 0u;
-      if (on[1] && r.prefix[1] > r.key_min) r.key_min = r.prefix[1];
-    }
+  const float m = best.v;
+  if (part == 0 && tid == 0) {
+    FiltRow r;
+    r.m = m, r.best = best.i, r.listed = 0, r.key_min = 0u, r.kept_by_k = 0ull;
     rows[row] = r;
   }
+  __syncthreads();
+  const int share = part_share(V);
+  const int begin = part * share, end = begin + share < V ? begin + share : V;
+  const float T = row_scale_of(params.temperature, params.top_k, row), scale = T == 0.f ? 1.f : T;
+  float sum = 0.f;
+  for_part(logits + (size_t)row * ld, begin, end, [&](float v, int, int) {
+    const float z = clean_logit(v) / scale, e = expf(z - m);
+    sum += e;
+    const int bin = filt_bin(z, m);
+    if (on_p) atomicAdd(&mass_s[bin], filt_fixed(e));
+    if (on_k) atomicAdd(&count_s[bin], 1u);
+  });
+  sum = block_sum(sum, red);
+  if (tid == 0) parts[((size_t)row * ROW_PARTS + part) * 4 + 2] = begin < end && m > -INFINITY ? sum : 0.f;
+  unsigned long long* h = hist + (size_t)row * 2 * FILT_BINS;
+  if (on_k && count_s[tid]) atomicAdd(&h[tid], (unsigned long long)count_s[tid]);
+  if (on_p && mass_s[tid]) atomicAdd(&h[FILT_BINS + tid], mass_s[tid]);
 }
 
-// Late rows: the mass of the keys that top-k kept, as the histograms count it (integers).
+// Where a row's thresholds lie: for each of the two searches the bin and the sum over the bins before it (nearer the
+// maximum).  A block of at least FILT_BINS threads, all of which get the result.
+struct FiltPlace {
+  bool on[2];     // top-k, top-p
+  bool largest[2];  // the target is nothing: the largest key alone is kept
+  int bin[2];
+  unsigned long long before[2], target[2];
+  int list;  // the bin whose keys are listed: that of the higher threshold; -1: none
+};
+__device__ __forceinline__ FiltPlace filt_place(const unsigned long long* __restrict__ h, const FiltParams& params, int V, int row,
+                                                const FiltRow& r, int late) {
+  __shared__ unsigned long long wave_sums[2][FILT_BINS / HAL_WAVE];
+  __shared__ unsigned long long before_s[2];
+  __shared__ int bin_s[2];
+  const int tid = threadIdx.x, lane = tid % HAL_WAVE, wave = tid / HAL_WAVE;
+  const int flags = filt_flags(params, V, row);
+  FiltPlace f;
+  f.on[0] = !late && (flags & FILT_K) != 0;
+  f.on[1] = (flags & (late ? FILT_P_LATE : FILT_P)) != 0;
+  f.list = -1;
+  if (!f.on[0] && !f.on[1]) return f;
+  unsigned long long own[2] = {0ull, 0ull}, upto[2];
+  if (tid < FILT_BINS) own[0] = f.on[0] ? h[tid] : 0ull, own[1] = f.on[1] ? h[FILT_BINS + tid] : 0ull;
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    upto[w] = own[w];
+#pragma unroll
+    for (int off = 1; off < HAL_WAVE; off <<= 1) {
+      const uint32_t lo = __shfl_up((uint32_t)upto[w], off, HAL_WAVE), hi = __shfl_up((uint32_t)(upto[w] >> 32), off, HAL_WAVE);
+      if (lane >= off) upto[w] += ((unsigned long long)hi << 32) | lo;
+    }
+    if (lane == HAL_WAVE - 1 && tid < FILT_BINS) wave_sums[w][wave] = upto[w];
+  }
+  if (tid < 2) bin_s[tid] = FILT_BINS - 1, before_s[tid] = 0ull;
+  __syncthreads();
+  unsigned long long all = 0ull;
+#pragma unroll
+  for (int w = 0; w < FILT_BINS / HAL_WAVE; ++w) {
+    if (w < wave) upto[0] += wave_sums[0][w], upto[1] += wave_sums[1][w];
+    all += wave_sums[1][w];
+  }
+  f.target[0] = (unsigned long long)params.top_k[row];
+  // top-p of the whole mass, as the bins have it, or of what top-k kept
+  f.target[1] = (unsigned long long)((double)params.top_p[row] * (double)(late ? r.kept_by_k : all));
+#pragma unroll
+  for (int w = 0; w < 2; ++w)
+    if (tid < FILT_BINS && f.on[w] && upto[w] - own[w] < f.target[w] && upto[w] >= f.target[w]) bin_s[w] = tid, before_s[w] = upto[w] - own[w];
+  __syncthreads();
+#pragma unroll
+  for (int w = 0; w < 2; ++w) {
+    f.bin[w] = bin_s[w], f.before[w] = before_s[w];
+    f.largest[w] = f.on[w] && f.target[w] == 0ull;
+    if (f.largest[w]) f.bin[w] = 0;
+    if (f.on[w] && !f.largest[w] && (f.list < 0 || f.bin[w] < f.list)) f.list = f.bin[w];
+  }
+  if (f.largest[0] || f.largest[1]) f.list = -1;  // (nothing to search for: the largest key is the threshold)
+  return f;
+}
+
 __global__ void __launch_bounds__(PART_THREADS)
-filt_kept_by_k_kernel(const float* __restrict__ logits, int ld, int V,
-                      const float* __restrict__ temperature, FiltRow* __restrict__ rows) {
-  __shared__ unsigned long long tmp[PART_THREADS / HAL_WAVE];
+filt_list_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, FiltRow* __restrict__ rows, int late,
+                 const unsigned long long* __restrict__ hist, uint32_t* __restrict__ lists) {  // [rows][V]
+  __shared__ uint32_t found[PART_BATCH * PART_THREADS];
+  __shared__ int n_found, first;
   const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
-  const int lane = tid % HAL_WAVE, wave = tid / HAL_WAVE;
   const FiltRow r = rows[row];
-  if (!(r.flags & FILT_P_LATE)) return;
+  const FiltPlace f = filt_place(hist + (size_t)row * 2 * FILT_BINS, params, V, row, r, late);
+  if (f.list < 0) return;
   const int share = part_share(V);
   const int begin = part * share, end = begin + share < V ? begin + share : V;
   const float* x = logits + (size_t)row * ld;
-  const float T = temperature[row];
-  unsigned long long mine = 0ull;
-  for_part(x, begin, end, [&](float v, int, int) {
-    const uint32_t key = sort_key(clean_logit(v) / T);
-    if (key >= r.key_min) mine += (unsigned long long)(expf(key_value(key) - r.m) * 1099511627776.0f);
-  });
-#pragma unroll
-  for (int off = HAL_WAVE / 2; off > 0; off >>= 1) {
-    const uint32_t lo = __shfl_xor((uint32_t)mine, off, HAL_WAVE);
-    const uint32_t hi = __shfl_xor((uint32_t)(mine >> 32), off, HAL_WAVE);
-    mine += ((unsigned long long)hi << 32) | lo;
-  }
-  if (lane == 0) tmp[wave] = mine;
-  __syncthreads();
-  if (tid == 0) {
-    unsigned long long all = 0ull;
-    for (int w = 0; w < PART_THREADS / HAL_WAVE; ++w) all += tmp[w];
-    if (all) atomicAdd(&rows[row].kept_by_k, all);
+  const float T = params.temperature[row];
+  // Logits that are surely outside the bin are left out by two comparisons (the bounds are a 100,000th of
+  // the numbers they are made of wider than the bin), the others go through the quotient.
+  const float wide = 1e-5f * (fabsf(r.m) + 32.f) * T;
+  const float high = (r.m - 0.125f * f.list) * T + wide;
+  const float low = f.list == FILT_BINS - 1 ? -INFINITY : (r.m - 0.125f * (f.list + 1)) * T - wide;
+  for (int from = begin; from < end; from += PART_BATCH * PART_THREADS) {
+    const int to = from + PART_BATCH * PART_THREADS < end ? from + PART_BATCH * PART_THREADS : end;
+    if (tid == 0) n_found = 0;
+    __syncthreads();
+    for_part(x, from, to, [&](float v, int, int) {
+      v = clean_logit(v);
+      if (v > high || v < low) return;
+      const float z = v / T;
+      if (filt_bin(z, r.m) == f.list) found[atomicAdd(&n_found, 1)] = sort_key(z);
+    });
+    __syncthreads();
+    if (tid == 0 && n_found) first = atomicAdd(&rows[row].listed, n_found);
+    __syncthreads();
+    for (int i = tid; i < n_found; i += PART_THREADS) lists[(size_t)row * V + first + i] = found[i];
+    __syncthreads();
   }
 }
 
-__device__ __forceinline__ float kept_mass_of(float v, float T, const FiltRow& r, float mp, float& z) {
+// The smallest key that a row keeps by the searches of this pass, and after the first pass of a late row the mass that
+// top-k kept; a block a row.  The keys of the row's list are searched bit by bit of those in which they differ, ten at a
+// time from the top, from histograms over the keys that share the bits found so far (the keys of a bin differ in some
+// eighteen bits: two rounds).  (Every block of the next pass finding it for itself instead: 24 us more there.)
+#define FILT_DIGIT 10
+#define FILT_STAGED 2048  // keys of a list that are kept in LDS
+// Sum of `v` over the threads after this one (exclusive) in a block of PART_THREADS; ends with a barrier.
+__device__ __forceinline__ unsigned long long part_suffix_u64(unsigned long long v, unsigned long long* tmp) {
+  const int lane = threadIdx.x % HAL_WAVE, wave = threadIdx.x / HAL_WAVE;
+  unsigned long long inc = v;
+#pragma unroll
+  for (int off = 1; off < HAL_WAVE; off <<= 1) {
+    const uint32_t lo = __shfl_down((uint32_t)inc, off, HAL_WAVE), hi = __shfl_down((uint32_t)(inc >> 32), off, HAL_WAVE);
+    if (lane + off < HAL_WAVE) inc += ((unsigned long long)hi << 32) | lo;
+  }
+  if (lane == 0) tmp[wave] = inc;
+  __syncthreads();
+  unsigned long long after = 0ull;
+#pragma unroll
+  for (int w = 1; w < PART_THREADS / HAL_WAVE; ++w)
+    if (w > wave) after += tmp[w];
+  __syncthreads();
+  return inc - v + after;
+}
+__global__ void __launch_bounds__(PART_THREADS)
+filt_find_kernel(FiltRow* __restrict__ rows, const unsigned long long* __restrict__ hists, FiltParams params, int V, int late,
+                 const uint32_t* __restrict__ lists) {
+  constexpr int BINS = 1 << FILT_DIGIT, EACH = BINS / PART_THREADS;
+  __shared__ unsigned long long bins[BINS];
+  __shared__ unsigned long long tmp[PART_THREADS / HAL_WAVE];
+  __shared__ uint32_t staged[FILT_STAGED];
+  __shared__ uint32_t ends[2];
+  __shared__ unsigned long long above_s;
+  __shared__ uint32_t bin_s;
+  const int row = blockIdx.x, tid = threadIdx.x;
+  const unsigned long long* hist = hists + (size_t)row * 2 * FILT_BINS;
+  const uint32_t* keys = lists + (size_t)row * V;
+  const FiltRow r = rows[row];
+  const FiltPlace f = filt_place(hist, params, V, row, r, late);
+  if (!f.on[0] && !f.on[1]) return;
+  uint32_t key_min = late ? r.key_min : 0u;
+  if (f.largest[0] || f.largest[1]) key_min = sort_key(r.m);
+  const int n = f.list < 0 ? 0 : r.listed, n_staged = n < FILT_STAGED ? n : FILT_STAGED;
+  auto each = [&](auto&& what) {
+    for (int i = tid; i < n_staged; i += PART_THREADS) what(staged[i]);
+    for (int i = FILT_STAGED + tid; i < n; i += PART_THREADS) what(keys[i]);
+  };
+  auto mass_of = [&](uint32_t key) { return filt_fixed(expf(key_value(key) - r.m)); };
+  if (n > 0) {
+    for (int i = tid; i < n_staged; i += PART_THREADS) staged[i] = keys[i];
+    if (tid == 0) ends[0] = 0xffffffffu, ends[1] = 0u;
+    __syncthreads();
+    uint32_t lowest = 0xffffffffu, highest = 0u;
+    each([&](uint32_t key) { lowest = min(lowest, key), highest = max(highest, key); });
+    atomicMin(&ends[0], lowest), atomicMax(&ends[1], highest);
+    __syncthreads();
+    lowest = ends[0];
+    const uint32_t range = ends[1] - lowest;
+#pragma unroll 1
+    for (int w = 0; w < 2; ++w) {
+      if (!f.on[w] || f.bin[w] != f.list) continue;
+      const unsigned long long target = f.target[w] - f.before[w];
+      uint32_t prefix = 0u;
+      unsigned long long above = 0ull;
+      int bits = range ? 32 - __builtin_clz(range) : 0;
+#pragma unroll 1
+      while (bits > 0) {
+        const int take = bits < FILT_DIGIT ? bits : FILT_DIGIT, shift = bits - take;
+#pragma unroll
+        for (int b = 0; b < EACH; ++b) bins[tid + b * PART_THREADS] = 0ull;
+        if (tid == 0) bin_s = 0u, above_s = above;
+        __syncthreads();
+        each([&](uint32_t key) {
+          const uint32_t rel = key - lowest;
+          if (((unsigned long long)rel >> bits) != prefix) return;
+          atomicAdd(&bins[(rel >> shift) & ((1u << take) - 1u)], w == 1 ? mass_of(key) : 1ull);
+        });
+        __syncthreads();
+        // in descending order: thread t has the bins EACH * t + EACH - 1 .. EACH * t
+        unsigned long long own[EACH], sum = 0ull;
+#pragma unroll
+        for (int b = 0; b < EACH; ++b) own[b] = bins[tid * EACH + b], sum += own[b];
+        unsigned long long higher = above + part_suffix_u64(sum, tmp);
+#pragma unroll
+        for (int b = EACH - 1; b >= 0; --b) {
+          if (higher < target && higher + own[b] >= target) bin_s = tid * EACH + b, above_s = higher;
+          higher += own[b];
+        }
+        __syncthreads();
+        prefix = (prefix << take) | bin_s;
+        above = above_s;
+        bits = shift;
+        __syncthreads();
+      }
+      key_min = max(key_min, lowest + prefix);
+    }
+  }
+  unsigned long long kept = 0ull;
+  if (!late && (filt_flags(params, V, row) & FILT_P_LATE)) {
+    kept = tid < f.bin[0] ? hist[FILT_BINS + tid] : 0ull;
+    each([&](uint32_t key) { kept += key >= key_min ? mass_of(key) : 0ull; });
+    kept += part_suffix_u64(kept, tmp);  // (thread 0: of all)
+  }
+  if (tid == 0) rows[row].key_min = key_min, rows[row].kept_by_k = kept, rows[row].listed = 0;
+}
+
+__device__ __forceinline__ float kept_mass_of(float v, float T, uint32_t key_min, float m, float mp, float& z) {
   const uint32_t key = sort_key(clean_logit(v) / T);
-  if (key < r.key_min) return 0.f;
+  if (key < key_min) return 0.f;
   z = key_value(key);
-  const float e = expf(z - r.m);
+  const float e = expf(z - m);
   return e >= mp ? e : 0.f;
 }
 
 // The kept mass of every share of a row.
 __global__ void __launch_bounds__(PART_THREADS)
-filt_mass_kernel(const float* __restrict__ logits, int ld, int V,
-                 const float* __restrict__ temperature, const float* __restrict__ min_p,
-                 const FiltRow* __restrict__ rows, float* __restrict__ kept) {  // [rows][ROW_PARTS]
+filt_mass_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, const FiltRow* __restrict__ rows,
+                 float* __restrict__ kept) {  // [rows][ROW_PARTS]
   __shared__ float red[16];
   const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
+  if (row_scale_of(params.temperature, params.top_k, row) == 0.f) return;
   const FiltRow r = rows[row];
-  if (r.flags & FILT_GREEDY) return;
   const int share = part_share(V);
   const int begin = part * share, end = begin + share < V ? begin + share : V;
   const float* x = logits + (size_t)row * ld;
-  const float T = temperature[row], mp = min_p[row];
+  const float T = params.temperature[row], mp = params.min_p[row];
   float mine = 0.f, z;
-  for_part(x, begin, end, [&](float v, int, int) { mine += kept_mass_of(v, T, r, mp, z); });
+  for_part(x, begin, end, [&](float v, int, int) { mine += kept_mass_of(v, T, r.key_min, r.m, mp, z); });
   mine = block_sum(mine, red);
   if (tid == 0) kept[(size_t)row * ROW_PARTS + part] = mine;
 }
 
-// The draw: the share in which the running kept mass passes u * (kept mass), then the walk
-// through that share, a quarter per wave.
-__global__ void __launch_bounds__(PART_THREADS)
-filt_pick_kernel(const float* __restrict__ logits, int ld, int V,
-                 const float* __restrict__ temperature, const float* __restrict__ min_p,
-                 const FiltRow* __restrict__ rows, const float* __restrict__ kept,
-                 const uint64_t* __restrict__ seeds, const int* __restrict__ draw_index,
-                 int* __restrict__ out_token, float* __restrict__ out_logprob) {
-  __shared__ float quarter_mass[PART_THREADS / HAL_WAVE];
+// The draw: the share in which the running kept mass passes u * (kept mass), then the walk through that share as four
+// waves would walk it, a quarter each, 64 logits at a time.  Sixteen waves make the masses and the running sums inside
+// every 64 and leave them in LDS; the sums over a quarter's runs of 64 and the runs' order are then a few additions.
+#define PICK_THREADS 1024
+#define PICK_QUARTERS 4
+__global__ void __launch_bounds__(PICK_THREADS)
+filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, const FiltRow* __restrict__ rows,
+                 const float* __restrict__ parts, const float* __restrict__ kept, const uint64_t* __restrict__ seeds,
+                 const int* __restrict__ draw_index, int* __restrict__ out_token, float* __restrict__ out_logprob) {
+  constexpr int RUNS = 16, WAVES = PICK_THREADS / HAL_WAVE, MINE = RUNS * PICK_QUARTERS / WAVES;  // runs in LDS a quarter; of a wave
+  __shared__ float e_s[PICK_QUARTERS][RUNS][HAL_WAVE], z_s[PICK_QUARTERS][RUNS][HAL_WAVE], inc_s[PICK_QUARTERS][RUNS][HAL_WAVE];
+  __shared__ float quarter_mass[PICK_QUARTERS];
   const int row = blockIdx.x, tid = threadIdx.x;
-  const int lane = tid % HAL_WAVE, wave = tid / HAL_WAVE;
+  const int lane = tid % HAL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / HAL_WAVE);
   const FiltRow r = rows[row];
-  if (r.flags & FILT_GREEDY) {
+  const float total = wave_sum(lane < ROW_PARTS ? parts[((size_t)row * ROW_PARTS + lane) * 4 + 2] : 0.f);
+  if (row_scale_of(params.temperature, params.top_k, row) == 0.f) {
     if (tid == 0) {
       out_token[row] = r.best < V ? r.best : 0;
-      out_logprob[row] = -logf(r.total);
+      out_logprob[row] = -logf(total);
     }
     return;
   }
-  const float mass = lane < ROW_PARTS ? kept[(size_t)row * ROW_PARTS + lane] : 0.f;
-  float incl = mass;
+  auto running = [&](float v) {
+    float inc = v;
 #pragma unroll
-  for (int off = 1; off < HAL_WAVE; off <<= 1) {
-    const float up = __shfl_up(incl, off, HAL_WAVE);
-    if (lane >= off) incl += up;
-  }
+    for (int off = 1; off < HAL_WAVE; off <<= 1) {
+      const float up = __shfl_up(inc, off, HAL_WAVE);
+      if (lane >= off) inc += up;
+    }
+    return inc;
+  };
+  const float mass = lane < ROW_PARTS ? kept[(size_t)row * ROW_PARTS + lane] : 0.f;
+  const float incl = running(mass);
   const float kept_mass = __shfl(incl, HAL_WAVE - 1, HAL_WAVE);
   const float target = uniform_draw(seeds[row], (uint32_t)draw_index[row]) * kept_mass;
   const unsigned long long some = __builtin_amdgcn_ballot_w64(mass > 0.f);
@@ -856,47 +1010,39 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V,
   const float before_part = __shfl(incl - mass, part, HAL_WAVE);
 
   const float* x = logits + (size_t)row * ld;
-  const float T = temperature[row], mp = min_p[row];
   const int share = part_share(V);
   const int p_begin = part * share, p_end = p_begin + share < V ? p_begin + share : V;
-  constexpr int n_waves = PART_THREADS / HAL_WAVE;
-  const int run_len = ((p_end - p_begin + n_waves - 1) / n_waves + HAL_WAVE - 1) / HAL_WAVE * HAL_WAVE;
-  const int begin = p_begin + wave * run_len;
-  const int end = begin + run_len < p_end ? begin + run_len : p_end;
-  float mine = 0.f, zz = 0.f;
-  // (the wave's run of the share, PICK_BATCH logits a lane of it in registers)
-  constexpr int PICK_BATCH = 16;
-  const int run_begin = __builtin_amdgcn_readfirstlane(begin), run_end = __builtin_amdgcn_readfirstlane(end);
-  float held[PICK_BATCH];
-  if (run_begin + (PICK_BATCH - 1) * HAL_WAVE < run_end) {
+  const int run_len = ((p_end - p_begin + PICK_QUARTERS - 1) / PICK_QUARTERS + HAL_WAVE - 1) / HAL_WAVE * HAL_WAVE;
+  const float T = params.temperature[row], mp = params.min_p[row];
+  auto quarter_end = [&](int q) { return p_begin + (q + 1) * run_len < p_end ? p_begin + (q + 1) * run_len : p_end; };
+  {  // (a wave's runs are all of one quarter)
+    const int q = wave * MINE / RUNS, run0 = wave * MINE % RUNS, from = p_begin + q * run_len, end = quarter_end(q);
+    float held[MINE];
 #pragma unroll
-    for (int u = 0; u < PICK_BATCH; ++u) {
-      const int i = begin + lane + u * HAL_WAVE;
+    for (int u = 0; u < MINE; ++u) {
+      const int i = from + (run0 + u) * HAL_WAVE + lane;
       held[u] = i < end ? x[i] : 0.f;
     }
 #pragma unroll
-    for (int u = 0; u < PICK_BATCH; ++u)
-      if (begin + lane + u * HAL_WAVE < end) mine += kept_mass_of(held[u], T, r, mp, zz);
-  } else {
-#pragma unroll
-    for (int u = 0; u < PICK_BATCH; ++u) {
-      if (run_begin + u * HAL_WAVE >= run_end) break;
-      const int i = begin + lane + u * HAL_WAVE;
-      held[u] = i < end ? x[i] : 0.f;
-    }
-#pragma unroll
-    for (int u = 0; u < PICK_BATCH; ++u) {
-      if (run_begin + u * HAL_WAVE >= run_end) break;
-      if (begin + lane + u * HAL_WAVE < end) mine += kept_mass_of(held[u], T, r, mp, zz);
+    for (int u = 0; u < MINE; ++u) {
+      float z = 0.f;
+      const float e = from + (run0 + u) * HAL_WAVE + lane < end ? kept_mass_of(held[u], T, r.key_min, r.m, mp, z) : 0.f;
+      e_s[q][run0 + u][lane] = e, z_s[q][run0 + u][lane] = z, inc_s[q][run0 + u][lane] = running(e);
     }
   }
-  for (int i = begin + lane + PICK_BATCH * HAL_WAVE; i < end; i += HAL_WAVE) mine += kept_mass_of(x[i], T, r, mp, zz);
+  __syncthreads();
+  if (wave >= PICK_QUARTERS) return;  // (the barrier below is met by the waves that are left)
+  const int begin = p_begin + wave * run_len, end = quarter_end(wave);
+  const int runs = end > begin ? (end - begin + HAL_WAVE - 1) / HAL_WAVE : 0;
+  float mine = 0.f, zz = 0.f;
+  for (int u = 0; u < runs && u < RUNS; ++u) mine += e_s[wave][u][lane];
+  for (int i = begin + RUNS * HAL_WAVE + lane; i < end; i += HAL_WAVE) mine += kept_mass_of(x[i], T, r.key_min, r.m, mp, zz);
   const float wave_mass = wave_sum(mine);
   if (lane == 0) quarter_mass[wave] = wave_mass;
   __syncthreads();
   float before = before_part;
   int pick = -1, last = -1;
-  for (int w = 0; w < n_waves; ++w) {
+  for (int w = 0; w < PICK_QUARTERS; ++w) {
     if (quarter_mass[w] > 0.f) last = w;
     if (pick < 0 && quarter_mass[w] > 0.f && before + quarter_mass[w] > target) pick = w;
     if (pick < 0) before += quarter_mass[w];
@@ -910,14 +1056,14 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V,
   float run = before;
   int tok = -1, last_kept = -1;
   float z_tok = 0.f, z_last = 0.f;
-  for (int i0 = begin; i0 < end && tok < 0; i0 += HAL_WAVE) {
-    float z = 0.f;
-    const float e = i0 + lane < end ? kept_mass_of(x[i0 + lane], T, r, mp, z) : 0.f;
-    float inc = e;
-#pragma unroll
-    for (int off = 1; off < HAL_WAVE; off <<= 1) {
-      const float up = __shfl_up(inc, off, HAL_WAVE);
-      if (lane >= off) inc += up;
+  for (int u = 0; u < runs && tok < 0; ++u) {
+    const int i0 = begin + u * HAL_WAVE;
+    float z = 0.f, e = 0.f, inc;
+    if (u < RUNS) {
+      e = e_s[wave][u][lane], z = z_s[wave][u][lane], inc = inc_s[wave][u][lane];
+    } else {
+      if (i0 + lane < end) e = kept_mass_of(x[i0 + lane], T, r.key_min, r.m, mp, z);
+      inc = running(e);
     }
     const unsigned long long kept_lanes = __builtin_amdgcn_ballot_w64(e > 0.f);
     const unsigned long long found = __builtin_amdgcn_ballot_w64(e > 0.f && run + inc > target);
@@ -939,7 +1085,7 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V,
   }
   if (lane == 0) {
     out_token[row] = tok;
-    out_logprob[row] = z_tok - r.m - logf(r.total);
+    out_logprob[row] = z_tok - r.m - logf(total);
   }
 }
 
@@ -1039,43 +1185,35 @@ extern "C" int hal_sample_unfiltered(const float* logits, int ld, int n_rows, in
 
 // Rows with filters (and greedy or unfiltered ones among them), every row spread over 32
 // blocks in every pass.  `any_late`: some row has top-k, top-p and min-p all at once (its
-// second search costs seven launches more; a wrong 0 leaves such a row without top-p).
-// Room: `parts` n_rows * 32 * 4 floats, `kept` n_rows * 32 floats, `state` n_rows * 20
-// words, `hist` n_rows * 2 * 2048 64-bit words.
+// second search costs two launches more; a wrong 0 leaves such a row without top-p).
+// Room: `parts` n_rows * 32 * 4 floats, `kept` n_rows * 32 floats, `state` n_rows * 6
+// words, `hist` n_rows * 2 * 256 64-bit words, `lists` n_rows * V words.
 extern "C" int hal_sample_spread(const float* logits, int ld, int n_rows, int V,
                                  const float* temperature, const int* top_k, const float* top_p,
                                  const float* min_p, const uint64_t* seeds, const int* draw_index,
-                                 float* parts, float* kept, void* state, void* hist, int any_late,
+                                 float* parts, float* kept, void* state, void* hist, uint32_t* lists, int any_late,
                                  int* out_token, float* out_logprob, hipStream_t stream) {
   HAL_REQUIRE(n_rows >= 0 && V > 0 && ld >= V, "hal_sample_spread: bad sizes rows=%d V=%d ld=%d",
               n_rows, V, ld);
   HAL_REQUIRE(n_rows <= 65535, "hal_sample_spread: %d rows exceed the grid limit", n_rows);
   if (n_rows == 0) return 0;
   HAL_REQUIRE(temperature && top_k && top_p && min_p && seeds && draw_index && parts && kept &&
-                  state && hist && ((uintptr_t)state % 8) == 0 && ((uintptr_t)hist % 8) == 0,
+                  state && hist && lists && ((uintptr_t)state % 8) == 0 && ((uintptr_t)hist % 8) == 0,
               "hal_sample_spread: arguments missing");
   FiltRow* rows = (FiltRow*)state;
   unsigned long long* h = (unsigned long long*)hist;
-  hipLaunchKernelGGL(row_part_kernel, dim3(ROW_PARTS, n_rows), dim3(PART_THREADS), 0, stream, logits,
-                     ld, V, temperature, top_k, parts);
-  hipLaunchKernelGGL(filt_join_kernel, dim3(n_rows), dim3(HAL_WAVE), 0, stream, parts, temperature,
-                     top_k, top_p, min_p, V, rows, h);
+  const FiltParams params = {temperature, top_p, min_p, top_k};
+  const dim3 shares(ROW_PARTS, n_rows);
+  hipLaunchKernelGGL(filt_max_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, parts, h);
+  hipLaunchKernelGGL(filt_coarse_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, parts, rows, h);
   // the searches; then, if some row has top-k, top-p and min-p all at once, its second search
   for (int late = 0; late <= (any_late ? 1 : 0); ++late) {
-    if (late)
-      hipLaunchKernelGGL(filt_kept_by_k_kernel, dim3(ROW_PARTS, n_rows), dim3(PART_THREADS), 0,
-                         stream, logits, ld, V, temperature, rows);
-    for (int level = 0; level < 3; ++level) {
-      hipLaunchKernelGGL(filt_hist_kernel, dim3(ROW_PARTS, n_rows), dim3(PART_THREADS), 0, stream,
-                         logits, ld, V, temperature, rows, level, late, h);
-      hipLaunchKernelGGL(filt_find_kernel, dim3(n_rows), dim3(SAMPLE_THREADS), 0, stream, rows, h,
-                         top_p, level, late);
-    }
+    hipLaunchKernelGGL(filt_list_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, rows, late, h, lists);
+    hipLaunchKernelGGL(filt_find_kernel, dim3(n_rows), dim3(PART_THREADS), 0, stream, rows, h, params, V, late, lists);
   }
-  hipLaunchKernelGGL(filt_mass_kernel, dim3(ROW_PARTS, n_rows), dim3(PART_THREADS), 0, stream, logits,
-                     ld, V, temperature, min_p, rows, kept);
-  hipLaunchKernelGGL(filt_pick_kernel, dim3(n_rows), dim3(PART_THREADS), 0, stream, logits, ld, V,
-                     temperature, min_p, rows, kept, seeds, draw_index, out_token, out_logprob);
+  hipLaunchKernelGGL(filt_mass_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, rows, kept);
+  hipLaunchKernelGGL(filt_pick_kernel, dim3(n_rows), dim3(PICK_THREADS), 0, stream, logits, ld, V, params, rows, parts,
+                     kept, seeds, draw_index, out_token, out_logprob);
   HAL_LAUNCH_CHECK();
   return 0;
 }

@@ -501,8 +501,8 @@ def sample(
     ``all_greedy`` promises that no row samples (``temperature`` 0 or ``top_k`` 1 in
     every row), ``unfiltered`` that every row is greedy or draws from its whole
     distribution (no top-k, top-p or min-p): the rows are then spread over many blocks,
-    in two launches.  ``spread``: every pass over a row is shared by 32 blocks (ten
-    launches; seven more unless ``late`` is false, which promises that no row has top-k,
+    in two launches.  ``spread``: every pass over a row is shared by 32 blocks (six
+    launches; two more unless ``late`` is false, which promises that no row has top-k,
     top-p and min-p all at once).  Otherwise, with
     ``key_scratch``, the kernel gets room for one 32-bit key per logit, which its passes
     over a row read instead of deriving it again."""
@@ -529,14 +529,13 @@ def sample(
             _ptr(parts), _ptr(tokens), _ptr(logprobs), _stream()))
         return tokens, logprobs
     if spread and logits.is_contiguous():
-        dev = logits.device
-        parts = torch.empty((n, 32, 4), dtype=torch.float32, device=dev)
-        kept = torch.empty((n, 32), dtype=torch.float32, device=dev)
-        state = torch.empty((n, 20), dtype=torch.int32, device=dev)
-        hist = torch.empty((n, 2, 2048), dtype=torch.int64, device=dev)
+        # (one buffer: histograms and the rows' state first, which are 64-bit words)
+        words = [n * 2 * 256 * 2, n * 6, n * 32 * 4, n * 32, n * vocab]
+        room = torch.empty(sum(words), dtype=torch.int32, device=logits.device)
+        hist, state, parts, kept, lists = (room.data_ptr() + 4 * sum(words[:i]) for i in range(5))
         _check(lib, lib.hal_sample_spread(
             _ptr(logits), vocab, n, vocab, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(min_p),
-            _ptr(seeds), _ptr(draw_index), _ptr(parts), _ptr(kept), _ptr(state), _ptr(hist),
+            _ptr(seeds), _ptr(draw_index), *(ctypes.c_void_p(p) for p in (parts, kept, state, hist, lists)),
             1 if late else 0, _ptr(tokens), _ptr(logprobs), _stream()))
         return tokens, logprobs
     keys = torch.empty((n, vocab), dtype=torch.int32, device=logits.device) if key_scratch and not all_greedy else None

@@ -1,0 +1,68 @@
+"""Filters found by bins of the distance from the maximum and a list of one bin's keys, against the one-block kernel
+(which selects by the keys' bits): lists of one key, of more than LDS holds and of all keys, thresholds in the last bin,
+equal logits, masked and infinite ones, temperatures at the type's ends, rows of every kind side by side."""
+
+import random
+
+import pytest
+import torch
+
+from halite_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def both(x, temperature, top_k, top_p, min_p, seed):
+    n = x.shape[0]
+    f = lambda v: torch.tensor(v, dtype=torch.float32, device=x.device)  # noqa: E731
+    args = (f(temperature), torch.tensor(top_k, dtype=torch.int32, device=x.device), f(top_p), f(min_p),
+            torch.arange(n, dtype=torch.int64, device=x.device) * 7919 + seed, torch.arange(n, dtype=torch.int32, device=x.device))
+    return [[t.cpu() for t in ops.sample(x, *args, spread=spread)] for spread in (False, True)]
+
+
+def agree(ways, rows, allowed=0):
+    (tok, lp), (tok2, lp2) = ways
+    same = tok == tok2
+    assert int((~same).sum()) <= allowed, (tok[~same].tolist(), tok2[~same].tolist())
+    assert torch.equal(lp.isnan(), lp2.isnan())
+    # (sums of up to 2e5 float32 exponentials in two orders, and their logarithm)
+    assert torch.allclose(lp[same & ~lp.isnan()], lp2[same & ~lp.isnan()], rtol=1e-5, atol=1e-5)
+    assert same.numel() == rows
+
+
+@pytest.mark.parametrize("vocab", [1, 2, 255, 4097, 32000, 131073])
+@pytest.mark.parametrize("spread", [0.01, 1.0, 30.0])
+def test_drawn_rows(vocab, spread):
+    """Where the draw falls within rounding of a token's edge the two may differ: a chance of some 1e-7 a kept token and
+    row, so one row in a hundred at most."""
+    rng, n = random.Random(vocab), 100
+    gen = torch.Generator().manual_seed(vocab)
+    x = (torch.randn((n, vocab), generator=gen) * spread)
+    x[::7] = x[::7].to(torch.bfloat16).float()  # many equal logits
+    x[1::7, ::3] = -float("inf")
+    ways = both(x.cuda(), [rng.choice([0.0, 0.1, 0.7, 1.0, 2.5]) for _ in range(n)],
+                [rng.choice([-1, -1, 1, 2, 40, max(1, vocab - 1), vocab, vocab + 5]) for _ in range(n)],
+                [rng.choice([0.01, 0.3, 0.9, 0.999, 1.0]) for _ in range(n)], [rng.choice([0.0, 0.0, 0.05, 1.0]) for _ in range(n)], 3)
+    agree(ways, n, allowed=1)
+
+
+def test_rows_at_the_ends():
+    n, vocab = 12, 6000
+    x = torch.randn((n, vocab), generator=torch.Generator().manual_seed(1))
+    x[0] = 0.0                                     # all equal: the list is the row
+    x[1], x[1, 17], x[1, 4000] = -float("inf"), 1.0, 1.0
+    x[2] = -float("inf")                           # nothing
+    x[3, 40], x[3, 700] = float("inf"), float("inf")
+    x[4, ::2] = float("nan")
+    x[5] = torch.linspace(0, -200, vocab)          # most keys in the last bin
+    x[6] = torch.linspace(0, -200, vocab)
+    x[7] = x[7] * 1e-38                            # quotients that are no normal numbers
+    x[8] = x[8] * 1e30
+    x[9, 100:] = x[9, 0]                           # one key and many of another
+    temperature = [1.0] * n
+    temperature[7], temperature[8] = 100.0, 1e-9   # ... and such that overflow
+    top_k = [3000, -1, 5, 5, -1, 5500, -1, 50, 50, 200, 1, -1]
+    top_p = [1.0, 0.4, 0.9, 0.9, 0.9, 1.0, 0.5, 0.9, 0.9, 0.9, 0.5, 0.0]
+    for seed in range(8):
+        agree(both(x.cuda(), temperature, top_k, top_p, [0.0] * n, seed), n)
+        agree(both(x.cuda(), temperature, top_k, top_p, [0.001] * n, seed), n)
