@@ -65,12 +65,18 @@ class Sampler:
         words[: 2 * n].view(np.int64)[:] = seeds
         f = words[2 * n : 5 * n].view(np.float32).reshape(3, n)
         i = words[5 * n : 7 * n].reshape(2, n)
-        for r, p in enumerate(params):
-            f[0, r] = 0.0 if p.greedy else p.temperature
-            f[1, r] = p.top_p
-            f[2, r] = p.min_p
-            i[0, r] = 1 if p.greedy else min(p.top_k, 2**31 - 1)
-            i[1, r] = draw_index[r]
+        # a list a parameter, and the rest on whole rows: a busy server's step has as many rows as requests
+        temperature, top_k = np.array([p.temperature for p in params], np.float64), np.array([p.top_k for p in params])
+        top_p, min_p = np.array([p.top_p for p in params], np.float64), np.array([p.min_p for p in params], np.float64)
+        greedy = (temperature == 0) | (top_k == 1)  # (``SamplingParams.greedy``)
+        f[0], f[1], f[2] = np.where(greedy, 0.0, temperature), top_p, min_p
+        i[0], i[1] = np.where(greedy, 1, np.minimum(top_k, 2**31 - 1)), draw_index
+        vocab = logits.shape[1]
+        by_k, by_p, by_min = (top_k > 0) & (top_k < vocab), top_p < 1.0, min_p > 0.0
+        unfiltered = not np.any(~greedy & (by_k | by_p | by_min))
+        # top-k, top-p and min-p all at once in one row: top-p then refers to what top-k kept,
+        # two searches one after the other
+        late = bool(np.any(~greedy & by_k & by_p & by_min))
         dev = torch.empty(7 * n, dtype=torch.int32, device=self.device)
         dev.copy_(host[: 7 * n], non_blocking=True)
         if self.device.type == "cuda":
@@ -80,10 +86,5 @@ class Sampler:
         fd = dev[2 * n : 5 * n].view(torch.float32).view(3, n)
         idv = dev[5 * n : 7 * n].view(2, n)
         sd = dev[: 2 * n].view(torch.int64)
-        vocab = logits.shape[1]
-        unfiltered = all(p.greedy or (not 0 < p.top_k < vocab and p.top_p >= 1.0 and p.min_p <= 0.0) for p in params)
-        # top-k, top-p and min-p all at once in one row: top-p then refers to what top-k kept,
-        # two searches one after the other
-        late = any(not p.greedy and 0 < p.top_k < vocab and p.top_p < 1.0 and p.min_p > 0.0 for p in params)
         return ops.sample(logits.contiguous(), fd[0], idv[0], fd[1], fd[2], sd, idv[1],
-                          all_greedy=all(p.greedy for p in params), unfiltered=unfiltered, spread=True, late=late)
+                          all_greedy=bool(greedy.all()), unfiltered=unfiltered, spread=True, late=late)
