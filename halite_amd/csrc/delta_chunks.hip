@@ -23,7 +23,7 @@
 // gate in a pass of their own: requests of 225, 450, 675 and 900 tokens 505 -> 192 us, one of 2,048 690 -> 290, one of 8,192
 // 2,640 -> 1,150, one of 300 128 -> 61, 32 of 16 tokens each 125 -> 86.  Distance from 64 bits (2-norm) of the normed rows
 // 1.55e-7 beside 1.47e-7, of the states 1.0e-7 beside 0.96e-7, largest differences 2.5e-7 beside 3.1e-7.
-#include "hal_common.h"
+#include "hal_lds.h"
 #include "hal_api.h"
 
 #define DK_D 64          // channels of a head
@@ -103,11 +103,6 @@ __device__ __forceinline__ bool dk_locate(const int* __restrict__ seg_q_len, int
     before += __shfl(upto, HAL_WAVE - 1, HAL_WAVE);
   }
   return false;
-}
-
-typedef __amdgpu_buffer_rsrc_t dk_memory;
-__device__ __forceinline__ dk_memory dk_memory_at(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
 }
 
 // ---- a chunk's record: a wave takes one head of one chunk.  Lane l is key channel l with all tokens in registers
@@ -207,7 +202,7 @@ delta_chunk_prep_kernel(const float* __restrict__ r, int ldr, const float* __res
   // what the tokens contribute; a place past the chunk's tokens decays nothing and adds nothing
   const float bias0 = to_f32(w0[ch0 + lane]), bias_a = to_f32(a_bias[ch0 + lane]);
   // (what lies past the record's bytes is not written: a wave without a head has a record of none)
-  const dk_memory rec = dk_memory_at(records + ((size_t)blockIdx.x * H + h) * DK_RECORD, real ? DK_RECORD * 4 : 0);
+  const hal_memory rec = hal_memory_at(records + ((size_t)blockIdx.x * H + h) * DK_RECORD, real ? DK_RECORD * 4 : 0);
   auto put = [&](float value, int at, bool if_lane = true) {
     __builtin_amdgcn_raw_buffer_store_b32(__float_as_uint(value), rec, if_lane ? lane * 4 : DK_RECORD * 4, at * 4, 0);
   };
@@ -308,18 +303,6 @@ delta_chunk_prep_kernel(const float* __restrict__ r, int ldr, const float* __res
   for (int t = 0; t < DK_TOKENS; ++t) put(x[1][t], DK_WM + t * DK_SMALL, lane < 16), put(y[1][t], DK_N + t * DK_SMALL, lane < 16);
 }
 
-// 16 bytes a lane from memory straight into LDS: lane l's from byte `each` (its own) + `all` of `from` to `to` + 16 l
-__device__ __forceinline__ void dk_load_lds(dk_memory from, uint32_t each, uint32_t all, float* to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, each, all, 0, 0);
-}
-// Until all but the last `LEFT` accesses to memory of this wave are done, and then until every wave is here.
-template <int LEFT>
-__device__ __forceinline__ void dk_meet() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-  __builtin_amdgcn_sched_barrier(0);
-}
-
 struct DeltaGate {  // of the heads' results: y / rms(y over the head) * weight * sigmoid(z)
   const float* z;
   int ldz;
@@ -362,7 +345,7 @@ delta_chunk_scan_kernel(const float* __restrict__ records, const float* __restri
       for (int i = 0; i < 4; ++i) Z[j][i] = st[(16 * j + 4 * g + i) * DK_D];
     __builtin_amdgcn_s_setprio(2);  // (the other waves have time)
     auto advance = [&](int c, const float* mine) {
-      dk_meet<0>();
+      hal_meet<0>();
       dk_f32x4 val, wu[DK_TILES], kt[DK_TILES], et[DK_TILES], add[DK_TILES], gone[DK_TILES], qs[DK_TILES];
       const dk_f32x4 wm = *(const dk_f32x4*)(mine + DK_WM + own16);
 #pragma unroll
@@ -412,8 +395,8 @@ delta_chunk_scan_kernel(const float* __restrict__ records, const float* __restri
     for (int j = 0; j < DK_TILES; ++j)
 #pragma unroll
       for (int i = 0; i < 4; ++i) st[(16 * j + 4 * g + i) * DK_D] = Z[j][i];
-    dk_meet<0>();  // (the others are two chunks behind)
-    dk_meet<0>();
+    hal_meet<0>();  // (the others are two chunks behind)
+    hal_meet<0>();
     return;
   }
 
@@ -423,17 +406,17 @@ delta_chunk_scan_kernel(const float* __restrict__ records, const float* __restri
   // (no branch: past the end the last chunk comes again and is not used)
   auto bring = [&](int chunk, float* to) {
     const int c = chunk < chunks ? chunk : chunks - 1;
-    const dk_memory rec = dk_memory_at(rec0 + (size_t)c * H * DK_RECORD, DK_RECORD * 4);
+    const hal_memory rec = hal_memory_at(rec0 + (size_t)c * H * DK_RECORD, DK_RECORD * 4);
 #pragma unroll
-    for (int j = 0; j < 5; ++j) dk_load_lds(rec, in_record, (j * 4 + wave) * 1024, to + (j * 4 + wave) * 256);
+    for (int j = 0; j < 5; ++j) hal_load_lds(rec, in_record, (j * 4 + wave) * 1024, to + (j * 4 + wave) * 256);
     const int before = c * DK_TOKENS, have = n - before < DK_TOKENS ? n - before : DK_TOKENS;
     int tok = wave * 4 + g;
     tok = tok < have ? tok : have - 1;
     const size_t row = t0 + before;
-    const dk_memory values = dk_memory_at(v + row * ldv + first, (uint32_t)((have - 1) * ldv + DK_D) * 4);
-    const dk_memory gates = dk_memory_at(gate.z + row * gate.ldz + first, (uint32_t)((have - 1) * gate.ldz + DK_D) * 4);
-    dk_load_lds(values, (uint32_t)(tok * ldv) * 4 + in_row, 0, to + DK_VALUES + wave * 256);
-    dk_load_lds(gates, (uint32_t)(tok * gate.ldz) * 4 + in_row, 0, to + DK_GATES + wave * 256);
+    const hal_memory values = hal_memory_at(v + row * ldv + first, (uint32_t)((have - 1) * ldv + DK_D) * 4);
+    const hal_memory gates = hal_memory_at(gate.z + row * gate.ldz + first, (uint32_t)((have - 1) * gate.ldz + DK_D) * 4);
+    hal_load_lds(values, (uint32_t)(tok * ldv) * 4 + in_row, 0, to + DK_VALUES + wave * 256);
+    hal_load_lds(gates, (uint32_t)(tok * gate.ldz) * 4 + in_row, 0, to + DK_GATES + wave * 256);
   };
   // of the rows that are written this lane has token 4 wave + g, columns 4 (l % 16) .. + 3
   const int mine_at = (4 * wave + g) * DK_ROW + 4 * col16;
@@ -443,7 +426,7 @@ delta_chunk_scan_kernel(const float* __restrict__ records, const float* __restri
   T* const to = out + (size_t)(t0 + 4 * wave + g) * H * DK_D + first + 4 * col16;
   // Turn c: the record of chunk c - 1 is in `last`, that of chunk c + 2 goes to `free`.
   auto turn = [&](int c, const float* last, float* free) {
-    dk_meet<DK_LOADS>();  // (chunk c is there, the next one may be on its way)
+    hal_meet<DK_LOADS>();  // (chunk c is there, the next one may be on its way)
     bring(c + 2, free);
     __builtin_amdgcn_sched_barrier(0);
     dk_f32x4 Z[DK_TILES], x[DK_TILES], os[DK_TILES], val;

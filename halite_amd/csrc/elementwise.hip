@@ -214,11 +214,34 @@ __global__ void rmsnorm_kernel(float* __restrict__ h, const T* __restrict__ delt
 // access, all loads issued before the first use.  d is a multiple of 4 and at most
 // 4 * RMS_MAXV * blockDim.x.
 #define RMS_MAXV 8
-template <typename T>
+// The sum of four neighbouring numbers over planes, in the planes' order; their loads are on their way four at a time.
+__device__ __forceinline__ void planes_sum4(const float* p, int n_planes, size_t stride, float (&sum)[4]) {
+  load4(p, sum);
+  int j = 1;
+  for (; j + 4 <= n_planes; j += 4) {
+    float v[4][4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) load4(p + (j + u) * stride, v[u]);
+#pragma unroll
+    for (int u = 0; u < 4; ++u)
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i] += v[u][i];
+  }
+  for (; j < n_planes; ++j) {
+    float v[4];
+    load4(p + j * stride, v);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) sum[i] += v[i];
+  }
+}
+
+// PLANES: delta is the sum of n_planes float32 planes [rows][d], rounded to T as a delta in one piece is.
+template <typename T, bool PLANES = false>
 __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const T* __restrict__ delta,
                                    const int* __restrict__ rows, const void* __restrict__ w,
                                    int w_dtype, float eps, T* __restrict__ out, int d,
-                                   int update_h) {
+                                   int update_h, const float* __restrict__ planes = nullptr, int n_planes = 0,
+                                   size_t plane_stride = 0) {
   __shared__ float scratch[16];
   const int r = blockIdx.x;
   const int src = rows ? rows[r] : r;
@@ -238,13 +261,19 @@ __global__ void rmsnorm_vec_kernel(float* __restrict__ h, const T* __restrict__ 
       load4_any(w, w_dtype, (size_t)v * 4, wv[u]);
     }
   }
-  if (dr) {
+  if (PLANES || dr) {
 #pragma unroll
     for (int u = 0; u < RMS_MAXV; ++u) {
       const int v = threadIdx.x + u * blockDim.x;
       if (v < nv) {
         float dv[4];
-        load4(dr + v * 4, dv);
+        if constexpr (PLANES) {
+          planes_sum4(planes + (size_t)src * d + v * 4, n_planes, plane_stride, dv);
+#pragma unroll
+          for (int i = 0; i < 4; ++i) dv[i] = to_f32(from_f32<T>(dv[i]));
+        } else {
+          load4(dr + v * 4, dv);
+        }
 #pragma unroll
         for (int i = 0; i < 4; ++i) x[u][i] += dv[i];
         if (update_h) store4(hr + v * 4, x[u]);
@@ -307,6 +336,46 @@ extern "C" int hal_rmsnorm(float* h, const void* delta, const int* rows, const v
     launch_rmsnorm<bf16_t>(h, delta, rows, w, w_dtype, eps, out, n_rows, d, update_h, stream);
   else
     return hal_fail("hal_rmsnorm: unknown dtype %d", dtype);
+  HAL_LAUNCH_CHECK();
+  return 0;
+}
+
+extern "C" int hal_rmsnorm_planes(float* h, const float* planes, int n_planes, int plane_rows, const int* rows, const void* w,
+                                  int w_dtype, float eps, void* out, int n_rows, int d, hipStream_t stream) {
+  HAL_REQUIRE(n_rows >= 0 && (rows || n_rows == plane_rows) && d > 0 && d % 4 == 0 && d <= 4096 * RMS_MAXV && n_planes > 0, "hal_rmsnorm_planes: bad sizes rows=%d d=%d planes=%d",
+              n_rows, d, n_planes);
+  HAL_REQUIRE(w_dtype == HAL_F32 || w_dtype == HAL_BF16, "hal_rmsnorm_planes: weight dtype %d", w_dtype);
+  HAL_REQUIRE((uintptr_t)h % 16 == 0 && (uintptr_t)planes % 16 == 0 && (uintptr_t)out % 8 == 0 &&
+                  (uintptr_t)w % (w_dtype == HAL_F32 ? 16 : 8) == 0, "hal_rmsnorm_planes: alignment");
+  if (n_rows == 0) return 0;
+  int threads = (d / 4 + HAL_WAVE - 1) / HAL_WAVE * HAL_WAVE;
+  threads = threads > 1024 ? 1024 : threads;
+  hipLaunchKernelGGL((rmsnorm_vec_kernel<bf16_t, true>), dim3(n_rows), dim3(threads), 0, stream, h, (const bf16_t*)nullptr,
+                     rows, w, w_dtype, eps, (bf16_t*)out, d, rows == nullptr, planes, n_planes, (size_t)plane_rows * d);
+  HAL_LAUNCH_CHECK();
+  return 0;
+}
+
+template <typename T>
+__global__ void sum_planes_kernel(const float* __restrict__ planes, int n_planes, T* __restrict__ out, size_t n4) {
+  for (size_t v = (size_t)blockIdx.x * blockDim.x + threadIdx.x; v < n4; v += (size_t)gridDim.x * blockDim.x) {
+    float sum[4];
+    planes_sum4(planes + v * 4, n_planes, n4 * 4, sum);
+    store4(out + v * 4, sum);
+  }
+}
+
+extern "C" int hal_sum_planes(const float* planes, int n_planes, void* out, int dtype, long long n, hipStream_t stream) {
+  HAL_REQUIRE(n >= 0 && n % 4 == 0 && n_planes > 0 && (uintptr_t)planes % 16 == 0 && (uintptr_t)out % 16 == 0,
+              "hal_sum_planes: %lld numbers of %d planes, or their places", n, n_planes);
+  HAL_REQUIRE(dtype == HAL_F32 || dtype == HAL_BF16, "hal_sum_planes: dtype %d", dtype);
+  if (n == 0) return 0;
+  const long long blocks = (n / 4 + 255) / 256;
+  const dim3 grid((unsigned)(blocks < 2048 ? blocks : 2048));
+  if (dtype == HAL_F32)
+    hipLaunchKernelGGL(sum_planes_kernel<float>, grid, dim3(256), 0, stream, planes, n_planes, (float*)out, (size_t)n / 4);
+  else
+    hipLaunchKernelGGL(sum_planes_kernel<bf16_t>, grid, dim3(256), 0, stream, planes, n_planes, (bf16_t*)out, (size_t)n / 4);
   HAL_LAUNCH_CHECK();
   return 0;
 }
@@ -847,6 +916,95 @@ rope_append_group_kernel(T* __restrict__ qkv, int row_stride, const int* __restr
 #pragma unroll
     for (int e = 0; e < 8; ++e) vp[kv_value_offset(tiled, page_size, D, s_off[i], d + e)] = vals[e];
   }
+}
+
+// The same for rows that lie as float32 planes (bf16 pages, pairs half a head apart, whole heads rotated): a workgroup
+// takes a share of a token's work, 128 pieces of eight pairs of q or k or of eight values, as the planes are
+// several times the rows' bytes and a token's alone keep a compute unit busy for 5 us.
+#define RP_THREADS 128
+__global__ void __launch_bounds__(RP_THREADS)
+rope_append_planes_kernel(const float* __restrict__ planes, int n_planes, bf16_t* __restrict__ q_out, const int* __restrict__ positions,
+                          const int* __restrict__ token_seg, const int* __restrict__ block_table, int bt_stride,
+                          const float* __restrict__ cos_t, const float* __restrict__ sin_t, int table_len, bf16_t* __restrict__ k_pages,
+                          bf16_t* __restrict__ v_pages, int H, int K, int D, int page_size, int n_pages, bool tiled) {
+  const int t = blockIdx.x, half = D / 2, cph = half / 8, turned = (H + K) * cph;
+  const int idx = blockIdx.y * RP_THREADS + threadIdx.x;
+  if (idx >= turned + K * (D / 8)) return;
+  const size_t row = (size_t)(H + 2 * K) * D, stride = gridDim.x * row;
+  const float* from = planes + t * row;
+  // (the row's pieces do not depend on the position: asked for before it is looked at)
+  const bool value = idx >= turned;
+  const int head = value ? H + K + (idx - turned) / (D / 8) : idx / cph, j = value ? (idx - turned) % (D / 8) * 8 : idx % cph * 8;
+  const int other = value ? j + 4 : j + half;  // the second four numbers of a value's eight; of a pair's partners the first
+  float a[2][4], b[2][4];
+  planes_sum4(from + (size_t)head * D + j, n_planes, stride, a[0]);
+  planes_sum4(from + (size_t)head * D + other, n_planes, stride, b[0]);
+  if (!value) {
+    planes_sum4(from + (size_t)head * D + j + 4, n_planes, stride, a[1]);
+    planes_sum4(from + (size_t)head * D + other + 4, n_planes, stride, b[1]);
+  }
+  const int pos = positions[t];
+  if (pos < 0 || pos >= table_len) return;
+  long long page = -1;
+  if (head >= H) {
+    page = block_table[(size_t)token_seg[t] * bt_stride + pos / page_size];
+    if (page < 0 || page >= n_pages) return;
+  }
+  const int off = pos % page_size;
+  if (value) {
+    bf16_t* vp = v_pages + ((size_t)page * K + (head - H - K)) * D * page_size;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      vp[kv_value_offset(tiled, page_size, D, off, j + i)] = f32_to_bf16(a[0][i]);
+      vp[kv_value_offset(tiled, page_size, D, off, j + 4 + i)] = f32_to_bf16(b[0][i]);
+    }
+    return;
+  }
+  float c[2][4], sn[2][4], y0[2][4], y1[2][4];
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    load4(cos_t + (size_t)pos * half + j + 4 * u, c[u]);
+    load4(sin_t + (size_t)pos * half + j + 4 * u, sn[u]);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      // the product is rounded to bf16 before the rotation, as rows in one piece are stored
+      const float x0 = to_f32(f32_to_bf16(a[u][i])), x1 = to_f32(f32_to_bf16(b[u][i]));
+      y0[u][i] = x0 * c[u][i] - x1 * sn[u][i];
+      y1[u][i] = x0 * sn[u][i] + x1 * c[u][i];
+    }
+  }
+  bf16_t* qp = q_out + ((size_t)t * H + head) * D;
+  bf16_t* kp = head >= H ? k_pages + ((size_t)page * K + (head - H)) * page_size * D : nullptr;
+#pragma unroll
+  for (int u = 0; u < 2; ++u) {
+    if (kp) {
+      store4(kp + kv_key_offset(tiled, page_size, D, off, j + 4 * u), y0[u]);
+      store4(kp + kv_key_offset(tiled, page_size, D, off, j + half + 4 * u), y1[u]);
+    } else {
+      store4(qp + j + 4 * u, y0[u]);
+      store4(qp + j + half + 4 * u, y1[u]);
+    }
+  }
+}
+
+extern "C" int hal_rope_append_planes(const float* planes, int n_planes, void* q_out, const int* positions, const int* token_seg,
+                                      const int* block_table, int bt_stride, const float* cos_t, const float* sin_t, int table_len,
+                                      void* k_pages, void* v_pages, int n_tokens, int H, int K, int D, int page_size, int n_pages,
+                                      int tiled, hipStream_t stream) {
+  HAL_REQUIRE(n_tokens >= 0 && n_planes > 0 && H > 0 && K > 0 && D > 0 && D % 16 == 0, "hal_rope_append_planes: bad sizes");
+  HAL_REQUIRE(planes && q_out && positions && token_seg && block_table && cos_t && sin_t && k_pages && v_pages && page_size > 0 &&
+                  n_pages > 0 && table_len > 0, "hal_rope_append_planes: arguments missing");
+  HAL_REQUIRE((uintptr_t)planes % 16 == 0 && (uintptr_t)q_out % 8 == 0 && (uintptr_t)cos_t % 16 == 0 && (uintptr_t)sin_t % 16 == 0 &&
+                  (uintptr_t)k_pages % 8 == 0, "hal_rope_append_planes: alignment");
+  HAL_REQUIRE(!tiled || (page_size % 32 == 0 && D % 32 == 0), "hal_rope_append_planes: the tiled page layout needs pages and heads of a "
+              "multiple of 32 (page %d, head %d)", page_size, D);
+  if (n_tokens == 0) return 0;
+  const int items = (H + K) * (D / 16) + K * (D / 8);
+  hipLaunchKernelGGL(rope_append_planes_kernel, dim3(n_tokens, (items + RP_THREADS - 1) / RP_THREADS), dim3(RP_THREADS), 0, stream, planes,
+                     n_planes, (bf16_t*)q_out, positions, token_seg, block_table, bt_stride, cos_t, sin_t, table_len, (bf16_t*)k_pages,
+                     (bf16_t*)v_pages, H, K, D, page_size, n_pages, tiled != 0);
+  HAL_LAUNCH_CHECK();
+  return 0;
 }
 
 extern "C" int hal_rope_append(void* qkv, int dtype, int row_stride, const int* positions,

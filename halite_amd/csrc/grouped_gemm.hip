@@ -18,7 +18,7 @@
 // results leave as vector stores: streaming tiles of 64 x 128 for experts of few rows and for heads
 // (grouped_stream_kernel), and tiles of up to 256 x 256 for prompts' experts (grouped_wide_kernel).
 // gg_experts_kernel says which of the four takes an expert's product, and why.
-#include "hal_common.h"
+#include "hal_lds.h"
 #include "hal_api.h"
 #include <math.h>
 
@@ -311,11 +311,6 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
 // through a group's row tiles (eight at a time) column by column: one die reads an expert's weights,
 // once (tiles of two experts side by side cost a third more reads from memory and 8% of the time).
 //
-// LDS holds 8 rows x 64 k as one KiB, eight lanes of a load a row: the piece of eight k that lies
-// at place p of row r is piece p ^ gw_turn(r % 16).  A 16-byte read of a wave goes through LDS in turns of
-// sixteen lanes, lanes 0-3, 12-15 and 20-27 in one and 4-11, 16-19 and 28-31 in the next (and so on from
-// lane 32); each turn then meets all 64 banks once.
-//
 // Measured beside tiles of 128 x 128 in registers and LDS (grouped_mfma_kernel): 9,000 rows of 16 experts,
 // 4096 x 4096: 469 -> 300 us (644 -> 1,007 TFLOP/s); 18,000 rows of 64 experts, gate and up 1024 x 4096
 // each: 537 -> 400 us, down 4096 x 1024 into float32 rows 352 -> 280 us; 49,152 rows of 64: 1,127 -> 745 us;
@@ -346,28 +341,10 @@ __device__ __forceinline__ void gw_store(const GroupedArgs& a, int dst, int n, g
   else *(uint2*)((bf16_t*)a.Y + at) = make_uint2(pack_bf16x2(v[0], v[1]), pack_bf16x2(v[2], v[3]));
 }
 
-// 16 bytes a lane from memory straight into LDS: from byte `each` (a lane's own) + `all` of `from`, lane l's to
-// `to` (the same in all lanes) + 16 l.  (Buffer loads: the compiler waits for every load where it meets
-// one in the flat form that goes into LDS.)
-typedef __amdgpu_buffer_rsrc_t gw_rows;
-__device__ __forceinline__ gw_rows gw_rows_at(const void* p, uint32_t bytes) {
-  return __builtin_amdgcn_make_buffer_rsrc(const_cast<void*>(p), 0, bytes, 0x00020000);
-}
 // The rows of X, K columns from `col0` on: up to the end of the last row's, so that rows that overlap (a row
 // length below K, or 0 where one row stands for all) lie in the range like any others.
-__device__ __forceinline__ gw_rows gw_rows_of_x(const GroupedArgs& a, int col0) {
-  return gw_rows_at((const bf16_t*)a.X + col0, ((uint32_t)(a.x_rows - 1) * a.ldx + a.K) * 2);
-}
-__device__ __forceinline__ void gw_load_lds(gw_rows from, uint32_t each, uint32_t all, char* to) {
-  __builtin_amdgcn_raw_ptr_buffer_load_lds(from, (__attribute__((address_space(3))) void*)to, 16, each, all, 0, 0);
-}
-__device__ __forceinline__ int gw_turn(int r) { return ((r >> 1) & 1) | ((r >> 2) & 2) | (((r >> 1) ^ r) & 4); }
-// Until all but the last `left` loads of this wave are there, and then until every wave is here.
-template <int LEFT>
-__device__ __forceinline__ void gw_meet() {
-  __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(LEFT) : "memory");
-  __builtin_amdgcn_sched_barrier(0);
+__device__ __forceinline__ hal_memory gw_rows_of_x(const GroupedArgs& a, int col0) {
+  return hal_memory_at((const bf16_t*)a.X + col0, ((uint32_t)(a.x_rows - 1) * a.ldx + a.K) * 2);
 }
 
 // What one wave does for a tile of at most 32 * NI rows.  The two buffers are two arrays, so that the
@@ -377,11 +354,11 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
   constexpr int AI = (NI + 1) / 2, LOADS = AI + 4;  // a wave's loads a step: 8 rows of every 64 of X, and of W
   const int steps = a.K / GW_TK;                    // even
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), wm = wave / 4, wn = wave % 4;
-  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ gw_turn(lr % 16)) * 16;
+  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ hal_turn(lr % 16)) * 16;
   // (GATED: of every 64 W rows, a wave's, the first 32 are the gate's and the others the up projection's)
   const void* w0 = GATED && wave >= 4 ? a.W2 : a.W;
-  const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
-  const gw_rows X = gw_rows_of_x(a, a.x_col0);
+  const hal_memory W = hal_memory_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
+  const hal_memory X = gw_rows_of_x(a, a.x_col0);
   uint32_t xo[AI], wo[4];
   // rows and columns past the end are read from the last one: nothing of them is stored
 #pragma unroll
@@ -400,12 +377,12 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
   auto bring = [&](char* lds, int step) {
     const uint32_t at = (uint32_t)(step < steps ? step : steps - 1) * (GW_TK * 2);
 #pragma unroll
-    for (int i = 0; i < AI; ++i) gw_load_lds(X, xo[i], at, lds + (i * 8 + wave) * 1024);
+    for (int i = 0; i < AI; ++i) hal_load_lds(X, xo[i], at, lds + (i * 8 + wave) * 1024);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) gw_load_lds(W, wo[i], at, lds + GW_A_BYTES + (i * 8 + wave) * 1024);
+    for (int i = 0; i < 4; ++i) hal_load_lds(W, wo[i], at, lds + GW_A_BYTES + (i * 8 + wave) * 1024);
   };
   const int q = lane / 16, r16 = lane % 16;
-  const int get[2] = {r16 * 128 + (q ^ gw_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ gw_turn(r16)) * 16};
+  const int get[2] = {r16 * 128 + (q ^ hal_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ hal_turn(r16)) * 16};
   struct Operands {
     gg_bf16x8 w[4], x[NI];
   };
@@ -438,7 +415,7 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
       __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
     }
     multiply(high, 0, HALF);
-    gw_meet<0>();
+    hal_meet<0>();
     bring(mine, s + 2);
     read(next, 0, low);
     multiply(high, HALF, NI);
@@ -451,7 +428,7 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
   };
   bring(b0, 0);
   bring(b1, 1);
-  gw_meet<LOADS>();
+  hal_meet<LOADS>();
   read(b0, 0, low);
   for (int s = 0; s < steps; s += 2) {
     advance(s, b0, b1);
@@ -566,11 +543,11 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
   // the order of K, as in the other tiles: their bits do not depend on which of the three the rows' number takes.)
   const int begin = a.turn ? (n0 / (GATED ? GT_COLS / 2 : GT_COLS) * 7 + g * 13) % steps : 0;
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
-  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ gw_turn(lr % 16)) * 16;
+  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ hal_turn(lr % 16)) * 16;
   // (GATED: of every 32 W rows, a wave's, the first 16 are the gate's and the others the up projection's)
   const void* w0 = GATED && wave % 4 >= 2 ? a.W2 : a.W;
-  const gw_rows W = gw_rows_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
-  const gw_rows X = gw_rows_of_x(a, a.x_col0 + (HEADS ? g * a.x_group_cols : 0));
+  const hal_memory W = hal_memory_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
+  const hal_memory X = gw_rows_of_x(a, a.x_col0 + (HEADS ? g * a.x_group_cols : 0));
   uint32_t xo[AI], wo[4];
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
@@ -588,12 +565,12 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
     step = (step < steps ? step : steps - 1) + begin;
     const uint32_t at = (uint32_t)(step < steps ? step : step - steps) * (GW_TK * 2);
 #pragma unroll
-    for (int i = 0; i < AI; ++i) gw_load_lds(X, xo[i], at, lds + (i * 4 + wave) * 1024);
+    for (int i = 0; i < AI; ++i) hal_load_lds(X, xo[i], at, lds + (i * 4 + wave) * 1024);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) gw_load_lds(W, wo[i], at, lds + GT_A_BYTES + (i * 4 + wave) * 1024);
+    for (int i = 0; i < 4; ++i) hal_load_lds(W, wo[i], at, lds + GT_A_BYTES + (i * 4 + wave) * 1024);
   };
   const int q = lane / 16, r16 = lane % 16;
-  const int get[2] = {r16 * 128 + (q ^ gw_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ gw_turn(r16)) * 16};
+  const int get[2] = {r16 * 128 + (q ^ hal_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ hal_turn(r16)) * 16};
   gg_f32x4 acc[NI][2];
 #pragma unroll
   for (int i = 0; i < NI; ++i)
@@ -617,14 +594,14 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
   const int odd = steps % 3;
   for (int s = 0; s < odd; ++s) {
     bring(b0, s);
-    gw_meet<0>();
+    hal_meet<0>();
     multiply(b0);
-    gw_meet<0>();
+    hal_meet<0>();
   }
   bring(b0, odd);
   bring(b1, odd + 1);
   auto advance = [&](int s, const char* mine, char* free) {
-    gw_meet<LOADS>();  // (this step's pieces are there, the next one's may be on their way)
+    hal_meet<LOADS>();  // (this step's pieces are there, the next one's may be on their way)
     bring(free, s + 2);
     multiply(mine);
   };

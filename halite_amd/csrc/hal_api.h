@@ -140,6 +140,26 @@ int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const floa
                       void* state, void* hist, uint32_t* lists, int any_late, int* out_token,
                       float* out_logprob, hipStream_t stream);
 
+// ---- products of 17 to 64 rows, W streamed through LDS (gemm_stream.hip) ----------------------
+// C = X W^T (with W2: act(X W^T) * (X W2^T)) for bf16 operands.  hal_gemm_bf16_stream_parts: 0 where the product is not
+// taken, else in how many parts of K (more than 1 only with may_part).  One part: Y [M, N] bf16 or float32; more:
+// float32 planes [parts][M][N] whose sum, in order, is the result.
+int hal_gemm_bf16_stream_parts(int N, int K, int gated, int may_part);
+int hal_gemm_bf16_stream(const void* X, int ldx, const void* W, const void* W2, int ldw, void* Y, int y_dtype,
+                         int parts, int act, float limit, float alpha, float up_shift, int M, int N, int K,
+                         hipStream_t stream);
+// What reads such planes: the residual add and norm (bf16; the sum is rounded to bf16 as a result in one piece is; of `rows`
+// alone the stream is not updated), the
+// rotation of whole heads in half-split pairs with the append (q to q_out [n, H * D], k and v to the pages), or a sum
+// rounded to `dtype`.
+int hal_rmsnorm_planes(float* h, const float* planes, int n_planes, int plane_rows, const int* rows, const void* w, int w_dtype,
+                       float eps, void* out, int n_rows, int d, hipStream_t stream);
+int hal_rope_append_planes(const float* planes, int n_planes, void* q_out, const int* positions, const int* token_seg,
+                           const int* block_table, int bt_stride, const float* cos_t, const float* sin_t, int table_len,
+                           void* k_pages, void* v_pages, int n_tokens, int H, int K, int D, int page_size, int n_pages,
+                           int tiled, hipStream_t stream);
+int hal_sum_planes(const float* planes, int n_planes, void* out, int dtype, long long n, hipStream_t stream);
+
 // ---- products in groups (grouped_gemm.hip) ---------------------------------------------
 // Y_g = X_g * W_g^T for G groups in one launch, float32 accumulation; operands of `dtype`.
 // Group g reads the columns from g * x_group_cols + x_col0 of X's rows (row length ldx) and

@@ -42,6 +42,7 @@ CORE_SOURCES = [
     "attention_simple.hip",
     "gemm_f32.hip",
     "gemm_bf16.hip",
+    "gemm_stream.hip",
     "sampling.hip",
     "grouped_gemm.hip",
     "latent_moe.hip",

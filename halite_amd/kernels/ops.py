@@ -9,6 +9,7 @@ functions: without a GPU and the built library they raise.
 from __future__ import annotations
 
 import ctypes
+import functools
 import math
 from dataclasses import dataclass
 
@@ -79,6 +80,10 @@ class NextNorm:
     h: torch.Tensor
     weight: torch.Tensor
     eps: float
+    sums: bool = False
+    """The norm adds up ``PartialSums`` itself."""
+    gathers: bool = False
+    """The norm reads some of the rows: it takes no ``NormedRows``."""
 
 
 @dataclass
@@ -112,6 +117,25 @@ class NormedRows:
         out = torch.empty((m, d), dtype=torch.bfloat16, device=x.device)
         _check(lib, lib.hal_scale_normed_rows(
             _ptr(x), x.stride(0), _ptr(ss), ss.shape[0], ss.shape[1], ctypes.c_float(self.eps), _ptr(out), m, d, _stream()))
+        return out
+
+
+@dataclass
+class PartialSums:
+    """A product's result as float32 planes ``[parts, rows, columns]`` that its reader adds up in order: what
+    ``linear`` returns to a caller that says ``sums``."""
+
+    planes: torch.Tensor
+
+    @property
+    def shape(self):
+        return self.planes.shape[1:]
+
+    def materialize(self, dtype: torch.dtype) -> torch.Tensor:
+        lib = library.core_library()
+        out = torch.empty(tuple(self.shape), dtype=dtype, device=self.planes.device)
+        _check(lib, lib.hal_sum_planes(_ptr(self.planes), self.planes.shape[0], _ptr(out), dtype_code(dtype),
+                                       ctypes.c_longlong(out.numel()), _stream()))
         return out
 
 
@@ -209,18 +233,33 @@ def take_tokens(src: torch.Tensor, tokens: torch.Tensor) -> None:
     _check(lib, lib.hal_take_tokens(_ptr(src), src.numel(), _ptr(tokens), tokens.numel(), _stream()))
 
 
+RMS_PLANES_WIDTH = 16384  # what the norm's kernel holds of a row
+
+
 def rmsnorm(
     h: torch.Tensor,
     weight: torch.Tensor,
     eps: float,
     out_dtype: torch.dtype,
-    delta: torch.Tensor | None = None,
+    delta: torch.Tensor | PartialSums | None = None,
     rows: torch.Tensor | None = None,
     update_h: bool = True,
 ):
     """RMSNorm of the float32 stream ``h`` (+ ``delta``), optionally only of
     ``rows``; with ``delta`` and ``update_h`` the sum is written back to ``h``."""
     lib = library.core_library()
+    if isinstance(delta, PartialSums):
+        if update_h and out_dtype == torch.bfloat16 and h.shape[1] % 4 == 0 and h.shape[1] <= RMS_PLANES_WIDTH:
+            planes, (n_tokens, d) = delta.planes, h.shape
+            n_rows = n_tokens if rows is None else rows.numel()
+            _dev(h, weight, planes, rows)
+            _i32(rows, "rows")
+            _need(h.dtype == torch.float32 and h.is_contiguous() and planes.shape[1:] == h.shape and weight.shape == (d,), "rmsnorm: bad planes")
+            out = torch.empty((n_rows, d), dtype=out_dtype, device=h.device)
+            _check(lib, lib.hal_rmsnorm_planes(_ptr(h), _ptr(planes), planes.shape[0], n_tokens, _ptr(rows), _ptr(weight),
+                                               dtype_code(weight.dtype), ctypes.c_float(eps), _ptr(out), n_rows, d, _stream()))
+            return out
+        delta = delta.materialize(out_dtype)
     _dev(h, weight, delta, rows)
     _i32(rows, "rows")
     _need(h.dtype == torch.float32 and h.dim() == 2, "rmsnorm: the stream is float32 [T, d]")
@@ -338,6 +377,31 @@ def rope_append(
             page_size, n_pages, 1 if tiled else 0, _stream(),
         ),
     )
+
+
+def rope_append_sums(qkv: PartialSums, positions: torch.Tensor, cos: torch.Tensor, sin: torch.Tensor, n_heads: int,
+                     n_kv_heads: int, head_dim: int, token_seg: torch.Tensor, block_table: torch.Tensor, k_pages: torch.Tensor,
+                     v_pages: torch.Tensor, page_size: int, tiled: bool) -> torch.Tensor:
+    """``rope_append`` of packed rows that come as planes: whole heads of bf16 pages rotated in pairs half a head
+    apart.  Returns the rotated queries ``[n, heads * dim]``; keys and values go to the pages."""
+    lib = library.core_library()
+    planes = qkv.planes
+    _dev(planes, positions, cos, sin, token_seg, block_table, k_pages, v_pages)
+    _i32(positions, "positions"), _i32(token_seg, "token_seg"), _i32(block_table, "block_table")
+    n, width = qkv.shape
+    _need(positions.numel() == n and token_seg.numel() == n and block_table.dim() == 2, "rope_append_sums: segment arrays")
+    _need(width == (n_heads + 2 * n_kv_heads) * head_dim, "rope_append_sums: row length")
+    _need(cos.dtype == torch.float32 and cos.shape == sin.shape and cos.shape[1] == head_dim // 2, "rope tables are float32 [positions, dim / 2]")
+    n_pages = k_pages.shape[0]
+    _need(k_pages.dtype == torch.bfloat16 and v_pages.dtype == torch.bfloat16
+          and k_pages.shape == (n_pages, n_kv_heads, page_size, head_dim)
+          and v_pages.shape == (n_pages, n_kv_heads, head_dim, page_size), "rope_append_sums: bf16 pages")
+    q = torch.empty((n, n_heads * head_dim), dtype=torch.bfloat16, device=planes.device)
+    _check(lib, lib.hal_rope_append_planes(
+        _ptr(planes), planes.shape[0], _ptr(q), _ptr(positions), _ptr(token_seg), _ptr(block_table), block_table.shape[1],
+        _ptr(cos), _ptr(sin), cos.shape[0], _ptr(k_pages), _ptr(v_pages), n, n_heads, n_kv_heads, head_dim, page_size, n_pages,
+        1 if tiled else 0, _stream()))
+    return q
 
 
 def pair_rows_for_rotation(w_qkv: torch.Tensor, head_dim: int) -> torch.Tensor:
@@ -552,6 +616,7 @@ def sample(
 SKINNY_MAX_ROWS = 64  # what the kernel takes
 SKINNY_ROWS = 16  # up to here it beats the library product
 FUSED_ROWS = 32  # what the epilogues that take other kernels' work take
+FUSED_BEST_ROWS = 20  # up to here they are the fastest way (``streams_instead``)
 FUSED_MID_ELEMENTS = 32 * 1024 * 1024  # the largest matrix on which they pay at 17 to 32 rows
 GATED_MID_ELEMENTS = 64 * 1024 * 1024  # the same for the gated product with SiLU*mul (each of its two matrices)
 # ... if the weights lie in its tiled order.  On row-major weights (a model too large for
@@ -638,6 +703,42 @@ def gemm_bf16_skinny(
     return out
 
 
+STREAM_ROWS = 64  # what the streaming product takes; from SKINNY_ROWS + 1 on
+
+
+@functools.lru_cache(maxsize=None)
+def _stream_parts(n: int, k: int, gated: bool, may_part: bool) -> int:
+    return library.core_library().hal_gemm_bf16_stream_parts(n, k, 1 if gated else 0, 1 if may_part else 0)
+
+
+def stream_parts(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, may_part: bool = False) -> int:
+    """In how many parts of K the streaming product takes ``x`` [17 to 64, k] against the bf16 weight ``w`` of ``n``
+    rows (``gated``: two of them); 0: another is the faster one, or it has none for these sizes or places."""
+    m, k = x.shape
+    if not (SKINNY_ROWS < m <= STREAM_ROWS and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.is_cuda
+            and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k and x.data_ptr() % 16 == 0 and w.stride(1) == 1
+            and w.stride(0) % 8 == 0 and w.stride(0) >= k and w.data_ptr() % 16 == 0 and n * w.stride(0) * 2 < 2**31):
+        return 0
+    return _stream_parts(n, k, gated, may_part)
+
+
+def gemm_bf16_stream(x: torch.Tensor, w: torch.Tensor, parts: int, w_up: torch.Tensor | None = None,
+                     out_dtype: torch.dtype = torch.bfloat16, activation: str = "silu", clamp: Clamp = Clamp()):
+    """``x @ w.T`` for 17 to 64 rows in the ``parts`` that ``stream_parts`` named: one gives the result, more give
+    ``PartialSums``; with ``w_up`` (one part) the gated form ``(x @ w_up.T) * act(x @ w.T)``."""
+    lib = library.core_library()
+    _need(x.is_cuda and w.is_cuda and (w_up is None or w_up.is_cuda), "kernel arguments must be on the GPU")
+    (m, k), n = x.shape, w.shape[0]
+    _need(w.shape[1] == k and (w_up is None or (w_up.shape == w.shape and w_up.stride() == w.stride() and w_up.dtype == w.dtype)),
+          "streaming product: weights' shapes")
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.stride(1) == 1, "streaming product: bf16 rows")
+    out = torch.empty((parts, m, n) if parts > 1 else (m, n), dtype=torch.float32 if parts > 1 else out_dtype, device=x.device)
+    _check(lib, lib.hal_gemm_bf16_stream(
+        _ptr(x), x.stride(0), _ptr(w), _ptr(w_up), w.stride(0), _ptr(out), dtype_code(out.dtype), parts, GATE_ACTIVATIONS[activation],
+        *clamp.args(), m, n, k, _stream()))
+    return PartialSums(out) if parts > 1 else out
+
+
 def norm_folds(m: int, n: int, k: int, tiled: torch.Tensor | None) -> bool:
     """Whether a product of ``m`` rows against an ``[n, k]`` weight with a tiled copy
     takes an RMSNorm before or after it, or the rotation and the append, into itself: up
@@ -650,6 +751,19 @@ def norm_folds(m: int, n: int, k: int, tiled: torch.Tensor | None) -> bool:
     # library product and a norm kernel; down 4096 x 14336 36-41 against 33-35, and
     # 3072 x 8192 22-25 against 21-22: two row tiles read the long rows of X twice as often)
     return m <= SKINNY_ROWS or (m <= FUSED_ROWS and n * k <= FUSED_MID_ELEMENTS and k <= 2 * n)
+
+
+def fold_pays(x: torch.Tensor | NormedRows, w: torch.Tensor, tiled: torch.Tensor | None) -> bool:
+    """Whether a product that ``norm_folds`` is to do so: not where the streaming product takes as many rows."""
+    (m, k), n = x.shape, w.shape[0]
+    return norm_folds(m, n, k, tiled) and not streams_instead(x, w, n)
+
+
+def streams_instead(x: torch.Tensor | NormedRows, w: torch.Tensor, n: int, gated: bool = False) -> bool:
+    """Whether the streaming product and the kernels between products beat the small-batch product with their work
+    in its epilogues (steps of 8 layers of the 8B shape: 17 rows 1,057 us against 1,012, 24 1,080 / 1,098, 32 1,136 / 1,197;
+    of the 3B shape 678 / 682, 694 / 717, 733 / 795)."""
+    return x.shape[0] > FUSED_BEST_ROWS and stream_parts(x.x if isinstance(x, NormedRows) else x, w, n, gated, may_part=True) > 0
 
 
 def gemm_bf16_skinny_norm(
@@ -709,15 +823,15 @@ def linear_add(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, tiled: torch.T
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = None,
-           tiled: torch.Tensor | None = None, next_norm: NextNorm | None = None):
+           tiled: torch.Tensor | None = None, next_norm: NextNorm | None = None, sums: bool = False):
     """``x @ w.T`` for a weight ``[out, in]``; ``tiled`` is ``tile_weight(w)`` if the
     model keeps that copy for small batches.  ``x`` may be ``NormedRows``; with
     ``next_norm`` the result may come back as ``NormedRows`` (already added into the
-    stream) instead of a tensor.
+    stream) instead of a tensor, with ``sums`` (or a norm that says so) as ``PartialSums``.
 
     float32 weights: the true 32-bit kernel (activations are widened if needed).
-    bf16 weights: the hand-written kernel where it is the faster one (``skinny_pays``:
-    up to 16 rows); otherwise the library product that the reference itself uses for
+    bf16 weights: the hand-written kernels where they are the faster ones (``skinny_pays``:
+    up to 16 rows; ``stream_parts``: 17 to 64); otherwise the library product that the reference itself uses for
     its linear layers (src/halite/transformers/infer/attention.py:21-24), except where
     float32 output is asked for and the library cannot give it, which the hand-written
     kernel does in passes of 64 rows.
@@ -725,9 +839,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
     if isinstance(x, NormedRows) or next_norm is not None:
         # ``next_norm``: where the product can, it adds its result into the stream itself
         # and returns ``NormedRows`` for that norm instead of the result
-        m, k = x.shape
-        if (w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and norm_folds(m, w.shape[0], k, tiled)
-                and out_dtype in (None, torch.bfloat16)):
+        folds = norm_folds(x.shape[0], w.shape[0], x.shape[1], tiled) if next_norm is None or not next_norm.sums else fold_pays(x, w, tiled)
+        if (w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and folds and out_dtype in (None, torch.bfloat16)
+                and (next_norm is None or not next_norm.gathers)):
             if isinstance(x, NormedRows):
                 return gemm_bf16_skinny_norm(x, tiled, tuple(w.shape))
             return gemm_bf16_skinny_norm(x, tiled, tuple(w.shape), next_norm=next_norm)
@@ -746,6 +860,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
         return gemm_bf16_skinny(x, tiled, out_dtype=out_dtype, tiled_shape=tuple(w.shape))
     if skinny_ok and skinny_pays(m, w.shape[0], k, False):
         return gemm_bf16_skinny(x, w, out_dtype=out_dtype)
+    parts = stream_parts(x, w, w.shape[0], may_part=sums or (next_norm is not None and next_norm.sums))
+    if parts:
+        return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)
     if out_dtype == torch.float32:
         global _MM_OUT_DTYPE
         if _MM_OUT_DTYPE is None:

@@ -114,7 +114,7 @@ class Attention(Mixer):
         group = ctx.group(kv.group_id)
         n_q = p.n_heads * p.head_dim
         if (run.appends and x.dtype == torch.bfloat16 and kv.k.dtype == torch.bfloat16
-                and ops.norm_folds(x.shape[0], self.w_qkv.shape[0], x.shape[1], self.t_qkv_paired)):
+                and ops.fold_pays(x, self.w_qkv, self.t_qkv_paired)):
             cos, sin = self.position.tables(ctx.max_position + 1)
             q = ops.qkv_rope_append(
                 x, self.t_qkv_paired, ctx.positions, cos, sin, p.n_heads, p.n_kv_heads, p.head_dim,
@@ -125,7 +125,16 @@ class Attention(Mixer):
         if isinstance(x, ops.NormedRows):
             x = x.materialize()
         if run.appends:
-            qkv = ops.linear(x, self.w_qkv, tiled=self.t_qkv)
+            pos = self.position  # (many requests: the rotation adds up the product's parts)
+            sums = (pos is not None and not pos.interleaved and pos.rotary_dim == p.head_dim and p.head_dim % 16 == 0
+                    and kv.k.dtype == torch.bfloat16)
+            qkv = ops.linear(x, self.w_qkv, tiled=self.t_qkv, sums=sums)
+            if isinstance(qkv, ops.PartialSums):
+                cos, sin = pos.tables(ctx.max_position + 1)
+                q = ops.rope_append_sums(qkv, ctx.positions, cos, sin, p.n_heads, p.n_kv_heads, p.head_dim, ctx.token_seg,
+                                         group.block_table, kv.k, kv.v, group.page_size, kv.tiled)
+                out = ctx.attention(q, q.shape[1], kv, group, p.n_heads, p.scale, p.window or 0)
+                return ops.linear(out, self.w_out, tiled=self.t_out, next_norm=then)
             n_kv_append = p.n_kv_heads
         else:  # the keys and values are an earlier run's
             qkv = ops.linear(x, self.w_qkv[:n_q], tiled=self.t_q)

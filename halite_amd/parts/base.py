@@ -226,7 +226,7 @@ class Norm(Part):
         (``kernels.ops.NormedRows``, see ``foldable``), which is handed on as it is."""
         raise NotImplementedError
 
-    def foldable(self, h: torch.Tensor):
+    def foldable(self, h: torch.Tensor, gathers: bool = False):
         """``kernels.ops.NextNorm`` if the product before this norm may add into ``h`` and
         prepare the norm's input itself, else None."""
         return None

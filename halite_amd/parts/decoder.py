@@ -146,6 +146,8 @@ class Decoder:
             next_norm = None
             if getattr(blocks[i], "takes_next_norm", False) and hasattr(ahead, "first_norm_for"):
                 next_norm = ahead.first_norm_for(h)
+            elif getattr(blocks[i], "takes_next_norm", False) and i + 1 == len(blocks) and hasattr(self.final_norm, "foldable"):
+                next_norm = self.final_norm.foldable(h, gathers=True)
             if next_norm is not None:
                 pending = blocks[i].forward(h, pending, ctx, run, next_norm=next_norm)
             else:

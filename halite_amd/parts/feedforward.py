@@ -97,10 +97,11 @@ class GatedFeedForward(FeedForward):
         # The gated product with SiLU·mul in its epilogue beats the library product and a
         # kernel for SiLU·mul up to 16 rows, and at 17 to 32 rows on matrices of up to 64 M
         # elements (measured in captured graphs: 50 against 56 us at 14336 x 4096, 23 against
-        # 25 at 8192 x 3072, 202 against 179 at 28672 x 8192).
+        # 25 at 8192 x 3072, 202 against 179 at 28672 x 8192), unless the streaming product takes it.
         m, d = x.shape
         small = (self.t_gate is not None and x.dtype == torch.bfloat16 and d % 8 == 0
-                 and (m <= ops.SKINNY_ROWS or (m <= ops.FUSED_ROWS and f * d <= ops.GATED_MID_ELEMENTS)))
+                 and (m <= ops.SKINNY_ROWS or (m <= ops.FUSED_ROWS and f * d <= ops.GATED_MID_ELEMENTS
+                                                  and not ops.streams_instead(x, w, f, gated=True))))
         if isinstance(x, ops.NormedRows):
             if small:
                 act = ops.gemm_bf16_skinny_norm(x, self.t_gate, (f, d), w_up_tiled=self.t_up)
@@ -118,6 +119,8 @@ class GatedFeedForward(FeedForward):
         )
         if fused:
             act = ops.gemm_bf16_skinny(x, w[:f], w_up=w[f:])
+        elif ops.stream_parts(x, w, f, gated=True):
+            act = ops.gemm_bf16_stream(x, w[:f], 1, w_up=w[f:])
         else:
             act = ops.silu_mul(ops.linear(x, w))
         return ops.linear(act, self.w_out, tiled=self.t_out, next_norm=then)

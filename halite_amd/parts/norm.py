@@ -78,7 +78,7 @@ class RMSNorm(Norm):
             return delta
         return ops.rmsnorm(h, self.weight, self.p.eps, self.build.dtype, delta=delta, rows=rows)
 
-    def foldable(self, h):
+    def foldable(self, h, gathers=False):
         if self.build.dtype != torch.bfloat16 or not h.is_cuda or not self.p.round_before_weight:
             return None
-        return ops.NextNorm(h, self.weight, self.p.eps)
+        return ops.NextNorm(h, self.weight, self.p.eps, sums=True, gathers=gathers)

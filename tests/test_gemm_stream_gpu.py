@@ -1,0 +1,109 @@
+"""The streaming product of 17 to 64 rows: rows and columns around its tiles, K around its turns through the buffers
+(three and six) and in parts, the gated form in both tile widths, rows that lie apart; and the kernels that add up its
+planes, against the same kernels on the sum."""
+
+import pytest
+import torch
+
+from halite_amd.kernels import ops
+
+pytestmark = pytest.mark.gpu
+
+
+def rand(gpu, *shape, seed=0, scale=1.0):
+    return (scale * torch.randn(*shape, generator=torch.Generator().manual_seed(seed))).to(gpu)
+
+
+def close(y, want, k):
+    """float32 sums of ``k`` exact products of bf16 numbers, rounded to bf16 at most: half a unit in the last
+    place (a significand of 8 bits: 2^-8 of the number) plus k roundings of 2^-24 of numbers of the sums' size."""
+    err, scale = float((y.double() - want).abs().max()), float(want.abs().max())
+    assert err <= (2.0**-8 if y.dtype == torch.bfloat16 else 0.0) * scale + 1e-6 * max(1.0, k / 1024) ** 0.5 * scale, (err, scale)
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 64])
+@pytest.mark.parametrize("n,k", [(16384, 256), (10244, 320), (20544, 384), (33000, 448), (16384, 1152)])
+def test_one_part(gpu, m, n, k):
+    x, w = rand(gpu, m, k + 8, seed=1).bfloat16()[:, :k], rand(gpu, n, k, seed=2, scale=0.05).bfloat16()
+    parts = ops.stream_parts(x, w, n)
+    assert parts == 1
+    want = x.double() @ w.double().t()
+    for dtype in (torch.bfloat16, torch.float32):
+        close(ops.gemm_bf16_stream(x, w, parts, out_dtype=dtype), want, k)
+
+
+@pytest.mark.parametrize("m", [17, 32, 33, 50, 64])
+@pytest.mark.parametrize("n,k,parts", [(4096, 4096, 4), (6144, 1024, 2), (6144, 4096, 5), (4096, 14336, 4), (2048, 3200, 8), (3000, 2112, 5), (6144, 832, 2)])
+def test_planes(gpu, m, n, k, parts):
+    x, w = rand(gpu, m, k, seed=3).bfloat16(), rand(gpu, n, k, seed=4, scale=0.05).bfloat16()
+    assert ops.stream_parts(x, w, n, may_part=True) == parts
+    got = ops.gemm_bf16_stream(x, w, parts)
+    want = x.double() @ w.double().t()
+    assert isinstance(got, ops.PartialSums) and got.shape == (m, n)
+    close(got.planes.sum(0), want, k)
+    close(got.materialize(torch.float32), want, k)
+    close(got.materialize(torch.bfloat16), want, k)
+
+
+@pytest.mark.parametrize("m", [17, 48, 64])
+@pytest.mark.parametrize("f,k", [(14336, 512), (8192, 320), (11008, 256), (5500, 704)])  # tiles of 64 + 64 and of 32 + 32 rows
+@pytest.mark.parametrize("activation", ["silu", "clamped"])
+def test_gated(gpu, m, f, k, activation):
+    x, w = rand(gpu, m, k, seed=5).bfloat16(), rand(gpu, 2 * f, k, seed=6, scale=0.1).bfloat16()
+    assert ops.stream_parts(x, w, f, gated=True) == 1
+    clamp = ops.Clamp(1.5, 1.7, 1.0) if activation == "clamped" else ops.Clamp()
+    y = ops.gemm_bf16_stream(x, w[:f], 1, w_up=w[f:], activation=activation, clamp=clamp)
+    g, u = x.double() @ w[:f].double().t(), x.double() @ w[f:].double().t()
+    if activation == "clamped":
+        g, u = g.clamp(max=1.5), u.clamp(-1.5, 1.5)
+        want = g * torch.sigmoid(1.7 * g) * (u + 1.0)
+    else:
+        want = g * torch.sigmoid(g) * u
+    assert float((y.double() - want).abs().max()) <= (2.0**-8 + 1e-5) * float(want.abs().max())
+
+
+def test_what_it_does_not_take(gpu):
+    w = torch.zeros((4096, 4096), dtype=torch.bfloat16, device=gpu)
+    x = lambda m, k=4096: torch.zeros((m, k), dtype=torch.bfloat16, device=gpu)  # noqa: E731
+    assert ops.stream_parts(x(17), w, 4096, may_part=True) == 4
+    assert not ops.stream_parts(x(16), w, 4096, may_part=True) and not ops.stream_parts(x(65), w, 4096, may_part=True)
+    assert not ops.stream_parts(x(17), w, 4096)  # (one part would leave the chip idle)
+    assert not ops.stream_parts(x(17, 4097)[:, 1:], w, 4096, may_part=True)  # off 16 bytes
+    assert not ops.stream_parts(x(17, 4000), w[:, :4000], 4096, may_part=True)  # K of half a step
+    assert not ops.stream_parts(x(17).float(), w, 4096, may_part=True)
+
+
+@pytest.mark.parametrize("rows,d,n_planes", [(17, 4096, 4), (64, 3072, 5), (33, 8192, 2), (20, 260, 9)])
+def test_the_norm_adds_up_planes(gpu, rows, d, n_planes):
+    planes = ops.PartialSums(rand(gpu, n_planes, rows, d, seed=7))
+    h, w = rand(gpu, rows, d, seed=8), rand(gpu, d, seed=9).bfloat16()
+    h2 = h.clone()
+    x = ops.rmsnorm(h, w, 1e-5, torch.bfloat16, delta=planes)
+    y = ops.rmsnorm(h2, w, 1e-5, torch.bfloat16, delta=planes.materialize(torch.bfloat16))
+    assert torch.equal(x, y) and torch.equal(h, h2)
+    some = torch.tensor([rows - 1, 3, 3], dtype=torch.int32, device=gpu)  # rows alone leave the stream as it is
+    x = ops.rmsnorm(h, w, 1e-5, torch.bfloat16, delta=planes, rows=some)
+    assert torch.equal(h, h2)
+    assert torch.equal(x, ops.rmsnorm(h2, w, 1e-5, torch.bfloat16, delta=planes.materialize(torch.bfloat16), rows=some))
+
+
+@pytest.mark.parametrize("H,K,D,page,tiled", [(32, 8, 128, 64, True), (24, 8, 128, 64, True), (6, 2, 48, 16, False), (4, 4, 16, 8, False)])
+def test_the_rotation_adds_up_planes(gpu, H, K, D, page, tiled):
+    n, segs, n_planes = 37, 5, 3
+    planes = ops.PartialSums(rand(gpu, n_planes, n, (H + 2 * K) * D, seed=10))
+    i32 = lambda t: t.to(torch.int32).to(gpu)  # noqa: E731
+    seg, pos = i32(torch.arange(n) % segs), i32(torch.arange(n) // segs * 3 + 50)
+    table = i32(torch.randperm(40, generator=torch.Generator().manual_seed(11))[: segs * 8].view(segs, 8))
+    angles = rand(gpu, 8 * page if 8 * page > 80 else 80, D // 2, seed=12)
+    pages = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16, device=gpu)  # noqa: E731
+    pos = pos % (8 * page)
+    k1, v1, k2, v2 = pages(40, K, page, D), pages(40, K, D, page), pages(40, K, page, D), pages(40, K, D, page)
+    cos, sin = torch.cos(angles), torch.sin(angles)
+    q = ops.rope_append_sums(planes, pos, cos, sin, H, K, D, seg, table, k1, v1, page, tiled)
+    rows = planes.materialize(torch.bfloat16)
+    ops.rope_append(rows, pos, cos, sin, H, K, D, D, False, token_seg=seg, block_table=table, k_pages=k2, v_pages=v2, page_size=page, tiled=tiled)
+    # (a turned pair's two products may be added with one rounding or with two: a step of bf16 where that decides, or of float32
+    # where the two nearly cancel)
+    for got, want in ((q, rows[:, : H * D]), (k1, k2)):
+        assert torch.allclose(got.float(), want.float(), rtol=2.0**-7, atol=1e-6) and float((got != want).float().mean()) < 1e-3
+    assert torch.equal(v1, v2)
