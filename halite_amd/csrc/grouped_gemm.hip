@@ -22,6 +22,9 @@
 #include "hal_api.h"
 #include <math.h>
 
+#include <algorithm>
+#include <type_traits>
+
 struct GroupedArgs {
   const void* X;
   int ldx, x_group_cols, x_col0;
@@ -291,7 +294,7 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
     }
 }
 
-// The experts' products of prompts (rows sorted by group): tiles of up to 256 rows x 256 W rows (GATED:
+// The experts' products of prompts (rows sorted by group): tiles of up to 352 rows x 256 W rows (GATED:
 // 128 of the gate's weight and the same 128 of the up projection's) by eight waves, a wave half the
 // tile's rows x 64 W rows, one workgroup a compute unit.
 //
@@ -305,20 +308,22 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
 // them runs.  W rows are the instruction's first operand, so lane l of a result holds row l % 16 and the
 // four neighbouring columns 4 * (l / 16) .. + 3: one vector store.
 //
-// A group's rows are cut into the fewest tiles of at most 256 and these are made equally high, in
-// steps of 32 rows, so that workgroups take equally long.  Workgroup b runs on compute die b % 8, and
+// A group's rows are cut into the fewest tiles of at most so many rows (gw_height) and these are made equally high,
+// in steps of 32 rows, so that workgroups take equally long.  Workgroup b runs on compute die b % 8, and
 // each die has an L2 of its own, so die x takes the x-th eighth of the list of all tiles, which goes
 // through a group's row tiles (eight at a time) column by column: one die reads an expert's weights,
 // once (tiles of two experts side by side cost a third more reads from memory and 8% of the time).
 //
 // Measured beside tiles of 128 x 128 in registers and LDS (grouped_mfma_kernel): 9,000 rows of 16 experts,
-// 4096 x 4096: 469 -> 300 us (644 -> 1,007 TFLOP/s); 18,000 rows of 64 experts, gate and up 1024 x 4096
-// each: 537 -> 400 us, down 4096 x 1024 into float32 rows 352 -> 280 us; 49,152 rows of 64: 1,127 -> 745 us;
-// 2,400 rows of 64 (the weights' 1.07 GB once): 252 -> 200 us.
-#define GW_ROWS 256
+// 4096 x 4096: 469 us -> 327 in tiles of at most 256 rows -> 286 of at most 352 (1,057 TFLOP/s); 18,000 rows of 64
+// experts, gate and up 1024 x 4096 each: 537 -> 391 -> 305 us, down 4096 x 1024 into float32 rows 352 -> 284 -> 237;
+// 49,152 rows of 64: 1,127 -> 787 -> 706; 2,400 rows of 8, gate and up 14336 x 4096: 660 -> 557, down 450 -> 338;
+// 3,600 rows of 64 (the weights' 1.07 GB once): 196 -> 197.
+#define GW_ROWS 352
 #define GW_COLS 256
 #define GW_TK 64
 #define GW_PANEL 8
+#define GG_UNITS 256  // compute units of the gfx950 parts that this library is built for
 #define GW_A_BYTES (GW_ROWS * GW_TK * 2)
 #define GW_BUFFER ((GW_ROWS + GW_COLS) * GW_TK * 2)
 
@@ -347,39 +352,45 @@ __device__ __forceinline__ hal_memory gw_rows_of_x(const GroupedArgs& a, int col
   return hal_memory_at((const bf16_t*)a.X + col0, ((uint32_t)(a.x_rows - 1) * a.ldx + a.K) * 2);
 }
 
+// The lane's number, counted anew at every call: kept over a tile's products, it and what follows from it would take registers.
+__device__ __forceinline__ int gw_lane() {
+  int zero = 0;
+  asm volatile("" : "+v"(zero));
+  return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
+}
+
 // What one wave does for a tile of at most 32 * NI rows.  The two buffers are two arrays, so that the
 // compiler can tell a load into one from a read of the other.
 template <bool GATED, int NI>
-__device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1) {
+__device__ __forceinline__ void gw_wave(const GroupedArgs& a, int wave, int g, int row0, int row_end, int n0, char* b0, char* b1) {
   constexpr int AI = (NI + 1) / 2, LOADS = AI + 4;  // a wave's loads a step: 8 rows of every 64 of X, and of W
+  constexpr bool FULL = NI > 10;  // no registers left for W's four addresses: added up for every load (elsewhere 1% slower)
   const int steps = a.K / GW_TK;                    // even
-  const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), wm = wave / 4, wn = wave % 4;
+  const int lane = gw_lane(), wm = wave / 4, wn = wave % 4;
   const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ hal_turn(lr % 16)) * 16;
   // (GATED: of every 64 W rows, a wave's, the first 32 are the gate's and the others the up projection's)
   const void* w0 = GATED && wave >= 4 ? a.W2 : a.W;
   const hal_memory W = hal_memory_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
   const hal_memory X = gw_rows_of_x(a, a.x_col0);
-  uint32_t xo[AI], wo[4];
-  // rows and columns past the end are read from the last one: nothing of them is stored
+  uint32_t xo[AI];
+  // (an odd NI's last load has rows for four waves: the others' bring their last rows again)
+  const int last_x = NI % 2 && wave >= 4 ? AI - 2 : AI - 1;
+  // rows past the end are read from the last one, columns as zeros: nothing of them is stored
 #pragma unroll
   for (int i = 0; i < AI; ++i) {
-    int r = row0 + lr + 64 * i;
+    int r = row0 + lr + 64 * (i == AI - 1 ? last_x : i);
     r = r < row_end ? r : row_end - 1;
     xo[i] = (uint32_t)(a.row_src ? a.row_src[r] / a.src_div : r) * (uint32_t)(a.ldx * 2) + c;
+    asm("v_mov_b32 %0, %1" : "=v"(xo[i]) : "v"(xo[i]));  // (one register, not the pair that a multiplication with addition writes)
   }
-#pragma unroll
-  for (int i = 0; i < 4; ++i) {
-    int n = GATED ? n0 + i * 32 + lr % 32 : n0 + i * 64 + lr;
-    n = n < a.N ? n : a.N - 1;
-    wo[i] = (uint32_t)n * (uint32_t)(a.ldw * 2) + c;
-  }
+  const uint32_t w_apart = (GATED ? 32u : 64u) * a.ldw * 2, wo = (uint32_t)(n0 + (GATED ? lr % 32 : lr)) * (uint32_t)(a.ldw * 2) + c;
   // (no branch: past the end the last step's pieces come again and are not multiplied)
   auto bring = [&](char* lds, int step) {
     const uint32_t at = (uint32_t)(step < steps ? step : steps - 1) * (GW_TK * 2);
 #pragma unroll
-    for (int i = 0; i < AI; ++i) hal_load_lds(X, xo[i], at, lds + (i * 8 + wave) * 1024);
+    for (int i = 0; i < AI; ++i) hal_load_lds(X, xo[i], at, lds + ((i == AI - 1 ? last_x : i) * 8 + wave) * 1024);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) hal_load_lds(W, wo[i], at, lds + GW_A_BYTES + (i * 8 + wave) * 1024);
+    for (int i = 0; i < 4; ++i) hal_load_lds(W, wo + i * w_apart + (FULL ? at : 0), FULL ? 0 : at, lds + GW_A_BYTES + (i * 8 + wave) * 1024);
   };
   const int q = lane / 16, r16 = lane % 16;
   const int get[2] = {r16 * 128 + (q ^ hal_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ hal_turn(r16)) * 16};
@@ -403,60 +414,98 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int g, int row0, i
 #pragma unroll
       for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[j], o.x[i], acc[i][j], 0, 0, 0);
   };
-  constexpr int HALF = NI / 2, REST = NI - HALF;
-  Operands low, high;
-  // One step: the operands of its first half are in `low`, the rest is in `mine`, the next step in `next`.
-  auto advance = [&](int s, char* mine, char* next) {
-    read(mine, 1, high);
-    multiply(low, 0, NI);
+  if constexpr (NI > 4) {
+    // Registers for few operands beside the results (up to 176 of 256): X's go through a ring of four, read while
+    // the 16 products before theirs run, W's of a half of the step with the last products of the half before.
+    gg_bf16x8 x[4], w[2][4];
+    auto get_x = [&](const char* lds, int t) { return *(const gg_bf16x8*)(lds + (wm * NI + t % NI) * 2048 + get[t / NI]); };
+    auto get_w = [&](const char* lds, int half, int j) { return *(const gg_bf16x8*)(lds + GW_A_BYTES + (wn * 4 + j) * 2048 + get[half]); };
+    auto lean = [&](int s, char* mine, char* next, auto turn) {
 #pragma unroll
-    for (int k = 0; k < NI; ++k) {  // (the order that the compiler is to emit)
-      __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + NI - 1) / NI, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-    }
-    multiply(high, 0, HALF);
-    hal_meet<0>();
-    bring(mine, s + 2);
-    read(next, 0, low);
-    multiply(high, HALF, NI);
-    __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
+      for (int t = 0; t < 2 * NI; ++t) {
+        if (t == 2 * NI - 4) {
+          hal_meet<0>();
+          bring(mine, s + 2);
+          __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
+        }
+        const int at = (t + decltype(turn)::value) % 4, ahead = t + 4;
 #pragma unroll
-    for (int k = 0; k < REST; ++k) {
-      __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + REST - 1) / REST, 0);
-      __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        for (int j = 0; j < 4; ++j) acc[t % NI][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t / NI][j], x[at], acc[t % NI][j], 0, 0, 0);
+        x[at] = ahead < 2 * NI ? get_x(mine, ahead) : get_x(next, ahead - 2 * NI);
+        if (t >= NI - 5 && t < NI - 1) w[1][t - (NI - 5)] = get_w(mine, 1, t - (NI - 5));
+        if (t >= 2 * NI - 4) w[0][t - (2 * NI - 4)] = get_w(next, 0, t - (2 * NI - 4));
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+        if ((t >= NI - 5 && t < NI - 1) || t >= 2 * NI - 4) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
+        else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
+      }
+    };
+    bring(b0, 0);
+    bring(b1, 1);
+    hal_meet<LOADS>();
+#pragma unroll
+    for (int t = 0; t < 4; ++t) x[t] = get_x(b0, t), w[0][t] = get_w(b0, 0, t);
+    for (int s = 0; s < steps; s += 2) {
+      lean(s, b0, b1, std::integral_constant<int, 0>());
+      lean(s + 1, b1, b0, std::integral_constant<int, 2 * NI % 4>());
     }
-  };
-  bring(b0, 0);
-  bring(b1, 1);
-  hal_meet<LOADS>();
-  read(b0, 0, low);
-  for (int s = 0; s < steps; s += 2) {
-    advance(s, b0, b1);
-    advance(s + 1, b1, b0);
+  } else {
+    constexpr int HALF = NI / 2, REST = NI - HALF;
+    Operands low, high;
+    // One step: the operands of its first half are in `low`, the rest is in `mine`, the next step in `next`.
+    auto advance = [&](int s, char* mine, char* next) {
+      read(mine, 1, high);
+      multiply(low, 0, NI);
+#pragma unroll
+      for (int k = 0; k < NI; ++k) {  // (the order that the compiler is to emit)
+        __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + NI - 1) / NI, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+      }
+      multiply(high, 0, HALF);
+      hal_meet<0>();
+      bring(mine, s + 2);
+      read(next, 0, low);
+      multiply(high, HALF, NI);
+      __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
+#pragma unroll
+      for (int k = 0; k < REST; ++k) {
+        __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + REST - 1) / REST, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
+      }
+    };
+    bring(b0, 0);
+    bring(b1, 1);
+    hal_meet<LOADS>();
+    read(b0, 0, low);
+    for (int s = 0; s < steps; s += 2) {
+      advance(s, b0, b1);
+      advance(s + 1, b1, b0);
+    }
   }
   asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // LDS is not given back while loads are on their way into it
+  const int end_lane = gw_lane();
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = row0 + (wm * NI + i) * 16 + r16;
+    const int r = row0 + (wm * NI + i) * 16 + end_lane % 16;
     if (r >= row_end) continue;
     const int dst = a.row_dst ? a.row_dst[r] : r;
 #pragma unroll
     for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-      const int n = n0 + wn * (GATED ? 32 : 64) + j * 16 + q * 4;
+      const int n = n0 + wn * (GATED ? 32 : 64) + j * 16 + end_lane / 16 * 4;
       if (n < a.N) gw_store<GATED>(a, dst, n, acc[i][j], GATED ? acc[i][j + 2] : acc[i][j]);
     }
   }
 }
 
-// Which tile a workgroup takes, written to `found` (group, first row, end row, column tile; group -1: none)
-// by its first wave: the groups' rows in tiles of at most ROWS, equally high in steps of 32.  A lane counts a
+// Which tile is a workgroup's `turn`-th, written to `found` (group, first row, end row, column tile, whether
+// there is one more after it; group -1: none),
+// by its first wave: the groups' rows in tiles of at most `most`, equally high in steps of 32.  A lane counts a
 // run of neighbouring groups (one where there are up to 64), so that one sum over the wave serves any number:
 // 64 at a time, 512 groups of 512 x 2048 (gate and up) took 27.9 us for 3 tokens of 10 and 69.0 for 8, now 23.4 and 62.7.
-template <int ROWS>
-__device__ __forceinline__ void gw_find(const GroupedArgs& a, int col_tiles, int* found) {
-  const int lane = threadIdx.x % 64, each = (a.G + 63) / 64;
+__device__ __forceinline__ void gw_find(const GroupedArgs& a, int most, int col_tiles, int turn, int* found) {
+  const int lane = gw_lane();
+  const int each = (a.G + 63) / 64;
   const int first = min(a.G, lane * each), last = min(a.G, first + each);
-  auto tiles_of = [&](int g) { return (a.group_offsets[g + 1] - a.group_offsets[g] + ROWS - 1) / ROWS; };
+  auto tiles_of = [&](int g) { return (a.group_offsets[g + 1] - a.group_offsets[g] + most - 1) / most; };
   int mine = 0;
   for (int g = first; g < last; ++g) mine += tiles_of(g);
   int upto = mine;
@@ -467,13 +516,13 @@ __device__ __forceinline__ void gw_find(const GroupedArgs& a, int col_tiles, int
   }
   const long long units = (long long)__shfl(upto, 63, 64) * col_tiles;
   const int die = blockIdx.x % 8;
-  const long long unit = units * die / 8 + blockIdx.x / 8;
-  if (lane == 0) found[0] = -1;
-  if (unit >= units * (die + 1) / 8) return;
+  const long long unit = units * die / 8 + blockIdx.x / 8 + (long long)turn * (gridDim.x / 8), end_of_die = units * (die + 1) / 8;
+  if (lane == 0) found[0] = -1, found[4] = unit + gridDim.x / 8 < end_of_die;
+  if (unit >= end_of_die) return;
   int before = upto - mine;  // row tiles of the groups before
   if (unit < (long long)before * col_tiles || unit >= (long long)upto * col_tiles) return;
   for (int g = first; g < last; ++g) {  // (one lane: its groups have the tile)
-    const int begin = a.group_offsets[g], end = a.group_offsets[g + 1], n = (end - begin + ROWS - 1) / ROWS;
+    const int begin = a.group_offsets[g], end = a.group_offsets[g + 1], n = (end - begin + most - 1) / most;
     if (unit < (long long)(before + n) * col_tiles) {
       const int in_group = (int)(unit - (long long)before * col_tiles);
       const int panel = in_group / (GW_PANEL * col_tiles), in_panel = in_group % (GW_PANEL * col_tiles);
@@ -489,26 +538,77 @@ __device__ __forceinline__ void gw_find(const GroupedArgs& a, int col_tiles, int
   }
 }
 
+// How high the wide tiles may be is chosen from the groups' sizes: the least of rounds of tiles, one a compute unit,
+// times what the highest tile asks of the second-level cache (X and W rows of a step: its rows and GW_COLS).  A result's
+// bits do not depend on it.  One group over a tile's height can be one more round: 18,000 rows dealt to 64 experts
+// at random (281 +- 17 each), gate and up, took 387 us in tiles of at most 320 rows (just over two rounds), 391 of at most
+// 256 (four of half the height), and now, of at most 352, 311.
+// (The first wave's work; the same in all its lanes.)
+#define GW_HEIGHTS 4
+#define GW_LEAST_ROWS 192
+__device__ __forceinline__ int gw_height(const GroupedArgs& a, int col_tiles) {
+  constexpr int heights[GW_HEIGHTS] = {GW_ROWS, 320, 256, GW_LEAST_ROWS};
+  const int lane = threadIdx.x % 64, each = (a.G + 63) / 64;
+  const int first = min(a.G, lane * each), last = min(a.G, first + each);
+  int tiles[GW_HEIGHTS] = {}, high[GW_HEIGHTS] = {}, most = 0;
+  for (int g = first; g < last; ++g) {
+    const int rows = a.group_offsets[g + 1] - a.group_offsets[g];
+    most = max(most, rows);
+#pragma unroll
+    for (int h = 0; h < GW_HEIGHTS; ++h) {
+      const int n = max(1, (rows + heights[h] - 1) / heights[h]);
+      tiles[h] += rows > 0 ? n : 0;
+      high[h] = max(high[h], (rows + n - 1) / n);
+    }
+  }
+  if (!__any(most > GW_LEAST_ROWS)) return GW_ROWS;  // (they are all the same)
+  int best = 0;
+  long long least = 0;
+#pragma unroll
+  for (int h = 0; h < GW_HEIGHTS; ++h) {
+#pragma unroll
+    for (int off = 32; off; off >>= 1) {
+      tiles[h] += __shfl_xor(tiles[h], off, 64);
+      high[h] = max(high[h], __shfl_xor(high[h], off, 64));
+    }
+    const long long cost = ((long long)tiles[h] * col_tiles + GG_UNITS - 1) / GG_UNITS * ((high[h] + 31) / 32 * 32 + GW_COLS);
+    if (h == 0 || cost < least) best = heights[h], least = cost;
+  }
+  return best;
+}
+
 template <bool GATED>
 __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GW_BUFFER], b1[GW_BUFFER];
-  __shared__ __attribute__((aligned(64))) int found[4];
-  if (threadIdx.x < 64) gw_find<GW_ROWS>(a, col_tiles, found);
-  __syncthreads();
-  const int g = __builtin_amdgcn_readfirstlane(found[0]);
-  if (g < 0) return;
-  const int row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
-  const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GW_COLS / 2 : GW_COLS);
-  const int rows = row_end - row0;
-  if (rows <= 0) return;  // (equal heights in steps of 32 can leave a group's last tile empty)
-#define GW_WAVE(NI_) gw_wave<GATED, NI_>(a, g, row0, row_end, n0, b0, b1)
-  if (rows <= 64) GW_WAVE(2);
-  else if (rows <= 128) GW_WAVE(4);
-  else if (rows <= 160) GW_WAVE(5);
-  else if (rows <= 192) GW_WAVE(6);
-  else if (rows <= 224) GW_WAVE(7);
-  else GW_WAVE(8);
+  __shared__ __attribute__((aligned(64))) int found[5];
+  __shared__ int most;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
+  if (wave == 0) most = gw_height(a, col_tiles);
+  // (as many workgroups as tiles of GW_ROWS can be, and one a compute unit: lower ones are some workgroups' second)
+  for (int turn = 0;; ++turn) {
+    __syncthreads();  // the tile before is done with the buffers and `found`
+    if (wave == 0) gw_find(a, most, col_tiles, turn, found);
+    __syncthreads();
+    const int g = __builtin_amdgcn_readfirstlane(found[0]), more = __builtin_amdgcn_readfirstlane(found[4]);
+    if (g < 0) return;
+    const int row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
+    const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GW_COLS / 2 : GW_COLS);
+    const int rows = row_end - row0;
+    // (equal heights in steps of 32 can leave a group's last tile empty)
+#define GW_WAVE(NI_) gw_wave<GATED, NI_>(a, wave, g, row0, row_end, n0, b0, b1)
+    if (rows <= 0);
+    else if (rows <= 64) GW_WAVE(2);
+    else if (rows <= 128) GW_WAVE(4);
+    else if (rows <= 160) GW_WAVE(5);
+    else if (rows <= 192) GW_WAVE(6);
+    else if (rows <= 224) GW_WAVE(7);
+    else if (rows <= 256) GW_WAVE(8);
+    else if (rows <= 288) GW_WAVE(9);
+    else if (rows <= 320) GW_WAVE(10);
+    else GW_WAVE(11);
 #undef GW_WAVE
+    if (!more) return;
+  }
 }
 
 // Groups of few rows (decode steps, short prompts): what counts is that the weights come at the memory's
@@ -636,7 +736,7 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
 template <bool GATED, bool HEADS>
 __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GT_BUFFER], b1[GT_BUFFER], b2[GT_BUFFER];
-  __shared__ __attribute__((aligned(64))) int found[4];
+  __shared__ __attribute__((aligned(64))) int found[5];
   int g, row0, row_end, col;
   if (HEADS) {
     // a die takes neighbouring heads, a head's columns beside each other: they read the same rows
@@ -646,7 +746,7 @@ __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, i
     g = (int)(unit / in_group), row0 = (int)(unit % in_group) / col_tiles * GT_ROWS;
     row_end = min(a.M, row0 + GT_ROWS), col = (int)(unit % in_group) % col_tiles;
   } else {
-    if (threadIdx.x < 64) gw_find<GT_ROWS>(a, col_tiles, found);
+    if (threadIdx.x < 64) gw_find(a, GT_ROWS, col_tiles, 0, found);
     __syncthreads();
     g = __builtin_amdgcn_readfirstlane(found[0]);
     if (g < 0) return;
@@ -769,7 +869,7 @@ static double gg_tiles_a_group(double rows, int tile) {
   for (double k = 0; tile * k < rows + 4 * sqrt(rows); k += 1) n += 0.5 * erfc((tile * k - rows) / sqrt(2 * rows));
   return n;
 }
-#define GG_UNITS 256  // compute units of the gfx950 parts that this library is built for
+#define GG_WIDE_ROWS 256  // of a wide tile, as the lines above were measured
 enum { GG_FEW_ROWS = 0, GG_STREAM = 1, GG_WIDE = 2, GG_TILES_128 = 3 };
 static int gg_experts_kernel(int M, int N, int K, int G, bool gated) {
   const double rows = (double)M / G;
@@ -782,10 +882,10 @@ static int gg_experts_kernel(int M, int N, int K, int G, bool gated) {
     return stream && tiles >= GG_UNITS / 2 && !begun ? GG_STREAM : GG_FEW_ROWS;
   }
   if (stream && M / G < GT_ROWS_A_GROUP) return GG_STREAM;
-  const double wide_tiles = G * gg_tiles_a_group(rows, GW_ROWS) * wide_cols;
+  const double wide_tiles = G * gg_tiles_a_group(rows, GG_WIDE_ROWS) * wide_cols;
   const double stream_tiles = G * gg_tiles_a_group(rows, GT_ROWS) * stream_cols;
   // (groups of many tiles make these lower where one more is needed, and the round begun is a short one)
-  const bool begun = rows < 2 * GW_ROWS && wide_tiles > 1.02 * GG_UNITS && wide_tiles < 1.1 * GG_UNITS;
+  const bool begun = rows < 2 * GG_WIDE_ROWS && wide_tiles > 1.02 * GG_UNITS && wide_tiles < 1.1 * GG_UNITS;
   const bool wide_fills = wide_tiles >= 0.625 * GG_UNITS && !begun;
   if (wide && (wide_fills || !stream)) return GG_WIDE;
   return stream && (stream_tiles <= 3 * GG_UNITS || K < 2048 || rows >= 512) ? GG_STREAM : GG_TILES_128;
@@ -854,7 +954,8 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
     if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
     else hipLaunchKernelGGL((grouped_stream_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
   } else if (kernel == GG_WIDE) {
-    const long long units = gw_most_tiles(M, G, GW_ROWS) * wide_cols, blocks = 8 * ((units + 7) / 8);
+    const long long most = gw_most_tiles(M, G, GW_LEAST_ROWS) * wide_cols, units = std::min(most, std::max(gw_most_tiles(M, G, GW_ROWS) * wide_cols, (long long)GG_UNITS));
+    const long long blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
     if (W2) hipLaunchKernelGGL(grouped_wide_kernel<true>, dim3((unsigned)blocks), dim3(512), 0, stream, a, wide_cols);
     else hipLaunchKernelGGL(grouped_wide_kernel<false>, dim3((unsigned)blocks), dim3(512), 0, stream, a, wide_cols);
