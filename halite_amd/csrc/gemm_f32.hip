@@ -7,13 +7,13 @@
 // its lanes take every 64th group of four k each (the rows of A come through LDS, shared by
 // the workgroup's four waves), and the partial sums of the lanes, and of the waves that share
 // columns, are added in a fixed order.  17 to about 100 rows: the matrix cores, k split over a
-// workgroup's waves, each staging whole rows through LDS of its own.  More rows: tiles of 128 rows and 128, 64 or 32
-// columns on the matrix cores, through LDS.  For sizes and addresses that are no multiples of
+// workgroup's waves, each staging whole rows through LDS of its own.  More rows: tiles of 128 rows and 128, 96, 64
+// or 32 columns on the matrix cores, straight into LDS.  For sizes and addresses that are no multiples of
 // four: tiles of 64 x 64 on the vector units, each output element one chain of K
 // multiply-adds in index order.
 // In all of them a token's result depends on its own row alone, not on what else is in the
 // batch; between them the order of the additions differs, i.e. the last bits may.
-#include "hal_common.h"
+#include "hal_lds.h"
 #include "hal_api.h"
 
 #define GF_BM 64
@@ -76,9 +76,8 @@ gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ 
 // ---- many rows: the matrix cores' float32 instruction -----------------------------------------
 // v_mfma_f32_32x32x2_f32 multiplies and adds in float32 (it is the instruction behind the
 // published float32 matrix rate, not one of the reduced-precision modes), at twice the rate of
-// the vector units' multiply-adds.  A workgroup of four waves takes 128 x 128 outputs, a wave
-// 64 x 64 as 2 x 2 products of 32 x 32; k goes through LDS 32 at a time, in two buffers, the
-// next stage on its way to registers while this one is multiplied.
+// the vector units' multiply-adds.  A workgroup takes 128 rows and 128, 64 (eight waves, a wave 64 x 32 or 32 x 32)
+// or 32 columns (four), or 96 (twelve).  k goes 32 at a time, whole 128-byte lines of both operands, straight into three LDS buffers.
 //
 // The instruction takes, from lane l, A[row l % 32][k l / 32] and B[k l / 32][column l % 32],
 // two k a call.  Which two k of the stage a call gets is free as long as A and B agree: the
@@ -87,136 +86,170 @@ gemm_f32_kernel(const float* __restrict__ A, int lda, const float* __restrict__ 
 // is the sum over k in that order, in stretches of 512 that each start from nothing (see the
 // kernel), rounded as the instruction rounds; it depends on its own row of A alone.
 #define MF_BM 128
-#define MF_BN 128
 #define MF_BK 32
 #define MF_KQ (MF_BK / 4)
+#define MF_THREADS(BN) ((BN) == 32 ? 256 : (BN) == 96 ? 768 : 512)
 #define MF_STRETCH 512  // k of a stretch that is summed from nothing
+#define MF_UNITS 256  // compute units of the gfx950 parts that this library is built for
+#define MF_ROW_LIMIT (1 << 23)  // numbers of a row: 128 of them lie within 32-bit offsets
 #define MF_XCDS 8  // dies of the gfx950 parts that this library is built for (a wrong count costs cache hits only)
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 
-// BN: columns of a workgroup's tile, 128 (four waves, a wave 64 x 64 as 2 x 2 products), 64 (eight
-// waves) or 32 (four; a wave 32 x 32): the narrower tiles are for products whose rows and columns would
-// leave units without a tile of 128.  What bounds them is the second-level cache (tiles of 32 columns
-// ask it for 20 bytes a clock and unit, all it gives; of 64 for 12).  An output element's sum is the same in all.
+// What bounds it: the instruction itself, 64 clocks for 32 x 32 x 2, as long as its operands are there: so the two stages
+// after the one that is multiplied are on their way to LDS, and the next one's operands to registers; a stage's one
+// barrier comes before its products, when no wave has anything left to read in the buffer that is filled anew.
+// LDS holds a row's eight 16-byte pieces in turned order, piece p of row r at place p ^ (r / 2 % 8): the sixteen lanes
+// of each of a read's turns (see hal_turn) have sixteen rows mod 16 and then meet all banks once.
+// The narrower tiles are for products whose rows and columns would leave units without a tile of 128; tiles of 32
+// columns ask the second-level cache for 20 bytes a clock and unit, all it gives, of 64 for 12.
+// An output element's sum is the same in all.
 template <int BN>
-__global__ void __launch_bounds__(BN == 64 ? 512 : 256, BN == 64 ? 4 : 2)
+__global__ void __launch_bounds__(MF_THREADS(BN), BN == 64 ? 4 : BN == 96 ? 3 : 2)
 gemm_f32_mfma_kernel(const float* __restrict__ A, int lda, const float* __restrict__ W, int ldw,
                      float* __restrict__ C, int ldc, int M, int N, int K, int tiles_m, int tiles_n) {
-  constexpr int THREADS = BN == 64 ? 512 : 256;
-  constexpr int NB = BN == 128 ? 2 : 1;           // 32 x 32 products of a wave, each way
-  constexpr int AV = MF_BM * MF_KQ / THREADS;     // 16-byte vectors of A's stage per thread
-  constexpr int WV = BN * MF_KQ / THREADS;        // and of W's
-  static_assert(BN == 128 || BN == 64 || BN == 32, "tiles of 128, 64 or 32 columns");
-  // [buffer][k / 4][row], a row more than there are so that the stores of a wave (a row's
-  // eight vectors side by side) spread over the banks
-  __shared__ float4 a_s[2][MF_KQ][MF_BM + 1];
-  __shared__ float4 w_s[2][MF_KQ][BN + 1];
-  const int tid = threadIdx.x, lane = tid % HAL_WAVE, wave = tid / HAL_WAVE;
+  static_assert(BN == 128 || BN == 96 || BN == 64 || BN == 32, "tiles of 128, 96, 64 or 32 columns");
+  constexpr int WAVES = MF_THREADS(BN) / HAL_WAVE, ACROSS = BN / 32;  // waves, and how many lie side by side
+  constexpr int NI = MF_BM / 32 * ACROSS / WAVES;            // 32 x 32 products of a wave, one above the other
+  constexpr int AL = (MF_BM / 8 + WAVES - 1) / WAVES, WL = BN / 8 / WAVES, LOADS = AL + WL;  // a wave's loads a stage
+  constexpr int A_BYTES = MF_BM * MF_BK * 4, BYTES = A_BYTES + BN * MF_BK * 4;
+  __shared__ __attribute__((aligned(16))) char b0[BYTES], b1[BYTES], b2[BYTES];
+  const int lane = threadIdx.x % HAL_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / HAL_WAVE);
   // Workgroups go to the eight dies in turn, each die with a cache of its own: renumber them
   // so that a die's workgroups are neighbours in the order of tiles (the same columns of W,
   // rows of A one after the other).
-  int id = blockIdx.x;
-  const int n_tiles = tiles_m * tiles_n;
-  if (n_tiles % MF_XCDS == 0) id = (id % MF_XCDS) * (n_tiles / MF_XCDS) + id / MF_XCDS;
+  const int n_tiles = tiles_m * tiles_n, die = blockIdx.x % MF_XCDS, rest = n_tiles % MF_XCDS;
+  const int id = die * (n_tiles / MF_XCDS) + min(die, rest) + blockIdx.x / MF_XCDS;  // (the first `rest` dies have one more)
   const int m0 = (id % tiles_m) * MF_BM, n0 = (id / tiles_m) * BN;
+  const int rows_here = min(MF_BM, M - m0), cols_here = min(BN, N - n0);
 
-  float4 a_next[AV], w_next[WV];
-  auto ask = [&](int k0) {  // vector e of a stage: row e / 8, k0 + 4 (e % 8)
+  const uint32_t a_bytes = ((uint32_t)(rows_here - 1) * lda + K) * 4, w_bytes = ((uint32_t)(cols_here - 1) * ldw + K) * 4;
+  const hal_memory a_all = hal_memory_at(A + (size_t)m0 * lda, a_bytes), w_all = hal_memory_at(W + (size_t)n0 * ldw, w_bytes);
+  // load i of a wave: rows 8 (i WAVES + wave) + lane / 8 of the operand (WAVES is even: they all turn alike);
+  // rows past the end are read from the last one: nothing of them is stored
+  const int piece = ((lane % 8) ^ ((wave % 2 * 4 + lane / 16) % 8)) * 4;  // of a stage's k, the first of four
+  uint32_t ao[AL], wo[WL];
+  // (of the last of A's there may be fewer than waves: the others bring their rows before again)
+  const int last_a = (AL - 1) * WAVES + wave < MF_BM / 8 ? (AL - 1) * WAVES + wave : (AL - 2) * WAVES + wave;
+  auto a_load = [&](int i) { return i == AL - 1 ? last_a : i * WAVES + wave; };
 #pragma unroll
-    for (int u = 0; u < AV; ++u) {
-      const int e = tid + u * THREADS, r = e / MF_KQ, k = k0 + (e % MF_KQ) * 4;
-      const bool in = k < K && m0 + r < M;  // (K is a multiple of 4)
-      a_next[u] = in ? *(const float4*)(A + (size_t)(m0 + r) * lda + k) : float4{0.f, 0.f, 0.f, 0.f};
-    }
+  for (int i = 0; i < AL; ++i) ao[i] = ((uint32_t)min(8 * a_load(i) + lane / 8, rows_here - 1) * lda + piece) * 4;
 #pragma unroll
-    for (int u = 0; u < WV; ++u) {
-      const int e = tid + u * THREADS, r = e / MF_KQ, k = k0 + (e % MF_KQ) * 4;
-      const bool in = k < K && n0 + r < N;
-      w_next[u] = in ? *(const float4*)(W + (size_t)(n0 + r) * ldw + k) : float4{0.f, 0.f, 0.f, 0.f};
-    }
-  };
-  auto put = [&](int buf) {
+  for (int i = 0; i < WL; ++i) wo[i] = ((uint32_t)min(8 * (i * WAVES + wave) + lane / 8, cols_here - 1) * ldw + piece) * 4;
+  // (past the end of K, also stages that fill the last turn through the buffers: zeros, read from past the operands' bytes)
+  auto bring = [&](char* lds, int stage) {
+    const bool in = stage * MF_BK + piece < K;  // (K is a multiple of 4)
+    const uint32_t at = (uint32_t)stage * (MF_BK * 4);
 #pragma unroll
-    for (int u = 0; u < AV; ++u) {
-      const int e = tid + u * THREADS;
-      a_s[buf][e % MF_KQ][e / MF_KQ] = a_next[u];
-    }
+    for (int i = 0; i < AL; ++i) hal_load_lds(a_all, in ? ao[i] + at : a_bytes, 0, lds + a_load(i) * 1024);
 #pragma unroll
-    for (int u = 0; u < WV; ++u) {
-      const int e = tid + u * THREADS;
-      w_s[buf][e % MF_KQ][e / MF_KQ] = w_next[u];
-    }
+    for (int i = 0; i < WL; ++i) hal_load_lds(w_all, in ? wo[i] + at : w_bytes, 0, lds + A_BYTES + (i * WAVES + wave) * 1024);
   };
 
   // An output element is summed in stretches of MF_STRETCH k, each from nothing, and the
   // stretches' sums are added in order: one chain of K additions would round K / 2 times on top
   // of each other (measured: four times the error of this at K = 14,336).
-  f32x16 acc[NB][NB], total[NB][NB];
+  f32x16 acc[NI], total[NI];
 #pragma unroll
-  for (int i = 0; i < NB; ++i)
+  for (int i = 0; i < NI; ++i)
 #pragma unroll
-    for (int j = 0; j < NB; ++j)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = total[i][j][v] = 0.f;
+    for (int v = 0; v < 16; ++v) acc[i][v] = total[i][v] = 0.f;
   // this wave's corner of the tile
-  const int wm = BN == 128 ? (wave / 2) * 64 : BN == 64 ? (wave / 2) * 32 : wave * 32;
-  const int wn = BN == 128 ? (wave % 2) * 64 : BN == 64 ? (wave % 2) * 32 : 0;
-  const int rows = wm + lane % 32, cols = wn + lane % 32, half = lane / 32;
-  const bool wave_has_rows = m0 + wm < M;  // (a wave whose rows are all beyond M only helps to load)
-
-  ask(0);
-  put(0);
-  __syncthreads();
-  int buf = 0;
-  for (int k0 = 0; k0 < K; k0 += MF_BK, buf ^= 1) {
-    const bool more = k0 + MF_BK < K;
-    if (more) ask(k0 + MF_BK);
-    if (wave_has_rows) {
+  const int wm = wave / ACROSS * 32 * NI, wn = wave % ACROSS * 32;
+  const int col = lane % 32, half = lane / 32;
+  const bool wave_has_rows = wm < rows_here;  // (a wave whose rows are all beyond M only helps to load)
+  struct Operands {
+    float4 a[NI][MF_KQ / 2], w[MF_KQ / 2];
+  };
+  const int first = (half ^ (col / 2 % 8)) * 16, a_at = (wm + col) * (MF_BK * 4) + first, w_at = A_BYTES + (wn + col) * (MF_BK * 4) + first;
+  auto read = [&](const char* lds, Operands& o) {
+    int a = a_at, w = w_at;
+    asm volatile("" : "+v"(a), "+v"(w));  // (the places of the other pieces derived anew: kept they would take registers)
 #pragma unroll
-      for (int s = 0; s < MF_KQ / 2; ++s) {
-        const int kq = 2 * s + half;
-        float av[NB][4], bv[NB][4];
+    for (int s = 0; s < MF_KQ / 2; ++s) {
 #pragma unroll
-        for (int i = 0; i < NB; ++i) {
-          const float4 a = a_s[buf][kq][rows + 32 * i], b = w_s[buf][kq][cols + 32 * i];
-          av[i][0] = a.x, av[i][1] = a.y, av[i][2] = a.z, av[i][3] = a.w;
-          bv[i][0] = b.x, bv[i][1] = b.y, bv[i][2] = b.z, bv[i][3] = b.w;
+      for (int i = 0; i < NI; ++i) o.a[i][s] = *(const float4*)(lds + (a ^ (s * 32)) + 32 * i * (MF_BK * 4));
+      o.w[s] = *(const float4*)(lds + (w ^ (s * 32)));
+    }
+  };
+  auto multiply = [&](const Operands& o) {
+#pragma unroll
+    for (int s = 0; s < MF_KQ / 2; ++s) {
+      const float wv[4] = {o.w[s].x, o.w[s].y, o.w[s].z, o.w[s].w};
+#pragma unroll
+      for (int e = 0; e < 4; ++e)
+#pragma unroll
+        for (int i = 0; i < NI; ++i) {
+          const float av[4] = {o.a[i][s].x, o.a[i][s].y, o.a[i][s].z, o.a[i][s].w};
+          acc[i] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[e], wv[e], acc[i], 0, 0, 0);
         }
-#pragma unroll
-        for (int e = 0; e < 4; ++e)
-#pragma unroll
-          for (int i = 0; i < NB; ++i)
-#pragma unroll
-            for (int j = 0; j < NB; ++j)
-              acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(av[i][e], bv[j][e], acc[i][j], 0, 0, 0);
-      }
     }
-    if ((k0 + MF_BK) % MF_STRETCH == 0 || !more) {  // (the same for every thread)
+  };
+  auto add_up = [&]() {
 #pragma unroll
-      for (int i = 0; i < NB; ++i)
-#pragma unroll
-        for (int j = 0; j < NB; ++j)
-#pragma unroll
-          for (int v = 0; v < 16; ++v) {
-            total[i][j][v] += acc[i][j][v];
-            acc[i][j][v] = 0.f;
-          }
-    }
-    if (more) put(buf ^ 1);  // (read last in the stage before the one that just ended)
-    __syncthreads();
-  }
-  // element v of a lane's 16: row 8 (v / 4) + 4 (lane / 32) + v % 4, column lane % 32
-#pragma unroll
-  for (int i = 0; i < NB; ++i)
-#pragma unroll
-    for (int j = 0; j < NB; ++j) {
-      const int gn = n0 + wn + j * 32 + lane % 32;
+    for (int i = 0; i < NI; ++i)
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
-        const int gm = m0 + wm + i * 32 + 8 * (v / 4) + 4 * half + v % 4;
-        if (gm < M && gn < N) C[(size_t)gm * ldc + gn] = total[i][j][v];
+        total[i][v] += acc[i][v];
+        acc[i][v] = 0.f;
       }
+  };
+  const int stages = (K + MF_BK - 1) / MF_BK;
+  Operands even, odd;
+  // One stage: its operands are in `now`, the next stage's pieces in `next`; `free` is the buffer that held its own.
+  auto advance = [&](int s, char* free, const char* next, const Operands& now, Operands& then) {
+    hal_meet<LOADS>();  // (the next stage's pieces are there, those of the one after it may be on their way)
+    if (wave_has_rows) {
+      bring(free, s + 3);
+      read(next, then);
+      multiply(now);
+      // (the order that the compiler is to emit: loads and reads are issued while the products run)
+      __builtin_amdgcn_sched_group_barrier(0x008, NI, 0);
+#pragma unroll
+      for (int i = 0; i < LOADS; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x020, 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, NI, 0);
+      }
+#pragma unroll
+      for (int i = 0; i < MF_KQ / 2; ++i) {
+        __builtin_amdgcn_sched_group_barrier(0x100, NI + 1, 0);
+        __builtin_amdgcn_sched_group_barrier(0x008, NI, 0);
+      }
+      __builtin_amdgcn_sched_group_barrier(0x008, NI * (2 * MF_KQ - 1 - LOADS - MF_KQ / 2), 0);
+      if ((s + 1) % (MF_STRETCH / MF_BK) == 0) add_up();
+    } else {
+      bring(free, s + 3);
     }
+  };
+  bring(b0, 0);
+  bring(b1, 1);
+  bring(b2, 2);
+  hal_meet<2 * LOADS>();
+  read(b0, even);
+  for (int s = 0;; s += 6) {
+    advance(s, b0, b1, even, odd);
+    if (s + 1 >= stages) break;
+    advance(s + 1, b1, b2, odd, even);
+    if (s + 2 >= stages) break;
+    advance(s + 2, b2, b0, even, odd);
+    if (s + 3 >= stages) break;
+    advance(s + 3, b0, b1, odd, even);
+    if (s + 4 >= stages) break;
+    advance(s + 4, b1, b2, even, odd);
+    if (s + 5 >= stages) break;
+    advance(s + 5, b2, b0, odd, even);
+    if (s + 6 >= stages) break;
+  }
+  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // LDS is not given back while loads are on their way into it
+  if (stages % (MF_STRETCH / MF_BK)) add_up();
+  // element v of a lane's 16: row 8 (v / 4) + 4 (lane / 32) + v % 4, column lane % 32
+  if (wn + col < cols_here)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const int r = wm + i * 32 + 8 * (v / 4) + 4 * half + v % 4;
+        if (r < rows_here) C[(size_t)(m0 + r) * ldc + n0 + wn + col] = total[i][v];
+      }
 }
 
 // ---- 17 to 128 rows: the same instruction, k split over a workgroup's waves -----------------
@@ -476,26 +509,38 @@ static void launch_skinny(const float* A, int lda, const float* W, int ldw, floa
                        A, lda, W, ldw, C, ldc, M, N, K);
 }
 
-// What tiles of BN columns cost, in microseconds at K = 4,096: rounds over the 256 compute units, a round
-// of tiles of 128 / 64 / 32 columns 270 / 147 / 83 (a compute unit whose only tile it is has too few waves
-// to hide what they wait for: 30 and 10 more; one or two tiles of 32 columns 125 and 183).  Measured at K =
-// 4,096 in tiles of 128 / 64 / 32: 500 rows x 4,096 columns 305 / 174 / 187 us, x 6,144 308 / 301 / 255,
-// x 28,672 1,085 / 1,017 / 1,129, x 32,000 1,093 / 1,161 / 1,285; 200 x 4,096 305 / 167 / 126; 1,500 x 4,096
-// 548 / 451 / 490; 2,048 x 4,096 554 / 594 / 661.
+// What tiles of 128, 64 or 32 columns cost, in microseconds at K = 4,096, by whole rounds over the 256 compute units.
+// Measured at K = 4,096 in tiles of 128 / 64 / 32: 500 rows x 4,096 columns 251 / 140 / 164 us, x 6,144 254 / 252 / 257,
+// x 28,672 1,026 / 888 / 1,119, x 32,000 1,032 / 1,010 / 1,277; 200 x 4,096 250 / 138 / 102; 1,500 x 4,096
+// 510 / 385 / 484; 2,048 x 4,096 517 / 518 / 647.  (With operands through registers and two buffers, same sums: 305 / 174 /
+// 187, 308 / 301 / 255, 1,085 / 1,017 / 1,129, 1,093 / 1,161 / 1,285; 305 / 167 / 126; 548 / 451 / 490; 554 / 594 / 661.)
 static double mf_rounds_cost(long long tiles_m, int N, int BN) {
-  const double n = (double)((tiles_m * ((N + BN - 1) / BN) + 255) / 256);
-  if (BN == 128) return 30 + 270 * n;
-  if (BN == 64) return 10 + 147 * n;
-  return n <= 1 ? 125 : n <= 2 ? 183 : 83 * n;
+  const double n = (double)((tiles_m * ((N + BN - 1) / BN) + MF_UNITS - 1) / MF_UNITS);
+  if (BN == 128) return 257 * n;
+  if (BN == 64) return 30 + 130 * n;
+  return n <= 1 ? 103 : n <= 2 ? 163 : 83 * n;
 }
 
-// The columns of the tiles that M rows by N columns take on the matrix cores (100 rows and fewer: see below).
+// The columns of the tiles that M rows by N columns take on the matrix cores by that count (100 rows and fewer: see below).
 extern "C" int hal_gemm_f32_tile_columns(int M, int N) {
   const long long tiles_m = (M + MF_BM - 1) / MF_BM;
   int bn = 128;
   for (int other = 64; other >= 32; other /= 2)
     if (mf_rounds_cost(tiles_m, N, other) < mf_rounds_cost(tiles_m, N, bn)) bn = other;
   return bn;
+}
+
+// The columns of the tiles that are launched: the count's, but
+// tiles of 96, whose one round takes 201 us, where they need no second one and the count's do (500 rows x 6,144 columns 201
+// instead of 257; 400 x 5,120 x 3,072 151 / 194; 640 x 4,096 200 / 256), and
+// tiles of 64 for those of 128 where these leave a part of their last round empty, since two of 64 share a unit and one
+// alone is done in 0.55 of their time (260 x 28,004 636 / 766, 300 x 28,672 646 / 766, 400 x 28,672 877 / 1,018,
+// 130 x 28,672 505 / 512; full rounds: 512 x 8,192 264 / 258).
+extern "C" int hal_gemm_f32_columns(int M, int N) {
+  const long long tiles_m = (M + MF_BM - 1) / MF_BM;
+  const int bn = hal_gemm_f32_tile_columns(M, N);
+  if (tiles_m * ((N + 95) / 96) <= MF_UNITS && mf_rounds_cost(tiles_m, N, bn) > 215) return 96;
+  return bn == 128 && tiles_m * ((N + 127) / 128) % MF_UNITS ? 64 : bn;
 }
 
 extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc,
@@ -526,20 +571,23 @@ extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, fl
       HAL_LAUNCH_CHECK();
       return 0;
     }
-    // more rows: the matrix cores, in the tiles whose rounds over the compute units are expected to end first
-    const int bn = hal_gemm_f32_tile_columns(M, N);
+  }
+  // more rows: the matrix cores, in the tiles whose rounds over the compute units are expected to end first (a tile's
+  // rows are reached by 32-bit offsets from its first)
+  if (K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0 && lda < MF_ROW_LIMIT &&
+      ldw < MF_ROW_LIMIT) {
+    const int bn = hal_gemm_f32_columns(M, N);
     const long long tiles_m = (M + MF_BM - 1) / MF_BM, tiles_n = (N + bn - 1) / bn;
     HAL_REQUIRE(tiles_m * tiles_n < (1ll << 31), "hal_gemm_f32: M=%d N=%d exceed the grid limit", M, N);
     const dim3 tiles((unsigned)(tiles_m * tiles_n));
-    if (bn == 128)
-      hipLaunchKernelGGL(gemm_f32_mfma_kernel<128>, tiles, dim3(256), 0, stream, A, lda, W, ldw, C, ldc, M, N, K,
-                         (int)tiles_m, (int)tiles_n);
-    else if (bn == 64)
-      hipLaunchKernelGGL(gemm_f32_mfma_kernel<64>, tiles, dim3(512), 0, stream, A, lda, W, ldw, C, ldc, M, N, K,
-                         (int)tiles_m, (int)tiles_n);
-    else
-      hipLaunchKernelGGL(gemm_f32_mfma_kernel<32>, tiles, dim3(256), 0, stream, A, lda, W, ldw, C, ldc, M, N, K,
-                         (int)tiles_m, (int)tiles_n);
+#define MF_LAUNCH(BN_)                                                                                                   \
+  hipLaunchKernelGGL(gemm_f32_mfma_kernel<BN_>, tiles, dim3(MF_THREADS(BN_)), 0, stream, A, lda, W, ldw, C, ldc, M, N, K, \
+                     (int)tiles_m, (int)tiles_n)
+    if (bn == 128) MF_LAUNCH(128);
+    else if (bn == 96) MF_LAUNCH(96);
+    else if (bn == 64) MF_LAUNCH(64);
+    else MF_LAUNCH(32);
+#undef MF_LAUNCH
     HAL_LAUNCH_CHECK();
     return 0;
   }
