@@ -119,7 +119,7 @@ static inline size_t plain_lds_floats(int D, int keys, int rows) {
 // (the entry of the block table is asked for in one step of the walk and put down in the
 // next, when the wave waits for its loads anyway)
 // NV: 16-byte vectors of a tile that a thread brings (KEYS * ceil(D / 64) / 16).
-template <typename T, int KEYS, int NV>
+template <typename T, int KEYS, int NV, int THREADS = PLAIN_THREADS>
 struct plain_tiles {
   const T* k_pages;
   const T* v_pages;
@@ -165,7 +165,7 @@ struct plain_tiles {
         if (w.x >= 0) load4(k_pages + ((size_t)w.x * page_size + w.y) * D + kc * 4, kreg[u]);
         else if (w.x == -1) kreg[u][0] = kreg[u][1] = kreg[u][2] = kreg[u][3] = __uint_as_float(0x7fc00000u);
       }
-      const int e = tid + u * PLAIN_THREADS;
+      const int e = tid + u * THREADS;
       const int d = e / (KEYS / 4), jj = (e % (KEYS / 4)) * 4;
       if (d < D) {
         if (page_size % 4 == 0) {  // the four keys lie side by side in one page
@@ -199,7 +199,7 @@ struct plain_tiles {
     for (int u = 0; u < NV; ++u) {
       const int row = kr0 + u * rows_per_pass;
       if (row < KEYS && kc < dv) store4(k_tile + (size_t)row * KS + kc * 4, kreg[u]);
-      const int e = tid + u * PLAIN_THREADS;
+      const int e = tid + u * THREADS;
       const int d = e / (KEYS / 4), jj = (e % (KEYS / 4)) * 4;
       if (d < D) store4(v_tile + (size_t)d * VS + jj, vreg[u]);
     }
@@ -521,35 +521,45 @@ attention_plain_merge_kernel(T* __restrict__ out, int out_row_stride, const int*
 // A row's maximum and sums are updated block by block; blocks outside a row's range change
 // nothing, so a row's result depends on its own position, window and request alone.
 // DB: blocks of 32 dimensions of a head (head sizes that are multiples of 8, up to 32 DB).
+// GROUPS: a block takes a wave alone on its SIMD 9 us, more than twice its products' time, and a prompt of a few hundred
+// tokens has few workgroups, of which the longest walks all keys.  So with up to one workgroup a compute unit (`groups`)
+// eight waves walk 64 keys at once, the first four the even blocks of 32 and the others the odd ones, and two waves join
+// their 32 rows' sums at the end by the log-sum-exp rule.  (32 heads of 128, 8 of the keys, float32, one group and two: one
+// request of 100 tokens 39 / 36 us, 500 146 / 114, 1,000 (256 workgroups) 279 / 216, 2,048 767 / 825; 16 of 500 615 / 740.)
 // Grid: x = groups of `tq` tokens, y = key/value head times chunk of 128 heads of its group.
 typedef __attribute__((ext_vector_type(16))) float plain_f32x16;
 #define ROWS_KEYS 32
 #define ROWS_MOST 128
+#define ROWS_UNITS 256  // compute units of the gfx950 parts that this library is built for
+#define ROWS_THREADS(GROUPS) (ROWS_MOST / 32 * (GROUPS) * HAL_WAVE)
 
-static inline size_t rows_lds_floats(int D, int db) {
-  return (size_t)ROWS_KEYS * (D + PLAIN_PAD) + (size_t)db * 32 * (ROWS_KEYS + PLAIN_PAD) + (size_t)2 * 2 * ROWS_KEYS;
+static inline size_t rows_lds_floats(int D, int db, int groups) {
+  const int keys = ROWS_KEYS * groups;
+  const size_t tiles = (size_t)keys * (D + PLAIN_PAD) + (size_t)db * 32 * (keys + PLAIN_PAD) + (size_t)2 * 2 * keys;
+  const size_t sums = groups == 1 ? 0 : (size_t)ROWS_MOST * 2 * (db * 16 + 2);  // of the waves with the odd blocks, where the tiles were
+  return tiles > sums ? tiles : sums;
 }
 
-template <typename T, int DB>
-__global__ void __launch_bounds__(PLAIN_THREADS, 2)
+template <typename T, int DB, int GROUPS>
+__global__ void __launch_bounds__(ROWS_THREADS(GROUPS), 2)
 attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__ out, int out_row_stride,
                       const int* __restrict__ positions, const int* __restrict__ token_seg,
                       const int* __restrict__ block_table, int bt_stride, const T* __restrict__ k_pages,
                       const T* __restrict__ v_pages, int n_tokens, int H, int K, int D, int page_size,
                       int n_pages, float scale, hal_score_rule rule, int tq, int chunks, int page_shift,
                       int cw_shift) {
-  constexpr int KEYS = ROWS_KEYS;
-  constexpr int NV = KEYS * ((DB + 1) / 2) / 16;
+  constexpr int THREADS = ROWS_THREADS(GROUPS), KEYS = ROWS_KEYS * GROUPS;
+  constexpr int NV = KEYS * ((DB + 1) / 2) * 16 / THREADS;
   extern __shared__ float smem[];
   const int tid = threadIdx.x;
   const int lane = tid % HAL_WAVE;
-  const int wave = __builtin_amdgcn_readfirstlane(tid / HAL_WAVE);
+  const int waves_at = __builtin_amdgcn_readfirstlane(tid / HAL_WAVE), wave = waves_at % (ROWS_MOST / 32), kg = waves_at / (ROWS_MOST / 32);
   const int half = lane / 32, col = lane % 32;
   const int KS = D + PLAIN_PAD, VS = KEYS + PLAIN_PAD;
   float* k_tile = smem;                             // [KEYS][D + pad]
   float* v_tile = k_tile + (size_t)KEYS * KS;        // [32 DB][KEYS + pad], zero from row D on
   int2* key_place = (int2*)(v_tile + (size_t)DB * 32 * VS);  // [2][KEYS]
-  for (int e = D * VS + tid; e < DB * 32 * VS; e += PLAIN_THREADS) v_tile[e] = 0.f;
+  for (int e = D * VS + tid; e < DB * 32 * VS; e += THREADS) v_tile[e] = 0.f;
 
   const int G = H / K;
   const int g = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
@@ -581,9 +591,9 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
     const bool wave_has_rows = wave * 32 < n_rows;
     int wave_lo = 0, wave_p = -1;
     if (wave_has_rows) {
-      const int p0 = positions[ta + wave * 32 / heads_here];
+      const int p0 = __builtin_amdgcn_readfirstlane(positions[ta + wave * 32 / heads_here]);
       wave_lo = hal_rule_lo(rule, p0);
-      wave_p = positions[ta + min(wave * 32 + 31, n_rows - 1) / heads_here];
+      wave_p = __builtin_amdgcn_readfirstlane(positions[ta + min(wave * 32 + 31, n_rows - 1) / heads_here]);
     }
     float qreg[DB * 16];
 #pragma unroll
@@ -600,12 +610,12 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
 #pragma unroll
       for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
 
-    plain_tiles<T, KEYS, NV> tiles;
+    plain_tiles<T, KEYS, NV, THREADS> tiles;
     tiles.k_pages = k_pages, tiles.v_pages = v_pages, tiles.bt = bt;
     tiles.k_tile = k_tile, tiles.v_tile = v_tile, tiles.key_place = key_place;
     tiles.KS = KS, tiles.VS = VS, tiles.D = D, tiles.dv = D / 4, tiles.page_size = page_size, tiles.page_shift = page_shift;
     tiles.n_pages = n_pages, tiles.K = K, tiles.g = g, tiles.lo_min = lo_min, tiles.p_max = p_max, tiles.tid = tid;
-    tiles.kc = tid & ((1 << cw_shift) - 1), tiles.kr0 = tid >> cw_shift, tiles.rows_per_pass = PLAIN_THREADS >> cw_shift;
+    tiles.kc = tid & ((1 << cw_shift) - 1), tiles.kr0 = tid >> cw_shift, tiles.rows_per_pass = THREADS >> cw_shift;
     tiles.asked_page = 0, tiles.asked_slot = -1, tiles.keep = rule.keep;
 
     __syncthreads();  // the walk before is done with the tiles and the places
@@ -624,13 +634,13 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
       if (j0 + KEYS < j_end) tiles.fetch(buf ^ 1);
       tiles.ask_place(walk.key(j0 + 3 * KEYS));
       __syncthreads();
-      const int key0 = walk.key(j0);
-      if (!wave_has_rows || key0 > wave_p || (key0 + KEYS <= wave_lo && key0 >= rule.keep)) continue;  // (the same for the whole wave)
+      const int key0 = walk.key(j0) + kg * ROWS_KEYS;
+      if (!wave_has_rows || key0 > wave_p || (key0 + ROWS_KEYS <= wave_lo && key0 >= rule.keep)) continue;  // (the same for the whole wave)
       // ---- S^T: lane = (key col, half) for the keys, (row col, half) for q ----
       plain_f32x16 st;
 #pragma unroll
       for (int v = 0; v < 16; ++v) st[v] = 0.f;
-      const float* kr = k_tile + (size_t)col * KS + half * hd;
+      const float* kr = k_tile + (size_t)(kg * ROWS_KEYS + col) * KS + half * hd;
 #pragma unroll
       for (int i = 0; i < DB * 4; ++i) {
         if (i * 4 < hd) {
@@ -673,7 +683,7 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
       for (int b = 0; b < DB; ++b) {
 #pragma unroll
         for (int v = 0; v < 16; ++v) acc[b][v] *= alpha;
-        const float* vr = v_tile + (size_t)(b * 32 + col) * VS + 4 * half;
+        const float* vr = v_tile + (size_t)(b * 32 + col) * VS + kg * ROWS_KEYS + 4 * half;
 #pragma unroll
         for (int t4 = 0; t4 < 4; ++t4) {
           const float4 vv = *(const float4*)(vr + 8 * t4);
@@ -690,7 +700,33 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
       plain_swap_32(l, other);
       l = l + other;
     }
-    if (have_row) {  // element v of a block's 16: dimension 32 b + 8 (v / 4) + 4 half + v % 4
+    if constexpr (GROUPS == 2) {
+      // the odd blocks' sums to those of the even ones, which are first
+      float* theirs = smem + (wave * HAL_WAVE + lane) * (DB * 16 + 2);
+      __syncthreads();  // every wave is done with the tiles
+      if (kg == 1) {
+        theirs[DB * 16] = m, theirs[DB * 16 + 1] = l;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) theirs[b * 16 + v] = acc[b][v];
+      }
+      __syncthreads();
+      if (kg == 0) {
+        const float m1 = theirs[DB * 16], m_all = fmaxf(m, m1);
+        const float w0 = m == -INFINITY ? 0.f : expf(m - m_all), w1 = m1 == -INFINITY ? 0.f : expf(m1 - m_all);
+        m = m_all, l = l * w0 + theirs[DB * 16 + 1] * w1;
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[b][v] = acc[b][v] * w0 + theirs[b * 16 + v] * w1;
+      }
+      if (tb < t_end) {  // (another run of tokens: rows of the values' tile from D on are zeros again)
+        __syncthreads();
+        for (int e = D * VS + tid; e < DB * 32 * VS; e += THREADS) v_tile[e] = 0.f;
+      }
+    }
+    if (kg == 0 && have_row) {  // element v of a block's 16: dimension 32 b + 8 (v / 4) + 4 half + v % 4
       T* op = out + (size_t)token * out_row_stride + (size_t)head * D;
       const float inv = hal_rule_inverse(rule, m, l, head);
 #pragma unroll
@@ -811,15 +847,29 @@ extern "C" int hal_attention_simple_ruled(const void* q, int q_row_stride, void*
   HAL_REQUIRE((long long)n_pages * K < (1ll << 31), "hal_attention_simple: %d pages of %d heads exceed the index range", n_pages, K);
   if (rw == 32) {
     const int chunks = (G + ROWS_MOST - 1) / ROWS_MOST, db = (D + 31) / 32;
-    const size_t smem = rows_lds_floats(D, db) * sizeof(float);
+    const int groups = (long long)((n_tokens + tq - 1) / tq) * K * chunks <= ROWS_UNITS ? 2 : 1;
+    const size_t smem = rows_lds_floats(D, db, groups) * sizeof(float);
     const long long gy = (long long)K * chunks;
     HAL_REQUIRE(gy <= 65535, "hal_attention_simple: %lld head chunks exceed the grid limit", gy);
     dim3 grid((n_tokens + tq - 1) / tq, (unsigned)gy);
-#define ROWS_LAUNCH(T_, DB_)                                                                          \
-  hipLaunchKernelGGL((attention_rows_kernel<T_, DB_>), grid, dim3(PLAIN_THREADS), smem, stream,        \
-                     (const T_*)q, q_row_stride, (T_*)out, out_row_stride, positions, token_seg,       \
-                     block_table, bt_stride, (const T_*)k_pages, (const T_*)v_pages, n_tokens, H, K, D, \
-                     page_size, n_pages, scale, rule, tq, chunks, page_shift, cw_shift)
+#define ROWS_LAUNCH_AS(T_, DB_, GROUPS_)                                                                \
+  do {                                                                                                \
+    static bool raised = false; /* more than 64 KB of LDS has to be asked for, once per kernel */      \
+    if (!raised && smem > 64 * 1024) {                                                                \
+      HAL_CHECK_HIP(hipFuncSetAttribute((const void*)attention_rows_kernel<T_, DB_, GROUPS_>,         \
+                                        hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));     \
+      raised = true;                                                                                  \
+    }                                                                                                 \
+    hipLaunchKernelGGL((attention_rows_kernel<T_, DB_, GROUPS_>), grid, dim3(ROWS_THREADS(GROUPS_)), smem, stream, \
+                       (const T_*)q, q_row_stride, (T_*)out, out_row_stride, positions, token_seg,    \
+                       block_table, bt_stride, (const T_*)k_pages, (const T_*)v_pages, n_tokens, H, K, D, \
+                       page_size, n_pages, scale, rule, tq, chunks, page_shift, cw_shift);            \
+  } while (0)
+#define ROWS_LAUNCH(T_, DB_)                    \
+  do {                                          \
+    if (groups == 2) ROWS_LAUNCH_AS(T_, DB_, 2); \
+    else ROWS_LAUNCH_AS(T_, DB_, 1);            \
+  } while (0)
 #define ROWS_BY_SIZE(T_)                  \
   do {                                    \
     if (db == 1) ROWS_LAUNCH(T_, 1);      \
@@ -835,6 +885,7 @@ extern "C" int hal_attention_simple_ruled(const void* q, int q_row_stride, void*
       return hal_fail("hal_attention_simple: unknown dtype %d", dtype);
 #undef ROWS_BY_SIZE
 #undef ROWS_LAUNCH
+#undef ROWS_LAUNCH_AS
     HAL_LAUNCH_CHECK();
     return 0;
   }
