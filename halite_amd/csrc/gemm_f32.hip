@@ -559,10 +559,13 @@ extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, fl
     return 0;
   }
   if (K % 4 == 0 && lda % 4 == 0 && ldw % 4 == 0 && ((uintptr_t)A % 16) == 0 && ((uintptr_t)W % 16) == 0) {
-    // up to 96 rows, and up to 128 on matrices of few columns: k split over a workgroup's waves (measured
-    // against the tiles below on the 8B shape's matrices: o-proj 31 / 50 / 74 / 100 us at 32 / 64 / 96 / 128
-    // rows against 120; gate and up together 129 / 204 / 287 / 414 us against 275 to 368)
-    if (M <= 96 || (M <= 128 && (N + 127) / 128 < 128)) {
+    // up to 96 rows, and up to 128 on matrices of few columns: k split over a workgroup's waves.  Both sides at 64 / 96 / 128
+    // rows, this and the tiles below, us: 4,096 x 4,096 50 / 69 / 93 against 102 / 101 / 101, x 14,336 147 / 225 / 297
+    // against 345 / 347 / 347; 16,384 x 3,072 76 / 101 / 143 against 71 / 104 / 107, 28,672 x 4,096 185 / 250 / 373 against
+    // 151 / 251 / 265, 128,256 x 4,096 747 / 1,003 / 1,476 against 645 / 995 / 1,111.  So not 33 to 64 rows of wide matrices
+    // either: half of a tile's waves have no rows then and leave the matrix cores to the others.
+    const bool wide = (N + 127) / 128 >= 128;
+    if (M <= (wide ? 32 : 128) || (M > 64 && M <= 96)) {
       if (M <= 32 ? launch_rows<1>(A, lda, W, ldw, C, ldc, M, N, K, stream)
           : M <= 64 ? launch_rows<2>(A, lda, W, ldw, C, ldc, M, N, K, stream)
           : M <= 96 ? launch_rows_with<3, 4>(A, lda, W, ldw, C, ldc, M, N, K, stream)
