@@ -93,7 +93,8 @@ __device__ __forceinline__ void plain_join_weights(float M, float m, float& M_ne
   w_new = (m == -INFINITY) ? 0.f : expf(m - M_new);
 }
 __device__ __forceinline__ float plain_join(float A, float w_old, float a, float w_new) {
-  return __fadd_rn(__fmul_rn(A, w_old), __fmul_rn(a, w_new));
+#pragma clang fp contract(off)
+  return A * w_old + a * w_new;
 }
 
 // The pieces of a row whose keys are lo .. p, where every piece is a workgroup of its own and
@@ -522,10 +523,13 @@ attention_plain_merge_kernel(T* __restrict__ out, int out_row_stride, const int*
 // nothing, so a row's result depends on its own position, window and request alone.
 // DB: blocks of 32 dimensions of a head (head sizes that are multiples of 8, up to 32 DB).
 // GROUPS: a block takes a wave alone on its SIMD 9 us, more than twice its products' time, and a prompt of a few hundred
-// tokens has few workgroups, of which the longest walks all keys.  So with up to one workgroup a compute unit (`groups`)
-// eight waves walk 64 keys at once, the first four the even blocks of 32 and the others the odd ones, and two waves join
-// their 32 rows' sums at the end by the log-sum-exp rule.  (32 heads of 128, 8 of the keys, float32, one group and two: one
-// request of 100 tokens 39 / 36 us, 500 146 / 114, 1,000 (256 workgroups) 279 / 216, 2,048 767 / 825; 16 of 500 615 / 740.)
+// tokens has few workgroups, of which the longest walks all keys.  So in float32 with up to one workgroup a compute unit
+// (`groups`) eight waves walk 64 keys at once, the first four the even blocks of 32 and the others the odd ones, and two
+// waves join their 32 rows' sums at the end by the log-sum-exp rule.  How many workgroups there are depends on what else the
+// step holds, so four waves add a float32 row up in the same order: all even blocks, all odd ones, and the same join
+// (TURNS; the even blocks' sums wait in the row's place of `out`, which bf16 rows do not have room for: they keep four waves).
+// (32 heads of 128, 8 of the keys, float32, four waves and eight: one request of 100 tokens 39 / 36 us, 500 146 / 114, 1,000
+// (256 workgroups) 279 / 214; four waves in one turn, in two, and eight: 2,048 772 / 787 / 825, 16 of 500 614 / 646 / 740.)
 // Grid: x = groups of `tq` tokens, y = key/value head times chunk of 128 heads of its group.
 typedef __attribute__((ext_vector_type(16))) float plain_f32x16;
 #define ROWS_KEYS 32
@@ -549,6 +553,7 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
                       int n_pages, float scale, hal_score_rule rule, int tq, int chunks, int page_shift,
                       int cw_shift) {
   constexpr int THREADS = ROWS_THREADS(GROUPS), KEYS = ROWS_KEYS * GROUPS;
+  constexpr int TURNS = GROUPS == 1 && sizeof(T) == 4 ? 2 : 1, STEP = KEYS * TURNS;  // walks of a row's keys, every TURNS-th block each
   constexpr int NV = KEYS * ((DB + 1) / 2) * 16 / THREADS;
   extern __shared__ float smem[];
   const int tid = threadIdx.x;
@@ -579,7 +584,7 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
     const int* bt = block_table + (size_t)seg * bt_stride;
     const int n_rows = (tb - ta) * heads_here;
     const hal_key_walk walk(rule, lo_min);  // (j: places in the walk)
-    const int j_begin = walk.first(lo_min) / KEYS * KEYS, j_end = walk.last(p_max) + 1;
+    const int j_begin = walk.first(lo_min) / STEP * STEP, j_end = walk.last(p_max) + 1;
 
     // this lane's row (both halves of the wave have the same 32 rows)
     const int r = wave * 32 + col;
@@ -603,13 +608,6 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
 #pragma unroll
       for (int x = 0; x < 4; ++x) qreg[i * 4 + x] = t[x];
     }
-    float m = -INFINITY, l = 0.f;  // (l: of this half's keys)
-    plain_f32x16 acc[DB];
-#pragma unroll
-    for (int b = 0; b < DB; ++b)
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
-
     plain_tiles<T, KEYS, NV, THREADS> tiles;
     tiles.k_pages = k_pages, tiles.v_pages = v_pages, tiles.bt = bt;
     tiles.k_tile = k_tile, tiles.v_tile = v_tile, tiles.key_place = key_place;
@@ -618,23 +616,61 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
     tiles.kc = tid & ((1 << cw_shift) - 1), tiles.kr0 = tid >> cw_shift, tiles.rows_per_pass = THREADS >> cw_shift;
     tiles.asked_page = 0, tiles.asked_slot = -1, tiles.keep = rule.keep;
 
+    T* const op = out + (size_t)token * out_row_stride + (size_t)head * D;
+    // element v of a block's 16: dimension 32 b + 8 (v / 4) + 4 half + v % 4
+    auto each_four = [&](auto&& what) {
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int v4 = 0; v4 < 4; ++v4)
+          if (b * 32 + 8 * v4 + 4 * half < D) what(b, 4 * v4, op + b * 32 + 8 * v4 + 4 * half);
+    };
+    float m = -INFINITY, l = 0.f, m_even = -INFINITY, l_even = 0.f;  // (l: of this half's keys, until the halves are joined)
+    plain_f32x16 acc[DB];
+    auto clear = [&]() {
+#pragma unroll
+      for (int b = 0; b < DB; ++b)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) acc[b][v] = 0.f;
+    };
+    auto join_halves = [&]() {
+      float other = l;
+      plain_swap_32(l, other);
+      l = l + other;
+    };
+    clear();
+    // the blocks: `n_even` of them in order, or, with two turns, those at even places and then those at odd ones
+    const int n_blocks = (j_end - j_begin + KEYS - 1) / KEYS, n_even = (n_blocks + TURNS - 1) / TURNS;
+    auto place = [&](int n) { return j_begin + (n < n_even ? n * STEP : (n - n_even) * STEP + KEYS); };
+
     __syncthreads();  // the walk before is done with the tiles and the places
-    tiles.ask_place(walk.key(j_begin));
+    tiles.ask_place(walk.key(place(0)));
     tiles.put_place(0);
-    tiles.ask_place(walk.key(j_begin + KEYS));
+    tiles.ask_place(walk.key(place(1)));
     tiles.put_place(1);
     __syncthreads();
     tiles.fetch(0);
-    tiles.ask_place(walk.key(j_begin + 2 * KEYS));
+    tiles.ask_place(walk.key(place(2)));
     int buf = 0;
-    for (int j0 = j_begin; j0 < j_end; j0 += KEYS, buf ^= 1) {
+    for (int n = 0; n < n_blocks; ++n, buf ^= 1) {
+#pragma clang fp contract(off)  // (the builds for one group and for two round alike)
       __syncthreads();  // every wave has read the block before
       tiles.commit();
       tiles.put_place(buf);  // of the block after the next
-      if (j0 + KEYS < j_end) tiles.fetch(buf ^ 1);
-      tiles.ask_place(walk.key(j0 + 3 * KEYS));
+      if (n + 1 < n_blocks) tiles.fetch(buf ^ 1);
+      tiles.ask_place(walk.key(place(n + 3)));
       __syncthreads();
-      const int key0 = walk.key(j0) + kg * ROWS_KEYS;
+      if (TURNS == 2 && n == n_even) {  // the even blocks' sums make room for the odd ones'
+        join_halves();
+        m_even = m, l_even = l;
+        if (have_row) each_four([&](int b, int v, T* at) {
+          const float t[4] = {acc[b][v], acc[b][v + 1], acc[b][v + 2], acc[b][v + 3]};
+          store4(at, t);
+        });
+        m = -INFINITY, l = 0.f;
+        clear();
+      }
+      const int key0 = walk.key(place(n)) + kg * ROWS_KEYS;
       if (!wave_has_rows || key0 > wave_p || (key0 + ROWS_KEYS <= wave_lo && key0 >= rule.keep)) continue;  // (the same for the whole wave)
       // ---- S^T: lane = (key col, half) for the keys, (row col, half) for q ----
       plain_f32x16 st;
@@ -695,11 +731,7 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
       }
     }
 
-    {
-      float other = l;
-      plain_swap_32(l, other);
-      l = l + other;
-    }
+    join_halves();
     if constexpr (GROUPS == 2) {
       // the odd blocks' sums to those of the even ones, which are first
       float* theirs = smem + (wave * HAL_WAVE + lane) * (DB * 16 + 2);
@@ -713,32 +745,36 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
       }
       __syncthreads();
       if (kg == 0) {
-        const float m1 = theirs[DB * 16], m_all = fmaxf(m, m1);
-        const float w0 = m == -INFINITY ? 0.f : expf(m - m_all), w1 = m1 == -INFINITY ? 0.f : expf(m1 - m_all);
-        m = m_all, l = l * w0 + theirs[DB * 16 + 1] * w1;
+        float m_all, w0, w1;
+        plain_join_weights(m, theirs[DB * 16], m_all, w0, w1);
+        m = m_all, l = plain_join(l, w0, theirs[DB * 16 + 1], w1);
 #pragma unroll
         for (int b = 0; b < DB; ++b)
 #pragma unroll
-          for (int v = 0; v < 16; ++v) acc[b][v] = acc[b][v] * w0 + theirs[b * 16 + v] * w1;
+          for (int v = 0; v < 16; ++v) acc[b][v] = plain_join(acc[b][v], w0, theirs[b * 16 + v], w1);
       }
       if (tb < t_end) {  // (another run of tokens: rows of the values' tile from D on are zeros again)
         __syncthreads();
         for (int e = D * VS + tid; e < DB * 32 * VS; e += THREADS) v_tile[e] = 0.f;
       }
     }
-    if (kg == 0 && have_row) {  // element v of a block's 16: dimension 32 b + 8 (v / 4) + 4 half + v % 4
-      T* op = out + (size_t)token * out_row_stride + (size_t)head * D;
+    if (TURNS == 2 && n_even < n_blocks) {
+      float m_all, w0, w1;
+      plain_join_weights(m_even, m, m_all, w0, w1);
+      m = m_all, l = plain_join(l_even, w0, l, w1);
+      if (have_row) each_four([&](int b, int v, T* at) {
+        float even[4];
+        load4(at, even);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) acc[b][v + i] = plain_join(even[i], w0, acc[b][v + i], w1);
+      });
+    }
+    if (kg == 0 && have_row) {
       const float inv = hal_rule_inverse(rule, m, l, head);
-#pragma unroll
-      for (int b = 0; b < DB; ++b)
-#pragma unroll
-        for (int v4 = 0; v4 < 4; ++v4) {
-          const int d = b * 32 + 8 * v4 + 4 * half;
-          if (d < D) {
-            const float t[4] = {acc[b][4 * v4] * inv, acc[b][4 * v4 + 1] * inv, acc[b][4 * v4 + 2] * inv, acc[b][4 * v4 + 3] * inv};
-            store4(op + d, t);
-          }
-        }
+      each_four([&](int b, int v, T* at) {
+        const float t[4] = {acc[b][v] * inv, acc[b][v + 1] * inv, acc[b][v + 2] * inv, acc[b][v + 3] * inv};
+        store4(at, t);
+      });
     }
     ta = tb;
   }
@@ -847,12 +883,12 @@ extern "C" int hal_attention_simple_ruled(const void* q, int q_row_stride, void*
   HAL_REQUIRE((long long)n_pages * K < (1ll << 31), "hal_attention_simple: %d pages of %d heads exceed the index range", n_pages, K);
   if (rw == 32) {
     const int chunks = (G + ROWS_MOST - 1) / ROWS_MOST, db = (D + 31) / 32;
-    const int groups = (long long)((n_tokens + tq - 1) / tq) * K * chunks <= ROWS_UNITS ? 2 : 1;
+    const int groups = dtype == HAL_F32 && (long long)((n_tokens + tq - 1) / tq) * K * chunks <= ROWS_UNITS ? 2 : 1;
     const size_t smem = rows_lds_floats(D, db, groups) * sizeof(float);
     const long long gy = (long long)K * chunks;
     HAL_REQUIRE(gy <= 65535, "hal_attention_simple: %lld head chunks exceed the grid limit", gy);
     dim3 grid((n_tokens + tq - 1) / tq, (unsigned)gy);
-#define ROWS_LAUNCH_AS(T_, DB_, GROUPS_)                                                                \
+#define ROWS_LAUNCH(T_, DB_, GROUPS_)                                                                   \
   do {                                                                                                \
     static bool raised = false; /* more than 64 KB of LDS has to be asked for, once per kernel */      \
     if (!raised && smem > 64 * 1024) {                                                                \
@@ -865,27 +901,23 @@ extern "C" int hal_attention_simple_ruled(const void* q, int q_row_stride, void*
                        block_table, bt_stride, (const T_*)k_pages, (const T_*)v_pages, n_tokens, H, K, D, \
                        page_size, n_pages, scale, rule, tq, chunks, page_shift, cw_shift);            \
   } while (0)
-#define ROWS_LAUNCH(T_, DB_)                    \
-  do {                                          \
-    if (groups == 2) ROWS_LAUNCH_AS(T_, DB_, 2); \
-    else ROWS_LAUNCH_AS(T_, DB_, 1);            \
+#define ROWS_BY_SIZE(T_, GROUPS_)                     \
+  do {                                                \
+    if (db == 1) ROWS_LAUNCH(T_, 1, GROUPS_);         \
+    else if (db == 2) ROWS_LAUNCH(T_, 2, GROUPS_);    \
+    else if (db == 3) ROWS_LAUNCH(T_, 3, GROUPS_);    \
+    else ROWS_LAUNCH(T_, 4, GROUPS_);                 \
   } while (0)
-#define ROWS_BY_SIZE(T_)                  \
-  do {                                    \
-    if (db == 1) ROWS_LAUNCH(T_, 1);      \
-    else if (db == 2) ROWS_LAUNCH(T_, 2); \
-    else if (db == 3) ROWS_LAUNCH(T_, 3); \
-    else ROWS_LAUNCH(T_, 4);              \
-  } while (0)
-    if (dtype == HAL_F32)
-      ROWS_BY_SIZE(float);
+    if (dtype == HAL_F32 && groups == 2)
+      ROWS_BY_SIZE(float, 2);
+    else if (dtype == HAL_F32)
+      ROWS_BY_SIZE(float, 1);
     else if (dtype == HAL_BF16)
-      ROWS_BY_SIZE(bf16_t);
+      ROWS_BY_SIZE(bf16_t, 1);
     else
       return hal_fail("hal_attention_simple: unknown dtype %d", dtype);
 #undef ROWS_BY_SIZE
 #undef ROWS_LAUNCH
-#undef ROWS_LAUNCH_AS
     HAL_LAUNCH_CHECK();
     return 0;
   }
