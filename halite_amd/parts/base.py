@@ -180,7 +180,7 @@ class Mixer(Part):
     ``kernels.ops.NormedRows`` for ``x`` (rows whose norm the part's first product
     finishes); ``folds_next_norm``, ``forward`` takes ``then=ops.NextNorm`` and may
     return ``NormedRows`` for that norm, with its result already added into the stream,
-    instead of the result."""
+    or, where the norm says ``sums``, ``PartialSums`` instead of the result."""
 
     takes_normed_rows: ClassVar[bool] = False
     folds_next_norm: ClassVar[bool] = False
@@ -208,6 +208,9 @@ class FeedForward(Part):
     takes_normed_rows: ClassVar[bool] = False
     folds_next_norm: ClassVar[bool] = False
     adds_to_stream: ClassVar[bool] = False
+    # True: ``then`` may also be what ``Norm.summable`` gives: a norm for which the result may come back as
+    # ``PartialSums``, as ``kernels.ops.linear`` gives them, and not as ``NormedRows``
+    leaves_sums: ClassVar[bool] = False
 
     def forward(self, x: torch.Tensor, ctx: "StepContext") -> torch.Tensor:
         raise NotImplementedError
@@ -226,9 +229,14 @@ class Norm(Part):
         (``kernels.ops.NormedRows``, see ``foldable``), which is handed on as it is."""
         raise NotImplementedError
 
-    def foldable(self, h: torch.Tensor, gathers: bool = False):
+    def foldable(self, h: torch.Tensor):
         """``kernels.ops.NextNorm`` if the product before this norm may add into ``h`` and
         prepare the norm's input itself, else None."""
+        return None
+
+    def summable(self, h: torch.Tensor):
+        """``kernels.ops.NextNorm`` (with ``gathers``) if this norm of some of ``h``'s rows adds up ``PartialSums`` that the
+        product before it leaves, else None: what the model's last product may be told of its final norm."""
         return None
 
 

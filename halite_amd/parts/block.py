@@ -29,6 +29,7 @@ class PreNormBlock(Arrangement):
     graph_safe = True
     roles = {"mixer_norm": NORMS, "mixer": MIXERS, "ff_norm": NORMS, "ff": FEED_FORWARDS}
     takes_next_norm = True  # forward() accepts next_norm=
+    takes_last_norm = True  # ... also where it is the model's final norm, which gathers rows
 
     def __init__(self, parts):
         super().__init__(parts)
@@ -47,7 +48,7 @@ class PreNormBlock(Arrangement):
             then = self.ff_norm.foldable(h)
         a = self.mixer.forward(x, ctx, run, then=then) if then is not None else self.mixer.forward(x, ctx, run)
         x = self.ff_norm.forward(h, delta=a)
-        if next_norm is not None and self.ff.folds_next_norm:
+        if next_norm is not None and self.ff.folds_next_norm and (self.ff.leaves_sums or not next_norm.gathers):
             return self.ff.forward(x, ctx, then=next_norm)
         return self.ff.forward(x, ctx)
 

@@ -141,13 +141,14 @@ class Decoder:
                 pending = None
             # what the next block's first norm lets this block's last product do for it
             # (both are optional abilities of an arrangement: `takes_next_norm` of the one that
-            # runs now, `first_norm_for` of the one that runs next)
+            # runs now, `first_norm_for` of the one that runs next), and the last block's for the final norm
+            # (`takes_last_norm` of the arrangement, `summable` of the norm)
             ahead = blocks[i + 1] if i + 1 < len(blocks) and self.spec.order[i + 1].junction is None else None
             next_norm = None
             if getattr(blocks[i], "takes_next_norm", False) and hasattr(ahead, "first_norm_for"):
                 next_norm = ahead.first_norm_for(h)
-            elif getattr(blocks[i], "takes_next_norm", False) and i + 1 == len(blocks) and hasattr(self.final_norm, "foldable"):
-                next_norm = self.final_norm.foldable(h, gathers=True)
+            elif i + 1 == len(blocks) and getattr(blocks[i], "takes_last_norm", False):
+                next_norm = self.final_norm.summable(h)
             if next_norm is not None:
                 pending = blocks[i].forward(h, pending, ctx, run, next_norm=next_norm)
             else:

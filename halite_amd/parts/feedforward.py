@@ -57,6 +57,7 @@ class GatedFeedForward(FeedForward):
     graph_safe = True
     takes_normed_rows = True
     folds_next_norm = True
+    leaves_sums = True
 
     def param_decls(self):
         f, d = self.p.intermediate_size, self.p.hidden_size

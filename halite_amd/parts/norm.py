@@ -2,6 +2,8 @@
 
 from __future__ import annotations
 
+from dataclasses import replace
+
 import torch
 from pydantic import BaseModel, Field, StrictBool, StrictInt, model_validator
 
@@ -78,7 +80,11 @@ class RMSNorm(Norm):
             return delta
         return ops.rmsnorm(h, self.weight, self.p.eps, self.build.dtype, delta=delta, rows=rows)
 
-    def foldable(self, h, gathers=False):
+    def foldable(self, h):
         if self.build.dtype != torch.bfloat16 or not h.is_cuda or not self.p.round_before_weight:
             return None
-        return ops.NextNorm(h, self.weight, self.p.eps, sums=True, gathers=gathers)
+        return ops.NextNorm(h, self.weight, self.p.eps, sums=True)
+
+    def summable(self, h):
+        norm = self.foldable(h)
+        return None if norm is None else replace(norm, gathers=True)
