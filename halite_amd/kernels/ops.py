@@ -860,7 +860,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
         return gemm_bf16_skinny(x, tiled, out_dtype=out_dtype, tiled_shape=tuple(w.shape))
     if skinny_ok and skinny_pays(m, w.shape[0], k, False):
         return gemm_bf16_skinny(x, w, out_dtype=out_dtype)
-    parts = stream_parts(x, w, w.shape[0], may_part=sums or (next_norm is not None and next_norm.sums))
+    # (who adds up the parts rounds their sum to bf16: a result that is wanted in float32 comes whole)
+    in_parts = out_dtype == torch.bfloat16 and (sums or (next_norm is not None and next_norm.sums))
+    parts = stream_parts(x, w, w.shape[0], may_part=in_parts)
     if parts:
         return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)
     if out_dtype == torch.float32:

@@ -94,3 +94,23 @@ def test_an_arrangement_with_the_plain_interface(norm):
     own = OwnBlock()
     step([own], norm())
     assert own.told == [None]
+
+
+def test_results_that_are_wanted_in_float32_come_whole():
+    """(the choice itself, without a GPU: only 16-bit results may come in parts, since the reader rounds their sum)"""
+    seen = []
+
+    def parts(x, w, n, gated=False, may_part=False):
+        seen.append(may_part)
+        raise StopIteration
+
+    x, w = torch.zeros((17, 64), dtype=torch.bfloat16), torch.zeros((128, 64), dtype=torch.bfloat16)
+    norm = ops.NextNorm(torch.zeros((17, 128)), torch.ones(128), 1e-5, sums=True, gathers=True)
+    kept, ops.stream_parts = ops.stream_parts, parts
+    try:
+        for how in (dict(sums=True), dict(next_norm=norm), dict(sums=True, out_dtype=torch.float32), dict(next_norm=norm, out_dtype=torch.float32)):
+            with pytest.raises(StopIteration):
+                ops.linear(x, w, **how)
+    finally:
+        ops.stream_parts = kept
+    assert seen == [True, True, False, False]
