@@ -717,7 +717,8 @@ def stream_parts(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, 
     m, k = x.shape
     if not (SKINNY_ROWS < m <= STREAM_ROWS and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.is_cuda
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k and x.data_ptr() % 16 == 0 and w.stride(1) == 1
-            and w.stride(0) % 8 == 0 and w.stride(0) >= k and w.data_ptr() % 16 == 0 and n * w.stride(0) * 2 < 2**31):
+            and w.stride(0) % 8 == 0 and w.stride(0) >= k and w.data_ptr() % 16 == 0 and n * w.stride(0) * 2 < 2**31
+            and m * x.stride(0) * 2 < 2**31):  # (the kernel's offsets)
         return 0
     return _stream_parts(n, k, gated, may_part)
 
