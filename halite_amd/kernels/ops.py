@@ -249,7 +249,9 @@ def rmsnorm(
     ``rows``; with ``delta`` and ``update_h`` the sum is written back to ``h``."""
     lib = library.core_library()
     if isinstance(delta, PartialSums):
-        if update_h and out_dtype == torch.bfloat16 and h.shape[1] % 4 == 0 and h.shape[1] <= RMS_PLANES_WIDTH:
+        # (the kernel reads four numbers at a time; weights at other places are read by the one for results in one piece)
+        if (update_h and out_dtype == torch.bfloat16 and h.shape[1] % 4 == 0 and h.shape[1] <= RMS_PLANES_WIDTH
+                and h.data_ptr() % 16 == 0 and weight.data_ptr() % (4 * weight.element_size()) == 0):
             planes, (n_tokens, d) = delta.planes, h.shape
             n_rows = n_tokens if rows is None else rows.numel()
             _dev(h, weight, planes, rows)

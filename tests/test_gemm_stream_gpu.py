@@ -87,6 +87,19 @@ def test_the_norm_adds_up_planes(gpu, rows, d, n_planes):
     assert torch.equal(x, ops.rmsnorm(h2, w, 1e-5, torch.bfloat16, delta=planes.materialize(torch.bfloat16), rows=some))
 
 
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("off_h, off_w", [(0, 1), (0, 2), (1, 0), (3, 3)])
+def test_a_norm_off_the_kernels_places(gpu, off_h, off_w, dtype):
+    """Weights and streams that begin inside a vector: taken as with a delta in one piece."""
+    rows, d = 18, 512
+    planes = ops.PartialSums(rand(gpu, 3, rows, d, seed=13))
+    w = rand(gpu, d + off_w, seed=14).to(dtype)[off_w:]
+    h, h2 = (rand(gpu, rows * d + off_h, seed=15)[off_h:].view(rows, d) for _ in range(2))
+    x = ops.rmsnorm(h, w, 1e-5, torch.bfloat16, delta=planes)
+    y = ops.rmsnorm(h2, w, 1e-5, torch.bfloat16, delta=planes.materialize(torch.bfloat16))
+    assert torch.equal(x, y) and torch.equal(h, h2)
+
+
 @pytest.mark.parametrize("H,K,D,page,tiled", [(32, 8, 128, 64, True), (24, 8, 128, 64, True), (6, 2, 48, 16, False), (4, 4, 16, 8, False)])
 def test_the_rotation_adds_up_planes(gpu, H, K, D, page, tiled):
     n, segs, n_planes = 37, 5, 3
