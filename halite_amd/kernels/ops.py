@@ -233,7 +233,7 @@ def take_tokens(src: torch.Tensor, tokens: torch.Tensor) -> None:
     _check(lib, lib.hal_take_tokens(_ptr(src), src.numel(), _ptr(tokens), tokens.numel(), _stream()))
 
 
-RMS_PLANES_WIDTH = 16384  # what the norm's kernel holds of a row
+RMS_PLANES_WIDTH = 32768  # what the norm's kernel holds of a row (1,024 threads of eight vectors of four)
 
 
 def rmsnorm(

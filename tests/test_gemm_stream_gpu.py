@@ -73,7 +73,7 @@ def test_what_it_does_not_take(gpu):
     assert not ops.stream_parts(x(17).float(), w, 4096, may_part=True)
 
 
-@pytest.mark.parametrize("rows,d,n_planes", [(17, 4096, 4), (64, 3072, 5), (33, 8192, 2), (20, 260, 9)])
+@pytest.mark.parametrize("rows,d,n_planes", [(17, 4096, 4), (64, 3072, 5), (33, 8192, 2), (20, 260, 9), (17, 16388, 2), (17, 32768, 2), (17, 32772, 2)])
 def test_the_norm_adds_up_planes(gpu, rows, d, n_planes):
     planes = ops.PartialSums(rand(gpu, n_planes, rows, d, seed=7))
     h, w = rand(gpu, rows, d, seed=8), rand(gpu, d, seed=9).bfloat16()
