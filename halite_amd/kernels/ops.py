@@ -398,6 +398,11 @@ def rope_append_sums(qkv: PartialSums, positions: torch.Tensor, cos: torch.Tenso
     _need(k_pages.dtype == torch.bfloat16 and v_pages.dtype == torch.bfloat16
           and k_pages.shape == (n_pages, n_kv_heads, page_size, head_dim)
           and v_pages.shape == (n_pages, n_kv_heads, head_dim, page_size), "rope_append_sums: bf16 pages")
+    if (cos.data_ptr() | sin.data_ptr()) % 16 or k_pages.data_ptr() % 8:  # (read and written a vector at a time)
+        rows = qkv.materialize(torch.bfloat16)
+        rope_append(rows, positions, cos, sin, n_heads, n_kv_heads, head_dim, head_dim, False, token_seg=token_seg,
+                    block_table=block_table, k_pages=k_pages, v_pages=v_pages, page_size=page_size, tiled=tiled)
+        return rows[:, : n_heads * head_dim].contiguous()
     q = torch.empty((n, n_heads * head_dim), dtype=torch.bfloat16, device=planes.device)
     _check(lib, lib.hal_rope_append_planes(
         _ptr(planes), planes.shape[0], _ptr(q), _ptr(positions), _ptr(token_seg), _ptr(block_table), block_table.shape[1],

@@ -100,8 +100,9 @@ def test_a_norm_off_the_kernels_places(gpu, off_h, off_w, dtype):
     assert torch.equal(x, y) and torch.equal(h, h2)
 
 
+@pytest.mark.parametrize("off", [0, 1])  # (tables that begin inside a vector)
 @pytest.mark.parametrize("H,K,D,page,tiled", [(32, 8, 128, 64, True), (24, 8, 128, 64, True), (6, 2, 48, 16, False), (4, 4, 16, 8, False)])
-def test_the_rotation_adds_up_planes(gpu, H, K, D, page, tiled):
+def test_the_rotation_adds_up_planes(gpu, H, K, D, page, tiled, off):
     n, segs, n_planes = 37, 5, 3
     planes = ops.PartialSums(rand(gpu, n_planes, n, (H + 2 * K) * D, seed=10))
     i32 = lambda t: t.to(torch.int32).to(gpu)  # noqa: E731
@@ -111,7 +112,7 @@ def test_the_rotation_adds_up_planes(gpu, H, K, D, page, tiled):
     pages = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16, device=gpu)  # noqa: E731
     pos = pos % (8 * page)
     k1, v1, k2, v2 = pages(40, K, page, D), pages(40, K, D, page), pages(40, K, page, D), pages(40, K, D, page)
-    cos, sin = torch.cos(angles), torch.sin(angles)
+    cos, sin = (torch.cat((t.new_zeros(off), t.flatten()))[off:].view(t.shape) for t in (torch.cos(angles), torch.sin(angles)))
     q = ops.rope_append_sums(planes, pos, cos, sin, H, K, D, seg, table, k1, v1, page, tiled)
     rows = planes.materialize(torch.bfloat16)
     ops.rope_append(rows, pos, cos, sin, H, K, D, D, False, token_seg=seg, block_table=table, k_pages=k2, v_pages=v2, page_size=page, tiled=tiled)
