@@ -110,7 +110,7 @@ __device__ __forceinline__ bool dk_locate(const int* __restrict__ seg_q_len, int
 // with the channels 16 j + 4 g .. + 3 (g = l / 16); the rows change sides through LDS.
 // The products of decays and what they multiply are made in 64 bits and rounded once: chains of float32 ones
 // showed in the results (distance from 64 bits of a head's normed rows 2.8e-7 instead of 1.7e-7).
-template <typename W, bool VEC>  // (VEC: rows of W2 are whole vectors of four)
+template <typename W, bool VEC>  // (VEC: rows of W2 are whole vectors of four, and lie at multiples of one)
 __global__ void __launch_bounds__(DK_HEADS * HAL_WAVE, 4)
 delta_chunk_prep_kernel(const float* __restrict__ r, int ldr, const float* __restrict__ k, int ldk,
                         const float* __restrict__ a_raw, int lda, const float* __restrict__ x1, int ldx1,
@@ -421,7 +421,9 @@ delta_chunk_scan_kernel(const float* __restrict__ records, const float* __restri
   // of the rows that are written this lane has token 4 wave + g, columns 4 (l % 16) .. + 3
   const int mine_at = (4 * wave + g) * DK_ROW + 4 * col16;
   float weight[4];
-  load4_any(gate.weight, gate.w_dtype, first + 4 * col16, weight);
+#pragma unroll
+  for (int i = 0; i < 4; ++i)  // (one by one, once a workgroup: the weight may begin anywhere)
+    weight[i] = gate.w_dtype == HAL_F32 ? ((const float*)gate.weight)[first + 4 * col16 + i] : to_f32(((const bf16_t*)gate.weight)[first + 4 * col16 + i]);
   dk_f32x4 zg = zero;  // the gates of the chunk that is written next
   T* const to = out + (size_t)(t0 + 4 * wave + g) * H * DK_D + first + 4 * col16;
   // Turn c: the record of chunk c - 1 is in `last`, that of chunk c + 2 goes to `free`.
@@ -520,23 +522,27 @@ extern "C" int hal_delta_chunks(const float* r, int ldr, const float* k, int ldk
                   (dtype == HAL_F32 || dtype == HAL_BF16),
               "hal_delta_chunks: dtypes %d, %d, %d", w_dtype, weight_dtype, dtype);
   HAL_REQUIRE(z && weight && out && records && state, "hal_delta_chunks: arguments missing");
+  HAL_REQUIRE((uintptr_t)records % 16 == 0 && (uintptr_t)out % (dtype == HAL_F32 ? 16 : 8) == 0, "hal_delta_chunks: records or results off a vector");
   if (n_tokens == 0 || n_segs == 0) return 0;
   const dim3 all((unsigned)(n_tokens / DK_TOKENS + n_segs), (H + DK_HEADS - 1) / DK_HEADS);
 #define DK_PREP(W_, VEC_)                                                                                                     \
   hipLaunchKernelGGL((delta_chunk_prep_kernel<W_, VEC_>), all, dim3(DK_HEADS * HAL_WAVE), 0, stream, r, ldr, k, ldk, a_raw, lda, \
                      x1, ldx1, (const W_*)w2, (const W_*)w0, (const W_*)a_bias, lora, decay_rate, unit_eps, seg_q_start,        \
                      seg_q_len, n_segs, records, H)
+  const bool vec = lora % 4 == 0 && (uintptr_t)w2 % (w_dtype == HAL_F32 ? 16 : 8) == 0;
   if (w_dtype == HAL_F32) {
-    if (lora % 4 == 0) DK_PREP(float, true);
+    if (vec) DK_PREP(float, true);
     else DK_PREP(float, false);
   } else {
-    if (lora % 4 == 0) DK_PREP(bf16_t, true);
+    if (vec) DK_PREP(bf16_t, true);
     else DK_PREP(bf16_t, false);
   }
 #undef DK_PREP
   HAL_LAUNCH_CHECK();
   const DeltaGate gate = {z, ldz, weight, weight_dtype, eps};
-#define DK_SCAN(T_)                                                                                                          hipLaunchKernelGGL(delta_chunk_scan_kernel<T_>, dim3(n_segs, H), dim3(512), 0, stream, records, v, ldv, state, seg_q_start,                      seg_q_len, token_slot, gate, (T_*)out, H)
+#define DK_SCAN(T_)                                                                                                        \
+  hipLaunchKernelGGL(delta_chunk_scan_kernel<T_>, dim3(n_segs, H), dim3(512), 0, stream, records, v, ldv, state, seg_q_start, \
+                     seg_q_len, token_slot, gate, (T_*)out, H)
   if (dtype == HAL_F32) DK_SCAN(float);
   else DK_SCAN(bf16_t);
 #undef DK_SCAN

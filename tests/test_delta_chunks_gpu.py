@@ -75,6 +75,16 @@ def test_rows_and_states(gpu, H, rank, lens, stored):
     assert torch.equal(rounded, y.to(torch.bfloat16))
 
 
+@pytest.mark.parametrize("stored", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("off", [1, 2, 3])
+def test_weights_that_begin_inside_a_vector(gpu, off, stored):
+    x = inputs(gpu, 3, 8, [33, 16], stored=stored)
+    moved = dict(x, **{name: torch.cat((x[name].new_zeros(off), x[name].flatten())).to(gpu)[off:].view(x[name].shape) for name in ("w2", "w0", "ab", "weight")})
+    assert moved["w2"].data_ptr() % (4 * moved["w2"].element_size()) != 0 and moved["weight"].data_ptr() % (4 * moved["weight"].element_size()) != 0
+    (y, state), (y2, state2) = run(gpu, x), run(gpu, moved)
+    assert torch.equal(y, y2) and torch.equal(state[1:-1], state2[1:-1])
+
+
 @pytest.mark.parametrize("what", [0, 1, 2, 3, 4])  # r, k, v, a, z
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_an_infinite_number_reaches_no_token_before_it(gpu, what, value):
