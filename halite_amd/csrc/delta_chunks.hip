@@ -10,8 +10,8 @@
 //   Q = Wu Z_0 + Wm V          Wu = (I + L)^-1 U~,  Wm = (I + L)^-1 M   (forward substitution)
 //   O = X Z_0 + N V            X = R~ - E Wu,       N = K - E Wm
 //   S_n = diag(G_n) (Z_0 + K~^T V - E~^T Q).
-// A decay is at least exp(-rate): 1 / G is at most exp(16 rate), which float32 holds far from its ends for the
-// rates that the host lets through.
+// A decay is at least exp(-rate): 1 / G is at most exp(16 rate), 2e17 for the largest rate that the host lets through, which
+// float32 holds far from its ends (k~ of keys above 1e21 would not be held, where the walk holds them).
 //
 // Two kernels.  delta_chunk_prep_kernel makes a chunk's record (Wu, X, E~, K~, Wm, N, G_n) for all chunks
 // side by side, a wave a (chunk, head).  delta_chunk_scan_kernel walks a segment's chunks, a workgroup a
@@ -22,7 +22,8 @@
 // dependent instructions of 32 clocks are 0.8).  Measured with 64 heads beside the walk token by token and the norm and
 // gate in a pass of their own: requests of 225, 450, 675 and 900 tokens 505 -> 192 us, one of 2,048 690 -> 290, one of 8,192
 // 2,640 -> 1,150, one of 300 128 -> 61, 32 of 16 tokens each 125 -> 86.  Distance from 64 bits (2-norm) of the normed rows
-// 1.55e-7 beside 1.47e-7, of the states 1.0e-7 beside 0.96e-7, largest differences 2.5e-7 beside 3.1e-7.
+// 1.55e-7 beside 1.47e-7, of the states 1.0e-7 beside 0.96e-7, largest differences 2.5e-7 beside 3.1e-7; at a rate of 2.5 and
+// decays next to exp(-2.5) 5.4e-7 beside 4.6e-7 and 6.3e-8 beside 4.7e-8, next to 1 1.8e-7 beside 1.7e-7 and 2.4e-7 each.
 #include "hal_lds.h"
 #include "hal_api.h"
 

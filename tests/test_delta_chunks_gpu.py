@@ -34,22 +34,22 @@ def inputs(gpu, H, rank, lens, stored=torch.float32, seed=1):
                 starts=i32([sum(lens[:i]) for i in range(S)]), counts=i32(lens), slot=i32([s for s, m in zip(slots, lens) for _ in range(m)]))
 
 
-def run(gpu, x, dtype=torch.float32):
+def run(gpu, x, dtype=torch.float32, rate=RATE):
     a, n = x["a"].to(gpu), x["H"] * D
     r, k, v, a_raw, z = (a[:, i * n : (i + 1) * n] for i in range(5))
     state = x["state"].clone().to(gpu)
     y = ops.delta_chunks(r, k, v, a_raw, a[:, 5 * n : 5 * n + x["rank"]], x["w2"].to(gpu), x["w0"].to(gpu), x["ab"].to(gpu), state,
-                         x["starts"], x["counts"], x["slot"], RATE, UNIT_EPS, z, x["weight"].to(gpu), EPS, dtype)
+                         x["starts"], x["counts"], x["slot"], rate, UNIT_EPS, z, x["weight"].to(gpu), EPS, dtype)
     return y.cpu(), state.cpu()
 
 
-def plain(x, segment):
+def plain(x, segment, rate=RATE):
     """The segment's rows and the state after it, in 64 bits."""
     H, n = x["H"], x["H"] * D
     t0 = sum(x["lens"][:segment])
     b = x["a"][t0 : t0 + x["lens"][segment]].to(F)
     r, k, v, a_raw, z = (b[:, i * n : (i + 1) * n].view(-1, H, D) for i in range(5))
-    decay = torch.exp(-RATE * torch.sigmoid(torch.tanh(b[:, 5 * n : 5 * n + x["rank"]]) @ x["w2"].to(F).T + x["w0"].to(F))).view(-1, H, D)
+    decay = torch.exp(-rate * torch.sigmoid(torch.tanh(b[:, 5 * n : 5 * n + x["rank"]]) @ x["w2"].to(F).T + x["w0"].to(F))).view(-1, H, D)
     rate = torch.sigmoid(a_raw + x["ab"].to(F).view(H, D))
     start = x["state"][x["slots"][segment]].to(F)
     heads = [P.delta_recurrence(r[:, h], k[:, h], v[:, h], decay[:, h], rate[:, h], start[h]) for h in range(H)]
@@ -73,6 +73,25 @@ def test_rows_and_states(gpu, H, rank, lens, stored):
     assert bool(torch.isnan(state[0]).all()) and bool(torch.isnan(state[-1]).all())
     rounded, _ = run(gpu, x, torch.bfloat16)
     assert torch.equal(rounded, y.to(torch.bfloat16))
+
+
+@pytest.mark.parametrize("rate", [1e-4, 1.5, 2.5])
+@pytest.mark.parametrize("bias", ["strong", "weak", "mixed"])
+def test_rates_up_to_the_largest(gpu, rate, bias):
+    """Decays near exp(-rate) in every token (a chunk's product is then exp(-16 rate), 4e-18 at the largest rate, which keys are
+    divided by), near 1, and both among a head's channels; the bound is that of the rows and states above."""
+    H, lens = 3, [16, 47, 33]
+    x = inputs(gpu, H, 8, lens, seed=9)
+    shift = torch.full((H * D,), 12.0)
+    if bias != "strong":
+        shift[(torch.arange(H * D) % 2 == 0) | (bias == "weak")] = -12.0
+    x["w0"] = x["w0"] + shift
+    y, state = run(gpu, x, rate=rate)
+    for i in range(len(lens)):
+        want, left = plain(x, i, rate)
+        t0 = sum(lens[:i])
+        assert float((y[t0 : t0 + lens[i]] - want).abs().max()) < 3e-5 * max(1.0, float(want.abs().max())), (i, lens[i])
+        assert float((state[x["slots"][i]] - left).abs().max()) < 3e-5 * max(1.0, float(left.abs().max())), (i, lens[i])
 
 
 @pytest.mark.parametrize("stored", [torch.float32, torch.bfloat16])
