@@ -1031,14 +1031,14 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams par
     }
   }
   __syncthreads();
-  if (wave >= PICK_QUARTERS) return;  // (the barrier below is met by the waves that are left)
+  // (a wave past the quarters begins at the share's end or behind it and has no runs)
   const int begin = p_begin + wave * run_len, end = quarter_end(wave);
   const int runs = end > begin ? (end - begin + HAL_WAVE - 1) / HAL_WAVE : 0;
   float mine = 0.f, zz = 0.f;
   for (int u = 0; u < runs && u < RUNS; ++u) mine += e_s[wave][u][lane];
   for (int i = begin + RUNS * HAL_WAVE + lane; i < end; i += HAL_WAVE) mine += kept_mass_of(x[i], T, r.key_min, r.m, mp, zz);
   const float wave_mass = wave_sum(mine);
-  if (lane == 0) quarter_mass[wave] = wave_mass;
+  if (lane == 0 && wave < PICK_QUARTERS) quarter_mass[wave] = wave_mass;
   __syncthreads();
   float before = before_part;
   int pick = -1, last = -1;
