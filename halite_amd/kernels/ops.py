@@ -554,6 +554,11 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor):
     return out
 
 
+# Room for the lists of the sampler's rows with filters: 256 MiB, 523 rows of 128,256.  So many rows keep the chip busy, and
+# more go in turns (1,024 rows 517 us at once, 515 in two turns; with room for 130 rows 765).
+SAMPLE_LIST_WORDS = 64 * 1024 * 1024
+
+
 def sample(
     logits: torch.Tensor,
     temperature: torch.Tensor,
@@ -600,14 +605,19 @@ def sample(
             _ptr(parts), _ptr(tokens), _ptr(logprobs), _stream()))
         return tokens, logprobs
     if spread and logits.is_contiguous():
+        # a row's list has room for all of its logits (they may all be alike), so many rows go in turns over one room
+        at_once = min(n, max(1, SAMPLE_LIST_WORDS // vocab))
         # (one buffer: histograms and the rows' state first, which are 64-bit words)
-        words = [n * 2 * 256 * 2, n * 6, n * 32 * 4, n * 32, n * vocab]
+        words = [at_once * 2 * 256 * 2, at_once * 6, at_once * 32 * 4, at_once * 32, at_once * vocab]
         room = torch.empty(sum(words), dtype=torch.int32, device=logits.device)
-        hist, state, parts, kept, lists = (room.data_ptr() + 4 * sum(words[:i]) for i in range(5))
-        _check(lib, lib.hal_sample_spread(
-            _ptr(logits), vocab, n, vocab, _ptr(temperature), _ptr(top_k), _ptr(top_p), _ptr(min_p),
-            _ptr(seeds), _ptr(draw_index), *(ctypes.c_void_p(p) for p in (parts, kept, state, hist, lists)),
-            1 if late else 0, _ptr(tokens), _ptr(logprobs), _stream()))
+        hist, state, parts, kept, lists = (ctypes.c_void_p(room.data_ptr() + 4 * sum(words[:i])) for i in range(5))
+        for r in range(0, n, at_once):
+            def row(t, width=1):
+                return ctypes.c_void_p(t.data_ptr() + r * width * t.element_size())
+
+            _check(lib, lib.hal_sample_spread(
+                row(logits, vocab), vocab, min(at_once, n - r), vocab, row(temperature), row(top_k), row(top_p), row(min_p),
+                row(seeds), row(draw_index), parts, kept, state, hist, lists, 1 if late else 0, row(tokens), row(logprobs), _stream()))
         return tokens, logprobs
     keys = torch.empty((n, vocab), dtype=torch.int32, device=logits.device) if key_scratch and not all_greedy else None
     _check(

@@ -46,6 +46,33 @@ def test_drawn_rows(vocab, spread):
     agree(ways, n, allowed=1)
 
 
+@pytest.mark.parametrize("rows_at_once", [1, 3, 7, 20, 21])
+def test_rows_in_turns(monkeypatch, rows_at_once):
+    """More rows than there is room for lists: the same tokens, turn by turn over one room."""
+    n, vocab, rng = 20, 5000, random.Random(5)
+    x = torch.randn((n, vocab), generator=torch.Generator().manual_seed(2)).cuda()
+    params = ([rng.choice([0.0, 0.7, 1.0]) for _ in range(n)], [rng.choice([-1, 1, 40, 4999]) for _ in range(n)],
+              [rng.choice([0.3, 0.9, 1.0]) for _ in range(n)], [rng.choice([0.0, 0.05]) for _ in range(n)], 11)
+    (_, _), (tok, lp) = both(x, *params)
+    monkeypatch.setattr(ops, "SAMPLE_LIST_WORDS", rows_at_once * vocab + 1)
+    (_, _), (tok2, lp2) = both(x, *params)
+    assert torch.equal(tok, tok2) and torch.equal(lp, lp2)
+
+
+def test_room_for_many_rows():
+    """What a step holds beside its logits does not grow with them: 256 MiB of lists, and 5 KiB a row of the rows in turn."""
+    n, vocab = 1100, 100000
+    x = torch.zeros((n, vocab), device="cuda")
+    full = lambda v, dt=torch.float32: torch.full((n,), v, dtype=dt, device="cuda")  # noqa: E731
+    args = (full(1.0), full(-1, torch.int32), full(0.9), full(0.0), full(1, torch.int64), full(1, torch.int32))
+    torch.cuda.synchronize()
+    torch.cuda.empty_cache()
+    torch.cuda.reset_peak_memory_stats()
+    before = torch.cuda.memory_allocated()
+    ops.sample(x, *args, spread=True)
+    assert torch.cuda.max_memory_allocated() - before < 272 * 2**20
+
+
 def test_rows_at_the_ends():
     n, vocab = 12, 6000
     x = torch.randn((n, vocab), generator=torch.Generator().manual_seed(1))
