@@ -522,7 +522,7 @@ static double mf_rounds_cost(long long tiles_m, int N, int BN) {
 }
 
 // The columns of the tiles that M rows by N columns take on the matrix cores by that count (100 rows and fewer: see below).
-extern "C" int hal_gemm_f32_tile_columns(int M, int N) {
+static int mf_columns_by_rounds(int M, int N) {
   const long long tiles_m = (M + MF_BM - 1) / MF_BM;
   int bn = 128;
   for (int other = 64; other >= 32; other /= 2)
@@ -538,7 +538,7 @@ extern "C" int hal_gemm_f32_tile_columns(int M, int N) {
 // 130 x 28,672 505 / 512; full rounds: 512 x 8,192 264 / 258).
 extern "C" int hal_gemm_f32_columns(int M, int N) {
   const long long tiles_m = (M + MF_BM - 1) / MF_BM;
-  const int bn = hal_gemm_f32_tile_columns(M, N);
+  const int bn = mf_columns_by_rounds(M, N);
   if (tiles_m * ((N + 95) / 96) <= MF_UNITS && mf_rounds_cost(tiles_m, N, bn) > 215) return 96;
   return bn == 128 && tiles_m * ((N + 127) / 128) % MF_UNITS ? 64 : bn;
 }

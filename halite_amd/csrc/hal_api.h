@@ -74,7 +74,6 @@ int hal_attention_simple_ruled(const void* q, int q_row_stride, void* out, int o
 
 int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M,
                  int N, int K, hipStream_t stream);
-int hal_gemm_f32_tile_columns(int M, int N);
 int hal_gemm_f32_columns(int M, int N);
 
 // X [M <= 64, K] bf16, W [N, K] bf16, optional W2 [N, K] (gated: up * act(gate), W the gate's;

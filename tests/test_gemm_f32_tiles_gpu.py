@@ -1,4 +1,4 @@
-"""The float32 product in tiles of 128, 64 and 32 columns: sizes at which each is chosen, with rows and
+"""The float32 product in tiles of 128, 64 and 32 columns: sizes at which each is launched, with rows and
 columns that end inside a tile, against the product in 64 bits."""
 
 import pytest
@@ -9,11 +9,13 @@ from halite_amd.kernels import library, ops
 pytestmark = pytest.mark.gpu
 
 
-# tiles of 32 in one, three and five rounds, of 64 in one and three, and of 128
-@pytest.mark.parametrize("m, n, k, columns", [(130, 4000, 36, 32), (300, 4100, 1028, 64), (500, 4090, 544, 64), (260, 28004, 64, 128),
-                                              (700, 4033, 96, 32), (1030, 4161, 512, 32), (1500, 4090, 1028, 64)])
+# tiles of 32 in one, three and five rounds, of 64 in one, two and three, and of 128 in full rounds: a last tile of one row more
+# than half of its waves take, of so few that half of them have none, and of nearly all
+@pytest.mark.parametrize("m, n, k, columns", [(130, 4000, 36, 32), (300, 4100, 1028, 64), (500, 4090, 544, 64), (260, 28004, 64, 64),
+                                              (700, 4033, 96, 32), (1030, 4161, 512, 32), (1500, 4090, 1028, 64),
+                                              (449, 16384, 132, 128), (400, 16378, 1060, 128), (1000, 8190, 100, 128), (2000, 4090, 516, 128)])
 def test_tiles(m, n, k, columns):
-    assert library.core_library().hal_gemm_f32_tile_columns(m, n) == columns
+    assert library.core_library().hal_gemm_f32_columns(m, n) == columns
     gen = torch.Generator().manual_seed(m)
     a, w = torch.randn(m, k, generator=gen).cuda(), torch.randn(n, k, generator=gen).cuda()
     got = ops.gemm_f32(a, w).double()
