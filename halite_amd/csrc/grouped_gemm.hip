@@ -16,7 +16,7 @@
 // from memory (grouped_skinny_kernel), and tiles of 128 x 128 staged through registers and LDS
 // (grouped_mfma_kernel).  Where moreover whole lines can go straight into LDS (K of whole 64s) and
 // results leave as vector stores: streaming tiles of 64 x 128 for experts of few rows and for heads
-// (grouped_stream_kernel), and tiles of up to 256 x 256 for prompts' experts (grouped_wide_kernel).
+// (grouped_stream_kernel), and tiles of up to 352 x 256 for prompts' experts (grouped_wide_kernel).
 // gg_experts_kernel says which of the four takes an expert's product, and why.
 #include "hal_lds.h"
 #include "hal_api.h"
