@@ -720,7 +720,10 @@ def gemm_bf16_skinny(
     return out
 
 
-STREAM_ROWS = 64  # what the streaming product takes; from SKINNY_ROWS + 1 on
+# What the streaming product takes; from SKINNY_ROWS + 1 on, where the small-batch product's epilogues begin to cost more than they
+# spare.  (Bare products were measured below that, too, 16 rows small-batch / streaming, us: 128256 x 4096 230 / 180, 16384 x 3072 25.0 /
+# 19.0, 6144 x 4096 16.2 / 12.5 in 5 parts, gate and up of 14336 x 4096 48.6 / 46.6: the line is drawn for layers, not for those.)
+STREAM_ROWS = 64
 
 
 @functools.lru_cache(maxsize=None)
