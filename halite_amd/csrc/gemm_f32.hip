@@ -8,7 +8,8 @@
 // the workgroup's four waves), and the partial sums of the lanes, and of the waves that share
 // columns, are added in a fixed order.  17 to about 100 rows: the matrix cores, k split over a
 // workgroup's waves, each staging whole rows through LDS of its own.  More rows: tiles of 128 rows and 128, 96, 64
-// or 32 columns on the matrix cores, straight into LDS.  For sizes and addresses that are no multiples of
+// or 32 columns on the matrix cores, straight into LDS (of K of 2,048 and more, and more rows than 64, gemm_f32_split.hip takes
+// them, in half to two thirds of the time).  For sizes and addresses that are no multiples of
 // four: tiles of 64 x 64 on the vector units, each output element one chain of K
 // multiply-adds in index order.
 // In all of them a token's result depends on its own row alone, not on what else is in the
@@ -563,7 +564,8 @@ extern "C" int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, fl
     // rows, this and the tiles below, us: 4,096 x 4,096 50 / 69 / 93 against 102 / 101 / 101, x 14,336 147 / 225 / 297
     // against 345 / 347 / 347; 16,384 x 3,072 76 / 101 / 143 against 71 / 104 / 107, 28,672 x 4,096 185 / 250 / 373 against
     // 151 / 251 / 265, 128,256 x 4,096 747 / 1,003 / 1,476 against 645 / 995 / 1,111.  So not 33 to 64 rows of wide matrices
-    // either: half of a tile's waves have no rows then and leave the matrix cores to the others.
+    // either: half of a tile's waves have no rows then and leave the matrix cores to the others.  (Of K of 2,048 and more
+    // only up to 64 rows come here: hal_gemm_f32_split_takes.)
     const bool wide = (N + 127) / 128 >= 128;
     if (M <= (wide ? 32 : 128) || (M > 64 && M <= 96)) {
       if (M <= 32 ? launch_rows<1>(A, lda, W, ldw, C, ldc, M, N, K, stream)

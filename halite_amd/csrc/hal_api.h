@@ -75,6 +75,12 @@ int hal_attention_simple_ruled(const void* q, int q_row_stride, void* out, int o
 int hal_gemm_f32(const float* A, int lda, const float* W, int ldw, float* C, int ldc, int M,
                  int N, int K, hipStream_t stream);
 int hal_gemm_f32_columns(int M, int N);
+// the same for prompts, by parts of bf16 whose sums are float32's (whether it is taken: hal_gemm_f32_split_takes); planes: room
+// for as many float32 numbers as hal_gemm_f32_split_planes says, or null where that is 0
+int hal_gemm_f32_split_takes(const float* A, int lda, const float* W, int ldw, int M, int K);
+long long hal_gemm_f32_split_planes(int M, int N);
+int hal_gemm_f32_split(const float* A, int lda, const float* W, int ldw, float* C, int ldc, float* planes, int M, int N, int K,
+                       hipStream_t stream);
 
 // X [M <= 64, K] bf16, W [N, K] bf16, optional W2 [N, K] (gated: up * act(gate), W the gate's;
 // act, limit, alpha, up_shift as for hal_gate_mul).

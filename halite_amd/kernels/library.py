@@ -41,6 +41,7 @@ CORE_SOURCES = [
     "elementwise.hip",
     "attention_simple.hip",
     "gemm_f32.hip",
+    "gemm_f32_split.hip",
     "gemm_bf16.hip",
     "gemm_stream.hip",
     "sampling.hip",

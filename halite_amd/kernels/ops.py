@@ -542,7 +542,8 @@ def attention_simple(
 
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor):
-    """``a @ w.T`` in true float32 (``a`` [M, K], ``w`` [N, K])."""
+    """``a @ w.T`` in float32 (``a`` [M, K], ``w`` [N, K]): float32 multiply-adds, or, for prompts, exact products
+    of three bf16 parts a number with float32 sums, whose error is no larger (``gemm_f32_split.hip``)."""
     lib = library.core_library()
     _dev(a, w)
     _need(a.dtype == torch.float32 and w.dtype == torch.float32, "gemm_f32 takes float32")
@@ -550,6 +551,12 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor):
     n, k2 = w.shape
     _need(k == k2, f"gemm_f32: inner sizes {k} and {k2}")
     out = torch.empty((m, n), dtype=torch.float32, device=a.device)
+    if n > 0 and lib.hal_gemm_f32_split_takes(_ptr(a), k, _ptr(w), k, m, k):
+        lib.hal_gemm_f32_split_planes.restype = ctypes.c_longlong
+        words = lib.hal_gemm_f32_split_planes(m, n)
+        planes = torch.empty(words, dtype=torch.float32, device=a.device) if words else None
+        _check(lib, lib.hal_gemm_f32_split(_ptr(a), k, _ptr(w), k, _ptr(out), n, _ptr(planes), m, n, k, _stream()))
+        return out
     _check(lib, lib.hal_gemm_f32(_ptr(a), k, _ptr(w), k, _ptr(out), n, m, n, k, _stream()))
     return out
 

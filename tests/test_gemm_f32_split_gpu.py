@@ -1,0 +1,55 @@
+"""Float32 products of prompts by parts of bf16: edges of tiles, parts of K, rows in turns, and numbers that have no parts."""
+
+import pytest
+import torch
+
+from halite_amd.kernels import library, ops
+
+pytestmark = pytest.mark.gpu
+
+
+def _operands(m, n, k):
+    gen = torch.Generator().manual_seed(m + n + k)
+    return torch.randn(m, k, generator=gen).cuda(), (torch.randn(n, k, generator=gen) * 0.02).cuda()
+
+
+# the fewest rows, a tile of each height and one row more; one part of K to eight, of unequal lengths, an odd number of stages in
+# a part, K that ends inside a stage; columns that end inside a tile and inside a vector; rows in two turns over their planes
+@pytest.mark.parametrize("m, n, k", [(65, 96, 2048), (128, 130, 2052), (96, 12300, 2056), (129, 4090, 2080), (257, 6147, 2116), (300, 8200, 2048),
+                                     (513, 16388, 2084), (1100, 3072, 2048), (1025, 4097, 4100), (200, 1000, 14336)])
+def test_sizes(m, n, k):
+    a, w = _operands(m, n, k)
+    lib = library.core_library()
+    assert lib.hal_gemm_f32_split_takes(ops._ptr(a), k, ops._ptr(w), k, m, k)
+    w[n // 2] = w[n // 2].abs()  # (sums without cancellation: of a stretch left out, doubled or rounded to one side)
+    a[m // 2] = a[m // 2].abs()
+    got = ops.gemm_f32(a, w)
+    want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
+    # a float32 addition a stage of 32; in a stage six sums that are cut off and the products left out: at most 2 and 1 / 2 each
+    assert bool(((got.double() - want).abs() <= (k // 32 + 16) * 2.0**-24 * size).all())
+    # a row's result is its own, whatever tile it is in and whatever rows are beside it
+    assert torch.equal(ops.gemm_f32(a[: m - 1].contiguous(), w) if m > 65 else got[:-1], got[: m - 1])
+    if m > 200:
+        assert torch.equal(ops.gemm_f32(a[m - 70 :].contiguous(), w), got[m - 70 :])
+
+
+@pytest.mark.parametrize("m, n, k", [(130, 300, 2052), (300, 8200, 2048)])
+def test_numbers_without_parts(m, n, k):
+    a, w = _operands(m, n, k)
+    inf, nan, most = float("inf"), float("nan"), 3.4e38  # (the last: a float32 number that rounds to a bf16 infinity)
+    w[:, 40] = 1e-30
+    a[3, 5], a[4, 7], a[4, 2047], a[100, 9], a[128, 40], a[129, 0] = inf, inf, -inf, nan, most, most
+    w[17, 11], w[n - 1, 2], w[18, 700] = -inf, nan, inf
+    a[7, 700] = 0.0
+    got = ops.gemm_f32(a, w)
+    want = a.double() @ w.double().T
+    want = torch.where(want.abs() > 3.4028235e38, want.sign() * inf, want)
+    assert torch.equal(got.isnan(), want.isnan())
+    finite = want.isfinite()
+    assert torch.equal(got[~finite & ~want.isnan()].double(), want[~finite & ~want.isnan()])
+    plain = a.nan_to_num(0, 0, 0).double().abs() @ w.nan_to_num(0, 0, 0).double().abs().T
+    assert bool(((got.double() - want).abs() <= (k // 32 + 16) * 2.0**-24 * plain)[finite].all())
+    # columns of W that begin off a vector go to the other tiles
+    off = torch.empty(n * k + 1, device="cuda")[1:].view(n, k).copy_(w)
+    assert not library.core_library().hal_gemm_f32_split_takes(ops._ptr(a), k, ops._ptr(off), k, m, k)
+    assert torch.equal(ops.gemm_f32(a, off).isnan(), got.isnan())
