@@ -1,4 +1,4 @@
-// C[M, N] = X[M, K] W[N, K]^T for 17 to 64 rows of bf16 X (decode steps of many requests): what counts is that W
+// C[M, N] = X[M, K] W[N, K]^T for up to 64 rows of bf16 X (decode steps of many requests; from how many on, the callers' rules say): what counts is that W
 // comes at the memory's rate.  Both operands go in whole 128-byte lines straight into LDS, two to five steps of 64 k on
 // their way while one is multiplied (v_mfma_f32_16x16x32_bf16, float32 sums).  A workgroup of four waves takes all rows
 // and 64 or 128 rows of W (of a gated product half of them the gate's and half the up projection's, act(gate) * up in the
@@ -184,7 +184,7 @@ extern "C" int hal_gemm_bf16_stream_parts(int N, int K, int gated, int may_part)
   return gs_cut(N, K, gated != 0, may_part != 0).parts;
 }
 
-// X [M, K], W (and W2 of a gated product: W is the gate's) [N, K] bf16, 17 to 64 rows.  parts: what
+// X [M, K], W (and W2 of a gated product: W is the gate's) [N, K] bf16, up to 64 rows.  parts: what
 // hal_gemm_bf16_stream_parts returned; 1: Y [M, N] of bf16 or float32, more: float32 planes [parts][M][N] whose sum is the result.
 extern "C" int hal_gemm_bf16_stream(const void* X, int ldx, const void* W, const void* W2, int ldw, void* Y, int y_dtype,
                                     int parts, int act, float limit, float alpha, float up_shift, int M, int N, int K,

@@ -146,7 +146,7 @@ int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const floa
                       void* state, void* hist, uint32_t* lists, int any_late, int* out_token,
                       float* out_logprob, hipStream_t stream);
 
-// ---- products of 17 to 64 rows, W streamed through LDS (gemm_stream.hip) ----------------------
+// ---- products of up to 64 rows, W streamed through LDS (gemm_stream.hip) ----------------------
 // C = X W^T (with W2: act(X W^T) * (X W2^T)) for bf16 operands.  hal_gemm_bf16_stream_parts: 0 where the product is not
 // taken, else in how many parts of K (more than 1 only with may_part).  One part: Y [M, N] bf16 or float32; more:
 // float32 planes [parts][M][N] whose sum, in order, is the result.

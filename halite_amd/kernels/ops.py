@@ -728,9 +728,14 @@ def gemm_bf16_skinny(
 
 
 # What the streaming product takes; from SKINNY_ROWS + 1 on, where the small-batch product's epilogues begin to cost more than they
-# spare.  (Bare products were measured below that, too, 16 rows small-batch / streaming, us: 128256 x 4096 230 / 180, 16384 x 3072 25.0 /
-# 19.0, 6144 x 4096 16.2 / 12.5 in 5 parts, gate and up of 14336 x 4096 48.6 / 46.6: the line is drawn for layers, not for those.)
+# spare.  A bare product that fills the chip without parts (a model's head) goes to it earlier: the small-batch kernel reads a row of
+# X for every 16 rows of W, streaming tiles for every 128.  Small-batch / streaming, us, at 8, 12 and 16 rows: 128256 x 4096 182 / 180,
+# 207 / 182, 230 / 184; 128256 x 3072 143 / 136, 169 / 139, 191 / 140; 32000 x 4096 47.7 / 45.9, 52.9 / 46.5, 58.3 / 46.4; of a shorter K
+# 32000 x 2048 27.7 / 30.9, 31.2 / 31.1, 34.0 / 31.3, 50256 x 2048 41.5 / 44.3, 46.7 / 44.6, 50.2 / 43.2; at 4 rows 170 / 178, 130 / 135.
+# (With a part of K a workgroup, 6144 x 4096 16.2 / 12.5 at 16 rows, but then the reader has planes to add up.)
 STREAM_ROWS = 64
+BARE_SKINNY_ROWS = 8  # up to here the small-batch kernel is the faster one
+BARE_SHORT_K, BARE_SHORT_ROWS = 3072, 12  # of rows below this length up to so many
 
 
 @functools.lru_cache(maxsize=None)
@@ -738,11 +743,11 @@ def _stream_parts(n: int, k: int, gated: bool, may_part: bool) -> int:
     return library.core_library().hal_gemm_bf16_stream_parts(n, k, 1 if gated else 0, 1 if may_part else 0)
 
 
-def stream_parts(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, may_part: bool = False) -> int:
-    """In how many parts of K the streaming product takes ``x`` [17 to 64, k] against the bf16 weight ``w`` of ``n``
-    rows (``gated``: two of them); 0: another is the faster one, or it has none for these sizes or places."""
+def stream_parts(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, may_part: bool = False, above: int = SKINNY_ROWS) -> int:
+    """In how many parts of K the streaming product takes ``x`` [17 to 64, k] (or from ``above`` + 1 rows on) against the bf16 weight
+    ``w`` of ``n`` rows (``gated``: two of them); 0: another is the faster one, or it has none for these sizes or places."""
     m, k = x.shape
-    if not (SKINNY_ROWS < m <= STREAM_ROWS and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.is_cuda
+    if not (above < m <= STREAM_ROWS and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.is_cuda
             and x.stride(1) == 1 and x.stride(0) % 8 == 0 and x.stride(0) >= k and x.data_ptr() % 16 == 0 and w.stride(1) == 1
             and w.stride(0) % 8 == 0 and w.stride(0) >= k and w.data_ptr() % 16 == 0 and n * w.stride(0) * 2 < 2**31
             and m * x.stride(0) * 2 < 2**31):  # (the kernel's offsets)
@@ -752,7 +757,7 @@ def stream_parts(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, 
 
 def gemm_bf16_stream(x: torch.Tensor, w: torch.Tensor, parts: int, w_up: torch.Tensor | None = None,
                      out_dtype: torch.dtype = torch.bfloat16, activation: str = "silu", clamp: Clamp = Clamp()):
-    """``x @ w.T`` for 17 to 64 rows in the ``parts`` that ``stream_parts`` named: one gives the result, more give
+    """``x @ w.T`` for up to 64 rows in the ``parts`` that ``stream_parts`` named: one gives the result, more give
     ``PartialSums``; with ``w_up`` (one part) the gated form ``(x @ w_up.T) * act(x @ w.T)``."""
     lib = library.core_library()
     _need(x.is_cuda and w.is_cuda and (w_up is None or w_up.is_cuda), "kernel arguments must be on the GPU")
@@ -859,7 +864,7 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
 
     float32 weights: the true 32-bit kernel (activations are widened if needed).
     bf16 weights: the hand-written kernels where they are the faster ones (``skinny_pays``:
-    up to 16 rows; ``stream_parts``: 17 to 64); otherwise the library product that the reference itself uses for
+    up to 16 rows; ``stream_parts``: 17 to 64, and from 9 on where nothing is folded in); otherwise the library product that the reference itself uses for
     its linear layers (src/halite/transformers/infer/attention.py:21-24), except where
     float32 output is asked for and the library cannot give it, which the hand-written
     kernel does in passes of 64 rows.
@@ -885,6 +890,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
     m, k = x.shape
     skinny_ok = k % 8 == 0 and w.stride(0) % 8 == 0 and w.data_ptr() % 16 == 0
     if m <= SKINNY_ROWS and tiled is not None and k % 8 == 0:
+        if stream_parts(x, w, w.shape[0], above=BARE_SKINNY_ROWS if k >= BARE_SHORT_K else BARE_SHORT_ROWS) == 1:
+            return gemm_bf16_stream(x, w, 1, out_dtype=out_dtype)
         return gemm_bf16_skinny(x, tiled, out_dtype=out_dtype, tiled_shape=tuple(w.shape))
     if skinny_ok and skinny_pays(m, w.shape[0], k, False):
         return gemm_bf16_skinny(x, w, out_dtype=out_dtype)

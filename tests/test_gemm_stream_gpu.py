@@ -62,6 +62,21 @@ def test_gated(gpu, m, f, k, activation):
     assert float((y.double() - want).abs().max()) <= (2.0**-8 + 1e-5) * float(want.abs().max())
 
 
+@pytest.mark.parametrize("n,k,rows", [(10304, 3072, 8), (16380, 2048, 12), (12801, 3072, 16), (4096, 3072, 16)])
+def test_bare_products_of_few_rows(gpu, n, k, rows):
+    """A product that folds nothing in leaves the small-batch kernel above ``rows`` rows, where one part fills the chip and columns are
+    whole vectors."""
+    w = rand(gpu, n, k, seed=14, scale=0.05).bfloat16()
+    tiled = ops.tile_weight(w)
+    for m in (1, rows, min(rows + 1, 16), 16):
+        x = rand(gpu, m, k, seed=m).bfloat16()
+        got = ops.linear(x, w, out_dtype=torch.float32, tiled=tiled)
+        close(got, x.double() @ w.double().t(), k)
+        same = ops.gemm_bf16_stream(x, w, 1, out_dtype=torch.float32) if m > rows else ops.gemm_bf16_skinny(x, tiled, out_dtype=torch.float32, tiled_shape=(n, k))
+        assert torch.equal(got, same)
+        assert torch.equal(ops.linear(x, w, tiled=tiled), got.bfloat16())
+
+
 def test_what_it_does_not_take(gpu):
     w = torch.zeros((4096, 4096), dtype=torch.bfloat16, device=gpu)
     x = lambda m, k=4096: torch.zeros((m, k), dtype=torch.bfloat16, device=gpu)  # noqa: E731
