@@ -146,6 +146,12 @@ int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const floa
                       void* state, void* hist, uint32_t* lists, int any_late, int* out_token,
                       float* out_logprob, hipStream_t stream);
 
+// a step's rows: their parameters into one buffer, and sampled by it (sampling.hip)
+int hal_sample_pack(const double* temperature, const double* top_p, const double* min_p, const long long* top_k, const long long* seeds,
+                    const long long* draws, int n, int V, int* words);
+int hal_sample_packed(const float* logits, int ld, int n, int V, const int* packed, int flags, int* room, int at_once, int* out,
+                      hipStream_t stream);
+
 // ---- products of up to 64 rows, W streamed through LDS (gemm_stream.hip) ----------------------
 // C = X W^T (with W2: act(X W^T) * (X W2^T)) for bf16 operands.  hal_gemm_bf16_stream_parts: 0 where the product is not
 // taken, else in how many parts of K (more than 1 only with may_part).  One part: Y [M, N] bf16 or float32; more:

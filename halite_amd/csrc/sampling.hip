@@ -11,6 +11,7 @@
 #include "hal_common.h"
 #include "hal_api.h"
 #include <mutex>
+#include <string.h>
 
 #define SAMPLE_THREADS 1024
 #define SAMPLE_BINS 2048  // two per thread
@@ -1215,5 +1216,56 @@ extern "C" int hal_sample_spread(const float* logits, int ld, int n_rows, int V,
   hipLaunchKernelGGL(filt_pick_kernel, dim3(n_rows), dim3(PICK_THREADS), 0, stream, logits, ld, V, params, rows, parts,
                      kept, seeds, draw_index, out_token, out_logprob);
   HAL_LAUNCH_CHECK();
+  return 0;
+}
+
+// ---- a step's rows as the host has them -------------------------------------------------
+// A row's parameters as they lie in one buffer of 7 n words, so that one copy brings a step's: seeds (64 bits), temperature, top_p,
+// min_p (float32), top_k, draw index.  Returns what holds for all rows, which decides how they are sampled.  (As two dozen numpy
+// calls on 64 rows this was 25 of the 50 us that the host had to do before a step's first launch.)
+enum { SAMPLE_ALL_GREEDY = 1, SAMPLE_UNFILTERED = 2, SAMPLE_LATE = 4 };
+extern "C" int hal_sample_pack(const double* temperature, const double* top_p, const double* min_p, const long long* top_k,
+                               const long long* seeds, const long long* draws, int n, int V, int* words) {
+  bool all_greedy = true, unfiltered = true, late = false;
+  float* f = (float*)(words + 2 * (size_t)n);
+  int* w = words + 5 * (size_t)n;
+  for (int r = 0; r < n; ++r) {
+    const bool greedy = temperature[r] == 0 || top_k[r] == 1;
+    const bool by_k = top_k[r] > 0 && top_k[r] < V, by_p = top_p[r] < 1.0, by_min = min_p[r] > 0.0;
+    all_greedy &= greedy;
+    unfiltered &= greedy || !(by_k || by_p || by_min);
+    // (top-k, top-p and min-p all at once: top-p then refers to what top-k kept, two searches one after the other)
+    late |= !greedy && by_k && by_p && by_min;
+    memcpy(words + 2 * (size_t)r, &seeds[r], 8);
+    f[r] = greedy ? 0.f : (float)temperature[r], f[n + r] = (float)top_p[r], f[2 * (size_t)n + r] = (float)min_p[r];
+    w[r] = greedy ? 1 : (int)(top_k[r] < 0x7fffffffll ? top_k[r] : 0x7fffffffll), w[n + r] = (int)draws[r];
+  }
+  return (all_greedy ? SAMPLE_ALL_GREEDY : 0) | (unfiltered ? SAMPLE_UNFILTERED : 0) | (late ? SAMPLE_LATE : 0);
+}
+
+// Samples n rows by such a buffer on the GPU.  `flags`: what hal_sample_pack returned.  `room`: for rows with filters, which go `at_once` at a time
+// over it, at_once * (1,190 + V) words that begin at a multiple of 8 bytes (64-bit histograms and the rows' state first), else n * 128.
+// `out`: n tokens, then n log-probabilities.
+extern "C" int hal_sample_packed(const float* logits, int ld, int n, int V, const int* packed, int flags, int* room, int at_once, int* out,
+                                 hipStream_t stream) {
+  HAL_REQUIRE(n >= 0 && V > 0 && ld >= V && at_once > 0, "hal_sample_packed: bad sizes rows=%d V=%d ld=%d, %d at once", n, V, ld, at_once);
+  if (n == 0) return 0;
+  HAL_REQUIRE(logits && packed && room && out && (uintptr_t)packed % 8 == 0 && (uintptr_t)room % 8 == 0, "hal_sample_packed: arguments missing");
+  const uint64_t* seeds = (const uint64_t*)packed;
+  const float *temperature = (const float*)(packed + 2 * (size_t)n), *top_p = temperature + n, *min_p = top_p + n;
+  const int *top_k = packed + 5 * (size_t)n, *draws = top_k + n;
+  float* logprobs = (float*)(out + n);
+  if (flags & SAMPLE_ALL_GREEDY) return hal_sample_greedy(logits, ld, n, V, (float*)room, out, logprobs, stream);
+  if (flags & SAMPLE_UNFILTERED) return hal_sample_unfiltered(logits, ld, n, V, temperature, top_k, seeds, draws, (float*)room, out, logprobs, stream);
+  int* hist = room;
+  int* state = hist + (size_t)at_once * 4 * FILT_BINS;
+  float* parts = (float*)(state + (size_t)at_once * 6);
+  float* kept = parts + (size_t)at_once * ROW_PARTS * 4;
+  uint32_t* lists = (uint32_t*)(kept + (size_t)at_once * ROW_PARTS);
+  for (int r = 0; r < n; r += at_once) {
+    if (hal_sample_spread(logits + (size_t)r * ld, ld, n - r < at_once ? n - r : at_once, V, temperature + r, top_k + r, top_p + r, min_p + r, seeds + r,
+                          draws + r, parts, kept, state, hist, lists, flags & SAMPLE_LATE ? 1 : 0, out + r, logprobs + r, stream))
+      return 1;
+  }
   return 0;
 }

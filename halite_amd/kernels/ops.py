@@ -637,6 +637,38 @@ def sample(
     return tokens, logprobs
 
 
+SAMPLE_ALL_GREEDY, SAMPLE_UNFILTERED = 1, 2  # (and 4: some row has top-k, top-p and min-p all at once)
+
+
+def pack_sample_rows(host: torch.Tensor, temperature, top_p, min_p, top_k, seeds, draw_index, vocab: int) -> int:
+    """The parameters of a step's rows (``array``s of doubles and of 64-bit integers) into the int32 buffer ``host`` of seven
+    words a row; returns what ``sample_packed`` takes as ``flags``."""
+    _need(host.dtype == torch.int32 and not host.is_cuda and host.is_contiguous() and host.numel() >= 7 * len(seeds), "sample: room for the rows")
+    at = [ctypes.c_void_p(a.buffer_info()[0]) for a in (temperature, top_p, min_p, top_k, seeds, draw_index)]
+    return library.core_library().hal_sample_pack(*at, len(seeds), vocab, _ptr(host))
+
+
+def sample_packed(logits: torch.Tensor, packed: torch.Tensor, flags: int):
+    """Next token and log-probability of every row of float32 ``logits`` by ``packed``, the buffer of ``pack_sample_rows`` on the
+    GPU, and its ``flags``: greedy rows and draws from whole distributions in two launches, others in six or eight."""
+    lib = library.core_library()
+    _dev(logits, packed)
+    n, vocab = logits.shape
+    _need(logits.dtype == torch.float32, "sample: logits are float32")
+    _need(packed.dtype == torch.int32 and packed.numel() == 7 * n, "sample: parameters of every row")
+    if flags & (SAMPLE_ALL_GREEDY | SAMPLE_UNFILTERED):
+        at_once, words = n, n * 128
+    else:
+        # a row's list has room for all of its logits (they may all be alike), so many rows go in turns over one room
+        at_once = min(n, max(1, SAMPLE_LIST_WORDS // vocab))
+        words = at_once * (2 * 256 * 2 + 6 + 32 * 4 + 32 + vocab)
+    room = torch.empty(words, dtype=torch.int32, device=logits.device)
+    # one buffer for both results, so that the host can fetch them with one copy
+    both = torch.empty(2 * n, dtype=torch.int32, device=logits.device)
+    _check(lib, lib.hal_sample_packed(_ptr(logits), vocab, n, vocab, _ptr(packed), flags, _ptr(room), at_once, _ptr(both), _stream()))
+    return both[:n], both[n:].view(torch.float32)
+
+
 SKINNY_MAX_ROWS = 64  # what the kernel takes
 SKINNY_ROWS = 16  # up to here it beats the library product
 FUSED_ROWS = 32  # what the epilogues that take other kernels' work take

@@ -4,6 +4,7 @@
 from __future__ import annotations
 
 import zlib
+from array import array
 
 import numpy as np
 import torch
@@ -21,6 +22,15 @@ def request_seed(params: SamplingParams, request_id, engine_seed: int = 0) -> in
     if params.seed is not None:
         return int(params.seed) & _MASK63
     return (zlib.crc32(repr(request_id).encode()) * 2654435761 + engine_seed * 40503) & _MASK63
+
+
+def _integers(values, most: int | None = None) -> array:
+    """Whole numbers as 64-bit integers (``most``: larger ones as that)."""
+    try:
+        return array("q", values)
+    except (TypeError, OverflowError):  # other number types, or numbers beyond 64 bits
+        numbers = np.asarray(values)
+        return array("q", (numbers if most is None else np.minimum(numbers, most)).astype(np.int64).tolist())
 
 
 class Sampler:
@@ -58,33 +68,14 @@ class Sampler:
         if n == 0:
             e = torch.empty(0, device=self.device)
             return e.to(torch.int32), e.to(torch.float32)
-        # all per-row parameters in one buffer, one copy: seeds (int64), then three float32
-        # rows and two int32 rows
+        # all per-row parameters in one buffer, one copy; a list a parameter, and the rest in one native call
         host = self._stage(7 * n)
-        words = host.numpy()
-        words[: 2 * n].view(np.int64)[:] = seeds
-        f = words[2 * n : 5 * n].view(np.float32).reshape(3, n)
-        i = words[5 * n : 7 * n].reshape(2, n)
-        # a list a parameter, and the rest on whole rows: a busy server's step has as many rows as requests
-        temperature, top_k = np.array([p.temperature for p in params], np.float64), np.array([p.top_k for p in params])
-        top_p, min_p = np.array([p.top_p for p in params], np.float64), np.array([p.min_p for p in params], np.float64)
-        greedy = (temperature == 0) | (top_k == 1)  # (``SamplingParams.greedy``)
-        f[0], f[1], f[2] = np.where(greedy, 0.0, temperature), top_p, min_p
-        i[0], i[1] = np.where(greedy, 1, np.minimum(top_k, 2**31 - 1)), draw_index
-        vocab = logits.shape[1]
-        by_k, by_p, by_min = (top_k > 0) & (top_k < vocab), top_p < 1.0, min_p > 0.0
-        unfiltered = not np.any(~greedy & (by_k | by_p | by_min))
-        # top-k, top-p and min-p all at once in one row: top-p then refers to what top-k kept,
-        # two searches one after the other
-        late = bool(np.any(~greedy & by_k & by_p & by_min))
+        flags = ops.pack_sample_rows(
+            host, array("d", [p.temperature for p in params]), array("d", [p.top_p for p in params]), array("d", [p.min_p for p in params]),
+            _integers([p.top_k for p in params], 2**31 - 1), _integers(seeds), _integers(draw_index), logits.shape[1])
         dev = torch.empty(7 * n, dtype=torch.int32, device=self.device)
         dev.copy_(host[: 7 * n], non_blocking=True)
-        if self.device.type == "cuda":
-            event = torch.cuda.Event()
-            event.record()
-            self._staging[self._turn] = (self._staging[self._turn][0], event)
-        fd = dev[2 * n : 5 * n].view(torch.float32).view(3, n)
-        idv = dev[5 * n : 7 * n].view(2, n)
-        sd = dev[: 2 * n].view(torch.int64)
-        return ops.sample(logits.contiguous(), fd[0], idv[0], fd[1], fd[2], sd, idv[1],
-                          all_greedy=bool(greedy.all()), unfiltered=unfiltered, spread=True, late=late)
+        event = torch.cuda.Event()
+        event.record()
+        self._staging[self._turn] = (host, event)
+        return ops.sample_packed(logits.contiguous(), dev, flags)
