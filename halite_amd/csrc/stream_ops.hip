@@ -1039,6 +1039,24 @@ __global__ void head_gate_cols_kernel(const T* __restrict__ x, int ldx, int x_he
   }
 }
 
+// The same without a rotation, four entries a thread, for sizes and addresses that allow it (a thread an entry asks for 128 bytes a
+// wave at a time: 2,250 rows of 32 heads of 128 took 20.9 us so, and take 8.3).
+template <typename T>
+__global__ void __launch_bounds__(256)
+head_gate_cols_vec_kernel(const T* __restrict__ x, int ldx, int x_head, const float* __restrict__ g, int ldg, T* __restrict__ y, int n, int H) {
+  const size_t t = blockIdx.x;
+  const int vectors = n / 4;
+  for (int e = blockIdx.y * 256 + threadIdx.x; e < H * vectors; e += gridDim.y * 256) {
+    const int h = e / vectors, j = e % vectors * 4;
+    const float gate = 1.0f / (1.0f + expf(-g[t * ldg + h]));
+    float f[4];
+    load4(x + t * ldx + (size_t)h * x_head + j, f);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) f[i] *= gate;
+    store4(y + t * H * n + (size_t)h * n + j, f);
+  }
+}
+
 // ---- q, k and v of float32 projections with their heads turned by the tokens' positions, packed
 // as [H heads of D | K heads of D | K heads of D] with zeros beyond a head's entries, keys and
 // values appended to the pages as well (k_pages null: not).  q and k: the pairs of their first `rot`
@@ -1138,6 +1156,14 @@ extern "C" int hal_head_gate_cols(const void* x, int ldx, int x_head, const floa
               "hal_head_gate_cols: bad sizes T=%d heads=%d n=%d of %d", n_tokens, H, n, x_head);
   HAL_REQUIRE(dtype == HAL_F32 || dtype == HAL_BF16, "hal_head_gate_cols: dtype %d", dtype);
   if (n_tokens == 0) return 0;
+  const int elt = dtype == HAL_F32 ? 16 : 8;  // bytes of four entries
+  if (!cos_t && n % 4 == 0 && x_head % 4 == 0 && ldx % 4 == 0 && (uintptr_t)x % elt == 0 && (uintptr_t)y % elt == 0) {
+    const dim3 rows(n_tokens, n_tokens <= 64 ? (H * n / 4 + 255) / 256 : 1);
+    if (dtype == HAL_F32) hipLaunchKernelGGL(head_gate_cols_vec_kernel<float>, rows, dim3(256), 0, stream, (const float*)x, ldx, x_head, g, ldg, (float*)y, n, H);
+    else hipLaunchKernelGGL(head_gate_cols_vec_kernel<bf16_t>, rows, dim3(256), 0, stream, (const bf16_t*)x, ldx, x_head, g, ldg, (bf16_t*)y, n, H);
+    HAL_LAUNCH_CHECK();
+    return 0;
+  }
   // (few tokens: several workgroups a row)
   const dim3 grid(n_tokens, n_tokens <= 64 ? (H * n + 511) / 512 : 1);
   if (dtype == HAL_F32)
