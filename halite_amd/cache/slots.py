@@ -13,6 +13,7 @@ from __future__ import annotations
 
 import torch
 
+from ..kernels import ops
 from ..parts.base import StateNeed
 
 
@@ -60,9 +61,12 @@ class StateStore:
             }
 
     def reset(self, slot: int) -> None:
-        for named in self.tensors.values():
-            for t in named.values():
-                t[slot].zero_()
+        rows = [t for named in self.tensors.values() for t in named.values()]
+        if rows and all(t.is_cuda for t in rows):
+            ops.zero_rows(rows, slot)
+            return
+        for t in rows:
+            t[slot].zero_()
 
     def bytes(self) -> int:
         return sum(t.numel() * t.element_size() for n in self.tensors.values() for t in n.values())

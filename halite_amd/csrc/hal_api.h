@@ -146,6 +146,9 @@ int hal_sample_spread(const float* logits, int ld, int n_rows, int V, const floa
                       void* state, void* hist, uint32_t* lists, int any_late, int* out_token,
                       float* out_logprob, hipStream_t stream);
 
+// zeros into n rows of so many 32-bit words each (elementwise.hip)
+int hal_zero_rows(void* const* rows, const unsigned long long* words, int n, hipStream_t stream);
+
 // a step's rows: their parameters into one buffer, and sampled by it (sampling.hip)
 int hal_sample_pack(const double* temperature, const double* top_p, const double* min_p, const long long* top_k, const long long* seeds,
                     const long long* draws, int n, int V, int* words);

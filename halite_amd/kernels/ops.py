@@ -561,6 +561,24 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor):
     return out
 
 
+def zero_rows(tensors: list[torch.Tensor], row: int) -> None:
+    """Row ``row`` of every one of ``tensors`` (contiguous, on one GPU) becomes zeros, in one launch; rows that are not whole
+    32-bit words one by one."""
+    lib = library.core_library()
+    whole = []
+    for t in tensors:
+        _dev(t)
+        _need(0 <= row < t.shape[0], f"zero_rows: row {row} of {t.shape[0]}")
+        size = t.numel() // t.shape[0] * t.element_size()
+        if size % 4 or (t.data_ptr() + row * size) % 4:
+            t[row].zero_()
+        elif size:
+            whole.append((t.data_ptr() + row * size, size // 4))
+    if whole:
+        at, words = zip(*whole)
+        _check(lib, lib.hal_zero_rows((ctypes.c_void_p * len(at))(*at), (ctypes.c_ulonglong * len(at))(*words), len(at), _stream()))
+
+
 # Room for the lists of the sampler's rows with filters: 256 MiB, 523 rows of 128,256.  So many rows keep the chip busy, and
 # more go in turns (1,024 rows 517 us at once, 515 in two turns; with room for 130 rows 765).
 SAMPLE_LIST_WORDS = 64 * 1024 * 1024

@@ -1,4 +1,5 @@
-"""Element-wise passes of prompts in vectors and runs: the convolution in runs of eight tokens, heads' gates four columns a thread."""
+"""Element-wise passes of prompts in vectors and runs: the convolution in runs of eight tokens, heads' gates four columns a thread, rows
+of zeros in several arrays."""
 
 import pytest
 import torch
@@ -56,3 +57,13 @@ def test_heads_gates(dtype, rows, heads, n, apart):
     got = ops.head_gate_cols(x, apart, g, n, heads)
     want = (x.view(rows, heads, apart)[:, :, :n].double() * torch.sigmoid(g.double())[:, :, None]).reshape(rows, heads * n)
     assert got.shape == want.shape and bool(((got.double() - want).abs() <= (2.0**-8 if dtype == torch.bfloat16 else 4e-7) * want.abs() + 1e-30).all())
+
+
+def test_rows_of_zeros():
+    shapes = [((5, 64, 64, 64), torch.float32), ((5, 3, 7), torch.float32), ((5, 3), torch.bfloat16), ((5, 6), torch.bfloat16), ((5, 0, 4), torch.float32)]
+    tensors = [torch.ones(shape, dtype=dtype, device="cuda") for shape, dtype in shapes * 20]  # (more than one launch takes)
+    ops.zero_rows(tensors, 3)
+    for t in tensors:
+        assert bool((t[3] == 0).all()) and bool((t[:3] == 1).all()) and bool((t[4:] == 1).all())
+    with pytest.raises(ops.KernelError):
+        ops.zero_rows(tensors, 5)
