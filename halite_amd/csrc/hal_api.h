@@ -220,12 +220,16 @@ int hal_latent_prep(const float* a, int lda, int q_col0, int q_rank, int kv_col0
 int hal_head_cols(const void* x, int ldx, int xs, int x0, void* y, int ldy, int ys, int y0, int n,
                   int z0, int n_zero, int H, int dtype, int n_tokens, hipStream_t stream);
 int hal_scale_f32(float* x, long long n, float s, hipStream_t stream);
-// Router of a mixture of experts on float32 logits z [T, E]: scores by sigmoid (softmax over
+// A router's logits: X [M, K] times W [N, K]^T of bf16 in parts of K, float32 planes Z [parts][M][N] (how many parts, 0 where
+// the product is not taken: hal_narrow_product_parts).
+int hal_narrow_product_parts(const void* X, int ldx, const void* W, int ldw, int M, int N, int K);
+int hal_narrow_product(const void* X, int ldx, const void* W, int ldw, float* Z, int parts, int M, int N, int K, hipStream_t stream);
+// Router of a mixture of experts on float32 logits z [T, E], or the sum of so many planes of them, `plane` numbers apart: scores by sigmoid (softmax over
 // the experts if `softmax`), the `top` largest (lower index on a tie) to idx [T, top], their
 // scores (divided by their sum + norm_eps if `normalize`), times scale, to wgt [T, top].  correction
 // (or null) [E]: added to the scores for the choice alone.  groups > 0: only experts of the `keep`
 // groups of neighbours with the largest sums of their two largest (corrected) scores are chosen from.
-int hal_moe_route(const float* z, int ldz, int E, int top, int softmax, int normalize, float norm_eps,
+int hal_moe_route(const float* z, int ldz, int planes, long long plane, int E, int top, int softmax, int normalize, float norm_eps,
                   float scale, const void* correction, int c_dtype, int groups, int keep, int* idx, float* wgt,
                   int n_tokens, hipStream_t stream);
 // Counting sort of the n (token, choice) pairs by expert (idx [n]); offsets, tile_offsets
@@ -238,7 +242,7 @@ int hal_moe_combine(float* h, const float* y, const float* wgt, const float* ext
                     const float* extra_gate, int ld_gate, int top, int d, int n_tokens, int overwrite,
                     hipStream_t stream);
 // hal_moe_route and hal_moe_sort in one workgroup (for steps of few tokens; at most 256 experts)
-int hal_moe_route_sort(const float* z, int ldz, int E, int top, int softmax, int normalize, float norm_eps,
+int hal_moe_route_sort(const float* z, int ldz, int planes, long long plane, int E, int top, int softmax, int normalize, float norm_eps,
                        float scale, const void* correction, int c_dtype, int groups, int keep, int* idx, float* wgt, int n_tokens, int tile, int* offsets, int* tile_offsets,
                        int* sorted, hipStream_t stream);
 

@@ -8,6 +8,7 @@
 //     the query latent and of the key/value latent, and the key and value rows that the
 //     paged attention kernels take;
 //   * column ranges copied head by head;
+//   * the product of a router's few columns, in parts of K;
 //   * the router of a mixture of experts: scores, the chosen `top` (also by corrected scores and
 //     among the best groups of neighbours), their weights;
 //   * a counting sort of the (token, choice) pairs by expert, on the device;
@@ -420,16 +421,123 @@ __device__ __forceinline__ void moe_close_groups(float (&s)[W], int E, int group
   }
 }
 
+// ---------------------------------------------------------------------------------
+// Z[p] = X W^T over the p-th part of K, for a bf16 W [N, K] of few rows (a router's): float32 planes [parts][M][N], which
+// whoever reads the logits adds up in order.
+//
+// What bounds it: a matrix of 64 columns is four tiles of an instruction, so that a whole product of few rows has four workgroups, each
+// of which waits for its K numbers a row alone.  In parts of K, four waves a part whose sums meet in LDS, one tile of columns a
+// workgroup: 8 rows, 64 x 4,096: 7.7 -> 2.9 us (the small-batch product before); 48 rows, 16 x 4,096: 6.0 -> 4.3 (the library).
+// Both operands come straight from memory in the instruction's order, four steps of 32 k at a time.
+// ---------------------------------------------------------------------------------
+typedef __attribute__((ext_vector_type(8))) __bf16 nw_bf16x8;
+typedef __attribute__((ext_vector_type(4))) float nw_f32x4;
+#define NW_WAVES 4
+template <int MT>  // tiles of 16 rows
+__global__ void __launch_bounds__(NW_WAVES * HAL_WAVE)
+narrow_product_kernel(const bf16_t* __restrict__ X, int ldx, const bf16_t* __restrict__ W, int ldw, float* __restrict__ Z, int M, int N, int K) {
+  constexpr int U = 4;  // steps of 32 k at a time
+  __shared__ __attribute__((aligned(16))) float sums[NW_WAVES][MT][256];
+  const int lane = threadIdx.x % HAL_WAVE, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / HAL_WAVE);
+  const int n0 = blockIdx.x * 16, part = blockIdx.y, parts = gridDim.y;
+  const int r = lane % 16, q = lane / 16, all = K / 32, shares = parts * NW_WAVES, mine = part * NW_WAVES + wave;
+  const int begin = (int)((long long)all * mine / shares), end = (int)((long long)all * (mine + 1) / shares);
+  // (rows and columns past the end are read from the last one: nothing of them is stored)
+  const bf16_t* x[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) x[i] = X + (size_t)min(i * 16 + r, M - 1) * ldx + q * 8;
+  const bf16_t* w = W + (size_t)min(n0 + r, N - 1) * ldw + q * 8;
+  nw_f32x4 acc[MT];
+#pragma unroll
+  for (int i = 0; i < MT; ++i) acc[i] = nw_f32x4{0.f, 0.f, 0.f, 0.f};
+  for (int s = begin; s < end; s += U) {
+    nw_bf16x8 a[U][MT], b[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = min(s + u, end - 1) * 32;  // (past the share's end the last step's numbers come again and are not multiplied)
+#pragma unroll
+      for (int i = 0; i < MT; ++i) a[u][i] = *(const nw_bf16x8*)(x[i] + k);
+      b[u] = *(const nw_bf16x8*)(w + k);
+    }
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      if (s + u >= end) break;
+#pragma unroll
+      for (int i = 0; i < MT; ++i) acc[i] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(b[u], a[u][i], acc[i], 0, 0, 0);
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < MT; ++i) *(nw_f32x4*)&sums[wave][i][lane * 4] = acc[i];
+  __syncthreads();
+  // lane l of a tile's result holds row l % 16 and columns 4 (l / 16) .. + 3; wave v adds up tile v
+  if (wave >= MT) return;
+  nw_f32x4 sum = *(const nw_f32x4*)&sums[0][wave][lane * 4];
+#pragma unroll
+  for (int v = 1; v < NW_WAVES; ++v) sum += *(const nw_f32x4*)&sums[v][wave][lane * 4];
+  const int m = wave * 16 + r, n = n0 + q * 4;
+  if (m >= M) return;
+  float* to = Z + ((size_t)part * M + m) * N + n;
+  if (N % 4 == 0 && n < N) {
+    *(nw_f32x4*)to = sum;
+  } else {
+#pragma unroll
+    for (int e = 0; e < 4; ++e)
+      if (n + e < N) to[e] = sum[e];
+  }
+}
+
+// Into how many parts K is cut; 0: the product is not taken.  Up to 64 rows (8 rows, 64 x 4,096: 7.7 us as one product, 2.9 in
+// parts; 64 rows: 6.2 and 4.5); at 65 rows and more the tiles of 64 columns that read X once take 10.6 us against the library's 6.2,
+// and no number of rows up to 8,192 turned that.  Past 256 columns (256 x 2,048, 64 rows: 5.3 and 3.6, of which the reader
+// of eight planes gives 1.1 back) the whole product has workgroups enough.
+#define NW_MAX_ROWS 64
+#define NW_MAX_COLS 256
+extern "C" int hal_narrow_product_parts(const void* X, int ldx, const void* W, int ldw, int M, int N, int K) {
+  if (M <= 0 || M > NW_MAX_ROWS || N <= 0 || N > NW_MAX_COLS || K % 32 || K < 512) return 0;
+  if (ldx % 8 || ldw % 8 || (uintptr_t)X % 16 || (uintptr_t)W % 16) return 0;
+  return K >= 2048 ? 8 : K / 256;  // (at least two steps of 32 k a wave)
+}
+
+extern "C" int hal_narrow_product(const void* X, int ldx, const void* W, int ldw, float* Z, int parts, int M, int N, int K, hipStream_t stream) {
+  HAL_REQUIRE(parts > 0 && parts == hal_narrow_product_parts(X, ldx, W, ldw, M, N, K), "hal_narrow_product: M=%d N=%d K=%d in %d parts", M, N, K, parts);
+  HAL_REQUIRE(ldx >= K && ldw >= K && (uintptr_t)Z % 16 == 0, "hal_narrow_product: rows of %d and %d, or the planes' place", ldx, ldw);
+  const dim3 grid((N + 15) / 16, parts), block(NW_WAVES * HAL_WAVE);
+#define NW_LAUNCH(MT_) \
+  hipLaunchKernelGGL((narrow_product_kernel<MT_>), grid, block, 0, stream, (const bf16_t*)X, ldx, (const bf16_t*)W, ldw, Z, M, N, K)
+  if (M <= 16) NW_LAUNCH(1);
+  else if (M <= 32) NW_LAUNCH(2);
+  else NW_LAUNCH(4);
+#undef NW_LAUNCH
+  HAL_LAUNCH_CHECK();
+  return 0;
+}
+
+// a router's logits: rows of `ld`, in planes that are added up
+#define MOE_MAX_PLANES 8
+struct MoeLogits {
+  const float* at;
+  int ld, planes;
+  long long plane;
+};
 template <int W>
-__device__ __forceinline__ void moe_route_token(const float* __restrict__ z, int ldz, int E, int top, const MoeChoice& how,
+__device__ __forceinline__ void moe_route_token(const MoeLogits& z, int E, int top, const MoeChoice& how,
                                                 int* __restrict__ idx, float* __restrict__ wgt, int t, int lane) {
-  const float* zr = z + (size_t)t * ldz;
+  const float* zr = z.at + (size_t)t * z.ld;
   float s[W], w[W];  // what the choice is made by, and the scores as weights
   float zmax = -INFINITY;
 #pragma unroll
   for (int u = 0; u < W; ++u) {
     const int e = lane + u * HAL_WAVE;
-    s[u] = e < E ? zr[e] : -INFINITY;
+    s[u] = -INFINITY;
+    if (e < E) {
+      float part[MOE_MAX_PLANES];  // (all asked for before they are added up)
+#pragma unroll
+      for (int p = 0; p < MOE_MAX_PLANES; ++p) part[p] = p < z.planes ? zr[(size_t)p * z.plane + e] : 0.f;
+      s[u] = part[0];
+#pragma unroll
+      for (int p = 1; p < MOE_MAX_PLANES; ++p)
+        if (p < z.planes) s[u] += part[p];
+    }
     zmax = fmaxf(zmax, s[u]);
   }
   if (how.softmax) {
@@ -503,9 +611,9 @@ __device__ __forceinline__ void moe_route_token(const float* __restrict__ z, int
 }
 
 template <int W>
-__global__ void __launch_bounds__(HAL_WAVE) moe_route_kernel(const float* __restrict__ z, int ldz, int E, int top, MoeChoice how,
+__global__ void __launch_bounds__(HAL_WAVE) moe_route_kernel(MoeLogits z, int E, int top, MoeChoice how,
                                                              int* __restrict__ idx, float* __restrict__ wgt, int n_tokens) {
-  moe_route_token<W>(z, ldz, E, top, how, idx, wgt, blockIdx.x, threadIdx.x);
+  moe_route_token<W>(z, E, top, how, idx, wgt, blockIdx.x, threadIdx.x);
 }
 
 static int moe_check_choice(const MoeChoice& how, int E, int top) {
@@ -524,16 +632,18 @@ static int moe_check_choice(const MoeChoice& how, int E, int top) {
     else if (MOST_ > 4) LAUNCH_(MOST_);            \
   } while (0)
 
-extern "C" int hal_moe_route(const float* z, int ldz, int E, int top, int softmax, int normalize, float norm_eps,
+extern "C" int hal_moe_route(const float* z, int ldz, int planes, long long plane, int E, int top, int softmax, int normalize, float norm_eps,
                              float scale, const void* correction, int c_dtype, int groups, int keep, int* idx,
                              float* wgt, int n_tokens, hipStream_t stream) {
   const MoeChoice how = {softmax, normalize, norm_eps, scale, correction, c_dtype, groups, keep};
+  HAL_REQUIRE(planes >= 1 && planes <= MOE_MAX_PLANES, "router: logits in %d planes", planes);
+  const MoeLogits logits = {z, ldz, planes, plane};
   HAL_REQUIRE(n_tokens >= 0 && E > 0 && E <= MOE_MAX_EXPERTS && top > 0 && top <= E && ldz >= E,
               "hal_moe_route: bad sizes T=%d E=%d top=%d", n_tokens, E, top);
   if (int rc = moe_check_choice(how, E, top)) return rc;
   if (n_tokens == 0) return 0;
 #define MOE_ROUTE(W_) \
-  hipLaunchKernelGGL(moe_route_kernel<W_>, dim3(n_tokens), dim3(HAL_WAVE), 0, stream, z, ldz, E, top, how, idx, wgt, n_tokens)
+  hipLaunchKernelGGL(moe_route_kernel<W_>, dim3(n_tokens), dim3(HAL_WAVE), 0, stream, logits, E, top, how, idx, wgt, n_tokens)
   MOE_BY_WORDS(MOE_ROUTE, 16);
 #undef MOE_ROUTE
   HAL_LAUNCH_CHECK();
@@ -600,8 +710,7 @@ __global__ void __launch_bounds__(1024) moe_sort_kernel(const int* __restrict__ 
 // Both in one workgroup, for steps of few tokens and up to 256 experts: its waves take the tokens in
 // turn, then all of it sorts the pairs.
 template <int W>
-__global__ void __launch_bounds__(1024) moe_route_sort_kernel(const float* __restrict__ z, int ldz, int E, int top,
-                                                              MoeChoice how, int* __restrict__ idx,
+__global__ void __launch_bounds__(1024) moe_route_sort_kernel(MoeLogits z, int E, int top, MoeChoice how, int* __restrict__ idx,
                                                               float* __restrict__ wgt, int n_tokens, int tile,
                                                               int* __restrict__ offsets, int* __restrict__ tile_offsets,
                                                               int* __restrict__ sorted) {
@@ -609,23 +718,25 @@ __global__ void __launch_bounds__(1024) moe_route_sort_kernel(const float* __res
   __shared__ int cursor[MOE_MAX_EXPERTS];
   const int wave = threadIdx.x / HAL_WAVE, lane = threadIdx.x % HAL_WAVE;
   for (int t = wave; t < n_tokens; t += blockDim.x / HAL_WAVE)
-    moe_route_token<W>(z, ldz, E, top, how, idx, wgt, t, lane);
+    moe_route_token<W>(z, E, top, how, idx, wgt, t, lane);
   __threadfence_block();
   __syncthreads();
   moe_sort_pairs(idx, n_tokens * top, E, tile, offsets, tile_offsets, sorted, count, cursor);
 }
 
-extern "C" int hal_moe_route_sort(const float* z, int ldz, int E, int top, int softmax, int normalize, float norm_eps,
+extern "C" int hal_moe_route_sort(const float* z, int ldz, int planes, long long plane, int E, int top, int softmax, int normalize, float norm_eps,
                                   float scale, const void* correction, int c_dtype, int groups, int keep,
                                   int* idx, float* wgt, int n_tokens, int tile, int* offsets, int* tile_offsets,
                                   int* sorted, hipStream_t stream) {
   const MoeChoice how = {softmax, normalize, norm_eps, scale, correction, c_dtype, groups, keep};
+  HAL_REQUIRE(planes >= 1 && planes <= MOE_MAX_PLANES, "router: logits in %d planes", planes);
+  const MoeLogits logits = {z, ldz, planes, plane};
   HAL_REQUIRE(n_tokens >= 0 && E > 0 && E <= 4 * HAL_WAVE && top > 0 && top <= E && ldz >= E && tile > 0,
               "hal_moe_route_sort: bad sizes T=%d E=%d top=%d", n_tokens, E, top);
   if (int rc = moe_check_choice(how, E, top)) return rc;
   int waves = n_tokens < 4 ? 4 : (n_tokens < 16 ? n_tokens : 16);
 #define MOE_ROUTE_SORT(W_)                                                                                                    \
-  hipLaunchKernelGGL(moe_route_sort_kernel<W_>, dim3(1), dim3(waves * HAL_WAVE), 0, stream, z, ldz, E, top, how, idx, wgt,    \
+  hipLaunchKernelGGL(moe_route_sort_kernel<W_>, dim3(1), dim3(waves * HAL_WAVE), 0, stream, logits, E, top, how, idx, wgt,    \
                      n_tokens, tile, offsets, tile_offsets, sorted)
   MOE_BY_WORDS(MOE_ROUTE_SORT, 4);
 #undef MOE_ROUTE_SORT

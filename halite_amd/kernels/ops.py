@@ -1129,17 +1129,43 @@ class RouterChoice:
                 _ptr(c), F32 if c is None else dtype_code(c.dtype), self.groups, self.keep)
 
 
-def moe_route(z: torch.Tensor, top: int, **how):
-    """The ``top`` experts of every token from float32 router logits ``z`` ``[T, E]``: indices
+def router_logits(x: torch.Tensor, w: torch.Tensor):
+    """``x @ w.T`` in float32 for a router's weight ``w`` of few rows: ``PartialSums``, which ``moe_route`` and ``moe_route_sort``
+    take, or a tensor where another product is taken."""
+    if x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.is_cuda and x.stride(1) == 1 and w.stride(1) == 1:
+        lib = library.core_library()
+        (m, k), n = x.shape, w.shape[0]
+        _need(w.shape[1] == k, f"router: inner sizes {k} and {w.shape[1]}")
+        parts = lib.hal_narrow_product_parts(_ptr(x), x.stride(0), _ptr(w), w.stride(0), m, n, k) if min(x.stride(0), w.stride(0)) >= k else 0
+        if parts:
+            planes = torch.empty((parts, m, n), dtype=torch.float32, device=x.device)
+            _check(lib, lib.hal_narrow_product(_ptr(x), x.stride(0), _ptr(w), w.stride(0), _ptr(planes), parts, m, n, k, _stream()))
+            return PartialSums(planes)
+    return linear(x, w, out_dtype=torch.float32)
+
+
+def _router_planes(z, what: str):
+    """Address, row length, number and distance of the planes of a router's logits."""
+    rows = z.planes[0] if isinstance(z, PartialSums) else z
+    _need(rows.is_cuda and rows.dtype == torch.float32 and rows.dim() == 2 and rows.stride(1) == 1,
+          f"{what}: float32 logits [T, E] (a row-strided view is allowed)")
+    if isinstance(z, PartialSums):
+        _dev(z.planes)
+        return _ptr(rows), rows.stride(0), z.planes.shape[0], ctypes.c_longlong(rows.numel())
+    return _ptr(rows), rows.stride(0), 1, ctypes.c_longlong(0)
+
+
+def moe_route(z, top: int, **how):
+    """The ``top`` experts of every token from float32 router logits ``z`` ``[T, E]`` (or ``PartialSums``): indices
     ``[T, top]`` int32 and weights ``[T, top]`` float32 (``how``: the fields of ``RouterChoice``)."""
     lib = library.core_library()
     choice = RouterChoice(**how)
-    _need(z.is_cuda and z.dtype == torch.float32 and z.dim() == 2 and z.stride(1) == 1,
-          "moe_route: float32 logits [T, E] (a row-strided view is allowed)")
+    logits = _router_planes(z, "moe_route")
     t, e = z.shape
-    idx = torch.empty((t, top), dtype=torch.int32, device=z.device)
-    wgt = torch.empty((t, top), dtype=torch.float32, device=z.device)
-    _check(lib, lib.hal_moe_route(_ptr(z), z.stride(0), e, top, *choice.args(e), _ptr(idx), _ptr(wgt), t, _stream()))
+    device = (z.planes if isinstance(z, PartialSums) else z).device
+    idx = torch.empty((t, top), dtype=torch.int32, device=device)
+    wgt = torch.empty((t, top), dtype=torch.float32, device=device)
+    _check(lib, lib.hal_moe_route(*logits, e, top, *choice.args(e), _ptr(idx), _ptr(wgt), t, _stream()))
     return idx, wgt
 
 
@@ -1147,19 +1173,20 @@ ROUTE_SORT_MAX_TOKENS = 16  # up to so many tokens (one a wave) one workgroup ro
 ROUTE_SORT_MAX_EXPERTS = 256  # of at most so many experts
 
 
-def moe_route_sort(z: torch.Tensor, top: int, n_experts: int, **how):
+def moe_route_sort(z, top: int, n_experts: int, **how):
     """``moe_route`` and ``moe_sort`` in one launch: ``(idx, wgt, offsets, tile_offsets, sorted)``."""
     lib = library.core_library()
     choice = RouterChoice(**how)
-    _need(z.is_cuda and z.dtype == torch.float32 and z.dim() == 2 and z.stride(1) == 1 and z.shape[1] == n_experts,
-          "moe_route_sort: float32 logits [T, E] (a row-strided view is allowed)")
+    _need(z.shape[1] == n_experts, "moe_route_sort: logits of every expert")
+    logits = _router_planes(z, "moe_route_sort")
     t = z.shape[0]
-    idx = torch.empty((t, top), dtype=torch.int32, device=z.device)
-    wgt = torch.empty((t, top), dtype=torch.float32, device=z.device)
-    offsets = torch.empty(n_experts + 1, dtype=torch.int32, device=z.device)
-    tile_offsets = torch.empty(n_experts + 1, dtype=torch.int32, device=z.device)
-    order = torch.empty(max(t * top, 1), dtype=torch.int32, device=z.device)
-    _check(lib, lib.hal_moe_route_sort(_ptr(z), z.stride(0), n_experts, top, *choice.args(n_experts), _ptr(idx), _ptr(wgt), t, GROUP_TILE_ROWS, _ptr(offsets),
+    device = (z.planes if isinstance(z, PartialSums) else z).device
+    idx = torch.empty((t, top), dtype=torch.int32, device=device)
+    wgt = torch.empty((t, top), dtype=torch.float32, device=device)
+    offsets = torch.empty(n_experts + 1, dtype=torch.int32, device=device)
+    tile_offsets = torch.empty(n_experts + 1, dtype=torch.int32, device=device)
+    order = torch.empty(max(t * top, 1), dtype=torch.int32, device=device)
+    _check(lib, lib.hal_moe_route_sort(*logits, n_experts, top, *choice.args(n_experts), _ptr(idx), _ptr(wgt), t, GROUP_TILE_ROWS, _ptr(offsets),
                                        _ptr(tile_offsets), _ptr(order), _stream()))
     return idx, wgt, offsets, tile_offsets, order
 

@@ -179,9 +179,12 @@ class MixtureOfExperts(FeedForward):
         """The result as the rows that its reader adds up."""
         p = self.p
         n, d = x.shape
-        z = ops.linear(x, self.w_router, out_dtype=torch.float32)
-        shared_gate = z[:, p.n_experts:] if p.shared_gate else None
-        z = z[:, : p.n_experts]
+        shared_gate = None
+        if p.shared_gate:  # (whose reader takes whole numbers)
+            z = ops.linear(x, self.w_router, out_dtype=torch.float32)
+            z, shared_gate = z[:, : p.n_experts], z[:, p.n_experts :]
+        else:
+            z = ops.router_logits(x, self.w_router)
         routing = dict(softmax=p.score == "softmax", normalize=p.normalize, norm_eps=p.norm_eps, scale=p.weight_scale,
                        correction=self.w_correction, groups=p.groups.count if p.groups else 0,
                        keep=p.groups.keep if p.groups else 0)
