@@ -425,6 +425,26 @@ static int skinny_waves(int blocks, int steps) {
   return waves;
 }
 
+// Tiles of 16 rows of W (sets of them) that a workgroup of up to 16 rows of X takes: one or two.  At 16 rows X is as many bytes
+// as a tile, and every workgroup reads all of it, so that what a CU's busiest round brings in counts beside the weights' way
+// from memory: with two tiles a workgroup half as many rounds, each with X once.  One tile / two, us, at 16 rows with the norm folded in:
+// plain 257 tiles of K 4,096 15.6 / 13.3, 320 x 3,072 14.3 / 11.5, 384 x 4,096 16.6 / 14.5, 512 x 4,096 17.8 / 16.4, 1,024 x 4,096 32.4 / 28.7,
+// but (without the norm) 256 x 4,096 9.8 / 12.9, 516 21.3 / 21.9, 640 x 5,120 30.1 / 29.7, 768 24.6 / 25.1; gated 257 x 4,096 22.0 / 20.0,
+// 344 x 2,048 13.8 / 12.6, 896 x 4,096 48.2 / 46.1, 896 x 5,120 62.6 / 56.0, but 512 x 3,072 22.5 / 22.5 and 21.7 / 22.9 between a
+// model's other kernels, 256 x 4,096 14.4 / 18.5, 688 37.0 / 42.2.  With fewer rows X weighs less: 9 rows 320 tiles 12.1 / 11.6, 384
+// 14.5 / 14.2; 12 rows 384 15.6 / 15.0, but 512 without the norm 14.9 / 15.5; 8 rows 384 13.2 / 13.1.  (Measured on tiled weights, which
+// is what a model's small batches read.)
+static int skinny_tiles(int M, int tiles, int sets, int ldw) {
+  if (ldw != 0 || M <= 8 || M > 16) return 1;
+  if (tiles <= 512) return tiles > 256 && (tiles <= 448 || (sets == 1 && M > 12)) ? 2 : 1;
+  return M > 12 && (tiles + 511) / 512 * (2 * sets + 1) < (tiles + 255) / 256 * (sets + 1) ? 2 : 1;
+}
+// (two tiles: at most 8 waves; 320 x 3,072 10.6 us with 16 and 10.4 with 8, gated 344 x 2,048 12.9 and 12.1)
+static int skinny_waves_of_two(int tiles, int steps) {
+  const int waves = skinny_waves((tiles + 1) / 2, steps);
+  return waves > 8 ? 8 : waves;
+}
+
 // X [M, K] bf16 (M <= 64), W [N, K] bf16, optional W2 [N, K] (gated form: W is the
 // gate's weight, W2 is up's; act: HAL_ACT_*).  out_mode: 0 bf16, 1 float32, 2 add into
 // float32, 3 the square of relu of the result, as bf16.
@@ -450,7 +470,7 @@ extern "C" int hal_gemm_bf16_skinny(const void* X, int ldx, const void* W, const
   // Rows of W per wave (16 * nt): more of them mean that a fragment of X, which every
   // block reads again, serves more of W.  The waves of a block split K, more of them
   // when there are few blocks.  Tunable through the environment for measurements.
-  int nt = mt >= 3 ? 2 : mt;
+  int nt = mt >= 2 ? 2 : skinny_tiles(M, (N + 15) / 16, sets, ldw);
   int u = 0, waves = 0;
   if (const char* e = getenv("HAL_SKINNY_NT")) nt = atoi(e);
   if (const char* e = getenv("HAL_SKINNY_U")) u = atoi(e);
@@ -460,7 +480,7 @@ extern "C" int hal_gemm_bf16_skinny(const void* X, int ldx, const void* W, const
   const int blocks = (N + 16 * nt - 1) / (16 * nt);
   const int steps = (K + 31) / 32;
   if (waves <= 0) {
-    waves = skinny_waves(blocks, steps);
+    waves = mt == 1 && nt == 2 ? skinny_waves_of_two((N + 15) / 16, steps) : skinny_waves(blocks, steps);
   }
   while (waves > 1 && (size_t)sets * nt * mt * 1024 > 64 * 1024) waves /= 2;  // one tile must fit
   // loads in flight per wave: about 16 fragments of 16 bytes
@@ -532,6 +552,14 @@ extern "C" int hal_gemm_bf16_skinny_norm(const void* X, int ldx, const void* W, 
 #define SK_NORM_LAUNCH(MT_, GATED_, U_, FLAGS_, W2_, MODE_)                                        \
   return launch_skinny<1, MT_, GATED_, U_, FLAGS_>(x, ldx, w, W2_, ldw, C, ldc, MODE_, M, N, K,    \
                                                    waves, stream, RopeEpilogue{}, nf)
+  if (!norm_w && skinny_tiles(M, blocks, w2 ? 2 : 1, ldw) == 2) {
+    const int fewer = skinny_waves_of_two(blocks, steps);
+    if (w2)
+      return launch_skinny<2, 1, true, 2, SK_SCALED>(x, ldx, w, w2, ldw, C, ldc, SK_OUT_BF16, M, N, K, fewer, stream,
+                                                     RopeEpilogue{}, nf);
+    return launch_skinny<2, 1, false, 4, SK_SCALED>(x, ldx, w, nullptr, ldw, C, ldc, SK_OUT_BF16, M, N, K, fewer, stream,
+                                                    RopeEpilogue{}, nf);
+  }
   if (M <= 16) {
     if (w2) SK_NORM_LAUNCH(1, true, 4, SK_SCALED, w2, SK_OUT_BF16);
     if (norm_w) SK_NORM_LAUNCH(1, false, 8, SK_PREP, nullptr, SK_OUT_F32_ADD);
@@ -587,6 +615,14 @@ extern "C" int hal_qkv_rope_append(const void* X, int ldx, const void* W, void* 
   return launch_skinny<1, MT_, false, U_, FLAGS_>((const bf16_t*)X, ldx, (const bf16_t*)W, nullptr, \
                                                   0, q_out, H * D, SK_OUT_BF16, M, N, K_in, waves,  \
                                                   stream, rope, nf)
+  if (skinny_tiles(M, blocks, 1, 0) == 2) {
+    const int fewer = skinny_waves_of_two(blocks, steps);
+    if (ss_in)
+      return launch_skinny<2, 1, false, 4, SK_ROPE | SK_SCALED>((const bf16_t*)X, ldx, (const bf16_t*)W, nullptr, 0, q_out, H * D,
+                                                                SK_OUT_BF16, M, N, K_in, fewer, stream, rope, nf);
+    return launch_skinny<2, 1, false, 4, SK_ROPE>((const bf16_t*)X, ldx, (const bf16_t*)W, nullptr, 0, q_out, H * D, SK_OUT_BF16, M,
+                                                  N, K_in, fewer, stream, rope, nf);
+  }
   if (M <= 16) {
     if (ss_in) SK_ROPE_LAUNCH(1, 8, SK_ROPE | SK_SCALED);
     SK_ROPE_LAUNCH(1, 8, SK_ROPE);
