@@ -376,8 +376,11 @@ int hal_head_norm_gate(const float* y, const float* z, int ldz, int silu, const 
 // read: u = sum_s in[s] x_s (in null: ones) of the new copies, written to result as it is
 // (norm_w null, float32) or as u / sqrt(mean(u^2) + eps) * (offset + norm_w).  rows (or null;
 // only without y): the rows to take, results in that order, ld_result elements from one to the next.
-int hal_streams_step(float* x, long long copy_stride, int S, const float* y, const void* mix,
-                     const void* outw, float m, const void* inw, int c_dtype, int read,
+// (terms > 0, in rows of a multiple of four elements up to 8,192 and up to four copies: y[t] is the sum of so many rows, y + t * y_token +
+// j * y_term, each times wgt[t, j] if there are weights, then with extra[t] (times sigmoid(extra_gate[t])) beside them)
+int hal_streams_step(float* x, long long copy_stride, int S, const float* y, int terms, long long y_token,
+                     long long y_term, const float* wgt, const float* extra, const float* extra_gate, int ld_gate,
+                     const void* mix, const void* outw, float m, const void* inw, int c_dtype, int read,
                      const void* norm_w, int norm_dtype, float offset, float eps, void* result,
                      int ld_result, int result_dtype, const int* rows, int n_rows, int W,
                      hipStream_t stream);

@@ -481,9 +481,22 @@ __global__ void streams_step_kernel(float* __restrict__ x, size_t copy_stride, i
 // Four copies of 4,096: 48 rows 14.4 -> 6.1, 1,024 39.7 -> 35.4.  Eight copies of one group a thread leave registers for a
 // single row a compute unit: 48 rows of 4,096 took 25.0 -> 12.0 us so, but 900 rows 60.7 -> 65.1, and of 1,028 24.2 ->
 // 32.4, and a row's bits are not to depend on the number of rows.  More than four copies stay above.
-template <typename TO, int MAXS, int V>
+//
+// SUMMED: y is made here, of `terms` rows a token: a product's planes, added up in order, or the results of the experts that the
+// token uses, weighted (and a row beside them): what hal_sum_planes or hal_moe_combine would write first and this pass read back.
+// Bound by memory, so what is saved is that row's way out and back and the launch: two copies of 4,096, four experts a token, apart / here:
+// 48 rows 6.4 / 4.6 us, 900 27.2 / 20.3, 3,600 116.8 / 78.1; four planes instead of one row 48 rows 4.0 -> 4.5.
+struct SummedRows {
+  long long token, term;  // from a token's first row to the next token's, and from a row to the next of the same token
+  int terms;
+  const float* wgt;    // [T, terms], or null: planes
+  const float* extra;  // [T, W], or null
+  const float* gate;   // [T] with rows of ld_gate, or null: sigmoid(gate) times the row beside
+  int ld_gate;
+};
+template <typename TO, int MAXS, int V, bool SUMMED>
 __global__ void __launch_bounds__(1024)
-streams_step_vec_kernel(float* __restrict__ x, size_t copy_stride, int S, const float* __restrict__ y,
+streams_step_vec_kernel(float* __restrict__ x, size_t copy_stride, int S, const float* __restrict__ y, SummedRows e,
                         const void* __restrict__ mix, const void* __restrict__ outw, float m,
                         const void* __restrict__ inw, int c_dtype, int read, const void* __restrict__ norm_w,
                         int norm_dtype, float offset, float eps, TO* __restrict__ result, int ld_result,
@@ -501,8 +514,38 @@ streams_step_vec_kernel(float* __restrict__ x, size_t copy_stride, int S, const 
         if (s < S) load4(x + s * copy_stride + t * W + v * 4, xs[u][s]);
         else xs[u][s][0] = xs[u][s][1] = xs[u][s][2] = xs[u][s][3] = 0.f;
       }
-      if (y) load4(y + t * W + v * 4, yv[u]);
+      if (!SUMMED && y) load4(y + t * W + v * 4, yv[u]);
       if (norm_w) load4_any(norm_w, norm_dtype, (size_t)v * 4, wn[u]);
+    }
+  }
+  if constexpr (SUMMED) {
+    const float eg = e.gate ? 1.0f / (1.0f + expf(-e.gate[t * e.ld_gate])) : 1.0f;
+#pragma unroll
+    for (int u = 0; u < V; ++u) {
+      const int v = threadIdx.x + u * threads;
+      if (v >= nv) continue;
+      const float* row = y + t * e.token + v * 4;
+      yv[u][0] = yv[u][1] = yv[u][2] = yv[u][3] = 0.f;
+      if (e.extra) {
+        load4(e.extra + t * W + v * 4, yv[u]);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) yv[u][i] *= eg;
+      }
+      for (int j0 = 0; j0 < e.terms; j0 += 4) {  // four rows on their way at a time
+        float part[4][4], c[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          const int at = j0 + j < e.terms ? j0 + j : j0;  // (past the end: a row that is there, not added)
+          load4(row + at * e.term, part[j]);
+          c[j] = e.wgt ? e.wgt[t * e.terms + at] : 1.0f;
+        }
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+          if (j0 + j >= e.terms) break;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) yv[u][i] = fmaf(c[j], part[j][i], yv[u][i]);
+        }
+      }
     }
   }
   float ci[MAXS];
@@ -579,11 +622,14 @@ streams_step_vec_kernel(float* __restrict__ x, size_t copy_stride, int S, const 
 #define STREAMS_VEC_MOST 8192     // the widest row of the vector kernel: 32 groups of 256
 #define STREAMS_VEC_COPIES 4      // and the most copies
 #define STREAMS_AT_ONCE (1 << 19)  // threads that the chip runs at once: 256 compute units of 2,048
-extern "C" int hal_streams_step(float* x, long long copy_stride, int S, const float* y, const void* mix,
-                                const void* outw, float m, const void* inw, int c_dtype, int read,
+extern "C" int hal_streams_step(float* x, long long copy_stride, int S, const float* y, int terms, long long y_token,
+                                long long y_term, const float* wgt, const float* extra, const float* extra_gate, int ld_gate,
+                                const void* mix, const void* outw, float m, const void* inw, int c_dtype, int read,
                                 const void* norm_w, int norm_dtype, float offset, float eps, void* result,
                                 int ld_result, int result_dtype, const int* rows, int n_rows, int W,
                                 hipStream_t stream) {
+  HAL_REQUIRE(terms >= 0 && (terms == 0 || (y && y_token % 4 == 0 && y_term % 4 == 0)), "hal_streams_step: %d rows to add up", terms);
+  const SummedRows e = {y_token, y_term, terms, wgt, wgt ? extra : nullptr, wgt ? extra_gate : nullptr, ld_gate};
   HAL_REQUIRE(!read || ld_result >= W, "hal_streams_step: rows of %d for a width of %d", ld_result, W);
   HAL_REQUIRE(S >= 1 && S <= 8, "hal_streams_step: %d copies of the stream (1 to 8)", S);
   HAL_REQUIRE(n_rows >= 0 && W > 0 && W <= 16384, "hal_streams_step: bad sizes rows=%d width=%d", n_rows, W);
@@ -594,14 +640,20 @@ extern "C" int hal_streams_step(float* x, long long copy_stride, int S, const fl
   if (n_rows == 0) return 0;
   const uintptr_t result_size = result_dtype == HAL_F32 ? 16 : 8, norm_size = norm_dtype == HAL_F32 ? 16 : 8;
   const long long nv = W / 4, groups = (long long)n_rows * nv;
-  if (W % 4 == 0 && W <= STREAMS_VEC_MOST && S <= STREAMS_VEC_COPIES && copy_stride % 4 == 0 && ((uintptr_t)x | (uintptr_t)y) % 16 == 0 &&
+  if (W % 4 == 0 && W <= STREAMS_VEC_MOST && S <= STREAMS_VEC_COPIES && copy_stride % 4 == 0 &&
+      ((uintptr_t)x | (uintptr_t)y | (uintptr_t)e.extra) % 16 == 0 &&
       (!read || (ld_result % 4 == 0 && (uintptr_t)result % result_size == 0 && (uintptr_t)norm_w % norm_size == 0))) {
     const int per = nv > 1024 || (S <= 2 && groups > STREAMS_AT_ONCE && groups <= 2 * STREAMS_AT_ONCE) ? 2 : 1;
     const int threads = (int)((nv + per - 1) / per + HAL_WAVE - 1) / HAL_WAVE * HAL_WAVE;
-#define STREAMS_LAUNCH(T_, M_, V_)                                                                                   \
-  hipLaunchKernelGGL((streams_step_vec_kernel<T_, M_, V_>), dim3(n_rows), dim3(threads), 0, stream, x,               \
-                     (size_t)copy_stride, S, y, mix, outw, m, inw, c_dtype, read, read ? norm_w : nullptr, norm_dtype, \
+#define STREAMS_LAUNCH_AS(T_, M_, V_, SUMMED_)                                                                       \
+  hipLaunchKernelGGL((streams_step_vec_kernel<T_, M_, V_, SUMMED_>), dim3(n_rows), dim3(threads), 0, stream, x,      \
+                     (size_t)copy_stride, S, y, e, mix, outw, m, inw, c_dtype, read, read ? norm_w : nullptr, norm_dtype, \
                      offset, eps, (T_*)result, ld_result, rows, W)
+#define STREAMS_LAUNCH(T_, M_, V_)                                \
+  do {                                                            \
+    if (terms) STREAMS_LAUNCH_AS(T_, M_, V_, true);               \
+    else STREAMS_LAUNCH_AS(T_, M_, V_, false);                    \
+  } while (0)
 #define STREAMS_BY_COUNT(T_)                                  \
   do {                                                        \
     if (S <= 2 && per == 1) STREAMS_LAUNCH(T_, 2, 1);         \
@@ -613,9 +665,11 @@ extern "C" int hal_streams_step(float* x, long long copy_stride, int S, const fl
     else STREAMS_BY_COUNT(bf16_t);
 #undef STREAMS_BY_COUNT
 #undef STREAMS_LAUNCH
+#undef STREAMS_LAUNCH_AS
     HAL_LAUNCH_CHECK();
     return 0;
   }
+  HAL_REQUIRE(terms == 0, "hal_streams_step: rows of these sizes or places are added up before");
   const size_t lds = (read && norm_w) ? (size_t)W * sizeof(float) : 0;
 #define STREAMS_LAUNCH(T_, M_)                                                                                      \
   hipLaunchKernelGGL((streams_step_kernel<T_, M_>), dim3(n_rows), dim3(256), lds, stream, x, (size_t)copy_stride, S, y, \

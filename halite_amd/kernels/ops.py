@@ -133,6 +133,11 @@ class PartialSums:
 
     def materialize(self, dtype: torch.dtype) -> torch.Tensor:
         lib = library.core_library()
+        if self.planes[0].numel() % 4:  # (the kernel takes four at a time)
+            total = self.planes[0].clone()
+            for plane in self.planes[1:]:
+                total += plane
+            return total.to(dtype)
         out = torch.empty(tuple(self.shape), dtype=dtype, device=self.planes.device)
         _check(lib, lib.hal_sum_planes(_ptr(self.planes), self.planes.shape[0], _ptr(out), dtype_code(dtype),
                                        ctypes.c_longlong(out.numel()), _stream()))
@@ -910,7 +915,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
     """``x @ w.T`` for a weight ``[out, in]``; ``tiled`` is ``tile_weight(w)`` if the
     model keeps that copy for small batches.  ``x`` may be ``NormedRows``; with
     ``next_norm`` the result may come back as ``NormedRows`` (already added into the
-    stream) instead of a tensor, with ``sums`` (or a norm that says so) as ``PartialSums``.
+    stream) instead of a tensor, with ``sums`` (or a norm that says so) as ``PartialSums``, whose reader
+    rounds their sum to ``out_dtype``.
 
     float32 weights: the true 32-bit kernel (activations are widened if needed).
     bf16 weights: the hand-written kernels where they are the faster ones (``skinny_pays``:
@@ -945,8 +951,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
         return gemm_bf16_skinny(x, tiled, out_dtype=out_dtype, tiled_shape=tuple(w.shape))
     if skinny_ok and skinny_pays(m, w.shape[0], k, False):
         return gemm_bf16_skinny(x, w, out_dtype=out_dtype)
-    # (who adds up the parts rounds their sum to bf16: a result that is wanted in float32 comes whole)
-    in_parts = out_dtype == torch.bfloat16 and (sums or (next_norm is not None and next_norm.sums))
+    # (a norm that adds up the parts rounds their sum to bf16: a result that is wanted in float32 comes to it whole)
+    in_parts = sums or (out_dtype == torch.bfloat16 and next_norm is not None and next_norm.sums)
     parts = stream_parts(x, w, w.shape[0], may_part=in_parts)
     if parts:
         return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)
@@ -1640,23 +1646,46 @@ def head_norm_gate(y: torch.Tensor, z: torch.Tensor | None, weight: torch.Tensor
     return out
 
 
-def streams_step(x: torch.Tensor, *, y: torch.Tensor | None = None, mix: torch.Tensor | None = None,
+STREAMS_STEP_MOST, STREAMS_STEP_COPIES = 8192, 4  # the widest row and the most copies for which ``streams_step`` adds up itself
+
+
+def streams_step(x: torch.Tensor, *, y: torch.Tensor | PartialSums | ExpertSum | None = None, mix: torch.Tensor | None = None,
                  out: torch.Tensor | None = None, mult: float = 1.0, read: bool = False,
                  inw: torch.Tensor | None = None, norm_weight: torch.Tensor | None = None, offset: float = 0.0,
                  eps: float = 0.0, dtype: torch.dtype = torch.float32, rows: torch.Tensor | None = None,
                  result: torch.Tensor | None = None):
     """One pass over the copies ``x`` (float32 ``[S, T, W]``) of the residual stream.  With
-    ``y`` (float32 ``[T, W]``) every copy is made anew from the old ones, ``x_t <- sum_s
+    ``y`` (float32 ``[T, W]``, or what adds up to it) every copy is made anew from the old ones, ``x_t <- sum_s
     mix[s, t] x_s + mult * out[t] * y``.  With ``read`` the row ``u = sum_s inw[s] x_s``
     (``inw`` None: the plain sum) of the new copies comes back, as it is (float32) or, with
     ``norm_weight``, as ``u / sqrt(mean(u^2) + eps) * (offset + norm_weight)`` in ``dtype``;
     ``rows`` (only without ``y``): of those rows alone; ``result``: rows to write them to (of
     any type, a column range of wider rows is allowed) instead of new ones."""
     lib = library.core_library()
-    _dev(x, y, mix, out, inw, norm_weight, rows)
-    _i32(rows, "rows")
     _need(x.dtype == torch.float32 and x.dim() == 3, "streams_step: float32 copies [S, T, W]")
     s, t, w = x.shape
+    terms, apart, wgt, extra, gate = 0, (0, 0), None, None, None
+    if isinstance(y, (PartialSums, ExpertSum)):
+        rows_at = (x, y.planes) if isinstance(y, PartialSums) else (x, y.y, y.extra)
+        if read:
+            rows_at += (result, norm_weight)
+        if (w % 4 or w > STREAMS_STEP_MOST or s > STREAMS_STEP_COPIES or any(v is not None and v.data_ptr() % 16 for v in rows_at)
+                or (read and result is not None and result.stride(0) % 4)):
+            y = y.materialize(torch.float32) if isinstance(y, PartialSums) else y.materialize()
+        elif isinstance(y, PartialSums):
+            _dev(y.planes)
+            _need(y.planes.dtype == torch.float32 and y.planes.shape[1:] == (t, w), "streams_step: float32 planes [parts, T, W]")
+            terms, apart, y = y.planes.shape[0], (w, t * w), y.planes[0]
+        else:
+            wgt, extra, gate = y.wgt, y.extra, y.gate
+            _dev(y.y, wgt, extra)
+            _need(wgt.dtype == torch.float32 and wgt.dim() == 2 and wgt.shape[0] == t and y.y.dtype == torch.float32
+                  and y.y.shape == (wgt.numel(), w) and (extra is None or (extra.dtype == torch.float32 and extra.shape == (t, w)))
+                  and (gate is None or (extra is not None and gate.is_cuda and gate.dtype == torch.float32 and gate.shape == (t, 1))),
+                  "streams_step: float32 rows of experts [T * top, W], weights [T, top], an extra row and its gate")
+            terms, apart, y = wgt.shape[1], (wgt.shape[1] * w, w), y.y[:t]
+    _dev(x, y, mix, out, inw, norm_weight, rows)
+    _i32(rows, "rows")
     _need(y is None or (y.dtype == torch.float32 and y.shape == (t, w) and mix is not None and out is not None
                         and mix.shape == (s, s) and out.numel() == s and mix.dtype == out.dtype and rows is None),
           "streams_step: an update takes float32 y [T, W], mix [S, S] and out [S] of one type, and all rows")
@@ -1669,7 +1698,8 @@ def streams_step(x: torch.Tensor, *, y: torch.Tensor | None = None, mix: torch.T
     elif read:
         result = torch.empty((n, w), dtype=dtype if norm_weight is not None else torch.float32, device=x.device)
     _check(lib, lib.hal_streams_step(
-        _ptr(x), ctypes.c_longlong(t * w), s, _ptr(y), _ptr(mix), _ptr(out), ctypes.c_float(mult), _ptr(inw),
+        _ptr(x), ctypes.c_longlong(t * w), s, _ptr(y), terms, *(ctypes.c_longlong(v) for v in apart), _ptr(wgt), _ptr(extra), _ptr(gate),
+        0 if gate is None else gate.stride(0), _ptr(mix), _ptr(out), ctypes.c_float(mult), _ptr(inw),
         dtype_code(c_dtype), 1 if read else 0, _ptr(norm_weight),
         dtype_code(norm_weight.dtype) if norm_weight is not None else F32, ctypes.c_float(offset), ctypes.c_float(eps),
         _ptr(result), 0 if result is None else result.stride(0), dtype_code(result.dtype) if result is not None else F32,

@@ -184,6 +184,8 @@ class Mixer(Part):
 
     takes_normed_rows: ClassVar[bool] = False
     folds_next_norm: ClassVar[bool] = False
+    # set by the arrangement: a float32 result may come back as ``PartialSums``, whose sum is the result
+    sums: bool = False
     # True: ``forward(..., add_to=h)`` adds the part's result into the float32 stream ``h``
     # itself (and returns None) instead of returning it; arrangements whose parts read the
     # same rows of the stream ask for this
@@ -205,6 +207,7 @@ class Mixer(Part):
 
 class FeedForward(Part):
     # as for Mixer
+    sums: bool = False
     takes_normed_rows: ClassVar[bool] = False
     folds_next_norm: ClassVar[bool] = False
     adds_to_stream: ClassVar[bool] = False
@@ -297,12 +300,15 @@ class Connection(Part):
     """How a part's input is read from the residual stream and how its result gets back
     there, for arrangements that keep the stream in ``copies`` copies ``[copies, T, width]``."""
 
+    adds_up = False
+    """Whether results that go back through it may be ``PartialSums`` or ``ExpertSum`` of float32 numbers."""
+
     @property
     def copies(self) -> int:
         raise NotImplementedError
 
     def step(self, x: torch.Tensor, pending, norm: "Norm") -> torch.Tensor:
-        """Writes what is ``pending`` (None, or ``(y, connection)``: a part's float32 result
+        """Writes what is ``pending`` (None, or ``(y, connection)``: a part's float32 result, or what adds up to it,
         and the connection it goes back through) into the copies ``x``, then returns the
         rows that the next part reads through this connection, normed by ``norm``."""
         raise NotImplementedError

@@ -202,6 +202,10 @@ class HyperPreNormBlock(Arrangement):
         for norm in (self.mixer_out_norm, self.ff_out_norm):
             if norm is not None and not (isinstance(norm, RMSNorm) and not norm.p.round_before_weight):
                 raise ValueError("a part's result is normed by an RMSNorm in the unrounded order")
+        # (what a part's result is added up from may stay apart for the pass that writes it, unless it is normed first)
+        self.mixer.sums = self.mixer_link.adds_up and self.mixer_out_norm is None
+        if self.ff is not None:
+            self.ff.sums = self.ff_link.adds_up and self.ff_out_norm is None
         if self.mixer_out_norm is not None and hasattr(self.mixer, "forward_normed_terms"):
             raise ValueError("a sum of normed results is not normed once more")
 
@@ -225,8 +229,9 @@ class HyperPreNormBlock(Arrangement):
         pending = (y, self.mixer_link)
         if self.ff is not None:
             x = self.ff_link.step(h, pending, self.ff_norm)
-            # (a mixture's weighted sum is made by the pass that norms and writes it)
-            sums = self.ff_out_norm is not None and hasattr(self.ff, "forward_sum")
+            # (a mixture's weighted sum is made by the pass that norms or writes it)
+            sums = hasattr(self.ff, "forward_sum") and (
+                self.ff_out_norm is not None or (self.ff.sums and getattr(self.ff.p, "float32_result", False)))
             y = self.ff.forward_sum(x, ctx) if sums else self.ff.forward(x, ctx)
             pending = (self._normed(y, self.ff_out_norm), self.ff_link)
         return pending

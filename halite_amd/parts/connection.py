@@ -67,6 +67,10 @@ class HyperConnection(Connection):
             self.w_out = torch.ones(1, dtype=torch.float32, device=dev)
             self.w_mix = torch.ones((1, 1), dtype=torch.float32, device=dev)
 
+    @property
+    def adds_up(self) -> bool:
+        return self.p.learned
+
     def _plain(self, pending) -> bool:
         """One copy and no learned weights, here and where the pending result goes back through."""
         return not self.p.learned and (pending is None or not pending[1].p.learned)
@@ -87,7 +91,7 @@ class HyperConnection(Connection):
         y, link = pending
         if isinstance(y, ops.NormedTerms):
             y = y.materialize()
-        if y.dtype != torch.float32:
+        if isinstance(y, torch.Tensor) and y.dtype != torch.float32:
             y = y.float()
         return dict(y=y, mix=link.w_mix, out=link.w_out, mult=link.p.mult)
 

@@ -132,9 +132,11 @@ class GatedFeedForward(FeedForward):
         m, d = x.shape
         if self.t_gate is not None and x.dtype == torch.bfloat16 and d % 8 == 0 and m <= ops.SKINNY_ROWS:
             act = ops.gemm_bf16_skinny(x, self.t_gate, w_up=self.t_up, tiled_shape=(f, d), activation=self.p.activation, clamp=self.p.clamp)
+        elif ops.stream_parts(x, self.w_gate_up, f, gated=True):
+            act = ops.gemm_bf16_stream(x, self.w_gate_up[:f], 1, w_up=self.w_gate_up[f:], activation=self.p.activation, clamp=self.p.clamp)
         else:
             act = ops.gate_mul(ops.linear(x, self.w_gate_up), self.p.activation, self.p.clamp)
-        return ops.linear(act, self.w_out, out_dtype=torch.float32, tiled=self.t_out)
+        return ops.linear(act, self.w_out, out_dtype=torch.float32, tiled=self.t_out, sums=self.sums)
 
 
 class DenseParams(BaseModel):
