@@ -911,12 +911,13 @@ def linear_add(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, tiled: torch.T
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = None,
-           tiled: torch.Tensor | None = None, next_norm: NextNorm | None = None, sums: bool = False):
+           tiled: torch.Tensor | None = None, next_norm: NextNorm | None = None, sums: bool = False,
+           unrounded: bool = False):
     """``x @ w.T`` for a weight ``[out, in]``; ``tiled`` is ``tile_weight(w)`` if the
     model keeps that copy for small batches.  ``x`` may be ``NormedRows``; with
     ``next_norm`` the result may come back as ``NormedRows`` (already added into the
-    stream) instead of a tensor, with ``sums`` (or a norm that says so) as ``PartialSums``, whose reader
-    rounds their sum to ``out_dtype``.
+    stream) instead of a tensor, with ``sums`` (or a norm that says so) a bfloat16 one as ``PartialSums``, whose reader
+    rounds their sum; ``unrounded``: a float32 one, whose reader does not.
 
     float32 weights: the true 32-bit kernel (activations are widened if needed).
     bf16 weights: the hand-written kernels where they are the faster ones (``skinny_pays``:
@@ -951,8 +952,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
         return gemm_bf16_skinny(x, tiled, out_dtype=out_dtype, tiled_shape=tuple(w.shape))
     if skinny_ok and skinny_pays(m, w.shape[0], k, False):
         return gemm_bf16_skinny(x, w, out_dtype=out_dtype)
-    # (a norm that adds up the parts rounds their sum to bf16: a result that is wanted in float32 comes to it whole)
-    in_parts = sums or (out_dtype == torch.bfloat16 and next_norm is not None and next_norm.sums)
+    # (the readers that ``sums`` and a norm mean round the sum of the parts: a result that is wanted in float32 comes to them whole)
+    in_parts = unrounded if out_dtype == torch.float32 else sums or (next_norm is not None and next_norm.sums)
     parts = stream_parts(x, w, w.shape[0], may_part=in_parts)
     if parts:
         return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)

@@ -136,7 +136,7 @@ class GatedFeedForward(FeedForward):
             act = ops.gemm_bf16_stream(x, self.w_gate_up[:f], 1, w_up=self.w_gate_up[f:], activation=self.p.activation, clamp=self.p.clamp)
         else:
             act = ops.gate_mul(ops.linear(x, self.w_gate_up), self.p.activation, self.p.clamp)
-        return ops.linear(act, self.w_out, out_dtype=torch.float32, tiled=self.t_out, sums=self.sums)
+        return ops.linear(act, self.w_out, out_dtype=torch.float32, tiled=self.t_out, unrounded=self.sums)
 
 
 class DenseParams(BaseModel):

@@ -99,4 +99,4 @@ class GeneralDelta(Mixer):
             y = ops.delta_chunks(*rule, gate, self.w_norm_weight, p.eps, x.dtype)
         else:
             y = ops.head_norm_gate(ops.delta_rule(*rule), gate, self.w_norm_weight, p.eps, p.n_heads, x.dtype)
-        return ops.linear(y, self.w_out_weight, out_dtype=torch.float32, tiled=self.t_out, sums=self.sums)
+        return ops.linear(y, self.w_out_weight, out_dtype=torch.float32, tiled=self.t_out, unrounded=self.sums)

@@ -138,4 +138,4 @@ class SigmoidAttention(Mixer):
                                     **(pages if run.appends else {}))
         out = ctx.attention(packed, packed.shape[1], kv, group, p.n_heads, p.scale, p.window or 0, rule=self.rule)
         heads = ops.head_gate_cols(out, D, gate, p.v_dim, p.n_heads)
-        return ops.linear(heads, self.w_out, out_dtype=torch.float32, tiled=self.t_out, sums=self.sums)
+        return ops.linear(heads, self.w_out, out_dtype=torch.float32, tiled=self.t_out, unrounded=self.sums)
