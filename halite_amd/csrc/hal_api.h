@@ -206,6 +206,11 @@ int hal_grouped_gemm_experts_kernel(int M, int N, int K, int G, int gated);
 int hal_norm_pair(const float* h, const int* rows, const void* w1, const void* w2, int w_dtype,
                   float eps, void* out1, void* out2, int dtype, int n_rows, int d,
                   hipStream_t stream);
+// The same after h[t] <- (h[t] + beside[t]) + sum_j wgt[t, j] y[t * top + j] (+ sigmoid(extra_gate[t]) extra[t]); with rows those rows
+// alone, and h stays as it is.
+int hal_norm_pair_added(float* h, const float* beside, const float* y, const float* wgt, const float* extra,
+                        const float* extra_gate, int ld_gate, int top, const int* rows, const void* w1, const void* w2,
+                        int w_dtype, float eps, void* out1, void* out2, int dtype, int n_rows, int d, hipStream_t stream);
 // From the float32 down projections of a latent attention (a [T, lda]: query latent of q_rank
 // columns from q_col0, none if q_rank == 0; key/value latent of kv_rank columns from kv_col0
 // followed by `rot` shared rotated-key columns): cq [T, q_rank] = the normed query latent,

@@ -131,6 +131,120 @@ extern "C" int hal_norm_pair(const float* h, const int* rows, const void* w1, co
 }
 
 // ---------------------------------------------------------------------------------
+// The same with what a layer left to be added: h[t] <- (h[t] + beside[t]) + s[t], s the weighted sum of a mixture's experts
+// (as hal_moe_combine adds it up), then the norms of the new row.  With `rows` those rows alone, and h stays as it is (the
+// last norm reads a few).  A thread holds its part of the new row; the rows of up to four experts are on their way together.
+// Bound by memory; what is saved is the stream's way out and back, twice, and two launches.  Three passes / this one, six experts, a row
+// beside and an extra one, two weights, us: 8 rows of 4,096 5.2 / 4.1, 64 8.3 / 4.4, 300 21.7 / 10.8, 3,000 130 / 101 (540 MB); 8,192 of
+// 2,048 with four 146 / 114.  One group of four numbers a thread where a workgroup can have as many (3,000 rows: two groups 105, four
+// 109, eight 121: a group's rows wait for the group's before).
+// ---------------------------------------------------------------------------------
+struct AddedRows {
+  const float* beside;  // [T, d], or null
+  const float* y;       // [T * top, d]
+  const float* wgt;     // [T, top]
+  const float* extra;   // [T, d], or null
+  const float* gate;    // [T] with rows of ld_gate, or null: sigmoid(gate) times `extra`
+  int ld_gate, top;
+};
+template <typename T, bool PAIR, int MAXV>
+__global__ void __launch_bounds__(1024) norm_added_vec_kernel(float* __restrict__ h, AddedRows e, const int* __restrict__ rows,
+                                                              const void* __restrict__ w1, const void* __restrict__ w2, int w_dtype,
+                                                              float eps, T* __restrict__ out1, T* __restrict__ out2, int d) {
+  __shared__ float scratch[16];
+  const int r = blockIdx.x, nv = d / 4;
+  const size_t t = rows ? rows[r] : r;
+  const float eg = e.gate ? 1.0f / (1.0f + expf(-e.gate[t * e.ld_gate])) : 1.0f;
+  const float* w = e.wgt + t * e.top;
+  float x[MAXV][4];
+  float ss = 0.f;
+#pragma unroll
+  for (int u = 0; u < MAXV; ++u) {
+    const int v = threadIdx.x + u * blockDim.x;
+    if (v >= nv) continue;
+    float b[4], s[4] = {0.f, 0.f, 0.f, 0.f};
+    load4(h + t * d + v * 4, x[u]);
+    if (e.beside) load4(e.beside + t * d + v * 4, b);
+    if (e.extra) load4(e.extra + t * d + v * 4, s);
+    const float* at = e.y + t * e.top * d + v * 4;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) s[i] *= eg;
+    for (int j0 = 0; j0 < e.top; j0 += 4) {
+      float part[4][4], c[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int which = j0 + j < e.top ? j0 + j : j0;  // (past the end: a row that is there, not added)
+        load4(at + (size_t)which * d, part[j]);
+        c[j] = w[which];
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        if (j0 + j >= e.top) break;
+#pragma unroll
+        for (int i = 0; i < 4; ++i) s[i] += c[j] * part[j][i];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      if (e.beside) x[u][i] += b[i];
+      x[u][i] += s[i];
+      ss += x[u][i] * x[u][i];
+    }
+    if (!rows) store4(h + t * d + v * 4, x[u]);
+  }
+  const float total = block_sum(ss, scratch);
+  const float rstd = 1.0f / sqrtf(total / (float)d + eps);
+#pragma unroll
+  for (int u = 0; u < MAXV; ++u) {
+    const int v = threadIdx.x + u * blockDim.x;
+    if (v >= nv) continue;
+    float a[4], b[4], y[4], z[4];
+    load4_any(w1, w_dtype, (size_t)v * 4, a);
+    if (PAIR) load4_any(w2, w_dtype, (size_t)v * 4, b);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      x[u][i] *= rstd;
+      y[i] = x[u][i] * a[i];
+      if (PAIR) z[i] = x[u][i] * b[i];
+    }
+    store4(out1 + (size_t)r * d + v * 4, y);
+    if (PAIR) store4(out2 + (size_t)r * d + v * 4, z);
+  }
+}
+
+// Rows of a multiple of four numbers up to NA_MOST, at places of 16 bytes.
+#define NA_MOST 16384
+extern "C" int hal_norm_pair_added(float* h, const float* beside, const float* y, const float* wgt, const float* extra,
+                                   const float* extra_gate, int ld_gate, int top, const int* rows, const void* w1, const void* w2,
+                                   int w_dtype, float eps, void* out1, void* out2, int dtype, int n_rows, int d, hipStream_t stream) {
+  HAL_REQUIRE(n_rows >= 0 && d > 0 && d % 4 == 0 && d <= NA_MOST && top > 0 && y && wgt, "hal_norm_pair_added: bad sizes rows=%d d=%d top=%d",
+              n_rows, d, top);
+  HAL_REQUIRE(dtype == HAL_F32 || dtype == HAL_BF16, "hal_norm_pair_added: dtype %d", dtype);
+  HAL_REQUIRE((w2 == nullptr) == (out2 == nullptr), "hal_norm_pair_added: a second weight and a second result come together");
+  HAL_REQUIRE(((uintptr_t)h | (uintptr_t)beside | (uintptr_t)y | (uintptr_t)extra | (uintptr_t)w1 | (uintptr_t)w2 | (uintptr_t)out1 |
+               (uintptr_t)out2) % 16 == 0, "hal_norm_pair_added: rows must be 16-byte aligned");
+  if (n_rows == 0) return 0;
+  const AddedRows e = {beside, y, wgt, extra, extra ? extra_gate : nullptr, ld_gate, top};
+  const int v = d <= 4096 ? 1 : 4;
+  const int lanes = ((d / 4 + v - 1) / v + 63) / 64 * 64;
+#define NA_LAUNCH(T_, PAIR_, V_) \
+  hipLaunchKernelGGL((norm_added_vec_kernel<T_, PAIR_, V_>), dim3(n_rows), dim3(lanes), 0, stream, h, e, rows, w1, w2, w_dtype, eps, (T_*)out1, (T_*)out2, d)
+#define NA_BY_WIDTH(T_, PAIR_)            \
+  do {                                    \
+    if (v == 1) NA_LAUNCH(T_, PAIR_, 1);  \
+    else NA_LAUNCH(T_, PAIR_, 4);         \
+  } while (0)
+  if (dtype == HAL_F32 && w2) NA_BY_WIDTH(float, true);
+  else if (dtype == HAL_F32) NA_BY_WIDTH(float, false);
+  else if (w2) NA_BY_WIDTH(bf16_t, true);
+  else NA_BY_WIDTH(bf16_t, false);
+#undef NA_BY_WIDTH
+#undef NA_LAUNCH
+  HAL_LAUNCH_CHECK();
+  return 0;
+}
+
+// ---------------------------------------------------------------------------------
 // a [T, lda] float32 holds, per token, the query latent (q_rank, from column q_col0; none
 // if q_rank == 0), then at kv_col0 the key/value latent (kv_rank) and the shared rotated key
 // part (rot, not normed).

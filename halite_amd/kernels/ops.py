@@ -900,14 +900,19 @@ def gemm_bf16_skinny_norm(
     return out
 
 
-def linear_add(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, tiled: torch.Tensor | None = None) -> None:
+def linear_add(h: torch.Tensor, x: torch.Tensor, w: torch.Tensor, tiled: torch.Tensor | None = None, apart: bool = False):
     """``h += x @ w.T`` for the float32 stream ``h``: the product is float32 and the sum is
-    made in float32; few bf16 rows do both in one kernel."""
+    made in float32; few bf16 rows do both in one kernel.  ``apart``: where they are two, the
+    product comes back and is not added."""
     m, k = x.shape
     if (w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and m <= SKINNY_ROWS and tiled is not None and k % 8 == 0):
         gemm_bf16_skinny(x, tiled, add_to=h, tiled_shape=tuple(w.shape))
-        return
-    residual_add(h, linear(x, w, out_dtype=torch.float32, tiled=tiled))
+        return None
+    y = linear(x, w, out_dtype=torch.float32, tiled=tiled)
+    if apart:
+        return y
+    residual_add(h, y)
+    return None
 
 
 def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = None,
@@ -983,12 +988,38 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
 GROUP_TILE_ROWS = 128  # rows of a tile of the grouped product (what ``moe_sort`` counts tiles in)
 
 
+ADDED_MOST = 16384  # the widest rows to which a norm adds a layer's results itself
+
+
 def rmsnorm_exact(h: torch.Tensor, weight: torch.Tensor, eps: float, out_dtype: torch.dtype,
-                  rows: torch.Tensor | None = None, second: torch.Tensor | None = None):
+                  rows: torch.Tensor | None = None, second: torch.Tensor | None = None, added: LayerResults | None = None):
     """RMSNorm of the float32 stream ``h`` (only of ``rows`` if given) as ``x * rstd * w``
     in float32 with one rounding at the end; with ``second`` (another weight for the same
-    rows) both results come back."""
+    rows) both results come back.  ``added``: what is added to the stream first (with ``rows`` it
+    may stay as it is)."""
     lib = library.core_library()
+    if added is not None:
+        e = added.experts
+        beside, (t, d) = added.beside, h.shape
+        places = (h, beside, e.y, e.extra, weight, second)
+        if d % 4 or d > ADDED_MOST or any(v is not None and v.data_ptr() % 16 for v in places):
+            added.add_to(h)
+            return rmsnorm_exact(h, weight, eps, out_dtype, rows, second)
+        _dev(h, weight, rows, second, beside, e.y, e.wgt, e.extra)
+        _i32(rows, "rows")
+        _need(h.dtype == e.y.dtype == e.wgt.dtype == torch.float32 and e.wgt.shape[0] == t and e.y.shape == (e.wgt.numel(), d)
+              and all(v is None or (v.dtype == torch.float32 and v.shape == h.shape) for v in (beside, e.extra))
+              and (e.gate is None or (e.extra is not None and e.gate.is_cuda and e.gate.dtype == torch.float32 and e.gate.shape == (t, 1))),
+              "rmsnorm: float32 rows to add, experts' results [T * top, d] and their weights [T, top]")
+        _need(weight.shape == (d,) and (second is None or (second.shape == (d,) and second.dtype == weight.dtype)),
+              "rmsnorm: weights of the stream's width and of one element type")
+        n = t if rows is None else rows.numel()
+        outs = [torch.empty((n, d), dtype=out_dtype, device=h.device) if w is not None else None for w in (weight, second)]
+        _check(lib, lib.hal_norm_pair_added(
+            _ptr(h), _ptr(beside), _ptr(e.y), _ptr(e.wgt), _ptr(e.extra), _ptr(e.gate), 0 if e.gate is None else e.gate.stride(0),
+            e.wgt.shape[1], _ptr(rows), _ptr(weight), _ptr(second), dtype_code(weight.dtype), ctypes.c_float(eps),
+            _ptr(outs[0]), _ptr(outs[1]), dtype_code(out_dtype), n, d, _stream()))
+        return outs[0] if second is None else tuple(outs)
     _dev(h, weight, rows, second)
     _i32(rows, "rows")
     _need(h.dtype == torch.float32 and h.dim() == 2, "rmsnorm: the stream is float32 [T, d]")
@@ -1293,6 +1324,20 @@ class ExpertSum:
         out = torch.empty(self.shape, dtype=torch.float32, device=self.y.device)
         moe_combine(out, self.y, self.wgt, self.extra, extra_gate=self.gate, overwrite=True)
         return out
+
+
+@dataclass
+class LayerResults:
+    """What a layer leaves to the norm that reads its stream next: ``h <- (h + beside) + experts``, all float32."""
+
+    beside: torch.Tensor | None
+    experts: ExpertSum
+
+    def add_to(self, h: torch.Tensor) -> None:
+        if self.beside is not None:
+            residual_add(h, self.beside)
+        e = self.experts
+        moe_combine(h, e.y, e.wgt, e.extra, extra_gate=e.gate)
 
 
 def normed_sum(terms: list[tuple[torch.Tensor, torch.Tensor, float]], eps: float) -> torch.Tensor:

@@ -190,6 +190,8 @@ class Mixer(Part):
     # itself (and returns None) instead of returning it; arrangements whose parts read the
     # same rows of the stream ask for this
     adds_to_stream: ClassVar[bool] = False
+    # True: with ``add_to`` and ``apart`` a result that takes a pass of its own to add comes back instead
+    adds_apart: ClassVar[bool] = False
 
     def attention_sizes(self) -> tuple[int, int, int] | None:
         """(query heads, key/value heads, head size) if the mixer has such sizes, for the

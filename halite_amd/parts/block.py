@@ -60,11 +60,13 @@ class ParallelBlock(Arrangement):
     feed-forward (and its norm) out.
 
     Both parts are handed the float32 stream to add their result into (``add_to``), so
-    the sum is float32 and nothing is left pending.  Where both norms are RMSNorms of one
-    eps in the unrounded order, one kernel computes the statistic once and writes both
-    results."""
+    the sum is float32.  Where both norms are RMSNorms of one eps in the unrounded order,
+    one kernel computes the statistic once and writes both results.  A mixture's weighted sum, with
+    the mixer's result where that is not in the stream yet, is left pending (``ops.LayerResults``) for the
+    norm that comes next; otherwise, and in float32 (whose stream is compared layer by layer), nothing is."""
 
     graph_safe = True
+    takes_layer_results = True
     roles = {"mixer_norm": NORMS, "mixer": MIXERS, "ff_norm": NORMS, "ff": FEED_FORWARDS}
     optional = ("ff_norm", "ff")
 
@@ -83,18 +85,23 @@ class ParallelBlock(Arrangement):
         )
 
     def forward(self, h, pending, ctx, run):
-        if pending is not None:
-            ops.residual_add(h, pending)
+        one_pass = self.ff is not None and self._one_pass and self.mixer_norm.weight.dtype == self.ff_norm.weight.dtype
+        added = pending if isinstance(pending, ops.LayerResults) and one_pass else None
+        if pending is not None and added is None:
+            pending.add_to(h) if isinstance(pending, ops.LayerResults) else ops.residual_add(h, pending)
         if self.ff is None:
             x = self.mixer_norm.forward(h)
             self.mixer.forward(x, ctx, run, add_to=h)
             return None
-        if self._one_pass and self.mixer_norm.weight.dtype == self.ff_norm.weight.dtype:
+        if one_pass:
             x, y = ops.rmsnorm_exact(h, self.mixer_norm.weight, self.mixer_norm.p.eps, self.mixer_norm.build.dtype,
-                                     second=self.ff_norm.weight)
+                                     second=self.ff_norm.weight, added=added)
         else:
             x, y = self.mixer_norm.forward(h), self.ff_norm.forward(h)
         # both results are computed before either is added: both parts read the same stream
+        if hasattr(self.ff, "forward_sum") and self.ff_norm.build.dtype == torch.bfloat16:
+            beside = self.mixer.forward(x, ctx, run, add_to=h, **(dict(apart=True) if self.mixer.adds_apart else {}))
+            return ops.LayerResults(beside, self.ff.forward_sum(y, ctx))
         self.mixer.forward(x, ctx, run, add_to=h)
         self.ff.forward(y, ctx, add_to=h)
         return None

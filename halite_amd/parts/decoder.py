@@ -27,6 +27,7 @@ from .base import (
     Part,
     RunBinding,
 )
+from .norm import RMSNorm
 
 
 EMBEDDING_RUN = -1  # the index of the embedding's state rows among the runs'
@@ -149,6 +150,8 @@ class Decoder:
                 next_norm = ahead.first_norm_for(h)
             elif i + 1 == len(blocks) and getattr(blocks[i], "takes_last_norm", False):
                 next_norm = self.final_norm.summable(h)
+            if isinstance(pending, ops.LayerResults) and not getattr(blocks[i], "takes_layer_results", False):
+                pending = pending.add_to(h)
             if next_norm is not None:
                 pending = blocks[i].forward(h, pending, ctx, run, next_norm=next_norm)
             else:
@@ -160,6 +163,8 @@ class Decoder:
             if x is None:
                 x = self.final_norm.forward(blocks[-1].leave(h, pending, ctx.logit_rows))
         else:
+            if isinstance(pending, ops.LayerResults) and not isinstance(self.final_norm, RMSNorm):
+                pending = pending.add_to(h)
             x = self.final_norm.forward(h, delta=pending, rows=ctx.logit_rows)
         return self.head.forward(x)
 
@@ -168,7 +173,9 @@ class Decoder:
         rows = junction.stream_rows(kept)
         ctx.rounded_rows = None
         if self.stream_copies is None:
-            if pending is not None:
+            if isinstance(pending, ops.LayerResults):
+                pending.add_to(h)
+            elif pending is not None:
                 ops.residual_add(h, pending)
             ops.cast_cols(h, rows)
             return junction.forward(kept)

@@ -61,6 +61,7 @@ class LatentAttention(Mixer):
     Params = LatentAttentionParams
     graph_safe = True
     adds_to_stream = True
+    adds_apart = True
 
     def __init__(self, params, build):
         super().__init__(params, build)
@@ -148,7 +149,7 @@ class LatentAttention(Mixer):
         if attention_kernels.mfma_supported(self.build.dtype, self.head_dim, group.page_size):
             ctx.plan_attention(group.group_id, self.p.n_heads, 1, self.p.window or 0, self.head_dim)
 
-    def forward(self, x, ctx, run, add_to=None):
+    def forward(self, x, ctx, run, add_to=None, apart=False):
         p = self.p
         kv = run.kv
         group = ctx.group(kv.group_id)
@@ -183,6 +184,5 @@ class LatentAttention(Mixer):
         ops.grouped_gemm(latent, self.w_uv3, heads, n_rows=n, x_group_cols=D, x_col0=p.rope_dim, y_group_cols=p.v_dim,
                          gate=a[:, gate_col0:] if p.output_gate else None, gate_per_group=p.gate_per_head)
         if add_to is not None:
-            ops.linear_add(add_to, heads, self.w_out, tiled=self.t_out)
-            return None
+            return ops.linear_add(add_to, heads, self.w_out, tiled=self.t_out, apart=apart)
         return ops.linear(heads, self.w_out, out_dtype=torch.float32 if p.float32_result else None, tiled=self.t_out)

@@ -62,6 +62,11 @@ class RMSNorm(Norm):
             self.multiplier = self.weight.float() + self.p.weight_offset
 
     def forward(self, h, delta=None, rows=None):
+        if isinstance(delta, ops.LayerResults):
+            if not (self.p.round_before_weight or self.p.layer_scale or self.p.weight_offset != 0.0):
+                return ops.rmsnorm_exact(h, self.weight, self.p.eps, self.build.dtype, rows=rows, added=delta)
+            delta.add_to(h)
+            delta = None
         if self.p.layer_scale:
             if delta is not None:
                 ops.residual_add(h, delta)
