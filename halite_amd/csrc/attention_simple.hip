@@ -195,6 +195,52 @@ struct plain_tiles {
       }
     }
   }
+  // The same, all places looked up before the first load and every load made, of a place that is there, so that none waits for
+  // the others' (pages of a multiple of four keys); which of them count is kept for `commit_together`.
+  uint32_t k_state[(NV + 15) / 16], v_state[(NV + 7) / 8];  // two bits a vector of keys (1: read, 2: a hole), four of values
+  __device__ __forceinline__ void fetch_together(int buf) {
+    const int2* place = key_place + buf * KEYS;
+    int2 wk[NV];
+    int4 wv[NV][2];
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int row = kr0 + u * rows_per_pass;
+      wk[u] = place[row < KEYS ? row : KEYS - 1];
+      const int jj = ((tid + u * THREADS) % (KEYS / 4)) * 4;
+      wv[u][0] = *(const int4*)(place + jj), wv[u][1] = *(const int4*)(place + jj + 2);
+    }
+#pragma unroll
+    for (int i = 0; i < (NV + 15) / 16; ++i) k_state[i] = 0;
+#pragma unroll
+    for (int i = 0; i < (NV + 7) / 8; ++i) v_state[i] = 0;
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const int row = kr0 + u * rows_per_pass;
+      const bool read = wk[u].x >= 0 && row < KEYS && kc < dv;
+      k_state[u / 16] |= (read ? 1u : wk[u].x == -1 ? 2u : 0u) << (2 * (u % 16));
+      load4(k_pages + (read ? ((size_t)wk[u].x * page_size + wk[u].y) * D + kc * 4 : 0), kreg[u]);
+      const int d = (tid + u * THREADS) / (KEYS / 4);
+      // the four keys lie side by side in one page; the range may begin and end among them
+      const int page[4] = {wv[u][0].x, wv[u][0].z, wv[u][1].x, wv[u][1].z}, slot[4] = {wv[u][0].y, wv[u][0].w, wv[u][1].y, wv[u][1].w};
+      int pg = -1, at = 0;
+#pragma unroll
+      for (int x = 3; x >= 0; --x)
+        if (page[x] >= 0) pg = page[x], at = slot[x] - x, v_state[u / 8] |= 1u << (4 * (u % 8) + x);
+      load4(v_pages + (pg >= 0 && d < D ? ((size_t)pg * D + d) * page_size + at : 0), vreg[u]);
+    }
+  }
+  __device__ __forceinline__ void commit_together() {
+#pragma unroll
+    for (int u = 0; u < NV; ++u) {
+      const uint32_t k = k_state[u / 16] >> (2 * (u % 16)) & 3, v = v_state[u / 8] >> (4 * (u % 8)) & 15;
+#pragma unroll
+      for (int x = 0; x < 4; ++x) {
+        kreg[u][x] = k == 1 ? kreg[u][x] : k == 2 ? __uint_as_float(0x7fc00000u) : 0.f;
+        vreg[u][x] = v >> x & 1 ? vreg[u][x] : 0.f;
+      }
+    }
+    commit();
+  }
   __device__ __forceinline__ void commit() {
 #pragma unroll
     for (int u = 0; u < NV; ++u) {
@@ -530,35 +576,41 @@ attention_plain_merge_kernel(T* __restrict__ out, int out_row_stride, const int*
 // (TURNS; the even blocks' sums wait in the row's place of `out`, which bf16 rows do not have room for: they keep four waves).
 // (32 heads of 128, 8 of the keys, float32, four waves and eight: one request of 100 tokens 39 / 36 us, 500 146 / 114, 1,000
 // (256 workgroups) 279 / 214; four waves in one turn, in two, and eight: 2,048 772 / 787 / 825, 16 of 500 614 / 646 / 740.)
-// Grid: x = groups of `tq` tokens, y = key/value head times chunk of 128 heads of its group.
+// ROWS: with workgroups of 128 rows for half of the compute units or fewer, workgroups of 64 (`rows`), four waves, a wave to a SIMD,
+// which has twice the registers then: the places of a block's keys are looked up together and its loads not waited for one
+// by one, a block's operands are on their way before its products begin, and scores that are only scaled take a loop of their own (in
+// the builds for 128 rows these spill: 2,048 tokens 780 -> 809).  A row's sums stay as they are.  100 tokens 34.6 -> 30.9 us, 300 71.5 -> 61.6,
+// 500 113.7 -> 92.0 (halving the rows alone 101.9), 64 after 8,000 1,598 -> 1,242.  513 tokens (129 workgroups of 128) 119.
+// Grid: x = groups of `tq` tokens, y = key/value head times chunk of ROWS heads of its group.
 typedef __attribute__((ext_vector_type(16))) float plain_f32x16;
 #define ROWS_KEYS 32
 #define ROWS_MOST 128
 #define ROWS_UNITS 256  // compute units of the gfx950 parts that this library is built for
-#define ROWS_THREADS(GROUPS) (ROWS_MOST / 32 * (GROUPS) * HAL_WAVE)
+#define ROWS_THREADS(ROWS, GROUPS) ((ROWS) / 32 * (GROUPS) * HAL_WAVE)
 
-static inline size_t rows_lds_floats(int D, int db, int groups) {
+static inline size_t rows_lds_floats(int D, int db, int rows, int groups) {
   const int keys = ROWS_KEYS * groups;
   const size_t tiles = (size_t)keys * (D + PLAIN_PAD) + (size_t)db * 32 * (keys + PLAIN_PAD) + (size_t)2 * 2 * keys;
-  const size_t sums = groups == 1 ? 0 : (size_t)ROWS_MOST * 2 * (db * 16 + 2);  // of the waves with the odd blocks, where the tiles were
+  const size_t sums = groups == 1 ? 0 : (size_t)rows * 2 * (db * 16 + 2);  // of the waves with the odd blocks, where the tiles were
   return tiles > sums ? tiles : sums;
 }
 
-template <typename T, int DB, int GROUPS>
-__global__ void __launch_bounds__(ROWS_THREADS(GROUPS), 2)
+template <typename T, int DB, int ROWS, int GROUPS>
+__global__ void __launch_bounds__(ROWS_THREADS(ROWS, GROUPS), ROWS == ROWS_MOST ? 2 : 1)
 attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__ out, int out_row_stride,
                       const int* __restrict__ positions, const int* __restrict__ token_seg,
                       const int* __restrict__ block_table, int bt_stride, const T* __restrict__ k_pages,
                       const T* __restrict__ v_pages, int n_tokens, int H, int K, int D, int page_size,
                       int n_pages, float scale, hal_score_rule rule, int tq, int chunks, int page_shift,
                       int cw_shift) {
-  constexpr int THREADS = ROWS_THREADS(GROUPS), KEYS = ROWS_KEYS * GROUPS;
+  constexpr int THREADS = ROWS_THREADS(ROWS, GROUPS), KEYS = ROWS_KEYS * GROUPS;
   constexpr int TURNS = GROUPS == 1 && sizeof(T) == 4 ? 2 : 1, STEP = KEYS * TURNS;  // walks of a row's keys, every TURNS-th block each
+  constexpr bool AHEAD = ROWS < ROWS_MOST;  // (a wave alone on its SIMD, with registers for a block's operands at once)
   constexpr int NV = KEYS * ((DB + 1) / 2) * 16 / THREADS;
   extern __shared__ float smem[];
   const int tid = threadIdx.x;
   const int lane = tid % HAL_WAVE;
-  const int waves_at = __builtin_amdgcn_readfirstlane(tid / HAL_WAVE), wave = waves_at % (ROWS_MOST / 32), kg = waves_at / (ROWS_MOST / 32);
+  const int waves_at = __builtin_amdgcn_readfirstlane(tid / HAL_WAVE), wave = waves_at % (ROWS / 32), kg = waves_at / (ROWS / 32);
   const int half = lane / 32, col = lane % 32;
   const int KS = D + PLAIN_PAD, VS = KEYS + PLAIN_PAD;
   float* k_tile = smem;                             // [KEYS][D + pad]
@@ -568,8 +620,8 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
 
   const int G = H / K;
   const int g = blockIdx.y / chunks, chunk = blockIdx.y % chunks;
-  const int heads_here = min(ROWS_MOST, G - chunk * ROWS_MOST);
-  const int h_first = g * G + chunk * ROWS_MOST;
+  const int heads_here = min(ROWS, G - chunk * ROWS);
+  const int h_first = g * G + chunk * ROWS;
   const int t_first = blockIdx.x * tq;
   const int t_end = min(n_tokens, t_first + tq);
   const int hd = D / 2;  // dimensions of a half of the lanes
@@ -615,6 +667,9 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
     tiles.n_pages = n_pages, tiles.K = K, tiles.g = g, tiles.lo_min = lo_min, tiles.p_max = p_max, tiles.tid = tid;
     tiles.kc = tid & ((1 << cw_shift) - 1), tiles.kr0 = tid >> cw_shift, tiles.rows_per_pass = THREADS >> cw_shift;
     tiles.asked_page = 0, tiles.asked_slot = -1, tiles.keep = rule.keep;
+    // (where there are registers for it)
+    const bool together = AHEAD && page_size % 4 == 0;
+    const bool scaled_only = AHEAD && rule.softcap == 0.f && !rule.bias && rule.sink != HAL_WEIGHTS_SIGMOID;
 
     T* const op = out + (size_t)token * out_row_stride + (size_t)head * D;
     // element v of a block's 16: dimension 32 b + 8 (v / 4) + 4 half + v % 4
@@ -649,15 +704,15 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
     tiles.ask_place(walk.key(place(1)));
     tiles.put_place(1);
     __syncthreads();
-    tiles.fetch(0);
+    together ? tiles.fetch_together(0) : tiles.fetch(0);
     tiles.ask_place(walk.key(place(2)));
     int buf = 0;
     for (int n = 0; n < n_blocks; ++n, buf ^= 1) {
 #pragma clang fp contract(off)  // (the builds for one group and for two round alike)
       __syncthreads();  // every wave has read the block before
-      tiles.commit();
+      together ? tiles.commit_together() : tiles.commit();
       tiles.put_place(buf);  // of the block after the next
-      if (n + 1 < n_blocks) tiles.fetch(buf ^ 1);
+      if (n + 1 < n_blocks) together ? tiles.fetch_together(buf ^ 1) : tiles.fetch(buf ^ 1);
       tiles.ask_place(walk.key(place(n + 3)));
       __syncthreads();
       if (TURNS == 2 && n == n_even) {  // the even blocks' sums make room for the odd ones'
@@ -677,19 +732,45 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
 #pragma unroll
       for (int v = 0; v < 16; ++v) st[v] = 0.f;
       const float* kr = k_tile + (size_t)(kg * ROWS_KEYS + col) * KS + half * hd;
+      float4 ahead[AHEAD ? DB * 4 : 1];
+      if constexpr (AHEAD) {
 #pragma unroll
-      for (int i = 0; i < DB * 4; ++i) {
-        if (i * 4 < hd) {
-          const float4 kk = *(const float4*)(kr + i * 4);
-          st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.x, qreg[i * 4 + 0], st, 0, 0, 0);
-          st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.y, qreg[i * 4 + 1], st, 0, 0, 0);
-          st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.z, qreg[i * 4 + 2], st, 0, 0, 0);
-          st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.w, qreg[i * 4 + 3], st, 0, 0, 0);
-        }
+        for (int i = 0; i < DB * 4; ++i) ahead[i] = *(const float4*)(kr + (i * 4 < hd ? i * 4 : 0));
+      }
+      auto four = [&](int i) {
+        const float4 kk = AHEAD ? ahead[AHEAD ? i : 0] : *(const float4*)(kr + i * 4);
+        st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.x, qreg[i * 4 + 0], st, 0, 0, 0);
+        st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.y, qreg[i * 4 + 1], st, 0, 0, 0);
+        st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.z, qreg[i * 4 + 2], st, 0, 0, 0);
+        st = __builtin_amdgcn_mfma_f32_32x32x2f32(kk.w, qreg[i * 4 + 3], st, 0, 0, 0);
+      };
+      if (AHEAD && hd == DB * 16) {
+#pragma unroll
+        for (int i = 0; i < DB * 4; ++i) four(i);
+      } else {
+#pragma unroll
+        for (int i = 0; i < DB * 4; ++i)
+          if (i * 4 < hd) four(i);
+      }
+      if constexpr (AHEAD) {  // (the values, while the probabilities are made)
+#pragma unroll
+        for (int b = 0; b < DB; ++b)
+#pragma unroll
+          for (int t4 = 0; t4 < 4; ++t4)
+            ahead[b * 4 + t4] = *(const float4*)(v_tile + (size_t)(b * 32 + col) * VS + kg * ROWS_KEYS + 4 * half + 8 * t4);
       }
       // ---- this row's 16 keys of the block (the other half of the wave has the other 16) ----
       float mx = -INFINITY;
       bool valid[16];
+      if (scaled_only) {  // (without sixteen looks at the rest of the rule: the same numbers)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) {
+          const int j = key0 + 8 * (v / 4) + 4 * half + v % 4;
+          valid[v] = hal_rule_sees(rule, lo, j) && j <= p;
+          st[v] = valid[v] ? st[v] * scale : -INFINITY;
+          mx = fmaxf(mx, st[v]);
+        }
+      } else
 #pragma unroll
       for (int v = 0; v < 16; ++v) {
         const int j = key0 + 8 * (v / 4) + 4 * half + v % 4;
@@ -722,7 +803,7 @@ attention_rows_kernel(const T* __restrict__ q, int q_row_stride, T* __restrict__
         const float* vr = v_tile + (size_t)(b * 32 + col) * VS + kg * ROWS_KEYS + 4 * half;
 #pragma unroll
         for (int t4 = 0; t4 < 4; ++t4) {
-          const float4 vv = *(const float4*)(vr + 8 * t4);
+          const float4 vv = AHEAD ? ahead[AHEAD ? b * 4 + t4 : 0] : *(const float4*)(vr + 8 * t4);
           acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.x, st[4 * t4 + 0], acc[b], 0, 0, 0);
           acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.y, st[4 * t4 + 1], acc[b], 0, 0, 0);
           acc[b] = __builtin_amdgcn_mfma_f32_32x32x2f32(vv.z, st[4 * t4 + 2], acc[b], 0, 0, 0);
@@ -882,38 +963,45 @@ extern "C" int hal_attention_simple_ruled(const void* q, int q_row_stride, void*
   while ((1 << cw_shift) < D / 4) ++cw_shift;
   HAL_REQUIRE((long long)n_pages * K < (1ll << 31), "hal_attention_simple: %d pages of %d heads exceed the index range", n_pages, K);
   if (rw == 32) {
-    const int chunks = (G + ROWS_MOST - 1) / ROWS_MOST, db = (D + 31) / 32;
-    const int groups = dtype == HAL_F32 && (long long)((n_tokens + tq - 1) / tq) * K * chunks <= ROWS_UNITS ? 2 : 1;
-    const size_t smem = rows_lds_floats(D, db, groups) * sizeof(float);
+    int chunks = (G + ROWS_MOST - 1) / ROWS_MOST;
+    const int db = (D + 31) / 32;
+    const long long blocks = (long long)((n_tokens + tq - 1) / tq) * K * chunks;
+    const int groups = dtype == HAL_F32 && blocks <= ROWS_UNITS ? 2 : 1;
+    // (half of the compute units without a workgroup: workgroups of half the rows)
+    const int rows = groups == 2 && blocks <= ROWS_UNITS / 2 ? ROWS_MOST / 2 : ROWS_MOST;
+    if (rows < ROWS_MOST) tq = G >= rows ? 1 : rows / G, chunks = (G + rows - 1) / rows;
+    const size_t smem = rows_lds_floats(D, db, rows, groups) * sizeof(float);
     const long long gy = (long long)K * chunks;
     HAL_REQUIRE(gy <= 65535, "hal_attention_simple: %lld head chunks exceed the grid limit", gy);
     dim3 grid((n_tokens + tq - 1) / tq, (unsigned)gy);
-#define ROWS_LAUNCH(T_, DB_, GROUPS_)                                                                   \
+#define ROWS_LAUNCH(T_, DB_, ROWS_, GROUPS_)                                                                   \
   do {                                                                                                \
     static bool raised = false; /* more than 64 KB of LDS has to be asked for, once per kernel */      \
     if (!raised && smem > 64 * 1024) {                                                                \
-      HAL_CHECK_HIP(hipFuncSetAttribute((const void*)attention_rows_kernel<T_, DB_, GROUPS_>,         \
+      HAL_CHECK_HIP(hipFuncSetAttribute((const void*)attention_rows_kernel<T_, DB_, ROWS_, GROUPS_>,  \
                                         hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));     \
       raised = true;                                                                                  \
     }                                                                                                 \
-    hipLaunchKernelGGL((attention_rows_kernel<T_, DB_, GROUPS_>), grid, dim3(ROWS_THREADS(GROUPS_)), smem, stream, \
+    hipLaunchKernelGGL((attention_rows_kernel<T_, DB_, ROWS_, GROUPS_>), grid, dim3(ROWS_THREADS(ROWS_, GROUPS_)), smem, stream, \
                        (const T_*)q, q_row_stride, (T_*)out, out_row_stride, positions, token_seg,    \
                        block_table, bt_stride, (const T_*)k_pages, (const T_*)v_pages, n_tokens, H, K, D, \
                        page_size, n_pages, scale, rule, tq, chunks, page_shift, cw_shift);            \
   } while (0)
-#define ROWS_BY_SIZE(T_, GROUPS_)                     \
-  do {                                                \
-    if (db == 1) ROWS_LAUNCH(T_, 1, GROUPS_);         \
-    else if (db == 2) ROWS_LAUNCH(T_, 2, GROUPS_);    \
-    else if (db == 3) ROWS_LAUNCH(T_, 3, GROUPS_);    \
-    else ROWS_LAUNCH(T_, 4, GROUPS_);                 \
+#define ROWS_BY_SIZE(T_, ROWS_, GROUPS_)                     \
+  do {                                                       \
+    if (db == 1) ROWS_LAUNCH(T_, 1, ROWS_, GROUPS_);         \
+    else if (db == 2) ROWS_LAUNCH(T_, 2, ROWS_, GROUPS_);    \
+    else if (db == 3) ROWS_LAUNCH(T_, 3, ROWS_, GROUPS_);    \
+    else ROWS_LAUNCH(T_, 4, ROWS_, GROUPS_);                 \
   } while (0)
-    if (dtype == HAL_F32 && groups == 2)
-      ROWS_BY_SIZE(float, 2);
+    if (dtype == HAL_F32 && rows < ROWS_MOST)
+      ROWS_BY_SIZE(float, ROWS_MOST / 2, 2);
+    else if (dtype == HAL_F32 && groups == 2)
+      ROWS_BY_SIZE(float, ROWS_MOST, 2);
     else if (dtype == HAL_F32)
-      ROWS_BY_SIZE(float, 1);
+      ROWS_BY_SIZE(float, ROWS_MOST, 1);
     else if (dtype == HAL_BF16)
-      ROWS_BY_SIZE(bf16_t, 1);
+      ROWS_BY_SIZE(bf16_t, ROWS_MOST, 1);
     else
       return hal_fail("hal_attention_simple: unknown dtype %d", dtype);
 #undef ROWS_BY_SIZE
