@@ -35,11 +35,11 @@ struct StreamArgs {
   hal_gate act;
 };
 
-// Tiles of 64 go through six buffers, one workgroup a compute unit; of 128 through three, two workgroups.
-template <int NI, int COLS, bool GATED>
+// Tiles of 64 go through six buffers, one workgroup a compute unit; of 128 through three, two workgroups, or six (`gs_deep`).
+template <int NI, int COLS, bool GATED, int BUFFERS>
 __global__ void __launch_bounds__(256)
 gemm_stream_kernel(StreamArgs a) {
-  constexpr int BUFFERS = COLS == 64 ? 6 : 3, NJ = COLS / 64, AI = NI / 2, WI = COLS / 32, LOADS = AI + WI;
+  constexpr int NJ = COLS / 64, AI = NI / 2, WI = COLS / 32, LOADS = AI + WI;
   constexpr int A_BYTES = NI * 16 * GS_K * 2, BYTES = A_BYTES + COLS * GS_K * 2, WIDE = GATED ? COLS / 2 : COLS;
   __shared__ __attribute__((aligned(16))) char b0[BYTES], b1[BYTES], b2[BYTES], b3[BUFFERS > 3 ? BYTES : 16], b4[BUFFERS > 3 ? BYTES : 16],
       b5[BUFFERS > 3 ? BYTES : 16];
@@ -178,6 +178,14 @@ static StreamCut gs_cut(int N, int K, bool gated, bool may_part) {
   return most >= GS_UNITS * 5 / 8 ? best : StreamCut{0, 0};
 }
 
+// Whether tiles of 128 go through six buffers: a compute unit has one of them then, so where there are no more tiles than units, and
+// where the longer start is made up for by the steps behind it.  Three / six buffers, us, at 48 rows: 161 tiles of K 4,096 39.7 / 37.0, 250 52.2 / 50.8,
+// gated 172 42.9 / 40.5, but gated 224 (which have the memory's rate) 49.2 / 49.5; 250 of 2,048 31.0 / 31.4; in parts 48 tiles x 5 of 4,096
+// 13.8 / 15.1, 97 x 2 25.5 / 27.2; at 17 rows 161 36.9 / 35.5, 172 42.5 / 39.8, 250 50.8 / 49.2.
+static bool gs_deep(int K, bool gated, int tiles, int parts) {
+  return parts == 1 && K >= 4096 && tiles <= (gated ? GS_UNITS * 3 / 4 : GS_UNITS);
+}
+
 // The cut above: parts of K, 0 for none (may_part: the reader adds up planes).
 extern "C" int hal_gemm_bf16_stream_parts(int N, int K, int gated, int may_part) {
   if (K % GS_K || K < 4 * GS_K || N % 4 || N < 128) return 0;
@@ -201,8 +209,12 @@ extern "C" int hal_gemm_bf16_stream(const void* X, int ldx, const void* W, const
   const int cols = gs_cut(N, K, W2 != nullptr, parts > 1).cols, tiles = ((W2 ? 2 * N : N) + cols - 1) / cols;
   const StreamArgs a = {(const bf16_t*)X, ldx, (const bf16_t*)W, (const bf16_t*)W2, ldw, Y, y_dtype == HAL_F32, M, N, K, tiles, parts,
                         {act, limit, alpha, up_shift}};
-#define GS_LAUNCH(NI_, COLS_, GATED_) \
-  hipLaunchKernelGGL((gemm_stream_kernel<NI_, COLS_, GATED_>), dim3(tiles * parts), dim3(256), 0, stream, a)
+  const bool deep = cols == 64 || gs_deep(K, W2 != nullptr, tiles, parts);
+#define GS_LAUNCH(NI_, COLS_, GATED_)                                                                                                  \
+  do {                                                                                                                                 \
+    if (deep) hipLaunchKernelGGL((gemm_stream_kernel<NI_, COLS_, GATED_, 6>), dim3(tiles * parts), dim3(256), 0, stream, a);            \
+    else hipLaunchKernelGGL((gemm_stream_kernel<NI_, COLS_, GATED_, COLS_ == 64 ? 6 : 3>), dim3(tiles * parts), dim3(256), 0, stream, a); \
+  } while (0)
 #define GS_ROWS(COLS_, GATED_)             \
   if (M <= 32) GS_LAUNCH(2, COLS_, GATED_); \
   else GS_LAUNCH(4, COLS_, GATED_)

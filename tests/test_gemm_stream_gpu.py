@@ -136,3 +136,25 @@ def test_the_rotation_adds_up_planes(gpu, H, K, D, page, tiled, off):
     for got, want in ((q, rows[:, : H * D]), (k1, k2)):
         assert torch.allclose(got.float(), want.float(), rtol=2.0**-7, atol=1e-6) and float((got != want).float().mean()) < 1e-3
     assert torch.equal(v1, v2)
+
+
+@pytest.mark.parametrize("m", [17, 48, 64])
+@pytest.mark.parametrize("n,k,gated", [(20544, 4096, False), (32001 // 4 * 4, 4160, False), (20484, 4224, False), (11008, 4096, True), (12288, 4160, True),
+                                       (12292, 4096, True), (20544, 4032, False)])
+def test_long_rows_through_six_buffers(gpu, m, n, k, gated):
+    """One workgroup a compute unit and 64 steps of K or more (4,032 and 12,292 gated: the three buffers still); steps that
+    do not fill the last turn through the buffers."""
+    x, w = rand(gpu, m, k, seed=21).bfloat16(), rand(gpu, n, k, seed=22, scale=0.05).bfloat16()
+    up = rand(gpu, n, k, seed=23, scale=0.05).bfloat16() if gated else None
+    assert ops.stream_parts(x, w, n, gated=gated) == 1
+    y = ops.gemm_bf16_stream(x, w, 1, w_up=up, out_dtype=torch.float32 if not gated else torch.bfloat16)
+    want, size = x.double() @ w.double().t(), x.double().abs() @ w.double().abs().t()
+    steps = (k / 32 + 8) * 2.0 ** -23  # a rounding of each partial sum
+    if gated:
+        u, u_size = x.double() @ up.double().t(), x.double().abs() @ up.double().abs().t()
+        s = want * torch.sigmoid(want)
+        bound = (1.1 * size * u.abs() + s.abs() * u_size) * steps + (s * u).abs() * 2.0 ** -7.9 + 1e-6
+        want = s * u
+    else:
+        bound = size * steps
+    assert bool(((y.double() - want).abs() <= bound).all())
