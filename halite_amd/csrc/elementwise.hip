@@ -587,6 +587,25 @@ __global__ void rope_append_kernel(T* __restrict__ qkv, int row_stride,
 
 // Eight elements per work item (rot a multiple of 16, or of 8 for adjacent pairs; D a
 // multiple of 8): all loads of an item are issued before its arithmetic.
+// The heads of q may come from rows of another product (`q`): `n` columns of each, which a head begins with, and zeros behind what
+// other kernels write there.  (A pass of its own took 4.6 us at 8 rows and 6.0 at 3,000; a decode step of four latent layers 1,171 -> 1,162 us.)
+template <typename T>
+struct QuerySource {
+  const T* at;  // the first head's first column of token 0, or null: the heads lie in their rows
+  int ld, head, n, zero_from, n_zero;
+};
+// the columns of a token's heads from `first` on that are taken as they are, and the zeros, 16 bytes at a time
+template <typename T>
+__device__ __forceinline__ void take_heads(const QuerySource<T>& q, T* row, size_t t, int first, int H, int D, int from, int step) {
+  constexpr int PER = 16 / sizeof(T);
+  const int copied = (q.n - first) / PER, per = copied + q.n_zero / PER;
+  for (int idx = from; idx < H * per; idx += step) {
+    const int head = idx / per, j = idx % per;
+    T* to = row + (size_t)head * D;
+    if (j < copied) *(uint4*)(to + first + j * PER) = *(const uint4*)(q.at + t * q.ld + (size_t)head * q.head + first + j * PER);
+    else *(uint4*)(to + q.zero_from + (j - copied) * PER) = make_uint4(0u, 0u, 0u, 0u);
+  }
+}
 template <typename T>
 __global__ void rope_append_vec_kernel(T* __restrict__ qkv, int row_stride,
                                        const int* __restrict__ positions,
@@ -596,7 +615,7 @@ __global__ void rope_append_vec_kernel(T* __restrict__ qkv, int row_stride,
                                        const float* __restrict__ sin_t, int table_len,
                                        T* __restrict__ k_pages, T* __restrict__ v_pages, int H,
                                        int K, int D, int rot, int interleaved, int page_size,
-                                       int n_pages, bool tiled) {
+                                       int n_pages, bool tiled, QuerySource<T> qs) {
   const int t = blockIdx.x;
   const int pos = positions[t];
   const int seg = K > 0 ? token_seg[t] : 0;
@@ -613,7 +632,9 @@ __global__ void rope_append_vec_kernel(T* __restrict__ qkv, int row_stride,
 #pragma unroll
     for (int i = 0; i < (int)(sizeof(T) / 2); ++i) vpre[i] = vr[i];
   }
-  if (rot > 0 && (pos < 0 || pos >= table_len)) return;
+  const bool turned = rot == 0 || (pos >= 0 && pos < table_len);
+  if (qs.at) take_heads(qs, row, t, turned ? rot : 0, H, D, threadIdx.x, blockDim.x);
+  if (!turned) return;
   long long page = -1;
   int off = 0;
   bool whole = false;
@@ -636,11 +657,12 @@ __global__ void rope_append_vec_kernel(T* __restrict__ qkv, int row_stride,
     for (int idx = threadIdx.x; idx < (H + K) * cph; idx += blockDim.x) {
       const int head = idx / cph, j = (idx % cph) * 8;
       T* hp = row + (size_t)head * D;
+      const T* from = qs.at && head < H ? qs.at + (size_t)t * qs.ld + (size_t)head * qs.head : hp;
       float a[2][4], b[2][4], c[2][4], sn[2][4], y0[2][4], y1[2][4];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        load4(hp + j + 4 * u, a[u]);
-        load4(hp + j + half + 4 * u, b[u]);
+        load4(from + j + 4 * u, a[u]);
+        load4(from + j + half + 4 * u, b[u]);
         load4(cp + j + 4 * u, c[u]);
         load4(sp + j + 4 * u, sn[u]);
       }
@@ -668,9 +690,10 @@ __global__ void rope_append_vec_kernel(T* __restrict__ qkv, int row_stride,
     for (int idx = threadIdx.x; idx < (H + K) * cph; idx += blockDim.x) {
       const int head = idx / cph, e0 = (idx % cph) * 8, j = e0 / 2;
       T* hp = row + (size_t)head * D;
+      const T* from = qs.at && head < H ? qs.at + (size_t)t * qs.ld + (size_t)head * qs.head : hp;
       float a[2][4], c[4], sn[4], y[2][4];
-      load4(hp + e0, a[0]);
-      load4(hp + e0 + 4, a[1]);
+      load4(from + e0, a[0]);
+      load4(from + e0 + 4, a[1]);
       load4(cp + j, c);
       load4(sp + j, sn);
 #pragma unroll
@@ -757,7 +780,7 @@ rope_append_group_kernel(T* __restrict__ qkv, int row_stride, const int* __restr
                          int bt_stride, const float* __restrict__ cos_t,
                          const float* __restrict__ sin_t, int table_len, T* __restrict__ k_pages,
                          T* __restrict__ v_pages, int n_tokens, int H, int K, int D, int rot,
-                         int interleaved, int page_size, int n_pages, bool tiled) {
+                         int interleaved, int page_size, int n_pages, bool tiled, QuerySource<T> qs) {
   __shared__ int s_pos[RG_TOKENS], s_off[RG_TOKENS];
   __shared__ int s_lead[RG_TOKENS];  // 0: the token writes its own values; 1: its run's first does; 2: it is that first
   __shared__ long long s_page[RG_TOKENS];
@@ -791,6 +814,10 @@ rope_append_group_kernel(T* __restrict__ qkv, int row_stride, const int* __restr
   }
   __syncthreads();
 
+  if (qs.at) {
+    for (int i = 0; i < n; ++i)
+      take_heads(qs, qkv + (size_t)(t0 + i) * row_stride, t0 + i, s_pos[i] < 0 ? 0 : rot, H, D, threadIdx.x, blockDim.x);
+  }
   // ---- q and k: rotate in place, k also into its page --------------------------------
   const int cph = interleaved ? rot / 8 : half / 8;  // work items of a head
   const int per_token = (H + K) * cph;
@@ -805,6 +832,7 @@ rope_append_group_kernel(T* __restrict__ qkv, int row_stride, const int* __restr
     const float* sp = sin_t + (size_t)pos * half;
     const int head = idx / cph;
     T* hp = row + (size_t)head * D;
+    const T* from = qs.at && head < H ? qs.at + (size_t)(t0 + i) * qs.ld + (size_t)head * qs.head : hp;
     T* kp = (head >= H && page >= 0) ? k_pages + ((size_t)page * K + (head - H)) * page_size * D
                                      : nullptr;
     if (!interleaved) {
@@ -812,8 +840,8 @@ rope_append_group_kernel(T* __restrict__ qkv, int row_stride, const int* __restr
       float a[2][4], b[2][4], c[2][4], sn[2][4], y0[2][4], y1[2][4];
 #pragma unroll
       for (int u = 0; u < 2; ++u) {
-        load4(hp + j + 4 * u, a[u]);
-        load4(hp + j + half + 4 * u, b[u]);
+        load4(from + j + 4 * u, a[u]);
+        load4(from + j + half + 4 * u, b[u]);
         load4(cp + j + 4 * u, c[u]);
         load4(sp + j + 4 * u, sn[u]);
       }
@@ -836,8 +864,8 @@ rope_append_group_kernel(T* __restrict__ qkv, int row_stride, const int* __restr
     } else {
       const int e0 = (idx % cph) * 8, j = e0 / 2;
       float a[2][4], c[4], sn[4], y[2][4];
-      load4(hp + e0, a[0]);
-      load4(hp + e0 + 4, a[1]);
+      load4(from + e0, a[0]);
+      load4(from + e0 + 4, a[1]);
       load4(cp + j, c);
       load4(sp + j, sn);
 #pragma unroll
@@ -1011,8 +1039,8 @@ extern "C" int hal_rope_append(void* qkv, int dtype, int row_stride, const int* 
                                const int* token_seg, const int* block_table, int bt_stride,
                                const float* cos_t, const float* sin_t, int table_len,
                                void* k_pages, void* v_pages, int n_tokens, int H, int K, int D,
-                               int rot, int interleaved, int page_size, int n_pages, int tiled,
-                               hipStream_t stream) {
+                               int rot, int interleaved, int page_size, int n_pages, int tiled, const void* q, int ldq,
+                               int q_head, int n_q, int zero_from, int n_zero, hipStream_t stream) {
   HAL_REQUIRE(n_tokens >= 0 && H >= 0 && K >= 0 && D > 0, "hal_rope_append: bad sizes");
   HAL_REQUIRE(rot >= 0 && rot <= D && rot % 2 == 0, "hal_rope_append: rotary dim %d of %d", rot, D);
   HAL_REQUIRE(row_stride >= (H + 2 * K) * D, "hal_rope_append: row stride %d < %d", row_stride,
@@ -1026,6 +1054,9 @@ extern "C" int hal_rope_append(void* qkv, int dtype, int row_stride, const int* 
               "(page %d, head %d)", page_size, D);
   const bool vec = D % 8 == 0 && row_stride % 8 == 0 && ((uintptr_t)qkv % 16) == 0 &&
                    (interleaved ? rot % 8 == 0 : rot % 16 == 0);
+  HAL_REQUIRE(!q || (vec && n_q >= rot && n_q <= D && zero_from >= n_q && n_zero >= 0 && zero_from + n_zero <= D && q_head >= n_q && ldq >= H * q_head &&
+                     !((ldq | q_head | n_q | zero_from | n_zero) % 8) && (uintptr_t)q % 16 == 0),
+              "hal_rope_append: heads of q from rows of %d, %d a head", ldq, q_head);
   // many tokens: eight to a workgroup (the values of eight tokens must fit LDS)
   const size_t group_lds = (size_t)RG_TOKENS * K * D * (dtype == HAL_F32 ? 4 : 2);
   // (measured with 32 + 8 + 8 heads of 128: the same at 1,024 tokens, 14 against 18 us at
@@ -1037,12 +1068,14 @@ extern "C" int hal_rope_append(void* qkv, int dtype, int row_stride, const int* 
       hipLaunchKernelGGL(rope_append_group_kernel<float>, grid, dim3(RG_THREADS), group_lds, stream,
                          (float*)qkv, row_stride, positions, token_seg, block_table, bt_stride,
                          cos_t, sin_t, table_len, (float*)k_pages, (float*)v_pages, n_tokens, H, K,
-                         D, rot, interleaved, page_size, n_pages, tiled != 0);
+                         D, rot, interleaved, page_size, n_pages, tiled != 0,
+                         QuerySource<float>{(const float*)q, ldq, q_head, n_q, zero_from, n_zero});
     else
       hipLaunchKernelGGL(rope_append_group_kernel<bf16_t>, grid, dim3(RG_THREADS), group_lds, stream,
                          (bf16_t*)qkv, row_stride, positions, token_seg, block_table, bt_stride,
                          cos_t, sin_t, table_len, (bf16_t*)k_pages, (bf16_t*)v_pages, n_tokens, H,
-                         K, D, rot, interleaved, page_size, n_pages, tiled != 0);
+                         K, D, rot, interleaved, page_size, n_pages, tiled != 0,
+                         QuerySource<bf16_t>{(const bf16_t*)q, ldq, q_head, n_q, zero_from, n_zero});
     HAL_LAUNCH_CHECK();
     return 0;
   }
@@ -1055,12 +1088,14 @@ extern "C" int hal_rope_append(void* qkv, int dtype, int row_stride, const int* 
       hipLaunchKernelGGL(rope_append_vec_kernel<float>, dim3(n_tokens), dim3(threads), 0, stream,
                          (float*)qkv, row_stride, positions, token_seg, block_table, bt_stride,
                          cos_t, sin_t, table_len, (float*)k_pages, (float*)v_pages, H, K, D, rot,
-                         interleaved, page_size, n_pages, tiled != 0);
+                         interleaved, page_size, n_pages, tiled != 0,
+                         QuerySource<float>{(const float*)q, ldq, q_head, n_q, zero_from, n_zero});
     else
       hipLaunchKernelGGL(rope_append_vec_kernel<bf16_t>, dim3(n_tokens), dim3(threads), 0, stream,
                          (bf16_t*)qkv, row_stride, positions, token_seg, block_table, bt_stride,
                          cos_t, sin_t, table_len, (bf16_t*)k_pages, (bf16_t*)v_pages, H, K, D,
-                         rot, interleaved, page_size, n_pages, tiled != 0);
+                         rot, interleaved, page_size, n_pages, tiled != 0,
+                         QuerySource<bf16_t>{(const bf16_t*)q, ldq, q_head, n_q, zero_from, n_zero});
     HAL_LAUNCH_CHECK();
     return 0;
   }

@@ -41,7 +41,8 @@ int hal_rope_append(void* qkv, int dtype, int row_stride, const int* positions,
                     const int* token_seg, const int* block_table, int bt_stride,
                     const float* cos_t, const float* sin_t, int table_len, void* k_pages,
                     void* v_pages, int n_tokens, int H, int K, int D, int rot, int interleaved,
-                    int page_size, int n_pages, int tiled, hipStream_t stream);
+                    int page_size, int n_pages, int tiled, const void* q, int ldq,
+                    int q_head, int n_q, int zero_from, int n_zero, hipStream_t stream);
 
 // `max_kv_len`: no request of the step has more keys (an upper bound will do); `min_q_len`:
 // none has fewer tokens in the step (a lower bound will do, 1 if not known).  They decide how

@@ -336,6 +336,19 @@ def silu_mul(gate_up: torch.Tensor):
     return gate_mul(gate_up)
 
 
+@dataclass(frozen=True)
+class QueryColumns:
+    """The first ``n`` columns of q's heads: columns ``h * head + col`` on of the rows ``x``; a head's ``n_zero`` columns from
+    ``zero_from`` on are zeros."""
+
+    x: torch.Tensor
+    head: int
+    col: int
+    n: int
+    zero_from: int = 0
+    n_zero: int = 0
+
+
 def rope_append(
     qkv: torch.Tensor,
     positions: torch.Tensor,
@@ -352,11 +365,26 @@ def rope_append(
     v_pages: torch.Tensor | None = None,
     page_size: int = 0,
     tiled: bool = False,
+    queries: QueryColumns | None = None,
 ):
     """Rotate q and k in place in the packed rows ``[q | k | v]`` and append k and
     v to the pages (``n_kv_heads == 0``: rows hold q only, nothing is appended);
-    ``tiled`` says that the pages are kept in the matrix-core kernel's own order."""
+    ``tiled`` says that the pages are kept in the matrix-core kernel's own order.  ``queries``: where the first
+    columns of q's heads lie before (they are brought into the rows first)."""
     lib = library.core_library()
+    source = (None, 0, 0, 0, 0, 0)
+    if queries is not None:
+        c = queries
+        per = 8  # columns that the kernel takes at a time
+        whole = (c.x.shape[1] | c.head | c.col | c.n | c.zero_from | c.n_zero | head_dim | qkv.shape[1]) % per == 0
+        if not (whole and c.x.data_ptr() % 16 == 0 and qkv.data_ptr() % 16 == 0 and rotary_dim <= c.n
+                and rotary_dim % (8 if interleaved else 16) == 0 and c.zero_from >= c.n):
+            head_cols(c.x, c.head, c.col, qkv, head_dim, 0, c.n, n_heads, zero_from=c.zero_from, n_zero=c.n_zero)
+        else:
+            _dev(c.x)
+            _need(c.x.dtype == qkv.dtype and c.x.dim() == 2 and c.x.shape[0] == qkv.shape[0] and c.x.shape[1] >= n_heads * c.head
+                  and c.col >= 0 and c.col + c.n <= c.head and c.zero_from + c.n_zero <= head_dim, "rope_append: columns of q")
+            source = (ctypes.c_void_p(c.x.data_ptr() + c.col * c.x.element_size()), c.x.shape[1], c.head, c.n, c.zero_from, c.n_zero)
     _dev(qkv, positions, cos, sin, token_seg, block_table, k_pages, v_pages)
     _i32(positions, "positions"), _i32(token_seg, "token_seg"), _i32(block_table, "block_table")
     n = qkv.shape[0]
@@ -381,7 +409,7 @@ def rope_append(
             _ptr(block_table), 0 if block_table is None else block_table.shape[1],
             _ptr(cos), _ptr(sin), cos.shape[0], _ptr(k_pages), _ptr(v_pages),
             n, n_heads, n_kv_heads, head_dim, rotary_dim, 1 if interleaved else 0,
-            page_size, n_pages, 1 if tiled else 0, _stream(),
+            page_size, n_pages, 1 if tiled else 0, *source, _stream(),
         ),
     )
 

@@ -165,8 +165,6 @@ class LatentAttention(Mixer):
                              p.eps, packed, h * D)
         q = ops.linear(cq, self.w_uq, tiled=self.t_uq)
         ops.grouped_gemm(q, self.w_ukt, packed, n_rows=n, x_group_cols=qh, y_group_cols=D, y_col0=p.rope_dim)
-        ops.head_cols(q, qh, p.nope_dim, packed, D, 0, p.rope_dim, h,
-                      zero_from=p.rope_dim + p.kv_rank, n_zero=D - p.rope_dim - p.kv_rank)
         if self.position is not None:
             cos, sin = self.position.tables(ctx.max_position + 1)
             rot = self.position.rotary_dim
@@ -178,6 +176,7 @@ class LatentAttention(Mixer):
             self.position.interleaved if self.position is not None else False,
             token_seg=ctx.token_seg, block_table=group.block_table,
             k_pages=kv.k, v_pages=kv.v, page_size=group.page_size, tiled=kv.tiled,
+            queries=ops.QueryColumns(q, qh, p.nope_dim, p.rope_dim, p.rope_dim + p.kv_rank, D - p.rope_dim - p.kv_rank),
         )
         latent = ctx.attention(packed, packed.shape[1], kv, group, h, p.scale, p.window or 0, rule=self.rule)
         heads = torch.empty((n, h * p.v_dim), dtype=x.dtype, device=x.device)
