@@ -8,7 +8,7 @@ import torch
 
 from halite_amd.kernels import ops
 from halite_amd.sampling import SamplingParams
-from halite_amd.sampling.sampler import _integers, array
+from halite_amd.sampling.sampler import Sampler, _integers, array
 
 
 def by_numpy(params, seeds, draws, vocab):
@@ -47,3 +47,30 @@ def test_other_numbers_than_integers():
     assert _integers([10**30, 5], 7).tolist() == [7, 5]
     with pytest.raises(OverflowError):
         _integers([10**30])
+
+
+@pytest.mark.parametrize("bad", [2**63, 2**63 + 5, -(2**63) - 1, 2**64])
+def test_seeds_out_of_range_are_refused(bad):
+    """Rounded or wrapped, two of them could become one."""
+    for values in ([bad], [bad, 1], [1, bad], [bad, -1]):
+        with pytest.raises(OverflowError):
+            _integers(values)
+
+
+@pytest.mark.parametrize("bad", [2**31, -(2**31) - 1, 2**32 + 3, 2**63])
+def test_draws_out_of_range_are_refused(bad):
+    with pytest.raises(OverflowError):
+        _integers([0, bad], code="i")
+    assert _integers([0, 2**31 - 1, np.int64(7), 2.0], code="i").tolist() == [0, 2**31 - 1, 7, 2]
+
+
+def test_sampler_refuses_them():
+    if not torch.cuda.is_available():
+        sampler = Sampler("cpu")
+        sampler._stage = lambda words: torch.empty(words, dtype=torch.int32)  # (no pinned memory without a GPU)
+    else:
+        sampler = Sampler("cuda:0")
+    logits = torch.zeros((2, 5), device=sampler.device)
+    for seeds, draws in (([2**63 + 5, 1], [0, 0]), ([1, 2], [0, 2**31])):
+        with pytest.raises(OverflowError):
+            sampler.forward(logits, [SamplingParams(), SamplingParams()], seeds, draws)
