@@ -11,6 +11,7 @@ from __future__ import annotations
 import ctypes
 import functools
 import math
+from array import array
 from dataclasses import dataclass
 
 import torch
@@ -694,8 +695,11 @@ SAMPLE_ALL_GREEDY, SAMPLE_UNFILTERED = 1, 2  # (and 4: some row has top-k, top-p
 def pack_sample_rows(host: torch.Tensor, temperature, top_p, min_p, top_k, seeds, draw_index, vocab: int) -> int:
     """The parameters of a step's rows (``array``s of doubles and of 64-bit integers) into the int32 buffer ``host`` of seven
     words a row; returns what ``sample_packed`` takes as ``flags``."""
+    rows = (temperature, top_p, min_p, top_k, seeds, draw_index)
+    _need(all(isinstance(a, array) and a.typecode == c and len(a) == len(seeds) for a, c in zip(rows, "dddqqq")),
+          "sample: arrays of one length, three of doubles and three of 64-bit integers")
     _need(host.dtype == torch.int32 and not host.is_cuda and host.is_contiguous() and host.numel() >= 7 * len(seeds), "sample: room for the rows")
-    at = [ctypes.c_void_p(a.buffer_info()[0]) for a in (temperature, top_p, min_p, top_k, seeds, draw_index)]
+    at = [ctypes.c_void_p(a.buffer_info()[0]) for a in rows]
     return library.core_library().hal_sample_pack(*at, len(seeds), vocab, _ptr(host))
 
 

@@ -74,3 +74,16 @@ def test_sampler_refuses_them():
     for seeds, draws in (([2**63 + 5, 1], [0, 0]), ([1, 2], [0, 2**31])):
         with pytest.raises(OverflowError):
             sampler.forward(logits, [SamplingParams(), SamplingParams()], seeds, draws)
+
+
+def test_arrays_of_other_lengths_and_types_are_refused():
+    """Six entries each are read from them."""
+    good = [array("d", [0.5] * 6)] * 3 + [array("q", [1] * 6)] * 3
+    host = torch.empty(42, dtype=torch.int32)
+    ops.pack_sample_rows(host, *good, 50)
+    for i in range(6):
+        for bad in (good[i][:5], good[i][:0], array("f" if i < 3 else "i", [1] * 6), array("q" if i < 3 else "d", [1] * 6), [1] * 6):
+            with pytest.raises(ops.KernelError):
+                ops.pack_sample_rows(host, *good[:i], bad, *good[i + 1 :], 50)
+    with pytest.raises(ops.KernelError):
+        ops.pack_sample_rows(host[:41], *good, 50)
