@@ -632,14 +632,15 @@ def sample(
     spread: bool = False,
     late: bool = True,
 ):
-    """Next token and log-probability of every row of float32 ``logits``.
+    """Next token and log-probability of every row of float32 ``logits`` by parameters that lie on the GPU.
     ``all_greedy`` promises that no row samples (``temperature`` 0 or ``top_k`` 1 in
     every row), ``unfiltered`` that every row is greedy or draws from its whole
     distribution (no top-k, top-p or min-p): the rows are then spread over many blocks,
     in two launches.  ``spread``: every pass over a row is shared by 32 blocks (six
     launches; two more unless ``late`` is false, which promises that no row has top-k,
-    top-p and min-p all at once).  Otherwise, with
-    ``key_scratch``, the kernel gets room for one 32-bit key per logit, which its passes
+    top-p and min-p all at once).  All three go through ``sample_packed``, which is what the engine's sampler calls.
+    Otherwise a row is one block's, which selects by the bits of its keys (what the others are compared
+    with); with ``key_scratch`` the kernel gets room for one 32-bit key per logit, which its passes
     over a row read instead of deriving it again."""
     lib = library.core_library()
     _dev(logits, temperature, top_k, top_p, min_p, seeds, draw_index)
@@ -650,35 +651,13 @@ def sample(
     _need(seeds.dtype == torch.int64, "sample: seeds are int64")
     for t in (temperature, top_k, top_p, min_p, seeds, draw_index):
         _need(t.numel() == n, "sample: one parameter per row")
-    # one buffer for both results, so that the host can fetch them with one copy
-    both = torch.empty(2 * n, dtype=torch.int32, device=logits.device)
-    tokens, logprobs = both[:n], both[n:].view(torch.float32)
-    if all_greedy and logits.is_contiguous():  # every row spread over many blocks
-        parts = torch.empty((n, 32, 4), dtype=torch.float32, device=logits.device)
-        _check(lib, lib.hal_sample_greedy(_ptr(logits), vocab, n, vocab, _ptr(parts), _ptr(tokens), _ptr(logprobs), _stream()))
-        return tokens, logprobs
-    if unfiltered and logits.is_contiguous():
-        parts = torch.empty((n, 32, 4), dtype=torch.float32, device=logits.device)
-        _check(lib, lib.hal_sample_unfiltered(
-            _ptr(logits), vocab, n, vocab, _ptr(temperature), _ptr(top_k), _ptr(seeds), _ptr(draw_index),
-            _ptr(parts), _ptr(tokens), _ptr(logprobs), _stream()))
-        return tokens, logprobs
-    if spread and logits.is_contiguous():
-        # a row's list has room for all of its logits (they may all be alike), so many rows go in turns over one room
-        at_once = min(n, max(1, SAMPLE_LIST_WORDS // vocab))
-        # (one buffer: histograms and the rows' state first, which are 64-bit words)
-        words = [at_once * 2 * 256 * 2, at_once * 6, at_once * 32 * 4, at_once * 32, at_once * vocab]
-        room = torch.empty(sum(words), dtype=torch.int32, device=logits.device)
-        hist, state, parts, kept, lists = (ctypes.c_void_p(room.data_ptr() + 4 * sum(words[:i])) for i in range(5))
-        for r in range(0, n, at_once):
-            def row(t, width=1):
-                return ctypes.c_void_p(t.data_ptr() + r * width * t.element_size())
-
-            _check(lib, lib.hal_sample_spread(
-                row(logits, vocab), vocab, min(at_once, n - r), vocab, row(temperature), row(top_k), row(top_p), row(min_p),
-                row(seeds), row(draw_index), parts, kept, state, hist, lists, 1 if late else 0, row(tokens), row(logprobs), _stream()))
-        return tokens, logprobs
-    keys = torch.empty((n, vocab), dtype=torch.int32, device=logits.device) if key_scratch and not all_greedy else None
+    if all_greedy or unfiltered or spread:
+        flags = (SAMPLE_ALL_GREEDY if all_greedy else 0) | (SAMPLE_UNFILTERED if unfiltered else 0) | (SAMPLE_LATE if late else 0)
+        packed = torch.cat([t.reshape(-1).view(torch.int32) for t in (seeds, temperature, top_p, min_p, top_k, draw_index)])
+        return sample_packed(logits, packed, flags)
+    tokens = torch.empty(n, dtype=torch.int32, device=logits.device)
+    logprobs = torch.empty(n, dtype=torch.float32, device=logits.device)
+    keys = torch.empty((n, vocab), dtype=torch.int32, device=logits.device) if key_scratch else None
     _check(
         lib,
         lib.hal_sample(
@@ -689,7 +668,7 @@ def sample(
     return tokens, logprobs
 
 
-SAMPLE_ALL_GREEDY, SAMPLE_UNFILTERED = 1, 2  # (and 4: some row has top-k, top-p and min-p all at once)
+SAMPLE_ALL_GREEDY, SAMPLE_UNFILTERED, SAMPLE_LATE = 1, 2, 4  # (the last: some row has top-k, top-p and min-p all at once)
 
 
 def pack_sample_rows(host: torch.Tensor, temperature, top_p, min_p, top_k, seeds, draw_index, vocab: int) -> int:
@@ -712,10 +691,10 @@ def sample_packed(logits: torch.Tensor, packed: torch.Tensor, flags: int):
     _need(logits.dtype == torch.float32, "sample: logits are float32")
     _need(packed.dtype == torch.int32 and packed.numel() == 7 * n, "sample: parameters of every row")
     if flags & (SAMPLE_ALL_GREEDY | SAMPLE_UNFILTERED):
-        at_once, words = n, n * 128
+        at_once, words = max(n, 1), n * 128
     else:
         # a row's list has room for all of its logits (they may all be alike), so many rows go in turns over one room
-        at_once = min(n, max(1, SAMPLE_LIST_WORDS // vocab))
+        at_once = max(1, min(n, SAMPLE_LIST_WORDS // vocab))
         words = at_once * (2 * 256 * 2 + 6 + 32 * 4 + 32 + vocab)
     room = torch.empty(words, dtype=torch.int32, device=logits.device)
     # one buffer for both results, so that the host can fetch them with one copy

@@ -59,6 +59,40 @@ def test_rows_in_turns(monkeypatch, rows_at_once):
     assert torch.equal(tok, tok2) and torch.equal(lp, lp2)
 
 
+@pytest.mark.parametrize("kind", ["greedy", "whole", "filtered", "late at the end"])
+@pytest.mark.parametrize("n, rows_at_once", [(1, 1), (20, 1), (20, 7), (21, 7), (22, 7), (23, 64)])
+def test_as_the_engine_samples(monkeypatch, kind, n, rows_at_once):
+    """The sampler with its requests' own parameters, rows in turns over one room, a cut last turn, the only row with all
+    three filters in it: the tokens of the one-block kernel."""
+    from halite_amd.sampling import SamplingParams
+    from halite_amd.sampling.sampler import Sampler
+
+    vocab, rng = 5000, random.Random(n + rows_at_once)
+    x = (torch.randn((n, vocab), generator=torch.Generator().manual_seed(n)) * 2).cuda()
+    pick = {"greedy": dict(temperature=[0.0, 0.7], top_k=[1]), "whole": dict(temperature=[0.0, 0.3, 1.0, 2.0]),
+            "filtered": dict(temperature=[0.0, 0.7, 1.0], top_k=[-1, 1, 40, 6000], top_p=[0.3, 0.9, 1.0]),
+            "late at the end": dict(temperature=[0.7, 1.0], top_k=[-1, 40], min_p=[0.0, 0.05])}[kind]
+    params = [SamplingParams(**{k: rng.choice(v) for k, v in pick.items()}) for _ in range(n)]
+    if kind == "late at the end":
+        params[-1] = SamplingParams(temperature=0.9, top_k=30, top_p=0.8, min_p=0.01)
+    seeds, draws = [rng.getrandbits(62) for _ in range(n)], [rng.randrange(1000) for _ in range(n)]
+    f = lambda v, dt=torch.float32: torch.tensor(v, dtype=dt, device="cuda")  # noqa: E731
+    want = ops.sample(x, f([p.temperature for p in params]), f([p.top_k for p in params], torch.int32), f([p.top_p for p in params]),
+                      f([p.min_p for p in params]), f(seeds, torch.int64), f(draws, torch.int32))
+    monkeypatch.setattr(ops, "SAMPLE_LIST_WORDS", rows_at_once * vocab + 1)
+    sampler = Sampler("cuda:0")
+    for _ in range(2):  # (the second time over a staging buffer of its own)
+        agree([[t.cpu() for t in want], [t.cpu() for t in sampler.forward(x, params, seeds, draws)]], n)
+    assert sampler.forward(x[:0], [], [], [])[0].numel() == 0
+
+
+def test_no_rows():
+    x = torch.zeros((0, 50), device="cuda")
+    for flags in range(8):
+        tok, lp = ops.sample_packed(x, torch.zeros(0, dtype=torch.int32, device="cuda"), flags)
+        assert tok.numel() == lp.numel() == 0
+
+
 def test_room_for_many_rows():
     """What a step holds beside its logits does not grow with them: 256 MiB of lists, and 5 KiB a row of the rows in turn."""
     n, vocab = 1100, 100000
