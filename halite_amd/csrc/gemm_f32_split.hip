@@ -5,11 +5,15 @@
 // most 2^-25 of the product, half of what its own rounding to float32 takes, and of either sign.  (Of numbers below 2^-102
 // the parts that fall below 2^-126, where float32's own numbers begin to lose bits, may be lost.)
 //
-// The instruction cuts its sums off where a float32 addition rounds, so how often a sum of full size goes through it decides
-// the error: each stage of 32 k starts from nothing, its five small products first, and is added to the total by a
-// float32 addition.  Distance to 64 bits, N(0, 1) times N(0, 0.02), K = 4,096 / 14,336, over the result's norm: 1.4e-7 / 2.4e-7 for a matrix
-// whose K is cut in four, 2.2e-7 / 4.1e-7 in one; the float32 instruction's tiles (gemm_f32.hip): 4.1e-7 / 4.2e-7.
-// (One sum of all six products over 64 stages: 7e-7, over all of 14,336: 1.9e-6.)
+// The instruction cuts its sums off where a float32 addition rounds, and a float32 addition to a long sum loses more than one
+// to a short one, so how often a sum of full size goes through either decides the error.  Two stages of 32 k at a time start from
+// nothing, each with its five small products first, and are added to the total by a float32 addition; a total takes 128 stages
+// at most (SP_WALK), the next one is added to it where it lies in memory.  Distance to 64 bits over the result's norm, for
+// K = 4,096 in four parts / two / one, 14,336 in four, 8,192 in one: N(0, 1) times N(0, 0.02) 1.4e-7 / 1.5e-7 / 1.8e-7, 2.0e-7, 1.9e-7;
+// the same without signs, where every sum is of full size, 0.5e-7 / 0.7e-7 / 1.2e-7, 0.7e-7, 0.9e-7.  The float32 instruction's tiles
+// (gemm_f32.hip) 4.1e-7, 4.2e-7, 4.1e-7 and 1.25e-7, 1.04e-7, 1.02e-7; its kernel for up to 128 rows 5.7e-7 (K = 4,096), 1.1e-6 (14,336) and
+// 2.4e-7, 4.6e-7.  (A total from each stage: 2.2e-7 and 1.65e-7 in one part of 4,096, and without walks 2.3e-7 for 8,192 without signs;
+// one sum of all six products over 64 stages: 7e-7, over all of 14,336: 1.9e-6.)
 //
 // What bounds it: the instruction at the clock that the chip holds under it (1,340 TFLOP/s of bf16 products, the
 // library's largest bf16 products reach 1,555), given that nothing else stands in the way.  So
@@ -22,8 +26,8 @@
 //    beside them: left to the compiler, conversions stood in front of a stage's products (686 us), or registers spilled;
 //  - one barrier a stage, before its last product: by then the next stage lies in LDS, and its first operands are read beside
 //    that product.
-// Measured beside the float32 instruction's tiles, 500 rows, us: x 28,672 x 4,096 990 -> 609; 32,000 x 4,096 1,095 -> 660; 4,096 x 14,336
-// 500 -> 298; 6,144 x 4,096 207 -> 160; 4,096 x 4,096 142 -> 104; 2,048 rows x 28,672 x 4,096 3,600 -> 2,230 (216 TFLOP/s).
+// Measured beside the float32 instruction's tiles, 500 rows, us: x 28,672 x 4,096 990 -> 602; 32,000 x 4,096 1,095 -> 629; 4,096 x 14,336
+// 500 -> 294; 6,144 x 4,096 207 -> 154; 4,096 x 4,096 142 -> 98; 2,048 rows x 28,672 x 4,096 3,600 -> 2,226 (216 TFLOP/s).
 //
 // A matrix of few columns fills the chip by its K, cut into parts whose sums go to planes that one more kernel adds up in order.  How many
 // depends on the matrix alone, so that a row's result is its own, whatever rows are beside it.
@@ -37,6 +41,7 @@
 #define SP_XCDS 8     // dies of the gfx950 parts that this library is built for (a wrong count costs cache hits only)
 #define SP_UNITS 256  // compute units of the same
 #define SP_MOST_PARTS 8
+#define SP_WALK 128   // most stages whose sums go into one total
 #define SP_PLANES (64ll << 20)  // bytes of planes up to which all rows go at once
 #define SP_ROW_LIMIT (1 << 22)  // numbers of a row: 256 of them lie within 32-bit offsets
 
@@ -67,7 +72,8 @@ struct SplitArgs {
   long long plane;  // numbers from one part's results to the next one's
 };
 
-template <int BM>
+// WALKS: for parts of more than SP_WALK stages.
+template <int BM, bool WALKS>
 __global__ void __launch_bounds__(SP_THREADS, BM == 64 ? 4 : 2)
 gemm_f32_split_kernel(SplitArgs g) {
   constexpr int WM = BM / 64, WN = 8 / WM, NI = 4, NJ = SP_BN / 16 / WN;  // WM x WN waves of NI x NJ results of 16 x 16
@@ -79,8 +85,8 @@ gemm_f32_split_kernel(SplitArgs g) {
   const int id = die * (n_tiles / SP_XCDS) + min(die, rest) + blockIdx.x / SP_XCDS;
   const int m0 = (id % g.tiles_m) * BM, n0 = (id / g.tiles_m % g.tiles_n) * SP_BN, part = id / g.tiles_m / g.tiles_n;
   const int rows_here = min(BM, g.M - m0), cols_here = min(SP_BN, g.N - n0);
-  const int all = (g.K + SP_BK - 1) / SP_BK, first = (int)((long long)all * part / g.parts);
-  const int stages = (int)((long long)all * (part + 1) / g.parts) - first, k_end = min(g.K, (first + stages) * SP_BK);
+  const int all = (g.K + SP_BK - 1) / SP_BK, part_first = (int)((long long)all * part / g.parts);
+  const int part_stages = (int)((long long)all * (part + 1) / g.parts) - part_first, walks = WALKS ? (part_stages + SP_WALK - 1) / SP_WALK : 1;
   const uint32_t a_bytes = ((uint32_t)(rows_here - 1) * g.lda + g.K) * 4, w_bytes = ((uint32_t)(cols_here - 1) * g.ldw + g.K) * 4;
   const hal_memory a_all = hal_memory_at(g.A + (size_t)m0 * g.lda, a_bytes), w_all = hal_memory_at(g.W + (size_t)n0 * g.ldw, w_bytes);
   uint32_t minus[2] = {0x0000bf80u, 0xbf800000u};
@@ -92,6 +98,7 @@ gemm_f32_split_kernel(SplitArgs g) {
   // (rows past the end begin past the operands' bytes and are read as zeros)
   const uint32_t a_from = ((uint32_t)(wave * 8 + lr) * g.lda + piece * 4) * 4, w_from = ((uint32_t)(wave * 8 + lr) * g.ldw + piece * 4) * 4;
   sp_f32x4 p[LOADS];
+  int first = 0, k_end = 0;  // the walk's first stage, and where its numbers end
   auto ask = [&](int stage, int i) {
     const int k = (first + stage) * SP_BK;
     const bool in = k + piece * 4 < k_end;  // (K is a multiple of 4; what lies past the end is read as zeros)
@@ -109,10 +116,6 @@ gemm_f32_split_kernel(SplitArgs g) {
   const int wm = wave / WN, wn = wave % WN;
   int get_a = wm * NI * 1024 + sp_slot(lane / 16, lane % 16), get_w = W_AT + wn * NJ * 1024 + sp_slot(lane / 16, lane % 16);
   sp_f32x4 acc[NI][NJ], total[NI][NJ];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) total[i][j] = sp_f32x4{0.f, 0.f, 0.f, 0.f};
   auto of_a = [&](int k, int i) { return *(const sp_bf16x8*)(lds + get_a + k * A_PLANE + i * 1024); };
   auto of_w = [&](int k, int j) { return *(const sp_bf16x8*)(lds + get_w + k * W_PLANE + j * 1024); };
   auto meet = [&]() {
@@ -123,8 +126,8 @@ gemm_f32_split_kernel(SplitArgs g) {
   sp_bf16x8 a_hi[NI], a_mid[NI], a_lo[NI], w_even[NJ], w_odd[NJ], w_mid[NJ], w_lo[NJ];
   // The last of stage s's six products (w_hi: W's high parts), and the first five of the stage after it, which lies in
   // `mine` (its own: w_next), in groups of NJ instructions; beside them the stage after that goes from registers to
-  // `next`, and one more is asked for.
-  auto turn = [&](int s, int to_mine, sp_bf16x8 (&w_hi)[NJ], sp_bf16x8 (&w_next)[NJ]) {
+  // `next`, and one more is asked for.  `fresh`: the sums so far go to the totals, and new ones begin.
+  auto turn = [&](int s, int to_mine, sp_bf16x8 (&w_hi)[NJ], sp_bf16x8 (&w_next)[NJ], const bool fresh) {
     // (one register each, whichever buffer it is: the compiler would keep both)
     get_a += to_mine, get_w += to_mine, put_at -= to_mine;
     asm volatile("" : "+v"(get_a), "+v"(get_w), "+v"(put_at));
@@ -145,7 +148,8 @@ gemm_f32_split_kernel(SplitArgs g) {
         if (t == 1) {
           a_mid[i] = of_a(1, i);
 #pragma unroll
-          for (int j = 0; j < NJ; ++j) total[i][j] += acc[i][j];
+          for (int j = 0; j < NJ; ++j)
+            if (fresh) total[i][j] += acc[i][j];
         }
         if (t == 2 && i < NJ) w_mid[i] = of_w(1, i);
         if (t == 3) a_hi[i] = of_a(0, i);
@@ -154,48 +158,64 @@ gemm_f32_split_kernel(SplitArgs g) {
         for (int j = 0; j < NJ; ++j) {
           const sp_bf16x8 w = t == 0 ? w_hi[j] : t < 3 ? w_next[j] : t < 5 ? w_mid[j] : w_lo[j];
           const sp_bf16x8 a = t == 1 ? a_lo[i] : t == 2 || t == 3 ? a_mid[i] : a_hi[i];
-          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, t == 1 ? sp_f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w, a, t == 1 && fresh ? sp_f32x4{0.f, 0.f, 0.f, 0.f} : acc[i][j], 0, 0, 0);
         }
         __builtin_amdgcn_sched_barrier(0);
       }
     meet();
   };
-  // (the stage before the first one: zeros)
-#pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    a_hi[i] = sp_bf16x8{};
-#pragma unroll
-    for (int j = 0; j < NJ; ++j) acc[i][j] = sp_f32x4{0.f, 0.f, 0.f, 0.f};
-  }
-#pragma unroll
-  for (int j = 0; j < NJ; ++j) w_odd[j] = sp_bf16x8{};
-#pragma unroll
-  for (int i = 0; i < LOADS; ++i) ask(0, i);
-#pragma unroll
-  for (int i = 0; i < LOADS; ++i) put(i), ask(1, i);
-  meet();
-  get_a += BYTES, get_w += BYTES;
-  for (int s = 0; s <= stages; s += 2) {  // (stages past the end are zeros; left in the middle, the loop would need more registers)
-    turn(s - 1, -BYTES, w_odd, w_even);
-    turn(s, BYTES, w_even, w_odd);
-  }
   float* C = g.C + part * g.plane;
   const bool vectors = g.ldc % 4 == 0 && (uintptr_t)C % 16 == 0;
   bool odd = false;
+  get_a += BYTES, get_w += BYTES;
+  for (int walk = 0; walk < walks; ++walk) {
+    first = part_first + part_stages * walk / walks;
+    const int stages = part_first + part_stages * (walk + 1) / walks - first;
+    k_end = min(g.K, (first + stages) * SP_BK);
+    // (the stage before the first one: zeros)
 #pragma unroll
-  for (int i = 0; i < NI; ++i) {
-    const int r = (wm * NI + i) * 16 + lane % 16;
-    if (r >= rows_here) continue;
+    for (int i = 0; i < NI; ++i) {
+      a_hi[i] = sp_bf16x8{};
 #pragma unroll
-    for (int j = 0; j < NJ; ++j) {
-      const int c = (wn * NJ + j) * 16 + lane / 16 * 4;
-      float* at = C + (size_t)(m0 + r) * g.ldc + n0 + c;
-      if (vectors && c + 3 < cols_here) *(sp_f32x4*)at = total[i][j];
+      for (int j = 0; j < NJ; ++j) acc[i][j] = total[i][j] = sp_f32x4{0.f, 0.f, 0.f, 0.f};
+    }
 #pragma unroll
-      for (int v = 0; v < 4; ++v) {
-        if (c + v >= cols_here) continue;
-        if (!(vectors && c + 3 < cols_here)) at[v] = total[i][j][v];
-        odd |= !(fabsf(total[i][j][v]) <= 3.4028235e38f);
+    for (int j = 0; j < NJ; ++j) w_odd[j] = sp_bf16x8{};
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) ask(0, i);
+#pragma unroll
+    for (int i = 0; i < LOADS; ++i) put(i), ask(1, i);
+    meet();
+    for (int s = 0; s < stages; s += 2) {  // (stages past the end are zeros; left in the middle, the loop would need more registers)
+      turn(s - 1, -BYTES, w_odd, w_even, true);
+      turn(s, BYTES, w_even, w_odd, false);
+    }
+    // (the last product of the last stage)
+#pragma unroll
+    for (int i = 0; i < NI; ++i)
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w_odd[j], a_hi[i], acc[i][j], 0, 0, 0);
+    int l = lane;
+    asm volatile("" : "+v"(l));  // (or where the results lie would be kept in registers over the walk)
+#pragma unroll
+    for (int i = 0; i < NI; ++i) {
+      const int r = (wm * NI + i) * 16 + l % 16;
+      if (r >= rows_here) continue;
+#pragma unroll
+      for (int j = 0; j < NJ; ++j) {
+        const int c = (wn * NJ + j) * 16 + l / 16 * 4;
+        float* at = C + (size_t)(m0 + r) * g.ldc + n0 + c;
+        sp_f32x4 sum = total[i][j] + acc[i][j];
+        if (vectors && c + 3 < cols_here) {
+          if (walk) sum += *(const sp_f32x4*)at;
+          *(sp_f32x4*)at = sum;
+        }
+#pragma unroll
+        for (int v = 0; v < 4; ++v) {
+          if (c + v >= cols_here) continue;
+          if (!(vectors && c + 3 < cols_here)) at[v] = sum[v] += walk ? at[v] : 0.f;
+          odd |= !(fabsf(sum[v]) <= 3.4028235e38f);
+        }
       }
     }
   }
@@ -203,7 +223,8 @@ gemm_f32_split_kernel(SplitArgs g) {
   // Infinities and NaN among the operands, and numbers that round to a bf16 infinity, have no parts: every result that is not
   // finite (they all are not then) is taken again as a float32 sum, by the whole wave.
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
-  const int k_begin = first * SP_BK;
+  const int k_begin = part_first * SP_BK;
+  k_end = min(g.K, (part_first + part_stages) * SP_BK);
   for (int r = wm * 64; r < min(rows_here, wm * 64 + 64); ++r) {
     const float* a = g.A + (size_t)(m0 + r) * g.lda;
     const int c = wn * NJ * 16 + lane;
@@ -294,15 +315,22 @@ extern "C" int hal_gemm_f32_split(const float* A, int lda, const float* W, int l
   const int parts = sp_parts(N), rows = parts == 1 ? M : sp_rows_at_once(M, N), pitch = sp_pitch(N);
   HAL_REQUIRE(parts == 1 || planes != nullptr, "hal_gemm_f32_split: no planes for %d parts", parts);
   const int tiles_n = (N + SP_BN - 1) / SP_BN;
+  const bool walks = ((K + SP_BK - 1) / SP_BK + parts - 1) / parts > SP_WALK;  // (parts differ by one stage at most)
   for (int m = 0; m < M; m += rows) {
     const int here = std::min(rows, M - m), tile = sp_tile_rows(here, N), tiles_m = (here + tile - 1) / tile;
     const long long blocks = (long long)tiles_m * tiles_n * parts, plane = (long long)here * pitch;
     HAL_REQUIRE(blocks < (1ll << 31), "hal_gemm_f32_split: M=%d N=%d exceed the grid limit", M, N);
     float* to = C + (size_t)m * ldc;
     const SplitArgs g = {A + (size_t)m * lda, W, parts > 1 ? planes : to, lda, ldw, parts > 1 ? pitch : ldc, here, N, K, tiles_m, tiles_n, parts, plane};
-    if (tile == 256) hipLaunchKernelGGL(gemm_f32_split_kernel<256>, dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);
-    else if (tile == 64) hipLaunchKernelGGL(gemm_f32_split_kernel<64>, dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);
-    else hipLaunchKernelGGL(gemm_f32_split_kernel<128>, dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);
+#define SP_LAUNCH(BM_)                                                                                                               \
+  do {                                                                                                                               \
+    if (walks) hipLaunchKernelGGL((gemm_f32_split_kernel<BM_, true>), dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);         \
+    else hipLaunchKernelGGL((gemm_f32_split_kernel<BM_, false>), dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);              \
+  } while (0)
+    if (tile == 256) SP_LAUNCH(256);
+    else if (tile == 64) SP_LAUNCH(64);
+    else SP_LAUNCH(128);
+#undef SP_LAUNCH
     if (parts > 1)
       hipLaunchKernelGGL(gemm_f32_planes_kernel, dim3((unsigned)((plane / 4 + 255) / 256)), dim3(256), 0, stream, planes, plane, pitch, to, ldc, N, parts);
     HAL_LAUNCH_CHECK();

@@ -5,8 +5,6 @@ import torch
 
 from halite_amd.kernels import library, ops
 
-pytestmark = pytest.mark.gpu
-
 
 def _operands(m, n, k):
     gen = torch.Generator().manual_seed(m + n + k)
@@ -15,6 +13,7 @@ def _operands(m, n, k):
 
 # the fewest rows, a tile of each height and one row more; one part of K to eight, of unequal lengths, an odd number of stages in
 # a part, K that ends inside a stage; columns that end inside a tile and inside a vector; rows in two turns over their planes
+@pytest.mark.gpu
 @pytest.mark.parametrize("m, n, k", [(65, 96, 2048), (128, 130, 2052), (96, 12300, 2056), (129, 4090, 2080), (257, 6147, 2116), (300, 8200, 2048),
                                      (513, 16388, 2084), (1100, 3072, 2048), (1025, 4097, 4100), (200, 1000, 14336)])
 def test_sizes(m, n, k):
@@ -33,6 +32,7 @@ def test_sizes(m, n, k):
         assert torch.equal(ops.gemm_f32(a[m - 70 :].contiguous(), w), got[m - 70 :])
 
 
+@pytest.mark.gpu
 @pytest.mark.parametrize("m, n, k", [(130, 300, 2052), (300, 8200, 2048)])
 def test_numbers_without_parts(m, n, k):
     a, w = _operands(m, n, k)
@@ -53,3 +53,29 @@ def test_numbers_without_parts(m, n, k):
     off = torch.empty(n * k + 1, device="cuda")[1:].view(n, k).copy_(w)
     assert not library.core_library().hal_gemm_f32_split_takes(ops._ptr(a), k, ops._ptr(off), k, m, k)
     assert torch.equal(ops.gemm_f32(a, off).isnan(), got.isnan())
+
+
+def _off(got, want):
+    return float((got.double() - want).norm() / want.norm())
+
+
+# (each in one part, several, several walks; the number of rows takes tiles of each height)
+EXACT_SIZES = [(65, 96, 2048), (128, 4096, 4096), (130, 16500, 4100), (300, 6144, 4096), (520, 8200, 2084), (70, 8300, 8192), (200, 8192, 14336), (80, 4096, 14336)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("kind", ["of both signs", "without signs", "beside one", "wide"])
+@pytest.mark.parametrize("m, n, k", EXACT_SIZES)
+def test_as_exact_as_the_float32_instruction(m, n, k, kind):
+    """The distance to 64 bits is no larger than that of the product in float32 multiply-adds."""
+    a, w = _operands(m, n, k)
+    if kind == "without signs":
+        a, w = a.abs(), w.abs()
+    elif kind == "beside one":
+        a, w = a + 1.0, w + 0.01
+    elif kind == "wide":
+        a = a * torch.exp(2.0 * torch.randn(a.shape, generator=torch.Generator().manual_seed(9))).cuda()
+    lib, before = library.core_library(), torch.empty((m, n), device="cuda")
+    assert lib.hal_gemm_f32(ops._ptr(a), k, ops._ptr(w), k, ops._ptr(before), n, m, n, k, ops._stream()) == 0
+    want = a.double() @ w.double().T
+    assert _off(ops.gemm_f32(a, w), want) <= _off(before, want) < 2e-6
