@@ -1,9 +1,11 @@
-// C[M, N] = A[M, K] * W[N, K]^T of float32 for prompts, on the matrix cores' bf16 instruction, as exact as float32 sums are:
-// a float32 number is the sum of three bf16 numbers (x = hi + mid + lo: hi = bf16(x), mid = bf16(x - hi), lo = x - hi - mid,
-// exactly, as 8 + 8 + 8 significant bits and two signs hold 24), a product of two bf16 numbers is exact in float32, and six
-// of the nine products of two such sums are added up in float32.  The other three, mid * lo, lo * mid and lo * lo, are at
-// most 2^-25 of the product, half of what its own rounding to float32 takes, and of either sign.  (Of numbers below 2^-102
-// the parts that fall below 2^-126, where float32's own numbers begin to lose bits, may be lost.)
+// C[M, N] = A[M, K] * W[N, K]^T of float32 for prompts, on the matrix cores' bf16 instruction, as exact as float32 sums are
+// (a published method: Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
+// Computations", 2019): a float32 number is the sum of three bf16 numbers (x = hi + mid + lo: hi = bf16(x), mid = bf16(x - hi),
+// lo = x - hi - mid, exactly, as 8 + 8 + 8 significant bits and two signs hold 24), a product of two bf16 numbers is exact in
+// float32, and six of the nine products of two such sums are added up in float32.  The other three, mid * lo, lo * mid and lo * lo, are at
+// most 2^-25 of the product, half of what its own rounding to float32 takes, and of either sign.  bf16 ends at 2^-133, float32 at 2^-149, so every number is multiplied by 2^16 (SP_SCALE) first, and a sum by
+// 2^-32 at the end: then no bit of any number is lost.  (Without: 2^-116 times N(0, 1) 2.2e-6, 2^-124 5.6e-4.)  Numbers from
+// 2^112 and sums from 2^96 on become infinities by that, and are taken again as below.
 //
 // The instruction cuts its sums off where a float32 addition rounds, and a float32 addition to a long sum loses more than one
 // to a short one, so how often a sum of full size goes through either decides the error.  Two stages of 32 k at a time start from
@@ -27,7 +29,9 @@
 //  - one barrier a stage, before its last product: by then the next stage lies in LDS, and its first operands are read beside
 //    that product.
 // Measured beside the float32 instruction's tiles, 500 rows, us: x 28,672 x 4,096 990 -> 602; 32,000 x 4,096 1,095 -> 629; 4,096 x 14,336
-// 500 -> 294; 6,144 x 4,096 207 -> 154; 4,096 x 4,096 142 -> 98; 2,048 rows x 28,672 x 4,096 3,600 -> 2,226 (216 TFLOP/s).
+// 500 -> 294; 6,144 x 4,096 207 -> 154; 4,096 x 4,096 142 -> 98; 2,048 rows x 28,672 x 4,096 3,600 -> 2,226 (216 TFLOP/s).  (The scale costs
+// two multiplications beside seven instructions a pair of numbers, 15 to 30 us of 600; the additions that every second stage spares
+// give that back.)
 //
 // A matrix of few columns fills the chip by its K, cut into parts whose sums go to planes that one more kernel adds up in order.  How many
 // depends on the matrix alone, so that a row's result is its own, whatever rows are beside it.
@@ -35,6 +39,7 @@
 #include "hal_api.h"
 #include <algorithm>
 
+#define SP_SCALE 65536.f  // 2^-149, float32's smallest number, is bf16's smallest, 2^-133, then
 #define SP_BN 128
 #define SP_BK 32  // k of a stage: a row's 128-byte line
 #define SP_THREADS 512
@@ -52,10 +57,11 @@ typedef __attribute__((ext_vector_type(4))) float sp_f32x4;
 // of its turns through LDS (see hal_turn) a quarter of it; and the 8-byte stores of four rows meet all banks.
 __device__ __forceinline__ int sp_slot(int q, int r) { return (q * 16 + (r ^ (12 * q & 15))) * 16; }
 
-// two neighbouring numbers as three words of two bf16 (minus: (-1, 0) and (0, -1) of bf16)
+// two neighbouring numbers, times the scale, as three words of two bf16 (minus: (-1, 0) and (0, -1) of bf16)
 typedef __attribute__((ext_vector_type(2))) __bf16 sp_bf16x2;
 __device__ __forceinline__ void sp_split(float a, float b, const uint32_t (&minus)[2], uint32_t& hi, uint32_t& mid, uint32_t& lo) {
   const sp_bf16x2 first = __builtin_bit_cast(sp_bf16x2, minus[0]), second = __builtin_bit_cast(sp_bf16x2, minus[1]);
+  a *= SP_SCALE, b *= SP_SCALE;
   hi = pack_bf16x2(a, b);
   const sp_bf16x2 h = __builtin_bit_cast(sp_bf16x2, hi);
   a = __builtin_amdgcn_fdot2_f32_bf16(h, first, a, false), b = __builtin_amdgcn_fdot2_f32_bf16(h, second, b, false);
@@ -205,7 +211,7 @@ gemm_f32_split_kernel(SplitArgs g) {
       for (int j = 0; j < NJ; ++j) {
         const int c = (wn * NJ + j) * 16 + l / 16 * 4;
         float* at = C + (size_t)(m0 + r) * g.ldc + n0 + c;
-        sp_f32x4 sum = total[i][j] + acc[i][j];
+        sp_f32x4 sum = (total[i][j] + acc[i][j]) * (1.f / SP_SCALE / SP_SCALE);
         if (vectors && c + 3 < cols_here) {
           if (walk) sum += *(const sp_f32x4*)at;
           *(sp_f32x4*)at = sum;
@@ -220,7 +226,7 @@ gemm_f32_split_kernel(SplitArgs g) {
     }
   }
   if (!__any(odd)) return;
-  // Infinities and NaN among the operands, and numbers that round to a bf16 infinity, have no parts: every result that is not
+  // Infinities and NaN among the operands, and numbers whose scaled parts are infinities, have no parts: every result that is not
   // finite (they all are not then) is taken again as a float32 sum, by the whole wave.
   __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "agent");
   const int k_begin = part_first * SP_BK;

@@ -577,7 +577,7 @@ def attention_simple(
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor):
     """``a @ w.T`` in float32 (``a`` [M, K], ``w`` [N, K]): float32 multiply-adds, or, for prompts, exact products
-    of three bf16 parts a number with float32 sums, whose error is no larger (``gemm_f32_split.hip``)."""
+    of three bf16 parts a number, which hold all of its bits, with float32 sums, whose error is no larger (``gemm_f32_split.hip``)."""
     lib = library.core_library()
     _dev(a, w)
     _need(a.dtype == torch.float32 and w.dtype == torch.float32, "gemm_f32 takes float32")

@@ -55,8 +55,31 @@ def test_numbers_without_parts(m, n, k):
     assert torch.equal(ops.gemm_f32(a, off).isnan(), got.isnan())
 
 
+# ---- as exact as float32 sums: what no bound on a sum's largest error can tell ----------------------------------------------
+def _by_parts(a, w, which, scale=2.0**16):
+    """The sum in 64 bits of chosen products of the parts."""
+    def parts(x):
+        out, x = [], x.double() * scale
+        for _ in range(3):
+            out.append(x.float().bfloat16().double())
+            x = x - out[-1]
+        return out
+
+    pa, pw = parts(a), parts(w)
+    return sum(pa[i] @ pw[j].T for i, j in which) / scale**2
+
+
 def _off(got, want):
     return float((got.double() - want).norm() / want.norm())
+
+
+@pytest.mark.parametrize("e_a, e_w", [(0, 0), (-125, 0), (0, -120), (-120, 100), (-100, -20)])
+def test_no_bit_of_a_small_number_is_lost(e_a, e_w):
+    """On the CPU: the parts of scaled numbers hold all bits down to float32's smallest."""
+    gen = torch.Generator().manual_seed(1)
+    a, w = torch.randn(6, 2048, generator=gen) * 2.0**e_a, torch.randn(5, 2048, generator=gen) * 2.0**e_w
+    all_nine = [(i, j) for i in range(3) for j in range(3)]
+    assert _off(_by_parts(a, w, all_nine), a.double() @ w.double().T) < 1e-15
 
 
 # (each in one part, several, several walks; the number of rows takes tiles of each height)
@@ -79,3 +102,13 @@ def test_as_exact_as_the_float32_instruction(m, n, k, kind):
     assert lib.hal_gemm_f32(ops._ptr(a), k, ops._ptr(w), k, ops._ptr(before), n, m, n, k, ops._stream()) == 0
     want = a.double() @ w.double().T
     assert _off(ops.gemm_f32(a, w), want) <= _off(before, want) < 2e-6
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("e_a, e_w", [(-104, 0), (-116, 0), (-125, 0), (0, -120), (-116, 100), (-60, -50), (100, -100), (108, -20), (113, -40)])
+def test_small_and_large_numbers_keep_their_bits(e_a, e_w):
+    """Below 2^-109 a number's low part would fall under bf16's smallest; from 2^112 on, results are taken as float32 sums."""
+    a, w = _operands(130, 300, 2052)
+    a, w = a * 2.0**e_a, (w * 64.0) * 2.0**e_w
+    want = a.double() @ w.double().T
+    assert float(want.abs().min()) > 2.0**-126 * 2.0**-20 and _off(ops.gemm_f32(a, w), want) < 4e-7
