@@ -2,8 +2,9 @@
 // (a published method: Henry, Tang, Heinecke, "Leveraging the bfloat16 Artificial Intelligence Datatype For Higher-Precision
 // Computations", 2019): a float32 number is the sum of three bf16 numbers (x = hi + mid + lo: hi = bf16(x), mid = bf16(x - hi),
 // lo = x - hi - mid, exactly, as 8 + 8 + 8 significant bits and two signs hold 24), a product of two bf16 numbers is exact in
-// float32, and six of the nine products of two such sums are added up in float32.  The other three, mid * lo, lo * mid and lo * lo, are at
-// most 2^-25 of the product, half of what its own rounding to float32 takes, and of either sign.  bf16 ends at 2^-133, float32 at 2^-149, so every number is multiplied by 2^16 (SP_SCALE) first, and a sum by
+// float32, and six of the nine products of two such sums are added up in float32.  The other three are left out: mid * lo and
+// lo * mid are at most 2^-25 of the product each, together (with lo * lo) under 2^-24, which is what its own rounding to
+// float32 takes.  bf16 ends at 2^-133, float32 at 2^-149, so every number is multiplied by 2^16 (SP_SCALE) first, and a sum by
 // 2^-32 at the end: then no bit of any number is lost.  (Without: 2^-116 times N(0, 1) 2.2e-6, 2^-124 5.6e-4.)  Numbers from
 // 2^112 and sums from 2^96 on become infinities by that, and are taken again as below.
 //

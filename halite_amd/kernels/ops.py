@@ -576,7 +576,7 @@ def attention_simple(
 
 
 def gemm_f32(a: torch.Tensor, w: torch.Tensor):
-    """``a @ w.T`` in float32 (``a`` [M, K], ``w`` [N, K]): float32 multiply-adds, or, for prompts, exact products
+    """``a @ w.T`` in float32 (``a`` [M, K], ``w`` [N, K]): float32 multiply-adds, or, for prompts, six exact products
     of three bf16 parts a number, which hold all of its bits, with float32 sums, whose error is no larger (``gemm_f32_split.hip``)."""
     lib = library.core_library()
     _dev(a, w)

@@ -24,7 +24,7 @@ def test_sizes(m, n, k):
     a[m // 2] = a[m // 2].abs()
     got = ops.gemm_f32(a, w)
     want, size = a.double() @ w.double().T, a.double().abs() @ w.double().abs().T
-    # a float32 addition a stage of 32; in a stage six sums that are cut off and the products left out: at most 2 and 1 / 2 each
+    # a float32 addition a stage of 32; in a stage six sums that are cut off and the products left out: at most 2 and 1 each
     assert bool(((got.double() - want).abs() <= (k // 32 + 16) * 2.0**-24 * size).all())
     # a row's result is its own, whatever tile it is in and whatever rows are beside it
     assert torch.equal(ops.gemm_f32(a[: m - 1].contiguous(), w) if m > 65 else got[:-1], got[: m - 1])
@@ -56,6 +56,22 @@ def test_numbers_without_parts(m, n, k):
 
 
 # ---- as exact as float32 sums: what no bound on a sum's largest error can tell ----------------------------------------------
+# Each of the six products that are added up, the bound that the tests below set on the error's norm over the result's, and
+# operands whose parts have one sign, so that a product left out or paired wrongly cannot cancel.
+SIX = [(0, 0), (0, 1), (1, 0), (0, 2), (2, 0), (1, 1)]  # parts of A and W (0: high, 1: middle, 2: low)
+
+
+def _parts_of_one_sign(m, n, k, gen):
+    """Numbers whose three parts are all positive: (128 + i) / 128 + j 2^-16 + l 2^-23, which float32 holds and whose last two
+    are under half of the first one's unit together; A's middle and low parts are near their largest, W's are smaller, so
+    that no two of the products are alike."""
+    def numbers(rows, middle, low):
+        i, j, l = (torch.randint(*between, (rows, k), generator=gen) for between in ((0, 128), middle, low))
+        return (((128 + i) * 2**16 + j * 2**7 + l).double() * 2.0**-23).float()
+
+    return numbers(m, (200, 255), (40, 64)), numbers(n, (128, 160), (10, 20))
+
+
 def _by_parts(a, w, which, scale=2.0**16):
     """The sum in 64 bits of chosen products of the parts."""
     def parts(x):
@@ -73,6 +89,30 @@ def _off(got, want):
     return float((got.double() - want).norm() / want.norm())
 
 
+# what the six products leave out is under 2^-24 of each product; a sum's float32 additions lose 1.5e-7 (see the kernel)
+ONE_SIGN_BOUND = 2.0**-24 + 1.5e-7
+
+
+@pytest.mark.parametrize("k", [2048, 4096])
+def test_the_bound_tells_each_product(k):
+    """On the CPU: all six products are far inside of the bounds, and with any one left out, or in the place of another, outside."""
+    gen = torch.Generator().manual_seed(k)
+    a, w = _parts_of_one_sign(6, 5, k, gen)
+    want = a.double() @ w.double().T
+    assert _off(_by_parts(a, w, SIX), want) < 2.0**-24
+    for left in SIX:
+        rest = [p for p in SIX if p != left]
+        assert _off(_by_parts(a, w, rest), want) > 3 * ONE_SIGN_BOUND
+        for other in rest:
+            assert _off(_by_parts(a, w, rest + [other]), want) > 3 * ONE_SIGN_BOUND
+    # and of ordinary numbers the low parts: more than ten times what float32 sums lose
+    a, w = torch.randn(6, k, generator=gen), torch.randn(5, k, generator=gen) * 0.02
+    want = a.double() @ w.double().T
+    assert _off(_by_parts(a, w, SIX), want) < 1e-7
+    for rest in (SIX[:3] + SIX[5:], SIX[:4] + SIX[5:], SIX[:3] + SIX[4:]):
+        assert _off(_by_parts(a, w, rest), want) > 1e-6
+
+
 @pytest.mark.parametrize("e_a, e_w", [(0, 0), (-125, 0), (0, -120), (-120, 100), (-100, -20)])
 def test_no_bit_of_a_small_number_is_lost(e_a, e_w):
     """On the CPU: the parts of scaled numbers hold all bits down to float32's smallest."""
@@ -84,6 +124,18 @@ def test_no_bit_of_a_small_number_is_lost(e_a, e_w):
 
 # (each in one part, several, several walks; the number of rows takes tiles of each height)
 EXACT_SIZES = [(65, 96, 2048), (128, 4096, 4096), (130, 16500, 4100), (300, 6144, 4096), (520, 8200, 2084), (70, 8300, 8192), (200, 8192, 14336), (80, 4096, 14336)]
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("m, n, k", EXACT_SIZES)
+def test_every_product_of_parts_is_there(m, n, k):
+    gen = torch.Generator().manual_seed(m)
+    a, w = (x.cuda() for x in _parts_of_one_sign(m, n, k, gen))
+    want = a.double() @ w.double().T
+    off = (ops.gemm_f32(a, w).double() - want) / want
+    assert float(off.norm() / off.numel() ** 0.5) < ONE_SIGN_BOUND
+    # and in every row and column
+    assert float(off.square().mean(0).sqrt().max()) < 2 * ONE_SIGN_BOUND and float(off.square().mean(1).sqrt().max()) < 2 * ONE_SIGN_BOUND
 
 
 @pytest.mark.gpu
