@@ -1336,6 +1336,10 @@ class ExpertSum:
         moe_combine(out, self.y, self.wgt, self.extra, extra_gate=self.gate, overwrite=True)
         return out
 
+    def drop(self) -> None:
+        """Lets the rows go, whoever still holds this: they have been added up."""
+        self.y = self.wgt = self.extra = self.gate = None
+
 
 @dataclass
 class LayerResults:
@@ -1349,6 +1353,20 @@ class LayerResults:
             residual_add(h, self.beside)
         e = self.experts
         moe_combine(h, e.y, e.wgt, e.extra, extra_gate=e.gate)
+
+    def drop(self) -> None:
+        """As ``ExpertSum.drop``."""
+        self.beside = None
+        self.experts.drop()
+
+
+def let_go(pending) -> None:
+    """What a block left ``pending`` (alone, or with the connection it goes back through) has been read: the rows of a mixture's
+    experts are given back now, and not when the block that read them ends, which needs as many of its own."""
+    what = pending[0] if isinstance(pending, tuple) else pending
+    for a in [t[0] for t in what.terms] if isinstance(what, NormedTerms) else [what]:
+        if isinstance(a, (ExpertSum, LayerResults)):
+            a.drop()
 
 
 def normed_sum(terms: list[tuple[torch.Tensor, torch.Tensor, float]], eps: float) -> torch.Tensor:

@@ -90,6 +90,7 @@ class ParallelBlock(Arrangement):
         if pending is not None and added is None:
             pending.add_to(h) if isinstance(pending, ops.LayerResults) else ops.residual_add(h, pending)
         if self.ff is None:
+            ops.let_go(pending)
             x = self.mixer_norm.forward(h)
             self.mixer.forward(x, ctx, run, add_to=h)
             return None
@@ -98,6 +99,7 @@ class ParallelBlock(Arrangement):
                                      second=self.ff_norm.weight, added=added)
         else:
             x, y = self.mixer_norm.forward(h), self.ff_norm.forward(h)
+        ops.let_go(pending)
         # both results are computed before either is added: both parts read the same stream
         if hasattr(self.ff, "forward_sum") and self.ff_norm.build.dtype == torch.bfloat16:
             beside = self.mixer.forward(x, ctx, run, add_to=h, **(dict(apart=True) if self.mixer.adds_apart else {}))
@@ -230,6 +232,7 @@ class HyperPreNormBlock(Arrangement):
 
     def forward(self, h, pending, ctx, run):
         x = self.mixer_link.step(h, pending, self.mixer_norm)
+        ops.let_go(pending)
         # (a sum of normed results is made by the pass that writes it)
         terms = self.mixer.forward_normed_terms(x, ctx, run) if hasattr(self.mixer, "forward_normed_terms") else None
         y = terms if terms is not None else self._normed(self.mixer.forward(x, ctx, run), self.mixer_out_norm)

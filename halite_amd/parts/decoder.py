@@ -151,7 +151,9 @@ class Decoder:
             elif i + 1 == len(blocks) and getattr(blocks[i], "takes_last_norm", False):
                 next_norm = self.final_norm.summable(h)
             if isinstance(pending, ops.LayerResults) and not getattr(blocks[i], "takes_layer_results", False):
-                pending = pending.add_to(h)
+                pending.add_to(h)
+                ops.let_go(pending)
+                pending = None
             if next_norm is not None:
                 pending = blocks[i].forward(h, pending, ctx, run, next_norm=next_norm)
             else:
@@ -164,8 +166,11 @@ class Decoder:
                 x = self.final_norm.forward(blocks[-1].leave(h, pending, ctx.logit_rows))
         else:
             if isinstance(pending, ops.LayerResults) and not isinstance(self.final_norm, RMSNorm):
-                pending = pending.add_to(h)
+                pending.add_to(h)
+                ops.let_go(pending)
+                pending = None
             x = self.final_norm.forward(h, delta=pending, rows=ctx.logit_rows)
+        ops.let_go(pending)
         return self.head.forward(x)
 
     def _through_junction(self, junction, kept, h, pending, block, ctx):
@@ -177,8 +182,10 @@ class Decoder:
                 pending.add_to(h)
             elif pending is not None:
                 ops.residual_add(h, pending)
+            ops.let_go(pending)
             ops.cast_cols(h, rows)
             return junction.forward(kept)
         block.leave(h, pending, None, out=rows)
+        ops.let_go(pending)
         x = junction.forward(kept)
         return x.unsqueeze(0) if self.stream_copies == 1 else x.unsqueeze(0).repeat(self.stream_copies, 1, 1)
