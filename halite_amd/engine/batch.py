@@ -196,7 +196,8 @@ class StepContext:
         lens = (self.seg_q_len_host, self.seg_kv_len_host, n_heads // n_kv_heads, n_kv_heads, window)
         if not attention_kernels.long_items_pay(*lens, head_dim, value_from, chunk):
             rows_big = attention_kernels.ROWS_PER_ITEM
-        plan = attention_kernels.plan_items(*lens, rows_big, chunk, keep, spread=True)
+        plan = attention_kernels.plan_items(*lens, rows_big, chunk, keep,
+                                            spread=attention_kernels.spread_from(head_dim))
         self._plan_host[key] = plan
         plan.name = f"plan{len(self._plan_host)}"
         if self._dev is None:

@@ -33,13 +33,24 @@ BIG_ITEM_INTS = 16  # an item of the kernel for long segments: 8, then what its 
 COMPUTE_UNITS = 256  # of the MI355X; the device that runs is asked (`compute_units`)
 MIN_PIECE_KEYS = 384
 # A plan that spreads (an engine's do) cuts shorter ones, a block of 32 keys a wave, where the merge kernel joins them anyway (its launch
-# is there whatever the lengths are) and where a range is long enough that the shorter walk outweighs the joins inside the
-# kernel.  Pieces of 384 / 128 keys, attention and merge, us: merge kernel's: one request, eight key/value heads of 128: 512 keys 8.2 / 7.2,
-# 2,000 10.7 / 9.2, 4,000 10.9 / 10.6, 8,192 14.4 / 13.7; latent heads of 256: one request of 1,549 13.6 / 11.2, eight of 1,092 to 1,980
-# 16.9 / 12.6, of 254 to 437 12.1 / 12.5; inside the kernel: four requests of 2,000 13.6 / 12.7, sixteen latent ones of 1,062 to 1,852 16.3 /
+# is there whatever the lengths are), from three pieces on (`spread_from`), and where a range is long enough that the shorter walk
+# outweighs the joins inside the kernel.  Pieces of 384 / 128 keys, attention and merge, us: merge kernel's: one request, eight key/value
+# heads of 128: 512 keys 8.2 / 7.2, 2,000 10.7 / 9.2, 4,000 10.9 / 10.6, 8,192 14.4 / 13.7; latent heads of 256: one request of 1,549 13.6 / 11.2,
+# eight of 1,092 to 1,980 16.9 / 12.6; inside the kernel: four requests of 2,000 13.6 / 12.7, sixteen latent ones of 1,062 to 1,852 16.3 /
 # 14.1, but four of 512 7.9 / 8.5 and eight 8.2 / 9.5.
 SPREAD_PIECE_KEYS = 128
 SPREAD_MERGED_KEYS = 1024  # inside the kernel for ranges from here on
+
+
+def spread_from(head_dim: int) -> int:
+    """The shortest range that a plan cuts into pieces of ``SPREAD_PIECE_KEYS`` where the merge kernel joins them.  A
+    second piece costs what it saves, a third one does not; with heads of 64, whose walk is the cheapest, a fourth.  One / two or three
+    pieces, us, at 256, 352, 384 and 448 keys: one request, eight key/value heads of 128 6.7 / 7.1, 7.4 / 7.6, 7.4 / 7.1, 8.0 / 7.6; two
+    6.8 / 7.4, 7.4 / 8.0, 7.5 / 7.5, 8.2 / 8.2; eight latent ones of 256 9.8 / 10.6, 11.1 / 12.0, 11.3 / 10.8, 12.4 / 11.9; one with heads of 64
+    5.7 / 6.6, 6.2 / 7.1, 6.3 / 6.7, 6.7 / 7.1, and four pieces of 512 keys 6.8 / 6.7."""
+    return (3 if head_dim >= 128 else 4) * SPREAD_PIECE_KEYS
+
+
 # Up to this many pieces a tile the attention kernel merges the partial results itself (the
 # workgroup that finishes a tile last does, in the same launch: 1 to 3 us less than a merge
 # kernel behind it); more go to the merge kernel, which spreads a tile's partial results over
@@ -278,7 +289,7 @@ def _cut_long(seg_ids, rho0s, kv_b, kv_e, chunk, slots_per_tile, first_slot, seg
     return _group_items(items, piece, WAVES_PER_GROUP, seg_scalars, kept), merges, first_slot + n_split * slots_per_tile
 
 
-def _cut_joined(seg_ids, rho0s, kv_b, kv_e, most_pieces, first_slot, seg_scalars, keep=0, spread=False):
+def _cut_joined(seg_ids, rho0s, kv_b, kv_e, most_pieces, first_slot, seg_scalars, keep=0, spread=0):
     """Items and merge entries of one-tile items whose key ranges are cut into at most
     ``most_pieces`` pieces, one per workgroup, and every piece into four, one per wave (in
     blocks of 32 keys, as evenly as they go; where a piece is short some of the four are
@@ -294,7 +305,7 @@ def _cut_joined(seg_ids, rho0s, kv_b, kv_e, most_pieces, first_slot, seg_scalars
     front = np.where(kv_b > 0, kept_units(keep) // KEYS_PER_BLOCK, 0)
     blocks = front + -(-(kv_e - base) // KEYS_PER_BLOCK)
     keys = front * KEYS_PER_BLOCK + kv_e - base
-    short = spread & ((most_pieces > MERGED_IN_KERNEL) | (keys >= SPREAD_MERGED_KEYS))
+    short = bool(spread) & (keys >= (spread if most_pieces > MERGED_IN_KERNEL else max(spread, SPREAD_MERGED_KEYS)))
     n_pieces = np.clip(keys // np.where(short, SPREAD_PIECE_KEYS, MIN_PIECE_KEYS), 1, most_pieces)
     total = int(n_pieces.sum())
     tile_of = np.repeat(np.arange(n), n_pieces)
@@ -412,13 +423,14 @@ def _group_tiles(seg_ids, rho0s, kv_b, kv_e, per_item: int):
 
 
 def plan_items(seg_q_len, seg_kv_len, group_size: int, n_kv_heads: int, window: int,
-               rows_big: int = 64, chunk: int = 0, keep: int = 0, spread: bool = False) -> AttentionPlan:
+               rows_big: int = 64, chunk: int = 0, keep: int = 0, spread: int = 0) -> AttentionPlan:
     """Cuts the step's query rows into tiles of 16 rows.  A segment of at most 16 rows or
     of one token (decode tokens) gives one-tile items, four to a workgroup, which takes a
     piece of the tile's key range; a longer segment gives items of ``rows_big / 16`` tiles
     that share the keys a wave loads.  ``keep`` (with a window): the first keys of a request
     that stay visible.  Where there are too few items to fill the GPU, a key range is cut
-    into pieces whose partial results are merged; ``spread``: into shorter ones where that pays."""
+    into pieces whose partial results are merged; ``spread``: into shorter ones where that pays, from so many keys
+    on where the merge kernel joins them (``spread_from``; 0: never)."""
     ql = np.asarray(seg_q_len, dtype=np.int64).reshape(-1)
     seg_scalars = np.stack((np.cumsum(ql) - ql, ql, np.asarray(seg_kv_len, dtype=np.int64).reshape(-1)), axis=1)
     per_item = max(1, rows_big // ROWS_PER_ITEM)

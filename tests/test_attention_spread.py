@@ -30,6 +30,39 @@ def test_where_shorter_pieces_are_taken():
     assert plan_items(ones(1), np.array([512]), 4, 8, 0).n_items == 4
 
 
+@pytest.mark.parametrize("head_dim, first", [(64, 512), (112, 512), (128, 384), (256, 384)])
+def test_two_pieces_are_never_cut(head_dim, first):
+    """What the merge kernel's launch and a second piece's start cost is more than half of so short a walk."""
+    assert attn_kernels.spread_from(head_dim) == first
+    for n, kv_heads in ((1, 8), (2, 8), (8, 1)):
+        count = lambda kv: plan_items(ones(n), np.full(n, kv, dtype=np.int32), 4, kv_heads, 0, spread=first).n_items // 4 // n  # noqa: E731
+        assert [count(kv) for kv in (1, 255, 256, 383, first - 1)] == [1] * 5
+        assert count(first) == first // 128 and count(first + 127) == first // 128 and count(first + 128) == first // 128 + 1
+    # lengths that differ: each by its own
+    plan = plan_items(ones(2), np.array([first - 1, first], dtype=np.int32), 4, 8, 0, spread=first)
+    assert plan.merges[:, 0].tolist() == [1] and plan.n_items == 4 * (1 + first // 128)
+    # inside the kernel as without a line of its own
+    for kv in (1023, 1024, 3000):
+        a, b = (plan_items(ones(4), np.full(4, kv, dtype=np.int32), 4, 8, 0, spread=s) for s in (first, True))
+        assert np.array_equal(a.items, b.items) and a.n_merges == b.n_merges == 0
+
+
+def test_the_engine_asks_for_that_line(monkeypatch):
+    from halite_amd.engine import batch
+
+    asked = []
+    monkeypatch.setattr(attn_kernels, "rows_per_big_item", lambda *a: 64)
+    monkeypatch.setattr(attn_kernels, "long_items_pay", lambda *a: True)
+    monkeypatch.setattr(attn_kernels, "plan_items", lambda *a, spread, **k: asked.append(spread) or plan_items(*a, spread=spread, **k))
+    for head_dim in (64, 128, 256):
+        ctx = object.__new__(batch.StepContext)
+        ctx._plan_host, ctx._dev, ctx.static, ctx.seg_q_len_host, ctx.seg_kv_len_host = {}, None, None, ones(1), np.array([300], np.int32)
+        ctx.cache = type("Cache", (), {"groups": [type("Group", (), {"need": object()})]})
+        ctx._packer = type("Packer", (), {"add": lambda *a: None})()
+        ctx.plan_attention(0, 32, 8, 0, head_dim)
+    assert asked == [512, 384, 384]
+
+
 def test_random_decode_steps_are_covered_and_fit_the_recorded_room():
     rng = np.random.default_rng(11)
     for case in range(300):
