@@ -185,6 +185,10 @@ def _check_device() -> None:
             raise KernelLibraryError(f"the HIP kernels are written for {ARCH} (MI355X); this GPU is {name}")
 
 
+# entry points that do not return an int, which is what ctypes takes results for
+RESULTS = {"hal_last_error": ctypes.c_char_p, "hal_gemm_f32_split_planes": ctypes.c_longlong, "hal_delta_chunks_room": ctypes.c_longlong}
+
+
 def load_library(name: str, sources: list[str], defines: dict[str, int] | None = None) -> ctypes.CDLL:
     defines = defines or {}
     key = name + repr(sorted(defines.items()))
@@ -197,7 +201,9 @@ def load_library(name: str, sources: list[str], defines: dict[str, int] | None =
             lib = ctypes.CDLL(path)
         except OSError as e:
             raise KernelLibraryError(f"cannot load {path}: {e}") from e
-        lib.hal_last_error.restype = ctypes.c_char_p
+        for entry, result in RESULTS.items():
+            if hasattr(lib, entry):
+                getattr(lib, entry).restype = result
         _loaded[key] = lib
         return lib
 

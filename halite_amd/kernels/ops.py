@@ -586,7 +586,6 @@ def gemm_f32(a: torch.Tensor, w: torch.Tensor):
     _need(k == k2, f"gemm_f32: inner sizes {k} and {k2}")
     out = torch.empty((m, n), dtype=torch.float32, device=a.device)
     if n > 0 and lib.hal_gemm_f32_split_takes(_ptr(a), k, _ptr(w), k, m, k):
-        lib.hal_gemm_f32_split_planes.restype = ctypes.c_longlong
         words = lib.hal_gemm_f32_split_planes(m, n)
         planes = torch.empty(words, dtype=torch.float32, device=a.device) if words else None
         _check(lib, lib.hal_gemm_f32_split(_ptr(a), k, _ptr(w), k, _ptr(out), n, _ptr(planes), m, n, k, _stream()))
@@ -1690,7 +1689,6 @@ def delta_chunks(r: torch.Tensor, k: torch.Tensor, v: torch.Tensor, a_raw: torch
     _need(w2.shape == (inner, lora) and w0.numel() == inner and a_bias.numel() == inner
           and w2.dtype == w0.dtype == a_bias.dtype, "delta_chunks: w2 [heads * dim, rank], w0 and a_bias [heads * dim] of one type")
     _need(token_slot.numel() == n and n_segs == seg_q_len.numel() and weight.numel() == inner, "delta_chunks: the step's arrays")
-    lib.hal_delta_chunks_room.restype = ctypes.c_longlong
     records = torch.empty(lib.hal_delta_chunks_room(n, n_segs, heads), dtype=torch.float32, device=r.device)
     out = torch.empty((n, inner), dtype=out_dtype, device=r.device)
     _check(lib, lib.hal_delta_chunks(
