@@ -181,7 +181,10 @@ static StreamCut gs_cut(int N, int K, bool gated, bool may_part) {
 // Whether tiles of 128 go through six buffers: a compute unit has one of them then, so where there are no more tiles than units, and
 // where the longer start is made up for by the steps behind it.  Three / six buffers, us, at 48 rows: 161 tiles of K 4,096 39.7 / 37.0, 250 52.2 / 50.8,
 // gated 172 42.9 / 40.5, but gated 224 (which have the memory's rate) 49.2 / 49.5; 250 of 2,048 31.0 / 31.4; in parts 48 tiles x 5 of 4,096
-// 13.8 / 15.1, 97 x 2 25.5 / 27.2; at 17 rows 161 36.9 / 35.5, 172 42.5 / 39.8, 250 50.8 / 49.2.
+// 13.8 / 15.1, 97 x 2 25.5 / 27.2; at 17 rows 161 36.9 / 35.5, 172 42.5 / 39.8, 250 50.8 / 49.2.  The lines are the cautious ones: of K 3,072
+// 161 tiles 34.6 / 29.4 at 48 rows and 31.9 / 31.7 at 64, 204 35.3 / 32.5 and 34.1 / 33.9, 250 38.0 / 37.0 and 37.5 / 37.8, gated 172 32.8 / 32.3 and
+// 35.5 / 35.6, 192 35.7 / 33.9 and 36.9 / 37.0, 224 36.0 / 36.0; 250 of 3,584 42.9 / 43.2 and 42.5 / 43.5; of 2,560 gated 172 32.0 / 32.0; of 5,120
+// gated 172 57.0 / 57.4 and 59.2 / 59.7 (17 rows 55.7 / 53.8), 224 60.3 / 61.0; gated 192 of 4,096 43.9 / 42.7, 204 45.0 / 44.5.
 static bool gs_deep(int K, bool gated, int tiles, int parts) {
   return parts == 1 && K >= 4096 && tiles <= (gated ? GS_UNITS * 3 / 4 : GS_UNITS);
 }
