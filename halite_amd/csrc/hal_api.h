@@ -153,6 +153,7 @@ int hal_zero_rows(void* const* rows, const unsigned long long* words, int n, hip
 // a step's rows: their parameters into one buffer, and sampled by it (sampling.hip)
 int hal_sample_pack(const double* temperature, const double* top_p, const double* min_p, const long long* top_k, const long long* seeds,
                     const long long* draws, int n, int V, int* words);
+long long hal_sample_row_words(int flags, int V);  // the words of room a row
 int hal_sample_packed(const float* logits, int ld, int n, int V, const int* packed, int flags, int* room, int at_once, int* out,
                       hipStream_t stream);
 

@@ -1243,9 +1243,15 @@ extern "C" int hal_sample_pack(const double* temperature, const double* top_p, c
   return (all_greedy ? SAMPLE_ALL_GREEDY : 0) | (unfiltered ? SAMPLE_UNFILTERED : 0) | (late ? SAMPLE_LATE : 0);
 }
 
-// Samples n rows by such a buffer on the GPU.  `flags`: what hal_sample_pack returned.  `room`: for rows with filters, which go `at_once` at a time
-// over it, at_once * (1,190 + V) words that begin at a multiple of 8 bytes (64-bit histograms and the rows' state first), else n * 128.
-// `out`: n tokens, then n log-probabilities.
+// The words of room a row: a histogram and its state (64-bit words, so they come first in the room), its blocks' partial results and kept
+// masses, a list as long as the row; partial results alone where no row is filtered.
+extern "C" long long hal_sample_row_words(int flags, int V) {
+  if (flags & (SAMPLE_ALL_GREEDY | SAMPLE_UNFILTERED)) return ROW_PARTS * 4;
+  return 4 * FILT_BINS + 6 + ROW_PARTS * 4 + ROW_PARTS + (long long)V;
+}
+
+// Samples n rows by such a buffer on the GPU.  `flags`: what hal_sample_pack returned.  `room`: hal_sample_row_words for each of the rows that go
+// over it at a time, from a multiple of 8 bytes on: `at_once` of those with filters, all others.  `out`: n tokens, then n log-probabilities.
 extern "C" int hal_sample_packed(const float* logits, int ld, int n, int V, const int* packed, int flags, int* room, int at_once, int* out,
                                  hipStream_t stream) {
   HAL_REQUIRE(n >= 0 && V > 0 && ld >= V && at_once > 0, "hal_sample_packed: bad sizes rows=%d V=%d ld=%d, %d at once", n, V, ld, at_once);

@@ -186,7 +186,8 @@ def _check_device() -> None:
 
 
 # entry points that do not return an int, which is what ctypes takes results for
-RESULTS = {"hal_last_error": ctypes.c_char_p, "hal_gemm_f32_split_planes": ctypes.c_longlong, "hal_delta_chunks_room": ctypes.c_longlong}
+RESULTS = {"hal_last_error": ctypes.c_char_p, "hal_gemm_f32_split_planes": ctypes.c_longlong, "hal_delta_chunks_room": ctypes.c_longlong,
+           "hal_sample_row_words": ctypes.c_longlong}
 
 
 def load_library(name: str, sources: list[str], defines: dict[str, int] | None = None) -> ctypes.CDLL:

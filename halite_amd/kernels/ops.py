@@ -681,6 +681,11 @@ def pack_sample_rows(host: torch.Tensor, temperature, top_p, min_p, top_k, seeds
     return library.core_library().hal_sample_pack(*at, len(seeds), vocab, _ptr(host))
 
 
+@functools.lru_cache(maxsize=256)
+def _sample_row_words(flags: int, vocab: int) -> int:
+    return library.core_library().hal_sample_row_words(flags, vocab)
+
+
 def sample_packed(logits: torch.Tensor, packed: torch.Tensor, flags: int):
     """Next token and log-probability of every row of float32 ``logits`` by ``packed``, the buffer of ``pack_sample_rows`` on the
     GPU, and its ``flags``: greedy rows and draws from whole distributions in two launches, others in six or eight."""
@@ -689,13 +694,11 @@ def sample_packed(logits: torch.Tensor, packed: torch.Tensor, flags: int):
     n, vocab = logits.shape
     _need(logits.dtype == torch.float32, "sample: logits are float32")
     _need(packed.dtype == torch.int32 and packed.numel() == 7 * n, "sample: parameters of every row")
-    if flags & (SAMPLE_ALL_GREEDY | SAMPLE_UNFILTERED):
-        at_once, words = max(n, 1), n * 128
-    else:
+    at_once = max(1, n)
+    if not flags & (SAMPLE_ALL_GREEDY | SAMPLE_UNFILTERED):
         # a row's list has room for all of its logits (they may all be alike), so many rows go in turns over one room
         at_once = max(1, min(n, SAMPLE_LIST_WORDS // vocab))
-        words = at_once * (2 * 256 * 2 + 6 + 32 * 4 + 32 + vocab)
-    room = torch.empty(words, dtype=torch.int32, device=logits.device)
+    room = torch.empty(at_once * _sample_row_words(flags, vocab), dtype=torch.int32, device=logits.device)
     # one buffer for both results, so that the host can fetch them with one copy
     both = torch.empty(2 * n, dtype=torch.int32, device=logits.device)
     _check(lib, lib.hal_sample_packed(_ptr(logits), vocab, n, vocab, _ptr(packed), flags, _ptr(room), at_once, _ptr(both), _stream()))
