@@ -15,7 +15,8 @@ def _operands(m, n, k):
 # a part, K that ends inside a stage; columns that end inside a tile and inside a vector; rows in two turns over their planes
 @pytest.mark.gpu
 @pytest.mark.parametrize("m, n, k", [(65, 96, 2048), (128, 130, 2052), (96, 12300, 2056), (129, 4090, 2080), (257, 6147, 2116), (300, 8200, 2048),
-                                     (513, 16388, 2084), (1100, 3072, 2048), (1025, 4097, 4100), (200, 1000, 14336)])
+                                     (513, 16388, 2084), (1100, 3072, 2048), (1025, 4097, 4100), (200, 1000, 14336),
+                                     (66, 8300, 4132), (129, 8201, 4100), (400, 8196, 8260)])  # the last three: totals in turns
 def test_sizes(m, n, k):
     a, w = _operands(m, n, k)
     lib = library.core_library()
@@ -33,7 +34,7 @@ def test_sizes(m, n, k):
 
 
 @pytest.mark.gpu
-@pytest.mark.parametrize("m, n, k", [(130, 300, 2052), (300, 8200, 2048)])
+@pytest.mark.parametrize("m, n, k", [(130, 300, 2052), (300, 8200, 2048), (130, 8201, 4132)])
 def test_numbers_without_parts(m, n, k):
     a, w = _operands(m, n, k)
     inf, nan, most = float("inf"), float("nan"), 3.4e38  # (the last: a float32 number that rounds to a bf16 infinity)
