@@ -1221,7 +1221,7 @@ extern "C" int hal_sample_spread(const float* logits, int ld, int n_rows, int V,
 
 // ---- a step's rows as the host has them -------------------------------------------------
 // A row's parameters as they lie in one buffer of 7 n words, so that one copy brings a step's: seeds (64 bits), temperature, top_p,
-// min_p (float32), top_k, draw index.  Returns what holds for all rows, which decides how they are sampled.  (As two dozen numpy
+// min_p (float32), top_k, draw index.  Returns what holds for all rows, which decides how they are sampled; -1: a draw index beyond 32 bits.  (As two dozen numpy
 // calls on 64 rows this was 25 of the 50 us that the host had to do before a step's first launch.)
 enum { SAMPLE_ALL_GREEDY = 1, SAMPLE_UNFILTERED = 2, SAMPLE_LATE = 4 };
 extern "C" int hal_sample_pack(const double* temperature, const double* top_p, const double* min_p, const long long* top_k,
@@ -1230,6 +1230,7 @@ extern "C" int hal_sample_pack(const double* temperature, const double* top_p, c
   float* f = (float*)(words + 2 * (size_t)n);
   int* w = words + 5 * (size_t)n;
   for (int r = 0; r < n; ++r) {
+    if (draws[r] != (int)draws[r]) return -1;
     const bool greedy = temperature[r] == 0 || top_k[r] == 1;
     const bool by_k = top_k[r] > 0 && top_k[r] < V, by_p = top_p[r] < 1.0, by_min = min_p[r] > 0.0;
     all_greedy &= greedy;

@@ -188,6 +188,8 @@ def _check_device() -> None:
 # entry points that do not return an int, which is what ctypes takes results for
 RESULTS = {"hal_last_error": ctypes.c_char_p, "hal_gemm_f32_split_planes": ctypes.c_longlong, "hal_delta_chunks_room": ctypes.c_longlong,
            "hal_sample_row_words": ctypes.c_longlong}
+# and those that are handed addresses as plain numbers, which ctypes would cut to 32 bits
+ARGUMENTS = {"hal_sample_pack": [ctypes.c_void_p] * 6 + [ctypes.c_int, ctypes.c_int, ctypes.c_void_p]}
 
 
 def load_library(name: str, sources: list[str], defines: dict[str, int] | None = None) -> ctypes.CDLL:
@@ -205,6 +207,9 @@ def load_library(name: str, sources: list[str], defines: dict[str, int] | None =
         for entry, result in RESULTS.items():
             if hasattr(lib, entry):
                 getattr(lib, entry).restype = result
+        for entry, kinds in ARGUMENTS.items():
+            if hasattr(lib, entry):
+                getattr(lib, entry).argtypes = kinds
         _loaded[key] = lib
         return lib
 

@@ -673,12 +673,19 @@ SAMPLE_ALL_GREEDY, SAMPLE_UNFILTERED, SAMPLE_LATE = 1, 2, 4  # (the last: some r
 def pack_sample_rows(host: torch.Tensor, temperature, top_p, min_p, top_k, seeds, draw_index, vocab: int) -> int:
     """The parameters of a step's rows (``array``s of doubles and of 64-bit integers) into the int32 buffer ``host`` of seven
     words a row; returns what ``sample_packed`` takes as ``flags``."""
-    rows = (temperature, top_p, min_p, top_k, seeds, draw_index)
-    _need(all(isinstance(a, array) and a.typecode == c and len(a) == len(seeds) for a, c in zip(rows, "dddqqq")),
+    n = len(seeds)
+    # (one by one: a step of few rows waits for this)
+    _need(type(temperature) is type(top_p) is type(min_p) is type(top_k) is type(seeds) is type(draw_index) is array
+          and temperature.typecode == top_p.typecode == min_p.typecode == "d" and top_k.typecode == seeds.typecode == draw_index.typecode == "q"
+          and len(temperature) == len(top_p) == len(min_p) == len(top_k) == len(draw_index) == n,
           "sample: arrays of one length, three of doubles and three of 64-bit integers")
-    _need(host.dtype == torch.int32 and not host.is_cuda and host.is_contiguous() and host.numel() >= 7 * len(seeds), "sample: room for the rows")
-    at = [ctypes.c_void_p(a.buffer_info()[0]) for a in rows]
-    return library.core_library().hal_sample_pack(*at, len(seeds), vocab, _ptr(host))
+    _need(host.dtype == torch.int32 and not host.is_cuda and host.is_contiguous() and host.numel() >= 7 * n, "sample: room for the rows")
+    flags = library.core_library().hal_sample_pack(
+        temperature.buffer_info()[0], top_p.buffer_info()[0], min_p.buffer_info()[0], top_k.buffer_info()[0], seeds.buffer_info()[0],
+        draw_index.buffer_info()[0], n, vocab, host.data_ptr())
+    if flags < 0:
+        raise OverflowError("sample: a draw index beyond 32 bits")
+    return flags
 
 
 @functools.lru_cache(maxsize=256)

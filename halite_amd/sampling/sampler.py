@@ -24,17 +24,17 @@ def request_seed(params: SamplingParams, request_id, engine_seed: int = 0) -> in
     return (zlib.crc32(repr(request_id).encode()) * 2654435761 + engine_seed * 40503) & _MASK63
 
 
-def _integers(values, most: int | None = None, code: str = "q") -> array:
-    """Whole numbers as integers of 64 bits, or of 32 (``code`` "i"); one that is out of their range raises ``OverflowError``
-    (``most``: larger ones count as that)."""
+def _integers(values, most: int | None = None) -> array:
+    """Whole numbers as 64-bit integers; one that is out of their range raises ``OverflowError`` (``most``: larger ones
+    count as that)."""
     try:
-        return array(code, values)
+        return array("q", values)
     except (TypeError, OverflowError):  # other number types, or numbers out of range
         if most is not None:
             values = np.minimum(values, most)
-        numbers = np.empty(len(values), np.dtype(code))
+        numbers = np.empty(len(values), np.int64)
         numbers[:] = values
-        return array(code, numbers.tolist())
+        return array("q", numbers.tolist())
 
 
 class Sampler:
@@ -76,7 +76,7 @@ class Sampler:
         host = self._stage(7 * n)
         flags = ops.pack_sample_rows(
             host, array("d", [p.temperature for p in params]), array("d", [p.top_p for p in params]), array("d", [p.min_p for p in params]),
-            _integers([p.top_k for p in params], 2**31 - 1), _integers(seeds), array("q", _integers(draw_index, code="i")), logits.shape[1])
+            _integers([p.top_k for p in params], 2**31 - 1), _integers(seeds), _integers(draw_index), logits.shape[1])
         dev = torch.empty(7 * n, dtype=torch.int32, device=self.device)
         dev.copy_(host[: 7 * n], non_blocking=True)
         event = torch.cuda.Event()
