@@ -18,7 +18,7 @@
 // results leave as vector stores: streaming tiles of 64 x 128 for experts of few rows and for heads
 // (grouped_stream_kernel), and tiles of up to 352 x 256 for prompts' experts (grouped_wide_kernel).
 // gg_experts_kernel says which of the four takes an expert's product, and why.
-#include "hal_lds.h"
+#include "wide_tile.h"
 #include "hal_api.h"
 #include <math.h>
 
@@ -298,15 +298,11 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
 // 128 of the gate's weight and the same 128 of the up projection's) by eight waves, a wave half the
 // tile's rows x 64 W rows, one workgroup a compute unit.
 //
-// What bounds it: what a compute unit gets from the second-level cache, 16 to 20 bytes a clock whatever
-// the kernel around it looked like (some seventy 128-byte requests in flight, 570 clocks each), and a
-// tile of 128 x 128 asks for twice as much a product.  So the tile is as large as the registers hold, K
-// goes 64 at a time (whole 128-byte lines: half lines are as many requests for half the bytes) through
-// two LDS buffers that the loads fill by themselves, and no load is waited for before a whole step's
-// products have run: a step's one barrier stands in the middle of its second half's products, and
-// behind it the buffer just read is filled anew and the next operands are read while the rest of
-// them runs.  W rows are the instruction's first operand, so lane l of a result holds row l % 16 and the
-// four neighbouring columns 4 * (l / 16) .. + 3: one vector store.
+// What bounds it: weights that come from memory while the matrix cores work at the clock that the chip holds under them.  Tiles are as large as
+// the registers hold, so that an expert's rows make one or two, and wide_tile.h says how a tile's steps go.  (4,000 to 5,440 rows of 4096 x 4096 in one round take 104 to
+// 136 us as rows of one group and 148 to 158 as rows of 16, whose 537 MB of weights take 106 at the memory's rate.)  Weights' rows are a power of two apart and
+// meet in a few of the memory's channels: rows a line further apart made prompts' products 5% faster, and those of decode steps, whose kernel reads whole
+// matrices in their order, 7% slower.
 //
 // A group's rows are cut into the fewest tiles of at most so many rows (gw_height) and these are made equally high,
 // in steps of 32 rows, so that workgroups take equally long.  Workgroup b runs on compute die b % 8, and
@@ -314,18 +310,14 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
 // through a group's row tiles (eight at a time) column by column: one die reads an expert's weights,
 // once (tiles of two experts side by side cost a third more reads from memory and 8% of the time).
 //
-// Measured beside tiles of 128 x 128 in registers and LDS (grouped_mfma_kernel): 9,000 rows of 16 experts,
-// 4096 x 4096: 469 us -> 327 in tiles of at most 256 rows -> 286 of at most 352 (1,057 TFLOP/s); 18,000 rows of 64
-// experts, gate and up 1024 x 4096 each: 537 -> 391 -> 305 us, down 4096 x 1024 into float32 rows 352 -> 284 -> 237;
-// 49,152 rows of 64: 1,127 -> 787 -> 706; 2,400 rows of 8, gate and up 14336 x 4096: 660 -> 557, down 450 -> 338;
-// 3,600 rows of 64 (the weights' 1.07 GB once): 196 -> 197.
+// Measured beside a schedule in which every wave read, loaded and multiplied for itself with one barrier a step, us: 9,000 rows of 16 experts, 4096 x 4096 302 ->
+// 280 (1,080 TFLOP/s; tiles of 128 x 128 in registers and LDS 469); 18,000 rows of 64, gate and up 1024 x 4096 each, 330 -> 320; 49,152 rows 730 -> 698;
+// 2,400 rows of 8, gate and up 14336 x 4096, 554 -> 551; 3,600 rows of 64 249 -> 234; 16 groups of 60, 128, 210, 280 and 340 rows 133 -> 129, 137 -> 135, 155 -> 150, 167 -> 159, 181 -> 170.
 #define GW_ROWS 352
 #define GW_COLS 256
 #define GW_TK 64
 #define GW_PANEL 8
 #define GG_UNITS 256  // compute units of the gfx950 parts that this library is built for
-#define GW_A_BYTES (GW_ROWS * GW_TK * 2)
-#define GW_BUFFER ((GW_ROWS + GW_COLS) * GW_TK * 2)
 
 // column n and the three behind it of the row that goes to row dst
 template <bool GATED>
@@ -359,138 +351,53 @@ __device__ __forceinline__ int gw_lane() {
   return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
 }
 
-// What one wave does for a tile of at most 32 * NI rows.  The two buffers are two arrays, so that the
-// compiler can tell a load into one from a read of the other.
+// What one wave does for a tile of at most 32 * NI rows.
 template <bool GATED, int NI>
-__device__ __forceinline__ void gw_wave(const GroupedArgs& a, int wave, int g, int row0, int row_end, int n0, char* b0, char* b1) {
-  constexpr int AI = (NI + 1) / 2, LOADS = AI + 4;  // a wave's loads a step: 8 rows of every 64 of X, and of W
-  constexpr bool FULL = NI > 10;  // no registers left for W's four addresses: added up for every load (elsewhere 1% slower)
-  const int steps = a.K / GW_TK;                    // even
-  const int lane = gw_lane(), wm = wave / 4, wn = wave % 4;
-  const int lr = wave * 8 + lane / 8, c = ((lane % 8) ^ hal_turn(lr % 16)) * 16;
-  // (GATED: of every 64 W rows, a wave's, the first 32 are the gate's and the others the up projection's)
-  const void* w0 = GATED && wave >= 4 ? a.W2 : a.W;
-  const hal_memory W = hal_memory_at((const bf16_t*)w0 + (size_t)g * a.w_group_stride, (uint32_t)a.N * a.ldw * 2);
+__device__ __forceinline__ void gw_wave(const GroupedArgs& a, int wave, int g, int row0, int row_end, int n0, const wt_lds& lds) {
+  using P = wt_part<NI>;
+  const int lane = gw_lane(), oct = lane / 8, c = ((lane % 8) ^ hal_turn(wave % 2 * 8 + oct)) * 16;
+  const size_t w_at = (size_t)g * a.w_group_stride;
+  const hal_memory W = hal_memory_at((const bf16_t*)a.W + w_at, (uint32_t)a.N * a.ldw * 2);
+  const hal_memory W2 = hal_memory_at((const bf16_t*)(GATED ? a.W2 : a.W) + w_at, (uint32_t)a.N * a.ldw * 2);
   const hal_memory X = gw_rows_of_x(a, a.x_col0);
-  uint32_t xo[AI];
-  // (an odd NI's last load has rows for four waves: the others' bring their last rows again)
-  const int last_x = NI % 2 && wave >= 4 ? AI - 2 : AI - 1;
+  const int last = a.K / GW_TK - 1;
   // rows past the end are read from the last one, columns as zeros: nothing of them is stored
+  uint32_t xo[P::loads(0) + P::loads(1)];
 #pragma unroll
-  for (int i = 0; i < AI; ++i) {
-    int r = row0 + lr + 64 * (i == AI - 1 ? last_x : i);
-    r = r < row_end ? r : row_end - 1;
-    xo[i] = (uint32_t)(a.row_src ? a.row_src[r] / a.src_div : r) * (uint32_t)(a.ldx * 2) + c;
-    asm("v_mov_b32 %0, %1" : "=v"(xo[i]) : "v"(xo[i]));  // (one register, not the pair that a multiplication with addition writes)
-  }
-  const uint32_t w_apart = (GATED ? 32u : 64u) * a.ldw * 2, wo = (uint32_t)(n0 + (GATED ? lr % 32 : lr)) * (uint32_t)(a.ldw * 2) + c;
-  // (no branch: past the end the last step's pieces come again and are not multiplied)
-  auto bring = [&](char* lds, int step) {
-    const uint32_t at = (uint32_t)(step < steps ? step : steps - 1) * (GW_TK * 2);
+  for (int p = 0; p < 2; ++p)
 #pragma unroll
-    for (int i = 0; i < AI; ++i) hal_load_lds(X, xo[i], at, lds + ((i == AI - 1 ? last_x : i) * 8 + wave) * 1024);
+    for (int u = 0; u < P::loads(p); ++u) {
+      int r = row0 + wt_octet_row<NI>(wt_octet<NI>(wave, p, u), p) + oct;
+      r = r < row_end ? r : row_end - 1;
+      uint32_t& to = xo[p * P::loads(0) + u];
+      to = (uint32_t)(a.row_src ? a.row_src[r] / a.src_div : r) * (uint32_t)(a.ldx * 2) + c;
+      asm("v_mov_b32 %0, %1" : "=v"(to) : "v"(to));  // (one register, not the pair that a multiplication with addition writes)
+    }
+  // (GATED: of a wave's 64 W rows the first 32 are the gate's and the others the up projection's)
+  const uint32_t row = (uint32_t)a.ldw * 2, wo = (uint32_t)(n0 + (GATED ? wave * 8 : wave / 4 * 64 + wave % 4 * 8) + oct) * row + c;
+  auto bring_x = [&](auto part, char* to, int step) {
+    constexpr int p = decltype(part)::value;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) hal_load_lds(W, wo + i * w_apart + (FULL ? at : 0), FULL ? 0 : at, lds + GW_A_BYTES + (i * 8 + wave) * 1024);
+    for (int u = 0; u < P::loads(p); ++u) hal_load_lds(X, xo[p * P::loads(0) + u], (uint32_t)min(step, last) * (GW_TK * 2), to + wt_octet<NI>(wave, p, u) * 1024);
   };
-  const int q = lane / 16, r16 = lane % 16;
-  const int get[2] = {r16 * 128 + (q ^ hal_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ hal_turn(r16)) * 16};
-  struct Operands {
-    gg_bf16x8 w[4], x[NI];
-  };
-  auto read = [&](const char* lds, int half, Operands& o) {  // the operands of 32 of a step's 64 k
+  auto bring_w = [&](int half, char* to, int step) {
 #pragma unroll
-    for (int j = 0; j < 4; ++j) o.w[j] = *(const gg_bf16x8*)(lds + GW_A_BYTES + (wn * 4 + j) * 2048 + get[half]);
-#pragma unroll
-    for (int i = 0; i < NI; ++i) o.x[i] = *(const gg_bf16x8*)(lds + (wm * NI + i) * 2048 + get[half]);
+    for (int u = 0; u < 2; ++u)
+      hal_load_lds(half ? W2 : W, wo + (GATED ? u * 64 : u * 128 + half * 32) * row, (uint32_t)min(step, last) * (GW_TK * 2), to + (wave + 8 * u) * 1024);
   };
   gg_f32x4 acc[NI][4];
-#pragma unroll
-  for (int i = 0; i < NI; ++i)
-#pragma unroll
-    for (int j = 0; j < 4; ++j) acc[i][j] = gg_f32x4{0.f, 0.f, 0.f, 0.f};
-  auto multiply = [&](const Operands& o, int from, int to) {
-#pragma unroll
-    for (int i = from; i < to; ++i)
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(o.w[j], o.x[i], acc[i][j], 0, 0, 0);
-  };
-  if constexpr (NI > 4) {
-    // Registers for few operands beside the results (up to 176 of 256): X's go through a ring of four, read while
-    // the 16 products before theirs run, W's of a half of the step with the last products of the half before.
-    gg_bf16x8 x[4], w[2][4];
-    auto get_x = [&](const char* lds, int t) { return *(const gg_bf16x8*)(lds + (wm * NI + t % NI) * 2048 + get[t / NI]); };
-    auto get_w = [&](const char* lds, int half, int j) { return *(const gg_bf16x8*)(lds + GW_A_BYTES + (wn * 4 + j) * 2048 + get[half]); };
-    auto lean = [&](int s, char* mine, char* next, auto turn) {
-#pragma unroll
-      for (int t = 0; t < 2 * NI; ++t) {
-        if (t == 2 * NI - 4) {
-          hal_meet<0>();
-          bring(mine, s + 2);
-          __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
-        }
-        const int at = (t + decltype(turn)::value) % 4, ahead = t + 4;
-#pragma unroll
-        for (int j = 0; j < 4; ++j) acc[t % NI][j] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[t / NI][j], x[at], acc[t % NI][j], 0, 0, 0);
-        x[at] = ahead < 2 * NI ? get_x(mine, ahead) : get_x(next, ahead - 2 * NI);
-        if (t >= NI - 5 && t < NI - 1) w[1][t - (NI - 5)] = get_w(mine, 1, t - (NI - 5));
-        if (t >= 2 * NI - 4) w[0][t - (2 * NI - 4)] = get_w(next, 0, t - (2 * NI - 4));
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-        if ((t >= NI - 5 && t < NI - 1) || t >= 2 * NI - 4) __builtin_amdgcn_sched_group_barrier(0x100, 2, 0);
-        else __builtin_amdgcn_sched_group_barrier(0x100, 1, 0);
-      }
-    };
-    bring(b0, 0);
-    bring(b1, 1);
-    hal_meet<LOADS>();
-#pragma unroll
-    for (int t = 0; t < 4; ++t) x[t] = get_x(b0, t), w[0][t] = get_w(b0, 0, t);
-    for (int s = 0; s < steps; s += 2) {
-      lean(s, b0, b1, std::integral_constant<int, 0>());
-      lean(s + 1, b1, b0, std::integral_constant<int, 2 * NI % 4>());
-    }
-  } else {
-    constexpr int HALF = NI / 2, REST = NI - HALF;
-    Operands low, high;
-    // One step: the operands of its first half are in `low`, the rest is in `mine`, the next step in `next`.
-    auto advance = [&](int s, char* mine, char* next) {
-      read(mine, 1, high);
-      multiply(low, 0, NI);
-#pragma unroll
-      for (int k = 0; k < NI; ++k) {  // (the order that the compiler is to emit)
-        __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + NI - 1) / NI, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-      }
-      multiply(high, 0, HALF);
-      hal_meet<0>();
-      bring(mine, s + 2);
-      read(next, 0, low);
-      multiply(high, HALF, NI);
-      __builtin_amdgcn_sched_group_barrier(0x020, LOADS, 0);
-#pragma unroll
-      for (int k = 0; k < REST; ++k) {
-        __builtin_amdgcn_sched_group_barrier(0x100, (4 + NI + REST - 1) / REST, 0);
-        __builtin_amdgcn_sched_group_barrier(0x008, 4, 0);
-      }
-    };
-    bring(b0, 0);
-    bring(b1, 1);
-    hal_meet<LOADS>();
-    read(b0, 0, low);
-    for (int s = 0; s < steps; s += 2) {
-      advance(s, b0, b1);
-      advance(s + 1, b1, b0);
-    }
-  }
-  asm volatile("s_waitcnt vmcnt(0)" ::: "memory");  // LDS is not given back while loads are on their way into it
+  wt_begin<NI>(lds, bring_x, bring_w);
+  wt_steps<NI>(lds, wave, lane, last + 1, acc, bring_x, bring_w);
+  wt_end();
   const int end_lane = gw_lane();
 #pragma unroll
   for (int i = 0; i < NI; ++i) {
-    const int r = row0 + (wm * NI + i) * 16 + end_lane % 16;
+    const int r = row0 + (wave / 4 * NI + i) * 16 + end_lane % 16;
     if (r >= row_end) continue;
     const int dst = a.row_dst ? a.row_dst[r] : r;
 #pragma unroll
     for (int j = 0; j < (GATED ? 2 : 4); ++j) {
-      const int n = n0 + wn * (GATED ? 32 : 64) + j * 16 + end_lane / 16 * 4;
+      const int n = n0 + wave % 4 * (GATED ? 32 : 64) + j * 16 + end_lane / 16 * 4;
       if (n < a.N) gw_store<GATED>(a, dst, n, acc[i][j], GATED ? acc[i][j + 2] : acc[i][j]);
     }
   }
@@ -579,7 +486,7 @@ __device__ __forceinline__ int gw_height(const GroupedArgs& a, int col_tiles) {
 
 template <bool GATED>
 __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int col_tiles) {
-  __shared__ __attribute__((aligned(16))) char b0[GW_BUFFER], b1[GW_BUFFER];
+  WT_LDS(lds);
   __shared__ __attribute__((aligned(64))) int found[5];
   __shared__ int most;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
@@ -595,7 +502,7 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
     const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GW_COLS / 2 : GW_COLS);
     const int rows = row_end - row0;
     // (equal heights in steps of 32 can leave a group's last tile empty)
-#define GW_WAVE(NI_) gw_wave<GATED, NI_>(a, wave, g, row0, row_end, n0, b0, b1)
+#define GW_WAVE(NI_) gw_wave<GATED, NI_>(a, wave, g, row0, row_end, n0, lds)
     if (rows <= 0);
     else if (rows <= 64) GW_WAVE(2);
     else if (rows <= 128) GW_WAVE(4);
