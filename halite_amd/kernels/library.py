@@ -44,6 +44,7 @@ CORE_SOURCES = [
     "gemm_f32_split.hip",
     "gemm_bf16.hip",
     "gemm_stream.hip",
+    "gemm_wide.hip",
     "sampling.hip",
     "grouped_gemm.hip",
     "latent_moe.hip",

@@ -847,6 +847,36 @@ def gemm_bf16_stream(x: torch.Tensor, w: torch.Tensor, parts: int, w_up: torch.T
     return PartialSums(out) if parts > 1 else out
 
 
+def wide_pays(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, out_dtype: torch.dtype = torch.bfloat16) -> bool:
+    """Whether the product of ``x`` [more than 64, k] against the bf16 weight ``w`` of ``n`` rows (``gated``: two of them) in wide tiles is
+    the faster one, and has a form for these sizes and places."""
+    m, k = x.shape
+    if not (m > STREAM_ROWS and x.is_cuda and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and x.stride(1) == 1 and w.stride(1) == 1
+            and n * w.stride(0) % 8 == 0):  # (where the gate's weight ends and the other begins)
+        return False
+    lib = library.core_library()
+    return bool(lib.hal_gemm_bf16_wide_pays(m, n, k, 1 if gated else 0, 1 if out_dtype == torch.float32 else 0)
+                and lib.hal_gemm_bf16_wide_takes(_ptr(x), x.stride(0), _ptr(w), None, w.stride(0), m, n, k))
+
+
+def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, w_up: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
+                   activation: str = "silu", clamp: Clamp = Clamp(), height: int = 0):
+    """``x @ w.T``, or with ``w_up`` the gated form ``(x @ w_up.T) * act(x @ w.T)``, in tiles of up to 352 x 256 (``height``: rows of a
+    tile in 32s, 4 to 11; 0: as it is best)."""
+    lib = library.core_library()
+    _need(x.is_cuda and w.is_cuda and (w_up is None or w_up.is_cuda), "kernel arguments must be on the GPU")
+    (m, k), n = x.shape, w.shape[0]
+    _need(w.shape[1] == k and (w_up is None or (w_up.shape == w.shape and w_up.stride() == w.stride() and w_up.dtype == w.dtype)),
+          "wide product: weights' shapes")
+    _need(x.dtype == torch.bfloat16 and w.dtype == torch.bfloat16 and x.stride(1) == 1 and w.stride(1) == 1, "wide product: bf16 rows")
+    _need(out_dtype in (torch.bfloat16, torch.float32), "wide product: output dtype")
+    out = torch.empty((m, n), dtype=out_dtype, device=x.device)
+    _check(lib, lib.hal_gemm_bf16_wide(
+        _ptr(x), x.stride(0), _ptr(w), _ptr(w_up), w.stride(0), _ptr(out), n, dtype_code(out_dtype), GATE_ACTIVATIONS[activation],
+        *clamp.args(), m, n, k, height, _stream()))
+    return out
+
+
 def norm_folds(m: int, n: int, k: int, tiled: torch.Tensor | None) -> bool:
     """Whether a product of ``m`` rows against an ``[n, k]`` weight with a tiled copy
     takes an RMSNorm before or after it, or the rotation and the append, into itself: up
@@ -946,7 +976,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
 
     float32 weights: the true 32-bit kernel (activations are widened if needed).
     bf16 weights: the hand-written kernels where they are the faster ones (``skinny_pays``:
-    up to 16 rows; ``stream_parts``: 17 to 64, and from 9 on where nothing is folded in); otherwise the library product that the reference itself uses for
+    up to 16 rows; ``stream_parts``: 17 to 64, and from 9 on where nothing is folded in; ``wide_pays``: more, where the tiles fill the
+    chip); otherwise the library product that the reference itself uses for
     its linear layers (src/halite/transformers/infer/attention.py:21-24), except where
     float32 output is asked for and the library cannot give it, which the hand-written
     kernel does in passes of 64 rows.
@@ -982,6 +1013,8 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
     parts = stream_parts(x, w, w.shape[0], may_part=in_parts)
     if parts:
         return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)
+    if wide_pays(x, w, w.shape[0], out_dtype=out_dtype):
+        return gemm_bf16_wide(x, w, out_dtype=out_dtype)
     if out_dtype == torch.float32:
         global _MM_OUT_DTYPE
         if _MM_OUT_DTYPE is None:

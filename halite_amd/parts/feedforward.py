@@ -122,6 +122,8 @@ class GatedFeedForward(FeedForward):
             act = ops.gemm_bf16_skinny(x, w[:f], w_up=w[f:])
         elif ops.stream_parts(x, w, f, gated=True):
             act = ops.gemm_bf16_stream(x, w[:f], 1, w_up=w[f:])
+        elif ops.wide_pays(x, w, f, gated=True):
+            act = ops.gemm_bf16_wide(x, w[:f], w_up=w[f:])
         else:
             act = ops.silu_mul(ops.linear(x, w))
         return ops.linear(act, self.w_out, tiled=self.t_out, next_norm=then)
@@ -134,6 +136,8 @@ class GatedFeedForward(FeedForward):
             act = ops.gemm_bf16_skinny(x, self.t_gate, w_up=self.t_up, tiled_shape=(f, d), activation=self.p.activation, clamp=self.p.clamp)
         elif ops.stream_parts(x, self.w_gate_up, f, gated=True):
             act = ops.gemm_bf16_stream(x, self.w_gate_up[:f], 1, w_up=self.w_gate_up[f:], activation=self.p.activation, clamp=self.p.clamp)
+        elif ops.wide_pays(x, self.w_gate_up, f, gated=True):
+            act = ops.gemm_bf16_wide(x, self.w_gate_up[:f], w_up=self.w_gate_up[f:], activation=self.p.activation, clamp=self.p.clamp)
         else:
             act = ops.gate_mul(ops.linear(x, self.w_gate_up), self.p.activation, self.p.clamp)
         return ops.linear(act, self.w_out, out_dtype=torch.float32, tiled=self.t_out, unrounded=self.sums)

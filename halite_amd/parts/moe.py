@@ -217,6 +217,9 @@ class MixtureOfExperts(FeedForward):
                 acts = torch.empty((n, fs), dtype=x.dtype, device=x.device)
                 ops.grouped_gemm(x, self.ws_gate_up[:fs].view(1, fs, d), acts, n_rows=n, w_up=self.ws_gate_up[fs:].view(1, fs, d),
                                  limit=p.shared.limit_or_inf, alpha=p.shared.alpha, up_shift=p.shared.up_shift)
+            elif ops.wide_pays(x, self.ws_gate_up, fs, gated=True):
+                clamp = ops.Clamp(p.shared.limit_or_inf, p.shared.alpha, p.shared.up_shift)
+                acts = ops.gemm_bf16_wide(x, self.ws_gate_up[:fs], w_up=self.ws_gate_up[fs:], activation="clamped", clamp=clamp)
             else:
                 acts = ops.clamped_gate_mul(ops.linear(x, self.ws_gate_up), p.shared.limit_or_inf, p.shared.alpha,
                                             p.shared.up_shift)
