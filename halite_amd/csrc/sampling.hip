@@ -383,15 +383,17 @@ __device__ __forceinline__ int part_share(int V) { return ((V + ROW_PARTS - 1) /
 // batch that lie past the share are passed over by all threads at once: worked through by none of them, 200 rows
 // of 1,000 logits without filters took 23.0 us, of 32,000 29.9, and take 16.5 and 23.4 so.
 #define PART_BATCH 16
-template <bool WHOLE, typename F>
-__device__ __forceinline__ void for_batch(const float* x, int from, int end, F&& each) {
-  float v[PART_BATCH];
+template <bool WHOLE>
+__device__ __forceinline__ void ask_batch(const float* x, int from, int end, float (&v)[PART_BATCH]) {
 #pragma unroll
   for (int u = 0; u < PART_BATCH; ++u) {
     if (!WHOLE && from + u * PART_THREADS >= end) break;
     const int i = from + u * PART_THREADS + (int)threadIdx.x;
     v[u] = x[i < end ? i : from];
   }
+}
+template <bool WHOLE, typename F>
+__device__ __forceinline__ void use_batch(const float (&v)[PART_BATCH], int from, int end, F&& each) {
 #pragma unroll
   for (int u = 0; u < PART_BATCH; ++u) {
     if (!WHOLE && from + u * PART_THREADS >= end) break;
@@ -402,9 +404,21 @@ __device__ __forceinline__ void for_batch(const float* x, int from, int end, F&&
 template <typename F>
 __device__ __forceinline__ void for_part(const float* x, int begin, int end, F&& each) {
   for (int from = begin; from < end; from += PART_BATCH * PART_THREADS) {
-    if (from + (PART_BATCH - 1) * PART_THREADS < end) for_batch<true>(x, from, end, each);
-    else for_batch<false>(x, from, end, each);
+    float v[PART_BATCH];
+    if (from + (PART_BATCH - 1) * PART_THREADS < end) ask_batch<true>(x, from, end, v), use_batch<true>(v, from, end, each);
+    else ask_batch<false>(x, from, end, v), use_batch<false>(v, from, end, each);
   }
+}
+// The same in two: the first batch of a share asked for before what its work needs is there, and then worked on with the others.
+__device__ __forceinline__ void ask_part(const float* x, int begin, int end, float (&v)[PART_BATCH]) {
+  if (begin + (PART_BATCH - 1) * PART_THREADS < end) ask_batch<true>(x, begin, end, v);
+  else ask_batch<false>(x, begin, end, v);
+}
+template <typename F>
+__device__ __forceinline__ void use_part(const float (&v)[PART_BATCH], const float* x, int begin, int end, F&& each) {
+  if (begin + (PART_BATCH - 1) * PART_THREADS < end) use_batch<true>(v, begin, end, each);
+  else use_batch<false>(v, begin, end, each);
+  for_part(x, begin + PART_BATCH * PART_THREADS, end, each);
 }
 
 // a row is greedy if it has no temperature array (all rows greedy), a temperature of 0 or top_k 1
@@ -590,30 +604,29 @@ row_join_kernel(const float* __restrict__ logits, int ld, int V, const float* __
 // ---- rows with filters, spread over many blocks -----------------------------------------
 // A row's passes are shared by ROW_PARTS blocks each; what a pass over 64 rows of 128,256 costs is its
 // launch, the logits' way from memory (33 MB, 6.5 us) and about fifty instructions a logit where it takes
-// an exponential.  So a row is passed over four times, and once with its share alone:
+// an exponential.  So a row is passed over three times, and once with its share alone:
 //   filt_max_kernel     its maximum;
 //   filt_coarse_kernel  the sum of exponentials, and how many logits and what mass lie in each of 256 bins of
 //                       the distance from the maximum (an eighth wide; the last takes the rest);
-//   filt_list_kernel    the keys in the bin that holds the threshold, as a list in memory;
-//   filt_find_kernel    (a block a row) the threshold among them, by radix selection over the bits in which
-//                       they differ;
-//   filt_mass_kernel    the kept mass of every share;
-//   filt_pick_kernel    the draw.
+//   filt_list_kernel    the keys in the bin that holds the threshold, as lists in memory, and the mass of what lies
+//                       before that bin, a share;
+//   filt_pick_kernel    (a block a row) the threshold among them, by radix selection over the bits in which
+//                       they differ, with it the kept mass of every share, and the draw.
 // Distances are monotone in the keys, so the bins hold the keys in order, and counts and masses are integers: the
-// thresholds are the same keys as the one-block kernel's.  The drawn token may differ where the draw is within
-// rounding of a token's edge, since the kept masses are added in another order.  A row with top-k, top-p and min-p
-// all at once, where top-p refers to what top-k kept, is searched twice: top-k first, then (`late`) top-p
+// thresholds are the same keys as the one-block kernel's, and the shares' kept masses do not depend on an order either.  The drawn token may differ where
+// the draw is within rounding of a token's edge, since the kept masses are made in another way.  A row with top-k, top-p and min-p
+// all at once, where top-p refers to what top-k kept, is searched twice: top-k first (filt_find_kernel), then (`late`) top-p
 // of the mass that top-k kept.
-// Before (three levels of 2,048 bins of the keys' bits, ten launches): 64 rows of 128,256 with top-p 112 us of kernels,
-// now 13.1 + 15.5 + 12.1 + 11.9 + 10.5 + 8.2 = 71.
+// 64 rows of 128,256 with top-p: 12.2 + 14.4 + 11.3 + 20.0 us of kernels, a call 59.7.  (A pass over the rows for the kept masses and the search and the
+// draw as kernels of their own: 12.4 + 14.7 + 10.7 + 12.8 + 9.8 + 8.3, 69.  With a share's logits asked for before what their work needs is there
+// the two middle passes take 1.5 and 5 us more.)
 struct FiltRow {
   float m;        // maximum of z
   int best;       // its first index
-  int listed;     // keys in the row's list
-  uint32_t key_min;
-  unsigned long long kept_by_k;  // late rows: the mass of the keys that top-k kept
+  uint32_t key_min;              // late rows: of their first search
+  unsigned long long kept_by_k;  // and the mass of the keys that it kept
 };
-static_assert(sizeof(FiltRow) == 24, "FiltRow is 6 words");
+static_assert(sizeof(FiltRow) == 24, "a row's state is 6 words");
 #define FILT_BINS 256
 // greedy; top-k is searched; top-p is searched beside it; top-p is searched after it (late)
 enum { FILT_GREEDY = 1, FILT_K = 2, FILT_P = 4, FILT_P_LATE = 8 };
@@ -623,13 +636,15 @@ struct FiltParams {
   const int* top_k;
 };
 
+// (all four parameters are asked for at once: one after the other, each is a trip to memory)
 __device__ __forceinline__ int filt_flags(const FiltParams& p, int V, int row) {
-  if (row_scale_of(p.temperature, p.top_k, row) == 0.f) return FILT_GREEDY;
+  const float T = p.temperature[row], tp = p.top_p[row], mp = p.min_p[row];
   const int k = p.top_k[row];
-  const bool want_k = k > 0 && k < V, want_p = p.top_p[row] < 1.f;
+  const bool want_k = (k > 0) & (k < V), want_p = tp < 1.f;
   // with min_p the reference renormalises after top-k, so top-p refers to what top-k kept
-  const bool late = want_k && want_p && p.min_p[row] > 0.f;
-  return (want_k ? FILT_K : 0) | (want_p ? (late ? FILT_P_LATE : FILT_P) : 0);
+  const bool late = want_k & want_p & (mp > 0.f);
+  const int flags = (want_k ? FILT_K : 0) | (want_p ? (late ? FILT_P_LATE : FILT_P) : 0);
+  return (T == 0.f) | (k == 1) ? FILT_GREEDY : flags;
 }
 
 // the bin of a z (the last one also where there is no distance: a maximum that is infinite)
@@ -701,6 +716,9 @@ filt_coarse_kernel(const float* __restrict__ logits, int ld, int V, FiltParams p
   const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x, lane = tid % HAL_WAVE;
   const int flags = filt_flags(params, V, row);
   const bool on_k = (flags & FILT_K) != 0, on_p = (flags & (FILT_P | FILT_P_LATE)) != 0;
+  const int share = part_share(V);
+  const int begin = part * share, end = begin + share < V ? begin + share : V;
+  const float* x = logits + (size_t)row * ld;
   count_s[tid] = 0u;
   mass_s[tid] = 0ull;
   // every wave joins the shares' maxima for itself
@@ -719,15 +737,13 @@ filt_coarse_kernel(const float* __restrict__ logits, int ld, int V, FiltParams p
   const float m = best.v;
   if (part == 0 && tid == 0) {
     FiltRow r;
-    r.m = m, r.best = best.i, r.listed = 0, r.key_min = 0u, r.kept_by_k = 0ull;
+    r.m = m, r.best = best.i, r.key_min = 0u, r.kept_by_k = 0ull;
     rows[row] = r;
   }
   __syncthreads();
-  const int share = part_share(V);
-  const int begin = part * share, end = begin + share < V ? begin + share : V;
   const float T = row_scale_of(params.temperature, params.top_k, row), scale = T == 0.f ? 1.f : T;
   float sum = 0.f;
-  for_part(logits + (size_t)row * ld, begin, end, [&](float v, int, int) {
+  for_part(x, begin, end, [&](float v, int, int) {
     const float z = clean_logit(v) / scale, e = expf(z - m);
     sum += e;
     const int bin = filt_bin(z, m);
@@ -761,9 +777,10 @@ __device__ __forceinline__ FiltPlace filt_place(const unsigned long long* __rest
   f.on[0] = !late && (flags & FILT_K) != 0;
   f.on[1] = (flags & (late ? FILT_P_LATE : FILT_P)) != 0;
   f.list = -1;
+  f.largest[0] = f.largest[1] = false;
   if (!f.on[0] && !f.on[1]) return f;
   unsigned long long own[2] = {0ull, 0ull}, upto[2];
-  if (tid < FILT_BINS) own[0] = f.on[0] ? h[tid] : 0ull, own[1] = f.on[1] ? h[FILT_BINS + tid] : 0ull;
+  if (tid < FILT_BINS) own[0] = h[tid], own[1] = h[FILT_BINS + tid];  // (zeros where there is no such search)
 #pragma unroll
   for (int w = 0; w < 2; ++w) {
     upto[w] = own[w];
@@ -800,146 +817,175 @@ __device__ __forceinline__ FiltPlace filt_place(const unsigned long long* __rest
   return f;
 }
 
+// What a share keeps for certain (its mass, to `kept`), and the keys among which the row's threshold lies, at the share's own place in the
+// row's list (their number is the fourth of the share's `parts`).  The logits that are not surely below the threshold's bin, a few in
+// a hundred, are gathered first and then go through quotient and exponential together; masses are added up as integers, so that their
+// order does not matter.
 __global__ void __launch_bounds__(PART_THREADS)
-filt_list_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, FiltRow* __restrict__ rows, int late,
-                 const unsigned long long* __restrict__ hist, uint32_t* __restrict__ lists) {  // [rows][V]
-  __shared__ uint32_t found[PART_BATCH * PART_THREADS];
-  __shared__ int n_found, first;
+filt_list_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, const FiltRow* __restrict__ rows, int late,
+                 const unsigned long long* __restrict__ hist, float* __restrict__ parts, float* __restrict__ kept,
+                 uint32_t* __restrict__ lists) {  // [rows][V]
+  __shared__ float found[PART_BATCH * PART_THREADS];
+  __shared__ unsigned long long mass_s[PART_THREADS / HAL_WAVE];
+  __shared__ int n_found, n_listed;
   const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
-  const FiltRow r = rows[row];
-  const FiltPlace f = filt_place(hist + (size_t)row * 2 * FILT_BINS, params, V, row, r, late);
-  if (f.list < 0) return;
+  const int flags = filt_flags(params, V, row);
+  if (flags == FILT_GREEDY || (late && !(flags & FILT_P_LATE))) return;
   const int share = part_share(V);
   const int begin = part * share, end = begin + share < V ? begin + share : V;
   const float* x = logits + (size_t)row * ld;
-  const float T = params.temperature[row];
-  // Logits that are surely outside the bin are left out by two comparisons (the bounds are a 100,000th of
-  // the numbers they are made of wider than the bin), the others go through the quotient.
+  const FiltRow r = rows[row];
+  if (tid == 0) n_listed = 0;
+  const FiltPlace f = filt_place(hist + (size_t)row * 2 * FILT_BINS, params, V, row, r, late);
+  const bool largest = f.largest[0] || f.largest[1];  // the largest key alone is kept; without a search and that, every key
+  const float T = params.temperature[row], mp = params.min_p[row];
+  // A bound a 100,000th of the numbers that it is made of below what counts: the bin's end, or without a search the largest key or min-p's.
   const float wide = 1e-5f * (fabsf(r.m) + 32.f) * T;
-  const float high = (r.m - 0.125f * f.list) * T + wide;
-  const float low = f.list == FILT_BINS - 1 ? -INFINITY : (r.m - 0.125f * (f.list + 1)) * T - wide;
+  float low = f.list < 0 || f.list == FILT_BINS - 1 ? -INFINITY : (r.m - 0.125f * (f.list + 1)) * T - wide;
+  if (f.list < 0 && (largest || mp > 0.f)) low = (largest ? r.m : r.m + logf(mp)) * T - wide;
+  const uint32_t top = sort_key(r.m);
+  uint32_t* list = lists + (size_t)row * V + begin;
+  unsigned long long mass = 0ull;
   for (int from = begin; from < end; from += PART_BATCH * PART_THREADS) {
     const int to = from + PART_BATCH * PART_THREADS < end ? from + PART_BATCH * PART_THREADS : end;
     if (tid == 0) n_found = 0;
     __syncthreads();
-    for_part(x, from, to, [&](float v, int, int) {
+    auto gather = [&](float v, int, int) {
       v = clean_logit(v);
-      if (v > high || v < low) return;
-      const float z = v / T;
-      if (filt_bin(z, r.m) == f.list) found[atomicAdd(&n_found, 1)] = sort_key(z);
-    });
+      if (v >= low) found[atomicAdd(&n_found, 1)] = v;
+    };
+    for_part(x, from, to, gather);
     __syncthreads();
-    if (tid == 0 && n_found) first = atomicAdd(&rows[row].listed, n_found);
-    __syncthreads();
-    for (int i = tid; i < n_found; i += PART_THREADS) lists[(size_t)row * V + first + i] = found[i];
+    for (int i = tid; i < n_found; i += PART_THREADS) {
+      const float z = found[i] / T;
+      const int bin = f.list < 0 ? 0 : filt_bin(z, r.m);
+      const bool sure = f.list < 0 ? !largest || sort_key(z) >= top : bin < f.list;
+      if (sure) {
+        const float e = expf(z - r.m);
+        if (e >= mp) mass += filt_fixed(e);
+      } else if (bin == f.list) {
+        list[atomicAdd(&n_listed, 1)] = sort_key(z);
+      }
+    }
     __syncthreads();
   }
+#pragma unroll
+  for (int off = HAL_WAVE / 2; off; off >>= 1) {
+    const uint32_t lo = __shfl_xor((uint32_t)mass, off, HAL_WAVE), hi = __shfl_xor((uint32_t)(mass >> 32), off, HAL_WAVE);
+    mass += ((unsigned long long)hi << 32) | lo;
+  }
+  if (tid % HAL_WAVE == 0) mass_s[tid / HAL_WAVE] = mass;
+  __syncthreads();
+  if (tid != 0) return;
+  for (int w = 1; w < PART_THREADS / HAL_WAVE; ++w) mass += mass_s[w];
+  kept[(size_t)row * ROW_PARTS + part] = (float)mass * (1.0f / 1099511627776.0f);
+  parts[((size_t)row * ROW_PARTS + part) * 4 + 3] = __int_as_float(n_listed);
 }
 
-// The smallest key that a row keeps by the searches of this pass, and after the first pass of a late row the mass that
-// top-k kept; a block a row.  The keys of the row's list are searched bit by bit of those in which they differ, ten at a
-// time from the top, from histograms over the keys that share the bits found so far (the keys of a bin differ in some
-// eighteen bits: two rounds).  (Every block of the next pass finding it for itself instead: 24 us more there.)
+// The smallest key that a row keeps by the searches of this pass, by a block a row; all its threads get it.  `listed`: lane l's is how many keys share l has.  The keys of the row's list are searched bit by
+// bit of those in which they differ, ten at a time from the top, from histograms over the keys that share the bits found so far (the keys of a bin
+// differ in some eighteen bits: two rounds).  A wave has two shares' keys.  (Every block of another pass finding it for itself: 24 us more there.)
+#define PICK_THREADS 1024
 #define FILT_DIGIT 10
-#define FILT_STAGED 2048  // keys of a list that are kept in LDS
-// Sum of `v` over the threads after this one (exclusive) in a block of PART_THREADS; ends with a barrier.
-__device__ __forceinline__ unsigned long long part_suffix_u64(unsigned long long v, unsigned long long* tmp) {
-  const int lane = threadIdx.x % HAL_WAVE, wave = threadIdx.x / HAL_WAVE;
-  unsigned long long inc = v;
+#define FILT_STAGED 4096  // keys of a list that are kept in LDS
+struct FiltSearch {
+  unsigned long long bins[1 << FILT_DIGIT], tmp[PICK_THREADS / HAL_WAVE], above;
+  uint32_t staged[FILT_STAGED], ends[2], bin;
+  int first[ROW_PARTS + 1];  // the shares' first keys, counted over the row
+};
+static_assert((1 << FILT_DIGIT) == PICK_THREADS && SAMPLE_THREADS == PICK_THREADS && PICK_THREADS / HAL_WAVE * 2 == ROW_PARTS, "a thread a bin, a wave two shares");
+// What a wave does with each key of each of its shares.
+template <typename F>
+__device__ __forceinline__ void filt_each(const FiltSearch& s, const uint32_t* keys, int V, F&& what) {
+  const int lane = threadIdx.x % HAL_WAVE, wave = threadIdx.x / HAL_WAVE, share = part_share(V);
 #pragma unroll
-  for (int off = 1; off < HAL_WAVE; off <<= 1) {
-    const uint32_t lo = __shfl_down((uint32_t)inc, off, HAL_WAVE), hi = __shfl_down((uint32_t)(inc >> 32), off, HAL_WAVE);
-    if (lane + off < HAL_WAVE) inc += ((unsigned long long)hi << 32) | lo;
+  for (int h = 0; h < 2; ++h) {
+    const int part = 2 * wave + h, first = s.first[part], n = s.first[part + 1] - first;
+    for (int k = lane; k < n; k += HAL_WAVE) what(first + k < FILT_STAGED ? s.staged[first + k] : keys[part * share + k], part);
   }
-  if (lane == 0) tmp[wave] = inc;
-  __syncthreads();
-  unsigned long long after = 0ull;
-#pragma unroll
-  for (int w = 1; w < PART_THREADS / HAL_WAVE; ++w)
-    if (w > wave) after += tmp[w];
-  __syncthreads();
-  return inc - v + after;
 }
-__global__ void __launch_bounds__(PART_THREADS)
-filt_find_kernel(FiltRow* __restrict__ rows, const unsigned long long* __restrict__ hists, FiltParams params, int V, int late,
+__device__ __forceinline__ uint32_t filt_search(FiltSearch& s, const FiltPlace& f, const FiltRow& r, int listed, const uint32_t* keys, int V, int late) {
+  const int tid = threadIdx.x, lane = tid % HAL_WAVE, wave = tid / HAL_WAVE, share = part_share(V);
+  uint32_t key_min = late ? r.key_min : 0u;
+  if (f.largest[0] || f.largest[1]) key_min = sort_key(r.m);
+  if (wave == 0) {
+    int upto = f.list >= 0 ? listed : 0;
+#pragma unroll
+    for (int off = 1; off < ROW_PARTS; off <<= 1) {
+      const int v = __shfl_up(upto, off, HAL_WAVE);
+      if (lane >= off) upto += v;
+    }
+    if (lane < ROW_PARTS) s.first[lane + 1] = upto;
+    if (lane == 0) s.first[0] = 0, s.ends[0] = 0xffffffffu, s.ends[1] = 0u;
+  }
+  __syncthreads();
+  if (s.first[ROW_PARTS] == 0) return key_min;
+  uint32_t lowest = 0xffffffffu, highest = 0u;
+#pragma unroll
+  for (int h = 0; h < 2; ++h) {
+    const int part = 2 * wave + h, first = s.first[part], n = s.first[part + 1] - first;
+    for (int k = lane; k < n; k += HAL_WAVE) {
+      const uint32_t key = keys[part * share + k];
+      if (first + k < FILT_STAGED) s.staged[first + k] = key;
+      lowest = min(lowest, key), highest = max(highest, key);
+    }
+  }
+#pragma unroll
+  for (int off = HAL_WAVE / 2; off; off >>= 1) lowest = min(lowest, (uint32_t)__shfl_xor((int)lowest, off, HAL_WAVE)), highest = max(highest, (uint32_t)__shfl_xor((int)highest, off, HAL_WAVE));
+  if (lane == 0) atomicMin(&s.ends[0], lowest), atomicMax(&s.ends[1], highest);
+  __syncthreads();
+  lowest = s.ends[0];
+  const uint32_t range = s.ends[1] - lowest;
+#pragma unroll 1
+  for (int w = 0; w < 2; ++w) {
+    if (!f.on[w] || f.bin[w] != f.list) continue;
+    const unsigned long long target = f.target[w] - f.before[w];
+    uint32_t prefix = 0u;
+    unsigned long long above = 0ull;
+    int bits = range ? 32 - __builtin_clz(range) : 0;
+#pragma unroll 1
+    while (bits > 0) {
+      const int take = bits < FILT_DIGIT ? bits : FILT_DIGIT, shift = bits - take;
+      s.bins[tid] = 0ull;
+      if (tid == 0) s.bin = 0u, s.above = above;
+      __syncthreads();
+      filt_each(s, keys, V, [&](uint32_t key, int) {
+        const uint32_t rel = key - lowest;
+        if (((unsigned long long)rel >> bits) != prefix) return;
+        atomicAdd(&s.bins[(rel >> shift) & ((1u << take) - 1u)], w == 1 ? filt_fixed(expf(key_value(key) - r.m)) : 1ull);
+      });
+      __syncthreads();
+      // in descending order
+      const unsigned long long own = s.bins[tid], higher = above + block_suffix_u64(own, s.tmp);
+      if (higher < target && higher + own >= target) s.bin = tid, s.above = higher;
+      __syncthreads();
+      prefix = (prefix << take) | s.bin;
+      above = s.above;
+      bits = shift;
+      __syncthreads();
+    }
+    key_min = max(key_min, lowest + prefix);
+  }
+  return key_min;
+}
+
+// The first search of late rows: the smallest key that top-k keeps, and the mass of those that it keeps.
+__global__ void __launch_bounds__(PICK_THREADS)
+filt_find_kernel(FiltRow* __restrict__ rows, const unsigned long long* __restrict__ hists, FiltParams params, int V, const float* __restrict__ parts,
                  const uint32_t* __restrict__ lists) {
-  constexpr int BINS = 1 << FILT_DIGIT, EACH = BINS / PART_THREADS;
-  __shared__ unsigned long long bins[BINS];
-  __shared__ unsigned long long tmp[PART_THREADS / HAL_WAVE];
-  __shared__ uint32_t staged[FILT_STAGED];
-  __shared__ uint32_t ends[2];
-  __shared__ unsigned long long above_s;
-  __shared__ uint32_t bin_s;
+  __shared__ FiltSearch s;
   const int row = blockIdx.x, tid = threadIdx.x;
+  if (!(filt_flags(params, V, row) & FILT_P_LATE)) return;
   const unsigned long long* hist = hists + (size_t)row * 2 * FILT_BINS;
   const uint32_t* keys = lists + (size_t)row * V;
   const FiltRow r = rows[row];
-  const FiltPlace f = filt_place(hist, params, V, row, r, late);
-  if (!f.on[0] && !f.on[1]) return;
-  uint32_t key_min = late ? r.key_min : 0u;
-  if (f.largest[0] || f.largest[1]) key_min = sort_key(r.m);
-  const int n = f.list < 0 ? 0 : r.listed, n_staged = n < FILT_STAGED ? n : FILT_STAGED;
-  auto each = [&](auto&& what) {
-    for (int i = tid; i < n_staged; i += PART_THREADS) what(staged[i]);
-    for (int i = FILT_STAGED + tid; i < n; i += PART_THREADS) what(keys[i]);
-  };
-  auto mass_of = [&](uint32_t key) { return filt_fixed(expf(key_value(key) - r.m)); };
-  if (n > 0) {
-    for (int i = tid; i < n_staged; i += PART_THREADS) staged[i] = keys[i];
-    if (tid == 0) ends[0] = 0xffffffffu, ends[1] = 0u;
-    __syncthreads();
-    uint32_t lowest = 0xffffffffu, highest = 0u;
-    each([&](uint32_t key) { lowest = min(lowest, key), highest = max(highest, key); });
-    atomicMin(&ends[0], lowest), atomicMax(&ends[1], highest);
-    __syncthreads();
-    lowest = ends[0];
-    const uint32_t range = ends[1] - lowest;
-#pragma unroll 1
-    for (int w = 0; w < 2; ++w) {
-      if (!f.on[w] || f.bin[w] != f.list) continue;
-      const unsigned long long target = f.target[w] - f.before[w];
-      uint32_t prefix = 0u;
-      unsigned long long above = 0ull;
-      int bits = range ? 32 - __builtin_clz(range) : 0;
-#pragma unroll 1
-      while (bits > 0) {
-        const int take = bits < FILT_DIGIT ? bits : FILT_DIGIT, shift = bits - take;
-#pragma unroll
-        for (int b = 0; b < EACH; ++b) bins[tid + b * PART_THREADS] = 0ull;
-        if (tid == 0) bin_s = 0u, above_s = above;
-        __syncthreads();
-        each([&](uint32_t key) {
-          const uint32_t rel = key - lowest;
-          if (((unsigned long long)rel >> bits) != prefix) return;
-          atomicAdd(&bins[(rel >> shift) & ((1u << take) - 1u)], w == 1 ? mass_of(key) : 1ull);
-        });
-        __syncthreads();
-        // in descending order: thread t has the bins EACH * t + EACH - 1 .. EACH * t
-        unsigned long long own[EACH], sum = 0ull;
-#pragma unroll
-        for (int b = 0; b < EACH; ++b) own[b] = bins[tid * EACH + b], sum += own[b];
-        unsigned long long higher = above + part_suffix_u64(sum, tmp);
-#pragma unroll
-        for (int b = EACH - 1; b >= 0; --b) {
-          if (higher < target && higher + own[b] >= target) bin_s = tid * EACH + b, above_s = higher;
-          higher += own[b];
-        }
-        __syncthreads();
-        prefix = (prefix << take) | bin_s;
-        above = above_s;
-        bits = shift;
-        __syncthreads();
-      }
-      key_min = max(key_min, lowest + prefix);
-    }
-  }
-  unsigned long long kept = 0ull;
-  if (!late && (filt_flags(params, V, row) & FILT_P_LATE)) {
-    kept = tid < f.bin[0] ? hist[FILT_BINS + tid] : 0ull;
-    each([&](uint32_t key) { kept += key >= key_min ? mass_of(key) : 0ull; });
-    kept += part_suffix_u64(kept, tmp);  // (thread 0: of all)
-  }
-  if (tid == 0) rows[row].key_min = key_min, rows[row].kept_by_k = kept, rows[row].listed = 0;
+  const int lane = tid % HAL_WAVE, listed = lane < ROW_PARTS ? __float_as_int(parts[((size_t)row * ROW_PARTS + lane) * 4 + 3]) : 0;
+  const FiltPlace f = filt_place(hist, params, V, row, r, 0);
+  const uint32_t key_min = filt_search(s, f, r, listed, keys, V, 0);
+  unsigned long long kept = tid < f.bin[0] ? hist[FILT_BINS + tid] : 0ull;
+  filt_each(s, keys, V, [&](uint32_t key, int) { kept += key >= key_min ? filt_fixed(expf(key_value(key) - r.m)) : 0ull; });
+  kept += block_suffix_u64(kept, s.tmp);  // (thread 0: of all)
+  if (tid == 0) rows[row].key_min = key_min, rows[row].kept_by_k = kept;
 }
 
 __device__ __forceinline__ float kept_mass_of(float v, float T, uint32_t key_min, float m, float mp, float& z) {
@@ -950,47 +996,61 @@ __device__ __forceinline__ float kept_mass_of(float v, float T, uint32_t key_min
   return e >= mp ? e : 0.f;
 }
 
-// The kept mass of every share of a row.
-__global__ void __launch_bounds__(PART_THREADS)
-filt_mass_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, const FiltRow* __restrict__ rows,
-                 float* __restrict__ kept) {  // [rows][ROW_PARTS]
-  __shared__ float red[16];
-  const int row = blockIdx.y, part = blockIdx.x, tid = threadIdx.x;
-  if (row_scale_of(params.temperature, params.top_k, row) == 0.f) return;
-  const FiltRow r = rows[row];
-  const int share = part_share(V);
-  const int begin = part * share, end = begin + share < V ? begin + share : V;
-  const float* x = logits + (size_t)row * ld;
-  const float T = params.temperature[row], mp = params.min_p[row];
-  float mine = 0.f, z;
-  for_part(x, begin, end, [&](float v, int, int) { mine += kept_mass_of(v, T, r.key_min, r.m, mp, z); });
-  mine = block_sum(mine, red);
-  if (tid == 0) kept[(size_t)row * ROW_PARTS + part] = mine;
-}
-
-// The draw: the share in which the running kept mass passes u * (kept mass), then the walk through that share as four
-// waves would walk it, a quarter each, 64 logits at a time.  Sixteen waves make the masses and the running sums inside
+// The threshold, what every share keeps, and the draw, a block a row: the share in which the running kept mass passes u * (kept mass), then the walk
+// through that share as four waves would walk it, a quarter each, 64 logits at a time.  Sixteen waves make the masses and the running sums inside
 // every 64 and leave them in LDS; the sums over a quarter's runs of 64 and the runs' order are then a few additions.
-#define PICK_THREADS 1024
 #define PICK_QUARTERS 4
 __global__ void __launch_bounds__(PICK_THREADS)
-filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, const FiltRow* __restrict__ rows,
-                 const float* __restrict__ parts, const float* __restrict__ kept, const uint64_t* __restrict__ seeds,
-                 const int* __restrict__ draw_index, int* __restrict__ out_token, float* __restrict__ out_logprob) {
+filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams params, const FiltRow* __restrict__ rows, int any_late,
+                 const unsigned long long* __restrict__ hists, const float* __restrict__ parts, const float* __restrict__ kept,
+                 const uint32_t* __restrict__ lists, const uint64_t* __restrict__ seeds, const int* __restrict__ draw_index,
+                 int* __restrict__ out_token, float* __restrict__ out_logprob) {
   constexpr int RUNS = 16, WAVES = PICK_THREADS / HAL_WAVE, MINE = RUNS * PICK_QUARTERS / WAVES;  // runs in LDS a quarter; of a wave
   __shared__ float e_s[PICK_QUARTERS][RUNS][HAL_WAVE], z_s[PICK_QUARTERS][RUNS][HAL_WAVE], inc_s[PICK_QUARTERS][RUNS][HAL_WAVE];
-  __shared__ float quarter_mass[PICK_QUARTERS];
+  __shared__ float quarter_mass[PICK_QUARTERS], kept_s[ROW_PARTS];
+  __shared__ FiltSearch search;
   const int row = blockIdx.x, tid = threadIdx.x;
   const int lane = tid % HAL_WAVE, wave = __builtin_amdgcn_readfirstlane(tid / HAL_WAVE);
   const FiltRow r = rows[row];
-  const float total = wave_sum(lane < ROW_PARTS ? parts[((size_t)row * ROW_PARTS + lane) * 4 + 2] : 0.f);
-  if (row_scale_of(params.temperature, params.top_k, row) == 0.f) {
+  // (what is read here does not wait for the search)
+  typedef __attribute__((ext_vector_type(4), aligned(4))) float any4;  // (the room's parts begin at any float)
+  any4 of_part = {0.f, 0.f, 0.f, 0.f};
+  if (lane < ROW_PARTS) of_part = *(const any4*)(parts + ((size_t)row * ROW_PARTS + lane) * 4);
+  const float for_sure = kept[(size_t)row * ROW_PARTS + 2 * wave + lane % 2];
+  const uint64_t seed = seeds[row];
+  const uint32_t drawn = (uint32_t)draw_index[row];
+  const int flags = filt_flags(params, V, row);
+  const float total = wave_sum(of_part.z);
+  if (flags == FILT_GREEDY) {
     if (tid == 0) {
       out_token[row] = r.best < V ? r.best : 0;
       out_logprob[row] = -logf(total);
     }
     return;
   }
+  const int late = any_late && (flags & FILT_P_LATE) ? 1 : 0;
+  const uint32_t* keys = lists + (size_t)row * V;
+  const FiltPlace f = filt_place(hists + (size_t)row * 2 * FILT_BINS, params, V, row, r, late);
+  const uint32_t key_min = filt_search(search, f, r, __float_as_int(of_part.w), keys, V, late);
+  {
+    const float mp = params.min_p[row];
+    unsigned long long listed[2] = {0ull, 0ull};
+    filt_each(search, keys, V, [&](uint32_t key, int part) {
+      if (key < key_min) return;
+      const float e = expf(key_value(key) - r.m);
+      if (e >= mp) listed[part % 2] += filt_fixed(e);
+    });
+#pragma unroll
+    for (int h = 0; h < 2; ++h) {
+#pragma unroll
+      for (int off = HAL_WAVE / 2; off; off >>= 1) {
+        const uint32_t lo = __shfl_xor((uint32_t)listed[h], off, HAL_WAVE), hi = __shfl_xor((uint32_t)(listed[h] >> 32), off, HAL_WAVE);
+        listed[h] += ((unsigned long long)hi << 32) | lo;
+      }
+      if (lane == h) kept_s[2 * wave + h] = for_sure + (float)listed[h] * (1.0f / 1099511627776.0f);
+    }
+  }
+  __syncthreads();
   auto running = [&](float v) {
     float inc = v;
 #pragma unroll
@@ -1000,10 +1060,10 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams par
     }
     return inc;
   };
-  const float mass = lane < ROW_PARTS ? kept[(size_t)row * ROW_PARTS + lane] : 0.f;
+  const float mass = lane < ROW_PARTS ? kept_s[lane] : 0.f;
   const float incl = running(mass);
   const float kept_mass = __shfl(incl, HAL_WAVE - 1, HAL_WAVE);
-  const float target = uniform_draw(seeds[row], (uint32_t)draw_index[row]) * kept_mass;
+  const float target = uniform_draw(seed, drawn) * kept_mass;
   const unsigned long long some = __builtin_amdgcn_ballot_w64(mass > 0.f);
   const unsigned long long hit = __builtin_amdgcn_ballot_w64(mass > 0.f && incl > target);
   // (the largest key is always kept, so some share holds something)
@@ -1027,7 +1087,7 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams par
 #pragma unroll
     for (int u = 0; u < MINE; ++u) {
       float z = 0.f;
-      const float e = from + (run0 + u) * HAL_WAVE + lane < end ? kept_mass_of(held[u], T, r.key_min, r.m, mp, z) : 0.f;
+      const float e = from + (run0 + u) * HAL_WAVE + lane < end ? kept_mass_of(held[u], T, key_min, r.m, mp, z) : 0.f;
       e_s[q][run0 + u][lane] = e, z_s[q][run0 + u][lane] = z, inc_s[q][run0 + u][lane] = running(e);
     }
   }
@@ -1037,7 +1097,7 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams par
   const int runs = end > begin ? (end - begin + HAL_WAVE - 1) / HAL_WAVE : 0;
   float mine = 0.f, zz = 0.f;
   for (int u = 0; u < runs && u < RUNS; ++u) mine += e_s[wave][u][lane];
-  for (int i = begin + RUNS * HAL_WAVE + lane; i < end; i += HAL_WAVE) mine += kept_mass_of(x[i], T, r.key_min, r.m, mp, zz);
+  for (int i = begin + RUNS * HAL_WAVE + lane; i < end; i += HAL_WAVE) mine += kept_mass_of(x[i], T, key_min, r.m, mp, zz);
   const float wave_mass = wave_sum(mine);
   if (lane == 0 && wave < PICK_QUARTERS) quarter_mass[wave] = wave_mass;
   __syncthreads();
@@ -1063,7 +1123,7 @@ filt_pick_kernel(const float* __restrict__ logits, int ld, int V, FiltParams par
     if (u < RUNS) {
       e = e_s[wave][u][lane], z = z_s[wave][u][lane], inc = inc_s[wave][u][lane];
     } else {
-      if (i0 + lane < end) e = kept_mass_of(x[i0 + lane], T, r.key_min, r.m, mp, z);
+      if (i0 + lane < end) e = kept_mass_of(x[i0 + lane], T, key_min, r.m, mp, z);
       inc = running(e);
     }
     const unsigned long long kept_lanes = __builtin_amdgcn_ballot_w64(e > 0.f);
@@ -1207,14 +1267,13 @@ extern "C" int hal_sample_spread(const float* logits, int ld, int n_rows, int V,
   const dim3 shares(ROW_PARTS, n_rows);
   hipLaunchKernelGGL(filt_max_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, parts, h);
   hipLaunchKernelGGL(filt_coarse_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, parts, rows, h);
-  // the searches; then, if some row has top-k, top-p and min-p all at once, its second search
-  for (int late = 0; late <= (any_late ? 1 : 0); ++late) {
-    hipLaunchKernelGGL(filt_list_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, rows, late, h, lists);
-    hipLaunchKernelGGL(filt_find_kernel, dim3(n_rows), dim3(PART_THREADS), 0, stream, rows, h, params, V, late, lists);
+  hipLaunchKernelGGL(filt_list_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, rows, 0, h, parts, kept, lists);
+  if (any_late) {  // rows with top-k, top-p and min-p all at once: what top-k keeps, and the second search's list
+    hipLaunchKernelGGL(filt_find_kernel, dim3(n_rows), dim3(PICK_THREADS), 0, stream, rows, h, params, V, parts, lists);
+    hipLaunchKernelGGL(filt_list_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, rows, 1, h, parts, kept, lists);
   }
-  hipLaunchKernelGGL(filt_mass_kernel, shares, dim3(PART_THREADS), 0, stream, logits, ld, V, params, rows, kept);
-  hipLaunchKernelGGL(filt_pick_kernel, dim3(n_rows), dim3(PICK_THREADS), 0, stream, logits, ld, V, params, rows, parts,
-                     kept, seeds, draw_index, out_token, out_logprob);
+  hipLaunchKernelGGL(filt_pick_kernel, dim3(n_rows), dim3(PICK_THREADS), 0, stream, logits, ld, V, params, rows, any_late, h, parts,
+                     kept, lists, seeds, draw_index, out_token, out_logprob);
   HAL_LAUNCH_CHECK();
   return 0;
 }

@@ -635,7 +635,7 @@ def sample(
     ``all_greedy`` promises that no row samples (``temperature`` 0 or ``top_k`` 1 in
     every row), ``unfiltered`` that every row is greedy or draws from its whole
     distribution (no top-k, top-p or min-p): the rows are then spread over many blocks,
-    in two launches.  ``spread``: every pass over a row is shared by 32 blocks (six
+    in two launches.  ``spread``: every pass over a row is shared by 32 blocks (four
     launches; two more unless ``late`` is false, which promises that no row has top-k,
     top-p and min-p all at once).  All three go through ``sample_packed``, which is what the engine's sampler calls.
     Otherwise a row is one block's, which selects by the bits of its keys (what the others are compared
@@ -695,7 +695,7 @@ def _sample_row_words(flags: int, vocab: int) -> int:
 
 def sample_packed(logits: torch.Tensor, packed: torch.Tensor, flags: int):
     """Next token and log-probability of every row of float32 ``logits`` by ``packed``, the buffer of ``pack_sample_rows`` on the
-    GPU, and its ``flags``: greedy rows and draws from whole distributions in two launches, others in six or eight."""
+    GPU, and its ``flags``: greedy rows and draws from whole distributions in two launches, others in four or six."""
     lib = library.core_library()
     _dev(logits, packed)
     n, vocab = logits.shape
