@@ -41,7 +41,8 @@
 #include <algorithm>
 
 #define SP_SCALE 65536.f  // 2^-149, float32's smallest number, is bf16's smallest, 2^-133, then
-#define SP_BN 128
+#define SP_BN 128  // columns of a tile
+#define SP_BN_LOW 96  // of 256 rows, where fewer end earlier
 #define SP_BK 32  // k of a stage: a row's 128-byte line
 #define SP_THREADS 512
 #define SP_XCDS 8     // dies of the gfx950 parts that this library is built for (a wrong count costs cache hits only)
@@ -80,18 +81,18 @@ struct SplitArgs {
 };
 
 // WALKS: for parts of more than SP_WALK stages.
-template <int BM, bool WALKS>
+template <int BM, int BN, bool WALKS>
 __global__ void __launch_bounds__(SP_THREADS, BM == 64 ? 4 : 2)
 gemm_f32_split_kernel(SplitArgs g) {
-  constexpr int WM = BM / 64, WN = 8 / WM, NI = 4, NJ = SP_BN / 16 / WN;  // WM x WN waves of NI x NJ results of 16 x 16
+  constexpr int WM = BM / 64, WN = 8 / WM, NI = 4, NJ = BN / 16 / WN;  // WM x WN waves of NI x NJ results of 16 x 16
   constexpr int AL = BM / 64, LOADS = AL + 2;                             // a wave's loads a stage, eight rows each
   constexpr int A_PLANE = BM * 64, W_PLANE = SP_BN * 64, W_AT = 3 * A_PLANE, BYTES = 3 * (A_PLANE + W_PLANE);
   __shared__ __attribute__((aligned(16))) char lds[2 * BYTES];
   const int lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int n_tiles = g.tiles_m * g.tiles_n * g.parts, die = blockIdx.x % SP_XCDS, rest = n_tiles % SP_XCDS;
   const int id = die * (n_tiles / SP_XCDS) + min(die, rest) + blockIdx.x / SP_XCDS;
-  const int m0 = (id % g.tiles_m) * BM, n0 = (id / g.tiles_m % g.tiles_n) * SP_BN, part = id / g.tiles_m / g.tiles_n;
-  const int rows_here = min(BM, g.M - m0), cols_here = min(SP_BN, g.N - n0);
+  const int m0 = (id % g.tiles_m) * BM, n0 = (id / g.tiles_m % g.tiles_n) * BN, part = id / g.tiles_m / g.tiles_n;
+  const int rows_here = min(BM, g.M - m0), cols_here = min(BN, g.N - n0);
   const int all = (g.K + SP_BK - 1) / SP_BK, part_first = (int)((long long)all * part / g.parts);
   const int part_stages = (int)((long long)all * (part + 1) / g.parts) - part_first, walks = WALKS ? (part_stages + SP_WALK - 1) / SP_WALK : 1;
   const uint32_t a_bytes = ((uint32_t)(rows_here - 1) * g.lda + g.K) * 4, w_bytes = ((uint32_t)(cols_here - 1) * g.ldw + g.K) * 4;
@@ -304,13 +305,37 @@ extern "C" long long hal_gemm_f32_split_planes(int M, int N) {
   return sp_parts(N) == 1 ? 0 : (long long)sp_parts(N) * sp_rows_at_once(M, N) * sp_pitch(N);
 }
 
+// How tiles of 256 rows go over the compute units: all of SP_BN columns, all of SP_BN_LOW, or SP_BN for whole rounds and SP_BN_LOW behind them (`first` columns
+// are the former's; K in one part), and what that costs beside rounds of SP_BN.
+struct SplitCut {
+  int first;
+  double rounds;
+};
+// (500 rows x 6,144 x 4,096 in parts, all lower: 153 -> 140 us; x 28,672 x 4,096, one round and a lower one for 448 tiles: 584 -> 574, less than the quarter of a round
+// that it spares, as the chip holds a higher clock with a quarter of its units idle; 200 rows x 20,608 x 4,096 268 -> 239, 400 x 32,000 x 4,096 610 -> 596.)
+#define SP_LOW_ROUND 0.79
+static SplitCut sp_cut(int M, int N, int parts) {
+  const long long rows = (M + 255) / 256;
+  auto tiles = [&](int n, int cols) { return rows * ((n + cols - 1) / cols) * parts; };
+  auto rounds = [&](long long n) { return (double)((n + SP_UNITS - 1) / SP_UNITS); };
+  SplitCut best = {N, rounds(tiles(N, SP_BN))};
+  if (SP_LOW_ROUND * rounds(tiles(N, SP_BN_LOW)) < best.rounds) best = {0, SP_LOW_ROUND * rounds(tiles(N, SP_BN_LOW))};
+  const long long whole = tiles(N, SP_BN) / SP_UNITS, cols = whole * SP_UNITS / rows;
+  if (parts == 1 && whole > 0 && cols > 0 && cols * SP_BN < N) {
+    const double then = (double)(cols * rows + SP_UNITS - 1) / SP_UNITS;  // (a few units may stay without a tile)
+    const double cost = (double)(long long)then + SP_LOW_ROUND * rounds(tiles(N - (int)cols * SP_BN, SP_BN_LOW)) + 0.02;
+    if (cost < best.rounds) best = {(int)cols * SP_BN, cost};
+  }
+  return best;
+}
+
 // The rows of a tile: those whose rounds over the compute units are expected to end first, in microseconds a round of 128 stages (500 rows x 28,672 x
 // 4,096 in tiles of 64 / 128 / 256: 743 / 730 / 629; 200 rows 396 / 356 / 304; 128 rows 207 / 195 / 304; 128 x 16,384 x 3,072 91 / 136 / 201;
 // 128, 256 and 500 x 4,096 x 4,096 40 / 54 / 82, 68 / 63 / 89, 126 / 118 / 104).  A result's bits do not depend on it.
 static int sp_tile_rows(int M, int N) {
   const long long n = (long long)((N + SP_BN - 1) / SP_BN) * sp_parts(N);
   auto cost = [&](int rows, int round) { return round * (((M + rows - 1) / rows * n + SP_UNITS - 1) / SP_UNITS); };
-  const long long low = cost(64, 100), middle = cost(128, 175), high = cost(256, 300);
+  const double low = (double)cost(64, 100), middle = (double)cost(128, 175), high = 300 * sp_cut(M, N, sp_parts(N)).rounds;
   return high <= middle && high <= low ? 256 : middle <= low ? 128 : 64;
 }
 
@@ -321,22 +346,30 @@ extern "C" int hal_gemm_f32_split(const float* A, int lda, const float* W, int l
   HAL_REQUIRE((uintptr_t)C % 4 == 0 && (uintptr_t)planes % 16 == 0, "hal_gemm_f32_split: addresses");
   const int parts = sp_parts(N), rows = parts == 1 ? M : sp_rows_at_once(M, N), pitch = sp_pitch(N);
   HAL_REQUIRE(parts == 1 || planes != nullptr, "hal_gemm_f32_split: no planes for %d parts", parts);
-  const int tiles_n = (N + SP_BN - 1) / SP_BN;
   const bool walks = ((K + SP_BK - 1) / SP_BK + parts - 1) / parts > SP_WALK;  // (parts differ by one stage at most)
   for (int m = 0; m < M; m += rows) {
     const int here = std::min(rows, M - m), tile = sp_tile_rows(here, N), tiles_m = (here + tile - 1) / tile;
-    const long long blocks = (long long)tiles_m * tiles_n * parts, plane = (long long)here * pitch;
-    HAL_REQUIRE(blocks < (1ll << 31), "hal_gemm_f32_split: M=%d N=%d exceed the grid limit", M, N);
+    const long long plane = (long long)here * pitch;
     float* to = C + (size_t)m * ldc;
-    const SplitArgs g = {A + (size_t)m * lda, W, parts > 1 ? planes : to, lda, ldw, parts > 1 ? pitch : ldc, here, N, K, tiles_m, tiles_n, parts, plane};
-#define SP_LAUNCH(BM_)                                                                                                               \
-  do {                                                                                                                               \
-    if (walks) hipLaunchKernelGGL((gemm_f32_split_kernel<BM_, true>), dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);         \
-    else hipLaunchKernelGGL((gemm_f32_split_kernel<BM_, false>), dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);              \
+    const int first = tile == 256 ? sp_cut(here, N, parts).first : N;
+#define SP_LAUNCH(BM_, BN_)                                                                                                               \
+  do {                                                                                                                                    \
+    if (walks) hipLaunchKernelGGL((gemm_f32_split_kernel<BM_, BN_, true>), dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);         \
+    else hipLaunchKernelGGL((gemm_f32_split_kernel<BM_, BN_, false>), dim3((unsigned)blocks), dim3(SP_THREADS), 0, stream, g);              \
   } while (0)
-    if (tile == 256) SP_LAUNCH(256);
-    else if (tile == 64) SP_LAUNCH(64);
-    else SP_LAUNCH(128);
+    for (int low = 0; low < 2; ++low) {  // the columns of the wider tiles, and those behind them
+      const int n0 = low ? first : 0, cols = low ? N - first : first, per = low ? SP_BN_LOW : SP_BN;
+      if (cols <= 0) continue;
+      const int tiles = (cols + per - 1) / per;
+      const long long blocks = (long long)tiles_m * tiles * parts;
+      HAL_REQUIRE(blocks < (1ll << 31), "hal_gemm_f32_split: M=%d N=%d exceed the grid limit", M, N);
+      const SplitArgs g = {A + (size_t)m * lda, W + (size_t)n0 * ldw, (parts > 1 ? planes : to) + n0, lda, ldw, parts > 1 ? pitch : ldc, here, cols, K,
+                           tiles_m, tiles, parts, plane};
+      if (low) SP_LAUNCH(256, SP_BN_LOW);
+      else if (tile == 256) SP_LAUNCH(256, SP_BN);
+      else if (tile == 64) SP_LAUNCH(64, SP_BN);
+      else SP_LAUNCH(128, SP_BN);
+    }
 #undef SP_LAUNCH
     if (parts > 1)
       hipLaunchKernelGGL(gemm_f32_planes_kernel, dim3((unsigned)((plane / 4 + 255) / 256)), dim3(256), 0, stream, planes, plane, pitch, to, ldc, N, parts);
