@@ -41,6 +41,14 @@ __device__ __forceinline__ bf16x8 load_frag(const bf16_t* p, bool valid) {
   return __builtin_bit_cast(bf16x8, raw);
 }
 
+// the same for weights in the kernel's own order, of which a wave reads whole lines and nobody reads them again (see HAL_ONCE)
+template <bool ONCE>
+__device__ __forceinline__ bf16x8 load_weight(const bf16_t* p, bool valid) {
+  u32x4 raw = {0u, 0u, 0u, 0u};
+  if (valid) raw = ONCE ? __builtin_nontemporal_load((const u32x4*)p) : *(const u32x4*)p;
+  return __builtin_bit_cast(bf16x8, raw);
+}
+
 enum { SK_OUT_BF16 = 0, SK_OUT_F32 = 1, SK_OUT_F32_ADD = 2, SK_OUT_BF16_RELU_SQUARED = 3 };
 
 // What the rotating epilogue needs beside the product.  Row r' = head * D + 16 * j + c of
@@ -75,7 +83,7 @@ struct NormFusion {
   bf16_t* xw_out;
   float* ss_out;
 };
-enum { SK_ROPE = 1, SK_SCALED = 2, SK_PREP = 4 };
+enum { SK_ROPE = 1, SK_SCALED = 2, SK_PREP = 4, SK_TILED = 8 };  // (the first three are for tiled weights alone)
 #define SK_MAX_PART_LOADS 4  // float4 loads of partial sums per thread that are asked for ahead
 
 // PL: float4 loads of partial sums per thread (SCALED), held in registers through the loop
@@ -187,8 +195,8 @@ __global__ void skinny_gemm_kernel(const bf16_t* __restrict__ X, int ldx,
       const size_t kw = (size_t)(step + u) * kstride;
 #pragma unroll
       for (int f = 0; f < NT; ++f) {
-        a[u][f] = load_frag(wrow[f] + kw, kv);
-        if (GATED) a2[u][f] = load_frag(w2row[f] + kw, kv);
+        a[u][f] = load_weight<FLAGS != 0>(wrow[f] + kw, kv);
+        if (GATED) a2[u][f] = load_weight<FLAGS != 0>(w2row[f] + kw, kv);
       }
 #pragma unroll
       for (int t = 0; t < MT; ++t) b[u][t] = load_frag(xrow[t] + k, kv && xvalid[t]);
@@ -394,6 +402,9 @@ static int launch_skinny(const bf16_t* X, int ldx, const bf16_t* W, const bf16_t
                          hipStream_t stream, RopeEpilogue rope = RopeEpilogue{},
                          NormFusion nf = NormFusion{}, hal_gate act = hal_gate{}) {
   constexpr int SETS = GATED ? 2 : 1;
+  if constexpr (FLAGS == 0) {
+    if (ldw == 0) return launch_skinny<NT, MT, GATED, U, SK_TILED, PL>(X, ldx, W, W2, ldw, C, ldc, out_mode, M, N, K, waves, stream, rope, nf, act);
+  }
   HAL_REQUIRE((FLAGS & SK_PREP) == 0 || waves >= 4,
               "small-batch product: the norm-preparing epilogue takes at least four waves (%d)", waves);
   // LDS for the partial sums of all waves, or of a half, a quarter ... if that is too much

@@ -79,7 +79,7 @@ gemm_stream_kernel(StreamArgs a) {
 #pragma unroll
     for (int i = 0; i < AI; ++i) hal_load_lds(X, past ? x_bytes : xo[i] + at, 0, lds + (i * 4 + wave) * 1024);
 #pragma unroll
-    for (int i = 0; i < WI; ++i) hal_load_lds(W, past ? w_bytes : wo[i] + at, 0, lds + A_BYTES + (i * 4 + wave) * 1024);
+    for (int i = 0; i < WI; ++i) hal_load_lds<HAL_ONCE>(W, past ? w_bytes : wo[i] + at, 0, lds + A_BYTES + (i * 4 + wave) * 1024);
   };
   const int q = lane / 16, r16 = lane % 16;
   const int get[2] = {r16 * 128 + (q ^ hal_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ hal_turn(r16)) * 16};
