@@ -540,7 +540,8 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
 // against 67.6, but 8,000 rows 131 / 121.
 #define GT_ONE_STEP_ROWS 4096
 typedef __attribute__((ext_vector_type(4), aligned(4))) float gt_f32x4_any;  // (a gate's rows begin at any float)
-template <bool GATED, bool HEADS, int NI>
+// ONCE: experts of so few rows that their weights are read once.
+template <bool GATED, bool HEADS, bool ONCE, int NI>
 __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1,
                                         char* b2) {
   constexpr int AI = NI / 2, LOADS = AI + 4;
@@ -574,7 +575,7 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
 #pragma unroll
     for (int i = 0; i < AI; ++i) hal_load_lds(X, xo[i], at, lds + (i * 4 + wave) * 1024);
 #pragma unroll
-    for (int i = 0; i < 4; ++i) hal_load_lds(W, wo[i], at, lds + GT_A_BYTES + (i * 4 + wave) * 1024);
+    for (int i = 0; i < 4; ++i) hal_load_lds<ONCE ? HAL_ONCE : 0>(W, wo[i], at, lds + GT_A_BYTES + (i * 4 + wave) * 1024);
   };
   const int q = lane / 16, r16 = lane % 16;
   const int get[2] = {r16 * 128 + (q ^ hal_turn(r16)) * 16, r16 * 128 + ((q + 4) ^ hal_turn(r16)) * 16};
@@ -640,7 +641,7 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
   }
 }
 
-template <bool GATED, bool HEADS>
+template <bool GATED, bool HEADS, bool ONCE>
 __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GT_BUFFER], b1[GT_BUFFER], b2[GT_BUFFER];
   __shared__ __attribute__((aligned(64))) int found[5];
@@ -663,8 +664,8 @@ __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, i
   const int n0 = col * (GATED ? GT_COLS / 2 : GT_COLS);
   const int rows = row_end - row0;
   if (rows <= 0) return;
-  if (rows <= 32) gt_wave<GATED, HEADS, 2>(a, g, row0, row_end, n0, b0, b1, b2);
-  else gt_wave<GATED, HEADS, 4>(a, g, row0, row_end, n0, b0, b1, b2);
+  if (rows <= 32) gt_wave<GATED, HEADS, ONCE, 2>(a, g, row0, row_end, n0, b0, b1, b2);
+  else gt_wave<GATED, HEADS, ONCE, 4>(a, g, row0, row_end, n0, b0, b1, b2);
 }
 
 // bf16, few rows a group (decode steps): a workgroup takes 64 rows of W (GATED: 32 of the
@@ -861,8 +862,14 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   if (kernel == GG_STREAM) {
     const long long units = gw_most_tiles(M, G, GT_ROWS) * stream_cols, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
-    else hipLaunchKernelGGL((grouped_stream_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+#define GT_LAUNCH(ONCE_)                                                                                                                        \
+  do {                                                                                                                                          \
+    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false, ONCE_>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);        \
+    else hipLaunchKernelGGL((grouped_stream_kernel<false, false, ONCE_>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);          \
+  } while (0)
+    if (a.turn) GT_LAUNCH(true);
+    else GT_LAUNCH(false);
+#undef GT_LAUNCH
   } else if (kernel == GG_WIDE) {
     const long long most = gw_most_tiles(M, G, GW_LEAST_ROWS) * wide_cols, units = std::min(most, std::max(gw_most_tiles(M, G, GW_ROWS) * wide_cols, (long long)GG_UNITS));
     const long long blocks = 8 * ((units + 7) / 8);
@@ -872,7 +879,7 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   } else if (heads && K % GW_TK == 0 && rows_per_group > 16 && (K > GW_TK || M <= GT_ONE_STEP_ROWS)) {
     const long long units = (long long)((M + GT_ROWS - 1) / GT_ROWS) * G * stream_cols, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31) && (long long)M * stream_cols < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    hipLaunchKernelGGL((grouped_stream_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+    hipLaunchKernelGGL((grouped_stream_kernel<false, true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
   } else if (dtype == HAL_BF16 && allow_mfma && aligned && kernel == GG_FEW_ROWS) {
     grid.x = W2 ? (N + 31) / 32 : (N + 63) / 64;
     if (W2) hipLaunchKernelGGL(grouped_skinny_kernel<true>, grid, dim3(256), 0, stream, a);
