@@ -756,10 +756,11 @@ static long long gw_most_tiles(int M, int G, int rows) {
 // groups have rows as M random picks meet).  Fewer of them than half of the compute units: 4 rows of 16
 // groups of 4096 x 4096 (116 tiles) 26.9 us against 26.3 of the kernel for few rows, whose workgroups are
 // smaller; 4096 x 8192, 2 of 8 groups (60) 42.5 / 36.4; 2048 x 512, 4 of 32 (61) 7.3 / 6.5, but 4608 x 4096,
-// 4 of 16 (131) 36.4 / 45.8.  Or the second or third round of two tiles a unit just begun, with less than a
-// row a group (the others are bound by the reads of all weights): 80 rows of 512 groups of 512 x 2048, gate
-// and up (1.16 rounds) 62.7 / 57.7, 64 of 128 of 768 x 2048 (1.18) 64.1 / 61.7, 48 of 64 of 4096 x 1024 (2.1)
-// 64.3 / 61.8; with a row or more in a group 1.02 to 0.57 of the other's time at any fraction of a round
+// 4 of 16 (131) 36.4 / 45.8.  (These before the streaming tiles' weights passed the caches by; since then 4 rows of 16 groups of 4096 x 4096 34.6 streaming / 25.1,
+// 12 of 64 of 1024 x 4096, gate and up (176 tiles), 36.1 / 45.8, 24 of 64 65.8 / 74.5, 8 of 16 of 4096 x 4096 (206) 39.5 / 49.3, in single calls.)  Or, of rows of up to 2,048, the second
+// round of two tiles a unit just begun, with less than a row a group (the others are bound by the reads of all weights): there the two are nearly alike (80 rows of 512 groups of
+// 512 x 2048, gate and up, 1.16 rounds, 63.0 / 64.3; 64 of 128 of 768 x 2048, 1.18, 64.1 / 69.9), of longer rows they are not (48 of 64 of 1024 x 4096, gate and up, 1.06 rounds, 109.6 /
+// 121.3; a third round, 48 of 64 of 4096 x 1024, 2.1, 56.7 / 58.4; 90 of 64, 3.0, 70.4 / 77.5).  With a row or more in a group 1.02 to 0.57 of the other's time at any fraction of a round
 // (4608 x 4096, 16 groups, 1.12 rounds: 48 rows 122 / 124, 256 rows 124 / 192).
 //
 // From 48 rows a group on the wide tiles, one a unit, where they fill the chip: below five eighths of a
@@ -789,7 +790,7 @@ static int gg_experts_kernel(int M, int N, int K, int G, bool gated) {
   const int stream_cols = (n_of + GT_COLS - 1) / GT_COLS, wide_cols = (n_of + GW_COLS - 1) / GW_COLS;
   if (M / G <= 16) {
     const double tiles = G * (1.0 - pow(1.0 - 1.0 / G, (double)M)) * stream_cols, rounds = tiles / (2 * GG_UNITS);
-    const bool begun = M < G && rounds > 1.0 && rounds < 3.0 && rounds - floor(rounds) < 0.2;
+    const bool begun = M < G && K <= 2048 && rounds > 1.0 && rounds < 1.2;
     return stream && tiles >= GG_UNITS / 2 && !begun ? GG_STREAM : GG_FEW_ROWS;
   }
   if (stream && M / G < GT_ROWS_A_GROUP) return GG_STREAM;
