@@ -96,7 +96,7 @@ __device__ __forceinline__ void wg_store(const WideArgs& a, const wg_place& p, i
 
 // Tiles of at most 32 * NI rows: `tile` and every `apart`-th after it below `end`, the next one's first pieces on their way while one's results are stored;
 // or, of one tile, a half of 32 * NI rows (0 or 1; -1: all of it).
-template <bool GATED, int NI>
+template <bool GATED, int NI, bool ONCE>
 __device__ __forceinline__ void wg_tiles(const WideArgs& a, const wt_lds& lds, int wave, int tile, int apart, int end, int half) {
   using P = wt_part<NI>;
   int lane = threadIdx.x % 64;
@@ -137,7 +137,7 @@ __device__ __forceinline__ void wg_tiles(const WideArgs& a, const wt_lds& lds, i
     const hal_memory W = hal_memory_at(half_of_w ? (over ? next.w2 : here.w2) : over ? next.w : here.w, over ? next.w_bytes : here.w_bytes);
     const uint32_t at = (uint32_t)(over ? step - steps : step) * (WT_TK * 2);
 #pragma unroll
-    for (int u = 0; u < 2; ++u) hal_load_lds(W, wo + (GATED ? u * 64 : u * 128 + half_of_w * 32) * row, at, to + (wave + 8 * u) * 1024);
+    for (int u = 0; u < 2; ++u) hal_load_lds<ONCE ? HAL_ONCE : 0>(W, wo + (GATED ? u * 64 : u * 128 + half_of_w * 32) * row, at, to + (wave + 8 * u) * 1024);
   };
   wt_begin<NI>(lds, bring_x, bring_w);
   for (;;) {
@@ -156,17 +156,18 @@ __device__ __forceinline__ void wg_tiles(const WideArgs& a, const wt_lds& lds, i
 
 // A die takes an eighth of the tiles, neighbours in an order that goes through WG_PANEL row tiles column by column, so that its 32
 // workgroups read few different rows.  Its last round, if at most half of its units have a tile in it, is of tiles of half the height.
-template <bool GATED, int NI>
+// ONCE: one row tile, so that W is read once and passes the caches by.
+template <bool GATED, int NI, bool ONCE>
 __global__ void __launch_bounds__(512, 2) gemm_wide_kernel(WideArgs a) {
   WT_LDS(lds);
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   const int tiles = a.row_tiles * a.col_tiles, die = blockIdx.x % WG_DIES, at = blockIdx.x / WG_DIES, apart = gridDim.x / WG_DIES;
   const int first = (int)((long long)tiles * die / WG_DIES), mine = (int)((long long)tiles * (die + 1) / WG_DIES) - first;
   const int rest = mine % WG_UNITS, whole = rest <= WG_UNITS / 2 ? mine - rest : mine;
-  if (at < whole) wg_tiles<GATED, NI>(a, lds, wave, first + at, apart, first + whole, -1);
+  if (at < whole) wg_tiles<GATED, NI, ONCE>(a, lds, wave, first + at, apart, first + whole, -1);
   if (at < 2 * (mine - whole)) {
     __syncthreads();
-    wg_tiles<GATED, (NI + 1) / 2>(a, lds, wave, first + whole + at / 2, 0, 0, at % 2);
+    wg_tiles<GATED, (NI + 1) / 2, false>(a, lds, wave, first + whole + at / 2, 0, 0, at % 2);
   }
 }
 
@@ -235,11 +236,14 @@ extern "C" int hal_gemm_bf16_wide(const void* X, int ldx, const void* W, const v
   // workgroups of a die: one a unit, or of fewer tiles one each, or two where they are cut in two
   const long long each = (tiles + WG_DIES - 1) / WG_DIES;
   const int blocks = each > WG_UNITS / 2 ? WG_UNITS : 2 * (int)each;
-#define WG_LAUNCH(NI_)                                                                                                                \
-  case NI_:                                                                                                                           \
-    if (gated) hipLaunchKernelGGL((gemm_wide_kernel<true, NI_>), dim3(WG_DIES * blocks), dim3(512), 0, stream, a);                     \
-    else hipLaunchKernelGGL((gemm_wide_kernel<false, NI_>), dim3(WG_DIES * blocks), dim3(512), 0, stream, a);                          \
+#define WG_LAUNCH(NI_)                                                                                                                         \
+  case NI_:                                                                                                                                    \
+    if (gated && once) hipLaunchKernelGGL((gemm_wide_kernel<true, NI_, true>), dim3(WG_DIES * blocks), dim3(512), 0, stream, a);                \
+    else if (gated) hipLaunchKernelGGL((gemm_wide_kernel<true, NI_, false>), dim3(WG_DIES * blocks), dim3(512), 0, stream, a);                  \
+    else if (once) hipLaunchKernelGGL((gemm_wide_kernel<false, NI_, true>), dim3(WG_DIES * blocks), dim3(512), 0, stream, a);                   \
+    else hipLaunchKernelGGL((gemm_wide_kernel<false, NI_, false>), dim3(WG_DIES * blocks), dim3(512), 0, stream, a);                            \
     break
+  const bool once = row_tiles == 1;
   switch (ni) {
     WG_LAUNCH(4);
     WG_LAUNCH(5);

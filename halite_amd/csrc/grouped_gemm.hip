@@ -313,6 +313,8 @@ __global__ void __launch_bounds__(256, 2) grouped_mfma_kernel(GroupedArgs a) {
 // Measured beside a schedule in which every wave read, loaded and multiplied for itself with one barrier a step, us: 9,000 rows of 16 experts, 4096 x 4096 302 ->
 // 280 (1,080 TFLOP/s; tiles of 128 x 128 in registers and LDS 469); 18,000 rows of 64, gate and up 1024 x 4096 each, 330 -> 320; 49,152 rows 730 -> 698;
 // 2,400 rows of 8, gate and up 14336 x 4096, 554 -> 551; 3,600 rows of 64 249 -> 234; 16 groups of 60, 128, 210, 280 and 340 rows 133 -> 129, 137 -> 135, 155 -> 150, 167 -> 159, 181 -> 170.
+// The weights of a group with one row tile, which are read once, pass the caches by (with two or three row tiles side by side 2 to 3% slower): 16 groups of 60, 210, 280 and 340 rows
+// 129 -> 120, 150 -> 133, 159 -> 136, 170 -> 147; 18,000 rows of 64, gate and up 320 -> 305, down 227 -> 219; 2,400 of 8 551 -> 530.
 #define GW_ROWS 352
 #define GW_COLS 256
 #define GW_TK 64
@@ -351,8 +353,8 @@ __device__ __forceinline__ int gw_lane() {
   return __builtin_amdgcn_mbcnt_hi(~0u, __builtin_amdgcn_mbcnt_lo(~0u, zero));
 }
 
-// What one wave does for a tile of at most 32 * NI rows.
-template <bool GATED, int NI>
+// What one wave does for a tile of at most 32 * NI rows.  ONCE: the group has one row tile, so that its weights are read once.
+template <bool GATED, int NI, bool ONCE>
 __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int wave, int g, int row0, int row_end, int n0, const wt_lds& lds) {
   using P = wt_part<NI>;
   const int lane = gw_lane(), oct = lane / 8, c = ((lane % 8) ^ hal_turn(wave % 2 * 8 + oct)) * 16;
@@ -383,7 +385,7 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int wave, int g, i
   auto bring_w = [&](int half, char* to, int step) {
 #pragma unroll
     for (int u = 0; u < 2; ++u)
-      hal_load_lds(half ? W2 : W, wo + (GATED ? u * 64 : u * 128 + half * 32) * row, (uint32_t)min(step, last) * (GW_TK * 2), to + (wave + 8 * u) * 1024);
+      hal_load_lds<ONCE ? HAL_ONCE : 0>(half ? W2 : W, wo + (GATED ? u * 64 : u * 128 + half * 32) * row, (uint32_t)min(step, last) * (GW_TK * 2), to + (wave + 8 * u) * 1024);
   };
   gg_f32x4 acc[NI][4];
   wt_begin<NI>(lds, bring_x, bring_w);
@@ -404,7 +406,7 @@ __device__ __forceinline__ void gw_wave(const GroupedArgs& a, int wave, int g, i
 }
 
 // Which tile is a workgroup's `turn`-th, written to `found` (group, first row, end row, column tile, whether
-// there is one more after it; group -1: none),
+// there is one more after it, whether the group has no other row tile; group -1: none),
 // by its first wave: the groups' rows in tiles of at most `most`, equally high in steps of 32.  A lane counts a
 // run of neighbouring groups (one where there are up to 64), so that one sum over the wave serves any number:
 // 64 at a time, 512 groups of 512 x 2048 (gate and up) took 27.9 us for 3 tokens of 10 and 69.0 for 8, now 23.4 and 62.7.
@@ -439,6 +441,7 @@ __device__ __forceinline__ void gw_find(const GroupedArgs& a, int most, int col_
       found[1] = begin + (panel * GW_PANEL + in_panel % high) * rows;
       found[2] = min(end, found[1] + rows);
       found[3] = in_panel / high;
+      found[5] = n == 1;
       return;
     }
     before += n;
@@ -487,7 +490,7 @@ __device__ __forceinline__ int gw_height(const GroupedArgs& a, int col_tiles) {
 template <bool GATED>
 __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int col_tiles) {
   WT_LDS(lds);
-  __shared__ __attribute__((aligned(64))) int found[5];
+  __shared__ __attribute__((aligned(64))) int found[6];
   __shared__ int most;
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64);
   if (wave == 0) most = gw_height(a, col_tiles);
@@ -500,9 +503,13 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
     if (g < 0) return;
     const int row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
     const int n0 = __builtin_amdgcn_readfirstlane(found[3]) * (GATED ? GW_COLS / 2 : GW_COLS);
-    const int rows = row_end - row0;
+    const int rows = row_end - row0, once = __builtin_amdgcn_readfirstlane(found[5]);
     // (equal heights in steps of 32 can leave a group's last tile empty)
-#define GW_WAVE(NI_) gw_wave<GATED, NI_>(a, wave, g, row0, row_end, n0, lds)
+#define GW_WAVE(NI_)                                                             \
+  do {                                                                           \
+    if (once) gw_wave<GATED, NI_, true>(a, wave, g, row0, row_end, n0, lds);      \
+    else gw_wave<GATED, NI_, false>(a, wave, g, row0, row_end, n0, lds);          \
+  } while (0)
     if (rows <= 0);
     else if (rows <= 64) GW_WAVE(2);
     else if (rows <= 128) GW_WAVE(4);
@@ -644,7 +651,7 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
 template <bool GATED, bool HEADS, bool ONCE>
 __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GT_BUFFER], b1[GT_BUFFER], b2[GT_BUFFER];
-  __shared__ __attribute__((aligned(64))) int found[5];
+  __shared__ __attribute__((aligned(64))) int found[6];
   int g, row0, row_end, col;
   if (HEADS) {
     // a die takes neighbouring heads, a head's columns beside each other: they read the same rows
