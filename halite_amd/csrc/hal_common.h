@@ -89,6 +89,12 @@ __device__ __forceinline__ void load4(const bf16_t* p, float (&v)[4]) {
   v[0] = __uint_as_float(t.x << 16); v[1] = __uint_as_float(t.x & 0xffff0000u);
   v[2] = __uint_as_float(t.y << 16); v[3] = __uint_as_float(t.y & 0xffff0000u);
 }
+// the same of what is read once and by nobody else: the caches pass it on
+__device__ __forceinline__ void load4_once(const float* p, float (&v)[4]) {
+  typedef __attribute__((ext_vector_type(4))) float f4;
+  const f4 t = __builtin_nontemporal_load((const f4*)p);
+  v[0] = t[0]; v[1] = t[1]; v[2] = t[2]; v[3] = t[3];
+}
 __device__ __forceinline__ void store4(float* p, const float (&v)[4]) {
   *(float4*)p = make_float4(v[0], v[1], v[2], v[3]);
 }

@@ -164,8 +164,8 @@ __global__ void __launch_bounds__(1024) norm_added_vec_kernel(float* __restrict_
     if (v >= nv) continue;
     float b[4], s[4] = {0.f, 0.f, 0.f, 0.f};
     load4(h + t * d + v * 4, x[u]);
-    if (e.beside) load4(e.beside + t * d + v * 4, b);
-    if (e.extra) load4(e.extra + t * d + v * 4, s);
+    if (e.beside) load4_once(e.beside + t * d + v * 4, b);
+    if (e.extra) load4_once(e.extra + t * d + v * 4, s);
     const float* at = e.y + t * e.top * d + v * 4;
 #pragma unroll
     for (int i = 0; i < 4; ++i) s[i] *= eg;
@@ -174,7 +174,7 @@ __global__ void __launch_bounds__(1024) norm_added_vec_kernel(float* __restrict_
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
         const int which = j0 + j < e.top ? j0 + j : j0;  // (past the end: a row that is there, not added)
-        load4(at + (size_t)which * d, part[j]);
+        load4_once(at + (size_t)which * d, part[j]);
         c[j] = w[which];
       }
 #pragma unroll
