@@ -1017,11 +1017,11 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
         return gemm_bf16_skinny(x, w, out_dtype=out_dtype)
     # (the readers that ``sums`` and a norm mean round the sum of the parts: a result that is wanted in float32 comes to them whole)
     in_parts = unrounded if out_dtype == torch.float32 else sums or (next_norm is not None and next_norm.sums)
-    parts = stream_parts(x, w, w.shape[0], may_part=in_parts)
-    if parts:
+    if m > STREAM_ROWS:
+        if wide_pays(x, w, w.shape[0], out_dtype=out_dtype):
+            return gemm_bf16_wide(x, w, out_dtype=out_dtype)
+    elif parts := stream_parts(x, w, w.shape[0], may_part=in_parts):
         return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)
-    if wide_pays(x, w, w.shape[0], out_dtype=out_dtype):
-        return gemm_bf16_wide(x, w, out_dtype=out_dtype)
     if out_dtype == torch.float32:
         global _MM_OUT_DTYPE
         if _MM_OUT_DTYPE is None:
