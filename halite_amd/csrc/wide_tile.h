@@ -47,14 +47,16 @@ __device__ __forceinline__ int wt_octet_row(int octet, int p) {
 }
 
 template <int LEFT>
-__device__ __forceinline__ void wt_meet_left() {  // the newest LEFT loads may be on their way, operands from LDS too
+__device__ __forceinline__ void wt_meet_left() {  // the newest LEFT loads may be on their way, this phase's operands from LDS too
   __builtin_amdgcn_sched_barrier(0);
   asm volatile("s_waitcnt vmcnt(%0)\n\ts_barrier" ::"n"(LEFT) : "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
+// The end of a phase: all that it read of LDS is there.  (Its products have waited for most of it, but not for what the next phase multiplies,
+// and that place is asked for anew by the other group of waves before this one's next products.)
 __device__ __forceinline__ void wt_meet() {
   __builtin_amdgcn_sched_barrier(0);
-  asm volatile("s_barrier" ::: "memory");
+  asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
   __builtin_amdgcn_sched_barrier(0);
 }
 
@@ -72,8 +74,8 @@ __device__ __forceinline__ int wt_get(int lane, int k) { return lane % 16 * 128 
 // multiplies, the other reads its next operands and asks for new pieces; a barrier ends each turn, and waves 4-7 are one turn behind.
 // A step is four such phases of a wave, a part of its rows times half of its columns each, in an order in which one operand
 // stays: (x0, A) (x0, B) (x1, B) (x1, A), A being the half of W that the step before ended without, so that a half's registers are free when its
-// next piece is read.  What phase p read of LDS is asked for anew in phase p + 2 (both groups of waves have multiplied it by then), for the
-// step after next, six phases before it is read: loads have the time of five to arrive.
+// next piece is read.  What phase p read of LDS is asked for anew in phase p + 2 (both groups of waves have ended phase p by then, with which its
+// reads have come, see wt_meet), for the step after next, six phases before it is read: loads have the time of five to arrive.
 // WT_SLIM blocks and more leave no registers for a part of X: there a phase is a part of the rows times all columns over 32 of the 64 k.
 #define WT_SLIM 10  // from so many blocks on
 template <int NI, typename BringX, typename BringW>
