@@ -70,9 +70,10 @@ typedef __attribute__((ext_vector_type(4))) uint32_t u32x4;
 __device__ __forceinline__ bf16x8 ld16(const bf16_t* p) {
   return __builtin_bit_cast(bf16x8, *(const u32x4*)p);
 }
-// What the pages' layout is to a kernel: the matrix cores' own order, and then whether a step reads a key once (no more heads share it than a tile has rows):
-// then the caches pass it on.  (8 requests of 8,192 keys, a step of eight layers 1,349 -> 1,309 us, 64 of 1,100 1,524 -> 1,461; eight latent ones, whose 32 heads are two
-// tiles, 1,090 -> 1,114.)
+// What the pages' layout is to a kernel: the matrix cores' own order, and then whether a step reads a key once (every segment is one tile, which the
+// plan says): then the caches pass it on.  (8 requests of 8,192 keys, a step of eight layers 1,349 -> 1,309 us, 64 of 1,100 1,524 -> 1,461; eight latent ones, whose 32 heads are two
+// tiles, 1,090 -> 1,114; in one-tile items of prompts every tile reads all keys before it: 16 heads of one latent, 800 tokens 45.8 -> 49.1, 8 requests beside a
+// prompt of 300 25.2 -> 36.4; 8 heads of 256 dimensions, 4,000 tokens 198 -> 264.)
 enum { ROWS = 0, TILED_SHARED = 1, TILED_ONCE = 2 };
 __device__ __forceinline__ bf16x8 ld16_once(const bf16_t* p) {
   return __builtin_bit_cast(bf16x8, __builtin_nontemporal_load((const u32x4*)p));
@@ -1265,7 +1266,7 @@ extern "C" int hal_attention_mfma(const void* q, int q_row_stride, void* out, in
                                   max_big, merges, max_merges, counts, seg_q_start, seg_q_len,
                                   seg_kv_len, block_table, bt_stride, k_pages, v_pages, part_o, part_ml,
                                   counters, n_counters, H, K, head_dim, page_size, tiled, scale, window,
-                                  0, nullptr, 0, 0, 0.f, nullptr, 0, 0, merge_parts, stream);
+                                  0, nullptr, 0, 0, 0.f, nullptr, 0, 0, 0, merge_parts, stream);
 }
 
 // The same with a rule for the scores.  `keep` (with a window): the first keys that stay visible;
@@ -1273,7 +1274,8 @@ extern "C" int hal_attention_mfma(const void* q, int q_row_stride, void* out, in
 // tile's first key is no earlier than the start of its first row's chunk).  `bias_log2`:
 // float32 [H][bias_len], the bias by distance times log2 e.  `value_from`: the values' dimensions
 // before it are zeros on every page (they need not be read; the result's are zeros; with kept keys
-// they are read, and the work lists are made for a value_from of 0: no layer has both).
+// they are read, and the work lists are made for a value_from of 0: no layer has both).  `keys_once`: every
+// segment of `items` has one tile of 16 rows, so that a key is read once (0 if that is not known; results do not depend on it).
 extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out_row_stride,
                                         const int* items, int max_items, const int* big_items,
                                         int max_big, const int* merges, int max_merges,
@@ -1285,7 +1287,7 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
                                         int page_size, int tiled, float scale, int window, int chunk,
                                         const float* bias_log2, int bias_len, int sink,
                                         float softcap, const float* sink_log2, int keep,
-                                        int value_from, int merge_parts, hipStream_t stream) {
+                                        int value_from, int keys_once, int merge_parts, hipStream_t stream) {
   HAL_REQUIRE(keep >= 0 && (keep == 0 || (window > 0 && chunk == 0)),
               "hal_attention_mfma: %d kept keys belong to a window alone (window %d, chunk %d)", keep, window, chunk);
   HAL_REQUIRE(chunk >= 0 && (bias_log2 == nullptr || bias_len > 0),
@@ -1316,11 +1318,10 @@ extern "C" int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* o
   if ((page_size & (page_size - 1)) == 0)
     for (page_shift = 0; (1 << page_shift) < page_size; ++page_shift) {}
   const int waves = WAVES;
-  const bool once = H / K <= 16;
 #define PICK_ATTENTION(RT_, SHARED_, KB_, HV_, RU_, KE_, VT_)                                       \
   {                                                                                               \
     kernel = attention_mfma_kernel<RT_, false, false, SHARED_, ROWS, KB_, HV_, RU_, KE_, VT_>;    \
-    if (tiled && once) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, D % 32 ? ROWS : SHARED_ ? TILED_SHARED : TILED_ONCE, KB_, HV_, RU_, KE_, VT_>; \
+    if (tiled && keys_once) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, D % 32 ? ROWS : SHARED_ ? TILED_SHARED : TILED_ONCE, KB_, HV_, RU_, KE_, VT_>; \
     else if (tiled) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, D % 32 ? ROWS : TILED_SHARED, KB_, HV_, RU_, KE_, VT_>; \
     else if (page_shift >= 5) kernel = attention_mfma_kernel<RT_, true, true, SHARED_, ROWS, KB_, HV_, RU_, KE_, VT_>; \
     else if (page_shift >= 0) kernel = attention_mfma_kernel<RT_, true, false, SHARED_, ROWS, KB_, HV_, RU_, KE_, VT_>; \

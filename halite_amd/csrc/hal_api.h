@@ -519,7 +519,7 @@ int hal_attention_mfma(const void* q, int q_row_stride, void* out, int out_row_s
 
 // hal_attention_mfma with a rule for the scores (see hal_attention_simple_ruled); the bias
 // table and the sinks' values come multiplied by log2 e, and the work lists are cut for the chunk.
-// The values' dimensions before value_from are zeros on every page.
+// The values' dimensions before value_from are zeros on every page.  keys_once: every segment of the one-tile items has one tile.
 int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out_row_stride,
                              const int* items, int max_items, const int* big_items, int max_big,
                              const int* merges, int max_merges, const int* counts,
@@ -529,6 +529,6 @@ int hal_attention_mfma_ruled(const void* q, int q_row_stride, void* out, int out
                              int n_counters, int H, int K, int head_dim, int page_size, int tiled,
                              float scale, int window, int chunk, const float* bias_log2,
                              int bias_len, int sink, float softcap, const float* sink_log2,
-                             int keep, int value_from, int merge_parts, hipStream_t stream);
+                             int keep, int value_from, int keys_once, int merge_parts, hipStream_t stream);
 
 }  // extern "C"

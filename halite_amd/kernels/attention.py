@@ -121,6 +121,9 @@ class AttentionPlan:
     max_parts: int = 0
     # some one-tile items ask the kernel to merge their tile's pieces itself (it needs counters)
     merged_in_kernel: bool = False
+    # every segment of the one-tile items has one tile: the kernel reads a key once, and the caches pass it on (of a step of one token a
+    # request this hangs on the heads alone, so that launches recorded for one such step serve the others)
+    keys_once: bool = False
 
     def __post_init__(self):
         if len(self.items) and int(self.items[:, 9].max()) > 1:
@@ -455,7 +458,7 @@ def plan_items(seg_q_len, seg_kv_len, group_size: int, n_kv_heads: int, window: 
         chunk = max(MIN_SPLIT_KEYS, -(-chunk // KEYS_PER_BLOCK) * KEYS_PER_BLOCK)
     big_items, merges_b, slot = _cut_long(*big, chunk, per_item, slot, seg_scalars, more, keep)
     merges = np.concatenate((merges_s, merges_b)) if len(merges_s) or len(merges_b) else np.zeros((0, 8), np.int32)
-    return AttentionPlan(items, big_items, merges, slot, rows_big)
+    return AttentionPlan(items, big_items, merges, slot, rows_big, keys_once=not bool((small[0][1:] == small[0][:-1]).any()))
 
 
 _COUNTERS: dict = {}
@@ -518,7 +521,7 @@ def attention_mfma(q, q_row_stride, plan_dev, ctx, group, kv, n_heads, scale, wi
         P(counters), N_COUNTERS, n_heads, n_kv, head_dim, page_size, 1 if getattr(kv, "tiled", False) else 0,
         ctypes.c_float(scale), window, rule.chunk, P(bias), 0 if bias is None else bias.shape[1],
         rule.weights_code(), ctypes.c_float(rule.softcap), P(sinks), rule.keep, 0 if rule.keep else getattr(kv, "value_from", 0),
-        plan.max_parts, ops._stream(),
+        1 if plan.keys_once else 0, plan.max_parts, ops._stream(),
     )
     ops._check(lib, rc)
     return out
