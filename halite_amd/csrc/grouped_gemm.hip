@@ -533,6 +533,9 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
 // once for every 16 rows, events around the call: 48 tokens, 4 of 16 experts of 4096 x 4096 (537 MB): 143 ->
 // 106 us; 16 tokens: 113 -> 104; 64 tokens: 178 -> 107; 48 tokens, 6 of 64 experts of 1024 x 4096, gate and
 // up: 211 -> 184.  All workgroups at one place of K (see `begin`): 122 instead of 106.
+// The weights of a group with one row tile pass the caches by, those of a group with several, side by side, do not.  None / all of groups of fewer than 48
+// rows on average / by group, us: 2,500 rows, 12 of 64 groups of 150, down of 4096 x 1024 123 / 139 / 120, gate and up of 1024 x 4096 220 / 213 / 210; 500
+// rows of 16 groups of 4096 x 4096, one of 300, 113 / 108 / 105; 900 rows of those, evenly, 111 / 111 / 101; 384 rows of 64, evenly, 182 / 161 / 162.
 #define GT_ROWS 64
 #define GT_ROWS_A_GROUP 48  // the streaming tiles are for fewer rows a group, on average
 #define GT_COLS 128
@@ -547,7 +550,7 @@ __global__ void __launch_bounds__(512, 2) grouped_wide_kernel(GroupedArgs a, int
 // against 67.6, but 8,000 rows 131 / 121.
 #define GT_ONE_STEP_ROWS 4096
 typedef __attribute__((ext_vector_type(4), aligned(4))) float gt_f32x4_any;  // (a gate's rows begin at any float)
-// ONCE: experts of so few rows that their weights are read once.
+// ONCE: the group has one row tile, so that its weights are read once.
 template <bool GATED, bool HEADS, bool ONCE, int NI>
 __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, int row_end, int n0, char* b0, char* b1,
                                         char* b2) {
@@ -648,11 +651,11 @@ __device__ __forceinline__ void gt_wave(const GroupedArgs& a, int g, int row0, i
   }
 }
 
-template <bool GATED, bool HEADS, bool ONCE>
+template <bool GATED, bool HEADS>
 __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, int col_tiles) {
   __shared__ __attribute__((aligned(16))) char b0[GT_BUFFER], b1[GT_BUFFER], b2[GT_BUFFER];
   __shared__ __attribute__((aligned(64))) int found[6];
-  int g, row0, row_end, col;
+  int g, row0, row_end, col, once = 0;
   if (HEADS) {
     // a die takes neighbouring heads, a head's columns beside each other: they read the same rows
     const int in_group = (a.M + GT_ROWS - 1) / GT_ROWS * col_tiles, die = blockIdx.x % 8;
@@ -666,13 +669,19 @@ __global__ void __launch_bounds__(256, 2) grouped_stream_kernel(GroupedArgs a, i
     g = __builtin_amdgcn_readfirstlane(found[0]);
     if (g < 0) return;
     row0 = __builtin_amdgcn_readfirstlane(found[1]), row_end = __builtin_amdgcn_readfirstlane(found[2]);
-    col = __builtin_amdgcn_readfirstlane(found[3]);
+    col = __builtin_amdgcn_readfirstlane(found[3]), once = __builtin_amdgcn_readfirstlane(found[5]);
   }
   const int n0 = col * (GATED ? GT_COLS / 2 : GT_COLS);
   const int rows = row_end - row0;
   if (rows <= 0) return;
-  if (rows <= 32) gt_wave<GATED, HEADS, ONCE, 2>(a, g, row0, row_end, n0, b0, b1, b2);
-  else gt_wave<GATED, HEADS, ONCE, 4>(a, g, row0, row_end, n0, b0, b1, b2);
+#define GT_WAVE(NI_)                                                                       \
+  do {                                                                                     \
+    if (!HEADS && once) gt_wave<GATED, HEADS, !HEADS, NI_>(a, g, row0, row_end, n0, b0, b1, b2); \
+    else gt_wave<GATED, HEADS, false, NI_>(a, g, row0, row_end, n0, b0, b1, b2);            \
+  } while (0)
+  if (rows <= 32) GT_WAVE(2);
+  else GT_WAVE(4);
+#undef GT_WAVE
 }
 
 // bf16, few rows a group (decode steps): a workgroup takes 64 rows of W (GATED: 32 of the
@@ -870,14 +879,8 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   if (kernel == GG_STREAM) {
     const long long units = gw_most_tiles(M, G, GT_ROWS) * stream_cols, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-#define GT_LAUNCH(ONCE_)                                                                                                                        \
-  do {                                                                                                                                          \
-    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false, ONCE_>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);        \
-    else hipLaunchKernelGGL((grouped_stream_kernel<false, false, ONCE_>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);          \
-  } while (0)
-    if (a.turn) GT_LAUNCH(true);
-    else GT_LAUNCH(false);
-#undef GT_LAUNCH
+    if (W2) hipLaunchKernelGGL((grouped_stream_kernel<true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+    else hipLaunchKernelGGL((grouped_stream_kernel<false, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
   } else if (kernel == GG_WIDE) {
     const long long most = gw_most_tiles(M, G, GW_LEAST_ROWS) * wide_cols, units = std::min(most, std::max(gw_most_tiles(M, G, GW_ROWS) * wide_cols, (long long)GG_UNITS));
     const long long blocks = 8 * ((units + 7) / 8);
@@ -887,7 +890,7 @@ extern "C" int hal_grouped_gemm(const void* X, int ldx, int x_group_cols, int x_
   } else if (heads && K % GW_TK == 0 && rows_per_group > 16 && (K > GW_TK || M <= GT_ONE_STEP_ROWS)) {
     const long long units = (long long)((M + GT_ROWS - 1) / GT_ROWS) * G * stream_cols, blocks = 8 * ((units + 7) / 8);
     HAL_REQUIRE(blocks < (1ll << 31) && (long long)M * stream_cols < (1ll << 31), "hal_grouped_gemm: %lld workgroups", blocks);
-    hipLaunchKernelGGL((grouped_stream_kernel<false, true, false>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
+    hipLaunchKernelGGL((grouped_stream_kernel<false, true>), dim3((unsigned)blocks), dim3(256), 0, stream, a, stream_cols);
   } else if (dtype == HAL_BF16 && allow_mfma && aligned && kernel == GG_FEW_ROWS) {
     grid.x = W2 ? (N + 31) / 32 : (N + 63) / 64;
     if (W2) hipLaunchKernelGGL(grouped_skinny_kernel<true>, grid, dim3(256), 0, stream, a);

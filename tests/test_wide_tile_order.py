@@ -2,37 +2,11 @@
 before the phase's last barrier.  The other group of waves asks for that place anew behind it, without a wait of its own for these reads."""
 
 import re
-import subprocess
 from concurrent.futures import ThreadPoolExecutor
 
-import pytest
-
-from halite_amd.kernels import library
+import assembly
 
 KERNELS = {"gemm_wide.hip": "gemm_wide_kernel", "grouped_gemm.hip": "grouped_wide_kernel"}
-
-
-@pytest.fixture(scope="module")
-def bodies(tmp_path_factory):
-    """Name and lines of every kernel that goes by wide tiles."""
-    folder = tmp_path_factory.mktemp("assembly")
-
-    def instructions(source):
-        out = folder / (source + ".s")
-        subprocess.run([library._hipcc(), *library.HIPCC_FLAGS, "--offload-device-only", "-S", "-I", library.CSRC,
-                        f"{library.CSRC}/{source}", "-o", str(out)], check=True, capture_output=True)
-        found, lines = {}, None
-        for line in out.read_text().splitlines():
-            if m := re.match(r"(_Z\w+):", line):
-                lines = found.setdefault(m[1], []) if KERNELS[source] in m[1] else None
-            elif line.startswith("\t.section"):
-                lines = None
-            elif lines is not None:
-                lines.append(line.split(";")[0].strip())
-        return found
-
-    with ThreadPoolExecutor() as pool:
-        return {name: lines for found in pool.map(instructions, KERNELS) for name, lines in found.items()}
 
 
 def late(lines):
@@ -50,7 +24,9 @@ def late(lines):
     return found
 
 
-def test_a_phase_has_its_operands_before_it_ends(bodies):
+def test_a_phase_has_its_operands_before_it_ends():
+    with ThreadPoolExecutor() as pool:
+        bodies = {name: lines for source, found in zip(KERNELS, pool.map(assembly.kernels, KERNELS)) for name, lines in found.items() if KERNELS[source] in name}
     assert len(bodies) == 34  # eight heights, plain and gated, read once or not; two of the experts'
     for name, lines in bodies.items():
         assert sum(line.startswith("s_barrier") for line in lines) >= 16 and sum(line.startswith("v_mfma") for line in lines) >= 64, name
