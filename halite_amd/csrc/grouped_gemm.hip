@@ -773,10 +773,12 @@ static long long gw_most_tiles(int M, int G, int rows) {
 // groups of 4096 x 4096 (116 tiles) 26.9 us against 26.3 of the kernel for few rows, whose workgroups are
 // smaller; 4096 x 8192, 2 of 8 groups (60) 42.5 / 36.4; 2048 x 512, 4 of 32 (61) 7.3 / 6.5, but 4608 x 4096,
 // 4 of 16 (131) 36.4 / 45.8.  (These before the streaming tiles' weights passed the caches by; since then 4 rows of 16 groups of 4096 x 4096 34.6 streaming / 25.1,
-// 12 of 64 of 1024 x 4096, gate and up (176 tiles), 36.1 / 45.8, 24 of 64 65.8 / 74.5, 8 of 16 of 4096 x 4096 (206) 39.5 / 49.3, in single calls.)  Or, of rows of up to 2,048, the second
-// round of two tiles a unit just begun, with less than a row a group (the others are bound by the reads of all weights): there the two are nearly alike (80 rows of 512 groups of
-// 512 x 2048, gate and up, 1.16 rounds, 63.0 / 64.3; 64 of 128 of 768 x 2048, 1.18, 64.1 / 69.9), of longer rows they are not (48 of 64 of 1024 x 4096, gate and up, 1.06 rounds, 109.6 /
-// 121.3; a third round, 48 of 64 of 4096 x 1024, 2.1, 56.7 / 58.4; 90 of 64, 3.0, 70.4 / 77.5).  With a row or more in a group 1.02 to 0.57 of the other's time at any fraction of a round
+// 12 of 64 of 1024 x 4096, gate and up (176 tiles), 36.1 / 45.8, 24 of 64 65.8 / 74.5, 8 of 16 of 4096 x 4096 (206) 39.5 / 49.3, in single calls.)  Or, of rows of up to 1,024, the second
+// round of two tiles a unit just begun, with less than a row a group (the others are bound by the reads of all weights).  Streaming / few rows, us, at 1.06, 1.12, 1.19 and 1.25
+// rounds: 64 groups of 4096 x 1024 33.6 / 30.5, 34.4 / 30.9, 36.3 / 32.6, 36.7 / 35.7; 256 of 2048 x 768 at 1.03 to 1.19 27.2 / 24.1, 27.9 / 25.3, 28.8 / 24.7; 64 of 2048 x 512 20.4 / 19.1,
+// 21.8 / 19.6, 22.3 / 20.0; 64 of 1024 x 1024, gate and up, 33.2 / 33.2, 34.1 / 34.0, 36.0 / 34.7; before the round, at 0.97 to 1.0, 25.3 / 28.5, 20.3 / 21.1, 14.8 / 17.5 and 25.3 / 29.7.  Of longer rows the streaming
+// tiles are the faster ones there too: 256 of 512 x 1536, gate and up, 46.4 / 51.5 to 48.2 / 53.7; 512 of 512 x 2048 60.5 / 61.6 to 64.0 / 65.0, 128 of 768 x 2048 58.8 / 61.9 to 63.1 / 65.0; 48 rows of 64 of
+// 1024 x 4096, 1.06 rounds, 109.6 / 121.3.  (A third round: 48 of 64 of 4096 x 1024, 2.1, 56.7 / 58.4; 90 of 64, 3.0, 70.4 / 77.5.)  With a row or more in a group 1.02 to 0.57 of the other's time at any fraction of a round
 // (4608 x 4096, 16 groups, 1.12 rounds: 48 rows 122 / 124, 256 rows 124 / 192).
 //
 // From 48 rows a group on the wide tiles, one a unit, where they fill the chip: below five eighths of a
@@ -806,7 +808,7 @@ static int gg_experts_kernel(int M, int N, int K, int G, bool gated) {
   const int stream_cols = (n_of + GT_COLS - 1) / GT_COLS, wide_cols = (n_of + GW_COLS - 1) / GW_COLS;
   if (M / G <= 16) {
     const double tiles = G * (1.0 - pow(1.0 - 1.0 / G, (double)M)) * stream_cols, rounds = tiles / (2 * GG_UNITS);
-    const bool begun = M < G && K <= 2048 && rounds > 1.0 && rounds < 1.2;
+    const bool begun = M < G && K <= 1024 && rounds > 1.0 && rounds < 1.2;
     return stream && tiles >= GG_UNITS / 2 && !begun ? GG_STREAM : GG_FEW_ROWS;
   }
   if (stream && M / G < GT_ROWS_A_GROUP) return GG_STREAM;

@@ -64,7 +64,9 @@ def test_which_kernel():
     # 48 tokens, 4 of 16 experts; half of the chip's units have a tile, or fewer; a begun round with less than a row a group, and more
     assert kernel_of(192, 4096, 4096, 16) == STREAM
     assert kernel_of(4, 4096, 4096, 16) == FEW and kernel_of(4, 4608, 4096, 16) == STREAM
-    assert kernel_of(64, 768, 2048, 128, True) == FEW and kernel_of(256, 4608, 4096, 16) == STREAM
+    assert kernel_of(40, 2048, 768, 256) == FEW and kernel_of(256, 4608, 4096, 16) == STREAM
+    # that round over longer rows
+    assert kernel_of(64, 768, 2048, 128, True) == STREAM and kernel_of(80, 512, 2048, 512, True) == STREAM and kernel_of(72, 512, 1536, 512, True) == STREAM
     # K of part of a line; many rows a group
     assert kernel_of(192, 4096, 4104, 16) == FEW and kernel_of(600, 4096, 4104, 16) == TILES
     # prompts: the wide tiles fill the chip or not, a round that has just begun, a long K
