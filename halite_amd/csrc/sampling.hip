@@ -381,7 +381,8 @@ __device__ __forceinline__ int part_share(int V) { return ((V + ROW_PARTS - 1) /
 // top-p: a pass over the rows 10.6 -> 10.1 us, the first one, which keeps its batch, 20.9 -> 15.1 us, a
 // histogram 19.4 -> 12.7 us on average (where it also leaves out what the row does not search by).  Places of the
 // batch that lie past the share are passed over by all threads at once: worked through by none of them, 200 rows
-// of 1,000 logits without filters took 23.0 us, of 32,000 29.9, and take 16.5 and 23.4 so.
+// of 1,000 logits without filters took 23.0 us, of 32,000 29.9, and take 16.5 and 23.4 so.  (Asking and working as two functions
+// schedules better than as one: a call of 64 rows with top-p 59.8 us / 60.7.)
 #define PART_BATCH 16
 template <bool WHOLE>
 __device__ __forceinline__ void ask_batch(const float* x, int from, int end, float (&v)[PART_BATCH]) {
@@ -408,17 +409,6 @@ __device__ __forceinline__ void for_part(const float* x, int begin, int end, F&&
     if (from + (PART_BATCH - 1) * PART_THREADS < end) ask_batch<true>(x, from, end, v), use_batch<true>(v, from, end, each);
     else ask_batch<false>(x, from, end, v), use_batch<false>(v, from, end, each);
   }
-}
-// The same in two: the first batch of a share asked for before what its work needs is there, and then worked on with the others.
-__device__ __forceinline__ void ask_part(const float* x, int begin, int end, float (&v)[PART_BATCH]) {
-  if (begin + (PART_BATCH - 1) * PART_THREADS < end) ask_batch<true>(x, begin, end, v);
-  else ask_batch<false>(x, begin, end, v);
-}
-template <typename F>
-__device__ __forceinline__ void use_part(const float (&v)[PART_BATCH], const float* x, int begin, int end, F&& each) {
-  if (begin + (PART_BATCH - 1) * PART_THREADS < end) use_batch<true>(v, begin, end, each);
-  else use_batch<false>(v, begin, end, each);
-  for_part(x, begin + PART_BATCH * PART_THREADS, end, each);
 }
 
 // a row is greedy if it has no temperature array (all rows greedy), a temperature of 0 or top_k 1
