@@ -221,16 +221,17 @@ extern "C" int hal_gemm_bf16_wide_pays(int M, int N, int K, int gated, int f32) 
   return !exact && part >= (K <= 2048 ? 0.15 : 0.5);
 }
 
-static bool wg_takes(const void* X, int ldx, const void* W, const void* W2, int ldw, int M, int N, int K) {
+// Whether there is a form for these sizes and distances of rows; operands begin at multiples of 16 bytes besides.
+extern "C" int hal_gemm_bf16_wide_takes(int M, int N, int K, int ldx, int ldw) {
   return M > 0 && N >= 4 && N % 4 == 0 && K >= 2 * WT_TK && K % (2 * WT_TK) == 0 && ldx >= K && ldw >= K && ldx % 8 == 0 && ldw % 8 == 0 && ldx < (1 << 21) &&
-         ldw < (1 << 21) && (uintptr_t)X % 16 == 0 && (uintptr_t)W % 16 == 0 && (uintptr_t)W2 % 16 == 0;
+         ldw < (1 << 21);
 }
 
 // X [M, K], W (and W2 of a gated product: W is the gate's) [N, K] bf16, Y [M, N] of bf16 or float32.  height: blocks of 16 rows of a wave (0: as
 // it is best), for tests and measurements.
 extern "C" int hal_gemm_bf16_wide(const void* X, int ldx, const void* W, const void* W2, int ldw, void* Y, int ldy, int y_dtype, int act, float limit,
                                   float alpha, float up_shift, int M, int N, int K, int height, hipStream_t stream) {
-  HAL_REQUIRE(wg_takes(X, ldx, W, W2, ldw, M, N, K), "hal_gemm_bf16_wide: M=%d N=%d K=%d, rows of %d and %d, or their places", M, N, K, ldx, ldw);
+  HAL_REQUIRE(hal_gemm_bf16_wide_takes(M, N, K, ldx, ldw) && ((uintptr_t)X | (uintptr_t)W | (uintptr_t)W2) % 16 == 0, "hal_gemm_bf16_wide: M=%d N=%d K=%d, rows of %d and %d, or their places", M, N, K, ldx, ldw);
   HAL_REQUIRE(ldy >= N && ldy % 4 == 0 && (uintptr_t)Y % 16 == 0, "hal_gemm_bf16_wide: results' rows of %d, or their place", ldy);
   HAL_REQUIRE(y_dtype == HAL_F32 || y_dtype == HAL_BF16, "hal_gemm_bf16_wide: result dtype %d", y_dtype);
   HAL_REQUIRE(act >= HAL_ACT_SILU && act <= HAL_ACT_CLAMPED, "hal_gemm_bf16_wide: activation %d", act);

@@ -166,7 +166,9 @@ int hal_gemm_bf16_stream(const void* X, int ldx, const void* W, const void* W2, 
                          int parts, int act, float limit, float alpha, float up_shift, int M, int N, int K,
                          hipStream_t stream);
 // ---- products of prompts in wide tiles (gemm_wide.hip) ------------------------------------------
-// The same result in one piece, for any number of rows; hal_gemm_bf16_wide_pays: whether it is the faster one.  height: 4 to 11 blocks of 32 rows a tile, 0 as it is best.
+// The same result in one piece, for any number of rows; hal_gemm_bf16_wide_takes: whether it has these sizes and distances of rows (operands begin at multiples of 16
+// bytes besides), hal_gemm_bf16_wide_pays: whether it is the faster one.  height: 4 to 11 blocks of 32 rows a tile, 0 as it is best.
+int hal_gemm_bf16_wide_takes(int M, int N, int K, int ldx, int ldw);
 int hal_gemm_bf16_wide_pays(int M, int N, int K, int gated, int f32);
 int hal_gemm_bf16_wide(const void* X, int ldx, const void* W, const void* W2, int ldw, void* Y, int ldy, int y_dtype, int act, float limit,
                        float alpha, float up_shift, int M, int N, int K, int height, hipStream_t stream);

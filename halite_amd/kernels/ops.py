@@ -849,21 +849,23 @@ def gemm_bf16_stream(x: torch.Tensor, w: torch.Tensor, parts: int, w_up: torch.T
 
 @functools.lru_cache(maxsize=8192)
 def _wide_pays(m: int, n: int, k: int, gated: bool, f32: bool) -> bool:
-    lib = library.core_library()
-    return n % 4 == 0 and k % 128 == 0 and bool(lib.hal_gemm_bf16_wide_pays(m, n, k, 1 if gated else 0, 1 if f32 else 0))
+    return bool(library.core_library().hal_gemm_bf16_wide_pays(m, n, k, 1 if gated else 0, 1 if f32 else 0))
+
+
+@functools.lru_cache(maxsize=8192)
+def _wide_takes(m: int, n: int, k: int, x_strides: tuple, w_strides: tuple) -> bool:
+    (ldx, one), (ldw, one_w) = x_strides, w_strides
+    return one == 1 and one_w == 1 and max(ldx, ldw) < 2**31 and bool(library.core_library().hal_gemm_bf16_wide_takes(m, n, k, ldx, ldw))
 
 
 def wide_pays(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, out_dtype: torch.dtype = torch.bfloat16) -> bool:
     """Whether the product of ``x`` [more than 64, k] against the bf16 weight ``w`` of ``n`` rows (``gated``: two of them) in wide tiles is
     the faster one, and has a form for these sizes and places."""
     m, k = x.shape
-    if not (m > STREAM_ROWS and x.is_cuda and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
-            and _wide_pays(m, n, k, gated, out_dtype == torch.float32)):
-        return False
-    (ldx, one), (ldw, one_w) = x.stride(), w.stride()
-    # (as the kernel's entry point checks; the second weight of a gated product begins n rows on)
-    return (one == 1 and one_w == 1 and ldx >= k and ldw >= k and ldx % 8 == 0 and ldw % 8 == 0 and ldx < 2**21 and ldw < 2**21
-            and x.data_ptr() % 16 == 0 and w.data_ptr() % 16 == 0)
+    # (the second weight of a gated product begins n rows on, whose distance is a multiple of 16 bytes)
+    return (m > STREAM_ROWS and x.is_cuda and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
+            and _wide_pays(m, n, k, gated, out_dtype == torch.float32) and _wide_takes(m, n, k, x.stride(), w.stride())
+            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
 
 
 def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, w_up: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
