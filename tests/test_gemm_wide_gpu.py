@@ -1,11 +1,14 @@
 """The product of prompts in wide tiles against products in 64 bits: every height, edges of tiles in rows and columns, last rounds of
 halved tiles, workgroups with several tiles, the shortest K, rows that lie apart, and the gates."""
 
+from types import SimpleNamespace
+
 import pytest
 import torch
 from test_grouped_wide_gpu import compare, rand
 
 from halite_amd.kernels import library, ops
+from halite_amd.parts.feedforward import GatedFeedForward
 
 pytestmark = pytest.mark.gpu
 
@@ -79,7 +82,7 @@ def test_a_row_does_not_depend_on_its_neighbours(gpu):
 
 
 def test_what_linear_takes(gpu):
-    """Where the rule says so, ``linear`` and the gated form go to the wide tiles; sizes and places that they do not have stay where they were."""
+    """Where the rule says so, ``linear`` goes to the wide tiles; sizes and places that they do not have stay where they were."""
     lib = library.core_library()
     assert lib.hal_gemm_bf16_wide_pays(2048, 4096, 4096, 0, 0) and lib.hal_gemm_bf16_wide_pays(2048, 14336, 4096, 1, 0)
     assert not lib.hal_gemm_bf16_wide_pays(8192, 4096, 4096, 0, 0) and not lib.hal_gemm_bf16_wide_pays(64, 14336, 4096, 1, 0)
@@ -91,4 +94,23 @@ def test_what_linear_takes(gpu):
             assert not ops.wide_pays(a, b, 2048)
         for dtype in (torch.bfloat16, torch.float32):
             y, xs, ws = ops.linear(a, b, out_dtype=dtype), a.double(), b.double()
+            assert not ops.wide_pays(a, b, 2048, out_dtype=dtype) or torch.equal(y, ops.gemm_bf16_wide(a, b, out_dtype=dtype))
             compare(y, xs @ ws.T, (b.shape[1], xs.abs() @ ws.abs().T), 2.0**-8 if dtype == torch.bfloat16 else 0.0)
+
+
+@pytest.mark.parametrize("f, wide", [(2048, True), (2056, False)])
+def test_what_the_gated_form_takes(gpu, monkeypatch, f, wide):
+    """The feed-forward's gated product goes to the wide tiles where the rule says so, and to the product and its gate's kernel where it does not."""
+    x, both, down = rand(2048, 512, seed=1), rand(2 * f, 512, seed=2, scale=0.1), rand(512, f, seed=3, scale=0.1)
+    x, both, down = (t.bfloat16().to(gpu) for t in (x, both, down))
+    took, real = [], ops.gemm_bf16_wide
+    monkeypatch.setattr(ops, "gemm_bf16_wide", lambda *a, **k: took.append("w_up" in k) or real(*a, **k))
+    if not wide:
+        monkeypatch.setattr(ops, "_wide_pays", lambda *a: False)
+    part = SimpleNamespace(p=SimpleNamespace(intermediate_size=f, float32_result=False), w_gate_up=both, w_out=down, t_gate=None, t_out=None)
+    y = GatedFeedForward.forward(part, x, None)
+    assert (True in took) == wide
+    act = torch.nn.functional.silu(x.double() @ both[:f].double().T) * (x.double() @ both[f:].double().T)
+    # act is rounded once or (in two kernels) three times to 8 bits, its error and the result's rounding
+    limit = 4 * 2.0**-8 * (act.abs() @ down.double().abs().T)
+    assert bool(((y.double() - act @ down.double().T).abs() <= limit).all())
