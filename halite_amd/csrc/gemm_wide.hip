@@ -6,8 +6,8 @@
 //  - one workgroup a compute unit goes through tiles, and the next tile's first two steps are on their way while one ends and its
 //    results are stored: with a workgroup a tile the same product took 1,372 us, now 1,261 (2,048 rows 367 -> 331);
 //  - the height of the tiles is chosen for the matrix, and a last round of half the units or fewer is of tiles of half the height;
-//  - the gate costs some fifteen instructions and two of the transcendental unit a number, 2.6 us a tile more than those two with nothing that makes up for
-//    their argument's rounding (8,192 rows x 28,672 x 4,096 1,346 us / 1,310), whose error grows with the gate; expf and a division: 6 us a tile;
+//  - the gate costs ten instructions and two of the transcendental unit a number, 1 us a tile more than those two with nothing that makes up for
+//    their argument's rounding (8,192 rows x 28,672 x 4,096 1,292 us / 1,278), whose error grows with the gate; expf and a division: 6 us a tile;
 //  - W's rows lie in LDS in such an order that bf16 results leave 16 bytes a lane.
 #include "wide_tile.h"
 #include "hal_api.h"
@@ -45,15 +45,15 @@ __device__ __forceinline__ wg_place wg_place_of(const WideArgs& a, int tile) {
   return p;
 }
 
-// sigmoid(z), to some 2^-22 of it (below 2^-126: 0): x = exp(-|z|) as a power of two whose argument's rounding is brought in behind it, and 1 or x over
-// 1 + x, a number from 1 to 2, by its reciprocal with a step of Newton's.
+// sigmoid(z), to some 2^-22 of it: 1 over 1 + exp(-z) by the reciprocal and a step of Newton's, and the exponential as a power of two behind which
+// is brought in what its argument's rounding lost.  (z is held where the power is finite: from there on down its reciprocal is 0, and up 1.)
 __device__ __forceinline__ float wg_sigmoid(float z) {
-  constexpr double LOG2_E = 1.4426950408889634;
-  constexpr float HIGH = (float)LOG2_E, LOW = (float)(LOG2_E - (double)HIGH), LN_2 = 0.6931471805599453f;
-  const float a = fminf(fabsf(z), 128.0f), t = a * -HIGH;
-  const float rest = fmaf(a, -LOW, fmaf(a, -HIGH, -t)), power = __builtin_amdgcn_exp2f(t);
-  const float x = fmaf(power * rest, LN_2, power), d = 1.0f + x, y = __builtin_amdgcn_rcpf(d);
-  return (z < 0.0f ? x : 1.0f) * fmaf(fmaf(-d, y, 1.0f), y, y);
+  constexpr double LN_2 = 0.6931471805599453;
+  constexpr float LOG2_E = 1.4426950408889634f, HIGH = (float)LN_2, LOW = (float)(LN_2 - (double)HIGH);
+  const float b = __builtin_amdgcn_fmed3f(z, -88.5f, 88.5f), t = b * -LOG2_E;
+  const float rest = fmaf(t, -LOW, fmaf(t, -HIGH, -b)), power = __builtin_amdgcn_exp2f(t);
+  const float d = 1.0f + fmaf(power, rest, power), y = __builtin_amdgcn_rcpf(d);
+  return fmaf(fmaf(-d, y, 1.0f), y, y);
 }
 __device__ __forceinline__ float wg_gated(const hal_gate& a, float g, float u) {
   float z = g;
@@ -211,7 +211,7 @@ static WideCut wg_cut(int M, int N, bool gated) {
 // 142.0 / 114.7; over a short K it is the slower one all the same (500 x 6,144 x 1,536 22.5 / 18.4, 500 x 4,096 x 2,048 21.4 / 20.8, 500 x 2,048 x 2,048
 // 20.7 / 19.9).  bf16 results whose tiles of 256 x 256 fill two rounds and more to the last unit are its best: 8,192 x 4,096 x 4,096 182.6 / 186.2,
 // x 14,336 598 / 626, but 8,192 x 5,120 x 3,072 (2.5 rounds) 290 / 183, 8,192 x 3,072 x 8,192 (1.5) 301 / 278.  Float32 results cost it more: 2,250 x 20,608 x 4,096
-// 368 / 296, 3,000 x 6,144 x 1,536 72 / 55, 8,192 x 6,144 x 4,096 309 / 282.  Gated, beside the kernel that multiplies (before the gate's 2.6 us a tile): 2,048 x 28,672 x 4,096 340 + 36 / 331,
+// 368 / 296, 3,000 x 6,144 x 1,536 72 / 55, 8,192 x 6,144 x 4,096 309 / 282.  Gated, beside the kernel that multiplies (before the gate's last us a tile): 2,048 x 28,672 x 4,096 340 + 36 / 331,
 // 8,192 x 28,672 x 4,096 1,238 + 128 / 1,261, 500 x 28,672 x 4,096 95 + 12 / 96, 2,250 x 22,016 x 4,096 377 + 32 / 285.
 extern "C" int hal_gemm_bf16_wide_pays(int M, int N, int K, int gated, int f32) {
   if (M <= 64 || N < 4 || K < 2 * WT_TK) return 0;
