@@ -458,7 +458,7 @@ def plan_items(seg_q_len, seg_kv_len, group_size: int, n_kv_heads: int, window: 
         chunk = max(MIN_SPLIT_KEYS, -(-chunk // KEYS_PER_BLOCK) * KEYS_PER_BLOCK)
     big_items, merges_b, slot = _cut_long(*big, chunk, per_item, slot, seg_scalars, more, keep)
     merges = np.concatenate((merges_s, merges_b)) if len(merges_s) or len(merges_b) else np.zeros((0, 8), np.int32)
-    return AttentionPlan(items, big_items, merges, slot, rows_big, keys_once=not bool((small[0][1:] == small[0][:-1]).any()))
+    return AttentionPlan(items, big_items, merges, slot, rows_big, keys_once=not small[1].any())
 
 
 _COUNTERS: dict = {}

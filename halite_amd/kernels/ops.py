@@ -862,10 +862,13 @@ def wide_pays(x: torch.Tensor, w: torch.Tensor, n: int, gated: bool = False, out
     """Whether the product of ``x`` [more than 64, k] against the bf16 weight ``w`` of ``n`` rows (``gated``: two of them) in wide tiles is
     the faster one, and has a form for these sizes and places."""
     m, k = x.shape
+    return (m > STREAM_ROWS and x.is_cuda and _wide_pays(m, n, k, gated, out_dtype == torch.float32)
+            and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16 and _wide_fits(x, w, m, n, k))
+
+
+def _wide_fits(x: torch.Tensor, w: torch.Tensor, m: int, n: int, k: int) -> bool:
     # (the second weight of a gated product begins n rows on, whose distance is a multiple of 16 bytes)
-    return (m > STREAM_ROWS and x.is_cuda and w.dtype == torch.bfloat16 and x.dtype == torch.bfloat16
-            and _wide_pays(m, n, k, gated, out_dtype == torch.float32) and _wide_takes(m, n, k, x.stride(), w.stride())
-            and (x.data_ptr() | w.data_ptr()) % 16 == 0)
+    return _wide_takes(m, n, k, x.stride(), w.stride()) and (x.data_ptr() | w.data_ptr()) % 16 == 0
 
 
 def gemm_bf16_wide(x: torch.Tensor, w: torch.Tensor, w_up: torch.Tensor | None = None, out_dtype: torch.dtype = torch.bfloat16,
@@ -1020,7 +1023,9 @@ def linear(x: torch.Tensor, w: torch.Tensor, out_dtype: torch.dtype | None = Non
     # (the readers that ``sums`` and a norm mean round the sum of the parts: a result that is wanted in float32 comes to them whole)
     in_parts = unrounded if out_dtype == torch.float32 else sums or (next_norm is not None and next_norm.sums)
     if m > STREAM_ROWS:
-        if wide_pays(x, w, w.shape[0], out_dtype=out_dtype):
+        # (``wide_pays`` of what is known here already: a prompt of few rows through few layers waits for the host)
+        n = w.shape[0]
+        if x.is_cuda and _wide_pays(m, n, k, False, out_dtype == torch.float32) and _wide_fits(x, w, m, n, k):
             return gemm_bf16_wide(x, w, out_dtype=out_dtype)
     elif parts := stream_parts(x, w, w.shape[0], may_part=in_parts):
         return gemm_bf16_stream(x, w, parts, out_dtype=out_dtype)

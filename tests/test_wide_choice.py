@@ -36,3 +36,12 @@ def test_what_the_answer_hangs_on_is_kept_for_it():
     """Answers are kept for sizes and distances, so that a matrix of the same size with rows elsewhere has its own."""
     for x, want in ((rows(2048, 4096, 4096), True), (rows(2048, 4096, 4100), False), (rows(2048, 4096, 4104), True), (rows(2048, 4096, 4096, step=2), False)):
         assert takes(2048, 4096, 4096, x=x) == want
+
+
+def test_tensors_on_the_host_ask_no_library(monkeypatch):
+    def asked(*sizes):
+        raise AssertionError("asked for the library")
+
+    monkeypatch.setattr(ops, "_wide_pays", asked)
+    x, w = torch.randn(2048, 128).bfloat16(), torch.randn(4096, 128).bfloat16()
+    assert not ops.wide_pays(x, w, 4096) and torch.equal(ops.linear(x, w), x @ w.t())
